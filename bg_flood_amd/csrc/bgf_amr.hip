@@ -4,35 +4,43 @@
 // copy of its neighbours' edge cells: it is a restriction (2x2 mean of a finer
 // neighbour), a barycentric prolongation from a coarser neighbour, a linear
 // reconstruction from the coarse gradients, and the coarse face fluxes are the
-// means of the fine ones.  These kernels keep the reference's Model<T> layout
-// (18x18 tiles; gradients and face fluxes stored per cell) because the
-// coarse/fine exchanges read other blocks' halos and faces, which the one-level
-// kernels never store.  Per stage:
+// means of the fine ones.  Blocks keep the reference's Model<T> layout (18x18
+// tiles).  Per step:
 //
-//   k_amr_halo_refine  halo of h, u, v (src/Halo.cu:2083-4609) and the wet/dry
-//                    restriction of h (src/ConserveElevation.cu:218-378,676-726);
-//                    zs = zb + h everywhere (src/Halo.cu:72-107) is formed where
-//                    it is read, never stored; beside a coarser block the linear
-//                    prolongation of h, u, v (src/Halo.cu:1044-1405), whose
-//                    coarse theta-minmod slopes (src/Gradients.cu:921-957: of
-//                    the reference's first gradient pass only these are read)
-//                    are formed from the cells the coarse block's fill reads;
-//                    and the wet/dry prolongation (src/ConserveElevation.cu:
-//                    80-205, 451-482) of the blocks beside a block on the
-//                    coarsest level.
-//   k_amr_prolong    the wet/dry prolongation of the finer levels, one launch
-//                    per level, finest last.
-//   k_amr_grad_flux  the gradients of h, zs, u, v and their halo values
-//                    (src/Gradients.cu:2584-3294), kept in LDS, then the 17x16 X and 16x17 Y
-//                    Kurganov faces (src/Kurganov.cu:474-641, 1404-1546) with the
-//                    coarse-face source substitution, the per-cell dtmax and the
-//                    block minimum of the step.
-//   k_amr_fix_advance  after the dt reduction: coarse face flux = mean of the
-//                    fine faces (src/Halo.cu:1441-1862) and the boundary patch
-//                    (src/Boundary.cu:587-760), then the tendencies
-//                    (src/Advection.cu:160-254), the advance
-//                    (src/Advection.cu:332-385), and in the corrector bottom
-//                    friction, cleanup and implicit rain.
+//   k_amr_stage      predictor: the block's halo of h, u, v
+//                    (src/Halo.cu:2083-4609) with the wet/dry restriction of h
+//                    (src/ConserveElevation.cu:218-378,676-726), and beside a
+//                    coarser block the linear prolongation
+//                    (src/Halo.cu:1044-1405), whose coarse theta-minmod slopes
+//                    (src/Gradients.cu:921-957: of the reference's first
+//                    gradient pass only these are read) are formed from the
+//                    cells the coarse block's fill reads, and the wet/dry
+//                    prolongation (src/ConserveElevation.cu:80-205, 451-482);
+//                    then the gradients with their halo values
+//                    (src/Gradients.cu:2584-3294), the faces
+//                    (src/Kurganov.cu:474-641, 1404-1546) with the coarse-face
+//                    source substitution, and the tendencies
+//                    (src/Advection.cu:160-254), all in LDS; zs = zb + h
+//                    (src/Halo.cu:72-107) is formed where it is read.  The
+//                    block's largest wave speed goes to the dt slots.
+//   k_amr_advance    after the dt reduction, U* = U + dt/2 L(U)
+//                    (src/Advection.cu:332-385).  A block beside a finer one
+//                    takes its shared faces as the means of the finer faces
+//                    first (src/Halo.cu:1441-1862), a block on an open
+//                    boundary the boundary's (src/Boundary.cu:587-760).
+//   k_amr_stage      corrector: the same on U*, and then the advance with
+//                    bottom friction, cleanup and implicit rain, except
+//   k_amr_fix_advance  in the blocks beside finer ones, or on open boundaries,
+//                    which wait for the others' faces.
+//
+// The step used to run as halo, prolongation, gradients and fluxes, and
+// fix-up and advance, two of each, with eight face arrays between them: 103 us
+// a step on a mesh of 1,607 blocks in FP32 and 2.01 ms on 39,348 blocks in
+// FP64; with the stage in one launch and faces stored only where another
+// block reads them 66 us and 0.98 ms.
+//
+// On meshes of four levels and more the halos are filled by a launch of their
+// own (k_amr_halo_refine) and prolonged level by level (k_amr_prolong).
 //
 // Threads map to halo cells by (side, j): side 0 left, 1 right, 2 bottom,
 // 3 top, j the position along the side.  Every formula keeps the reference
@@ -45,13 +53,11 @@
 // Sequential order.  The reference visits blocks in active-list order, and in
 // the wet/dry prolongation a block's test reads the halo of its coarser
 // neighbour, which that neighbour's own prolongation may already have
-// rewritten.  Levels are processed coarsest first (the level above the
-// coarsest with the halo itself: a coarsest-level block's halo is never
-// prolonged, so there the order does not matter), and a block reads its
-// coarse neighbour's halo from the current array if that neighbour comes
-// earlier in the active list, else from the copy taken before the
-// prolongation (hsnap).  Every other stage only reads cells that the same
-// launch does not write, so blocks run in parallel.
+// rewritten: it sees the prolonged value if that neighbour comes earlier in
+// the active list.  Only a halo cell of the coarser block beside a still
+// coarser one is ever rewritten, so with three levels the chain ends there and
+// a block evaluates that cell again (end_halo).  Every other stage only reads
+// cells that the same launch does not write, so blocks run in parallel.
 
 #include <hip/hip_runtime.h>
 
@@ -78,40 +84,45 @@ template <class T> __device__ __forceinline__ int ftoi(T v) {
     return v >= T(0) ? (int)(v + T(0.5)) : (int)(v - T(0.5));
 }
 
-// Neighbours covering the first half (bottom or left, k = 0) and second half
-// (top or right, k = 1) of a side; a block is its own neighbour at the domain
-// edge.  Read from the per-block record nbr (sides in the order left, right,
-// bottom, top, first and second half each, then the same places for each
-// neighbour's level and back flag): indexed loads where a selection among the
-// eight neighbour arrays by a per-thread side would index the parameter
-// struct itself, which puts the struct in per-thread scratch memory; and the
-// neighbours' levels come with the block's own record instead of a second
-// dependent load.
-__device__ __forceinline__ int nb_at(const KParams& P, int s, int b, int k) { return P.nbr[b * NBR + 2 * s + k]; }
-__device__ __forceinline__ int nb_first(const KParams& P, int s, int b) { return nb_at(P, s, b, 0); }
-__device__ __forceinline__ int nb_second(const KParams& P, int s, int b) { return nb_at(P, s, b, 1); }
-__device__ __forceinline__ int nb_lev(const KParams& P, int s, int b, int k) {
-    return (int)(signed char)(P.nbr[b * NBR + 8 + 2 * s + k] & 0xff);
+// A side of a block: the neighbours covering its first half (bottom or left)
+// and second half (top or right), itself at the domain edge; their levels;
+// and, beside a coarser neighbour, whether the block is that neighbour's
+// first-half neighbour.  Read from the block's record nbr (sides in the order
+// left, right, bottom, top, first and second half each, then the same places
+// for the levels and flags): one record instead of a selection among the
+// eight neighbour arrays, which would index the parameter struct by a
+// per-thread side and put it in scratch memory.
+struct Side {
+    int n1, n2, l1, l2;
+    bool back;
+};
+__device__ __forceinline__ int rec_level(int info) { return (int)(signed char)(info & 0xff); }
+__device__ __forceinline__ Side make_side(int n1, int n2, int i1, int i2) {
+    return Side{n1, n2, rec_level(i1), rec_level(i2), ((i1 & REC_BACK) != 0)};
 }
-__device__ __forceinline__ int lev_first(const KParams& P, int s, int b) { return nb_lev(P, s, b, 0); }
-__device__ __forceinline__ int lev_second(const KParams& P, int s, int b) { return nb_lev(P, s, b, 1); }
-// For a coarser neighbour C on side s of block b: whether b is C's first-half
-// neighbour on the shared side (b covers that half).
-__device__ __forceinline__ bool back_first(const KParams& P, int s, int b) {
-    return (P.nbr[b * NBR + 8 + 2 * s] >> 8) & 1;
+__device__ __forceinline__ Side side_of(const KParams& P, int s, int b) {
+    const int2 n = *(const int2*)(P.nbr + b * NBR + 2 * s), i = *(const int2*)(P.nbr + b * NBR + 8 + 2 * s);
+    return make_side(n.x, n.y, i.x, i.y);
+}
+// The same where s and b are uniform over the wave, in scalar loads.
+__device__ __forceinline__ Side side_of_uniform(const KParams& P, int s, int b) {
+    const int o = b * NBR + 2 * s;
+    return make_side(ldu(P.nbr, o), ldu(P.nbr, o + 1), ldu(P.nbr, o + 8), ldu(P.nbr, o + 9));
 }
 // Neighbours of a coarser block C next to the ends of the shared side: before
 // its first cell (j == 0) and after its last (j == 15), on the half facing us;
 // lev receives their level.
 __device__ __forceinline__ int corner_lo(const KParams& P, int s, int C, int& lev) {
-    const int side = s < 2 ? SB : SL, k = (s == SL || s == SB) ? 1 : 0;
-    lev = nb_lev(P, side, C, k);
-    return nb_at(P, side, C, k);
+    const Side S = side_of(P, s < 2 ? SB : SL, C);
+    const bool second = s == SL || s == SB;
+    lev = second ? S.l2 : S.l1;
+    return second ? S.n2 : S.n1;
 }
 __device__ __forceinline__ int corner_hi(const KParams& P, int s, int C, int& lev) {
-    const int side = s < 2 ? ST : SR, k = (s == SL || s == SB) ? 1 : 0;
-    lev = nb_lev(P, side, C, k);
-    return nb_at(P, side, C, k);
+    const Side S = side_of(P, s < 2 ? ST : SR, C);
+    const bool second = s == SL || s == SB;
+    lev = second ? S.l2 : S.l1;
+    return second ? S.n2 : S.n1;
 }
 // Cell at depth d from side s of block b, at position k along the side
 // (d = -1 is the halo cell).
@@ -175,16 +186,16 @@ template <class T> __device__ __forceinline__ Gather<T> mean_fine(int os, int n,
 }
 
 // Halo value of side s, position j (src/Halo.cu:2083-2286 and its three mirrors).
-// lev: the level of block ib.
+// S: side s of block ib; lev: the level of block ib.
 template <class T>
-__device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, int s, int j, int ib, int lev) {
+__device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, const Side& S, int s, int j, int ib, int lev) {
     const int os = s ^ 1;
-    const int n1 = nb_first(P, s, ib), n2 = nb_second(P, s, ib);
+    const int n1 = S.n1, n2 = S.n2;
     if (n1 == ib) {
         if (j < BW / 2 || n2 == ib) return g_copy<T>(edge_cell(s, 0, j, ib));
         return mean_fine<T>(os, n2, (j - BW / 2) * 2);
     }
-    const int l1 = lev_first(P, s, ib);
+    const int l1 = S.l1;
     if (l1 == lev) return g_copy<T>(edge_cell(os, 0, j, n1));
     if (l1 > lev) {
         if (j < BW / 2) return mean_fine<T>(os, n1, j * 2);
@@ -193,7 +204,7 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, int s, int j,
     }
     // coarser neighbour: 1/3 own edge cell + {1/6, 1/2} of the two nearest coarse cells
     const int C = n1;
-    const bool first = back_first(P, s, ib);
+    const bool first = S.back;
     const T cj = ceil(T(j) * T(0.5));
     const int jjc = first ? ftoi(cj) : ftoi(cj + T(BW / 2));
     const bool up = cj * T(2) > T(j);
@@ -219,7 +230,7 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, int s, int j,
             }
         }
     } else if (j == BW - 1) {
-        const int C2 = nb_second(P, s, ib), l2 = lev_second(P, s, ib);
+        const int C2 = S.n2, l2 = S.l2;
         int ln;
         const int n = corner_hi(P, s, C2, ln);
         if (n == C2) {
@@ -235,7 +246,7 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, int s, int j,
     return Gather<T>{G_W3, {ii, ir, it, ii}, w1, w2, w3};
 }
 template <class T> __device__ __forceinline__ T fill_value(const KParams& P, int s, int j, int ib, const T* z) {
-    const Gather<T> g = fill_recipe<T>(P, s, j, ib, P.level[ib]);
+    const Gather<T> g = fill_recipe<T>(P, side_of(P, s, ib), s, j, ib, P.level[ib]);
     T zz[4];
     g_load(g, z, zz);
     return g_apply(g, zz);
@@ -250,10 +261,10 @@ struct WetDry {
     int i[4];
     int w;
 };
-__device__ __forceinline__ WetDry wetdry_recipe(const KParams& P, int s, int j, int ib, int lev) {
+__device__ __forceinline__ WetDry wetdry_recipe(const KParams& P, const Side& S, int s, int j, int ib, int lev) {
     WetDry r;
-    const int n = j < BW / 2 ? nb_first(P, s, ib) : nb_second(P, s, ib);
-    r.on = P.wetdryfix && lev < (j < BW / 2 ? lev_first(P, s, ib) : lev_second(P, s, ib));
+    const int n = j < BW / 2 ? S.n1 : S.n2;
+    r.on = P.wetdryfix && lev < (j < BW / 2 ? S.l1 : S.l2);
     const int jr = (j & (BW / 2 - 1)) * 2;
     const int i0 = s == SL ? BW - 2 : s == SR ? 0 : jr;
     const int j0 = s == SB ? BW - 2 : s == ST ? 0 : jr;
@@ -305,7 +316,7 @@ template <class T>
 __device__ __forceinline__ T halo_depth(const KParams& P, const T* h, const T* zb, int s, int j, int ib) {
     const int lev = P.level[ib];
     T hv = fill_value(P, s, j, ib, h);
-    const WetDry wd = wetdry_recipe(P, s, j, ib, lev);
+    const WetDry wd = wetdry_recipe(P, side_of(P, s, ib), s, j, ib, lev);
     if (wd.on) {
         T hh[4], zz[4];
 #pragma unroll
@@ -373,9 +384,9 @@ template <class T> __device__ __forceinline__ T minmod2(T theta, T s0, T s1, T s
 
 // Value two cells beyond the edge on side s, the outer point of the limited
 // gradient at the halo cell (src/Gradients.cu:2713-3294); lev: block ib's level.
-template <class T> __device__ __forceinline__ Gather<T> far_recipe(const KParams& P, int s, int j, int ib, int lev) {
+template <class T> __device__ __forceinline__ Gather<T> far_recipe(const Side& S, int s, int j, int ib, int lev) {
     const int os = s ^ 1;
-    const int n1 = nb_first(P, s, ib), n2 = nb_second(P, s, ib);
+    const int n1 = S.n1, n2 = S.n2;
     // finer neighbour: mean of its depth-2 and depth-3 cells; the left and
     // bottom sides add the depth-2 cell first, the right and top sides the depth-3 cell
     const int da = (s == SL || s == SB) ? 2 : 3, db = 5 - da;
@@ -387,7 +398,7 @@ template <class T> __device__ __forceinline__ Gather<T> far_recipe(const KParams
         if (j < BW / 2 || n2 == ib) return g_copy<T>(edge_cell(s, 0, j, ib));
         return mean2(n2, (j - BW / 2) * 2);
     }
-    const int l1 = lev_first(P, s, ib);
+    const int l1 = S.l1;
     if (l1 == lev) return g_copy<T>(edge_cell(os, 1, j, n1));
     if (l1 > lev) {
         if (j < BW / 2) return mean2(n1, j * 2);
@@ -396,7 +407,7 @@ template <class T> __device__ __forceinline__ Gather<T> far_recipe(const KParams
     }
     const int C = n1;
     const T cj = ceil(T(j) * T(0.5));
-    const int jj = back_first(P, s, ib) ? ftoi(cj) : ftoi(cj + T(BW / 2));
+    const int jj = S.back ? ftoi(cj) : ftoi(cj + T(BW / 2));
     const T jr = cj * T(2) > T(j) ? T(0.25) : T(0.75);
     const int p0 = edge_cell(os, 0, jj, C), p1 = edge_cell(os, 1, jj, C);
     const int q0 = edge_cell(os, 0, jj - 1, C), q1 = edge_cell(os, 1, jj - 1, C);
@@ -407,126 +418,6 @@ template <class T> __device__ __forceinline__ Gather<T> far_recipe(const KParams
         case SB: return Gather<T>{G_BILIN, {q1, q0, p1, p0}, jr, T(0.75), T(0)};
         default: return Gather<T>{G_BILIN, {q0, q1, p0, p1}, jr, T(0.25), T(0)};
     }
-}
-
-// The limited slopes along x and y of field a at interior cell (x, y); at(x, y)
-// gives the cell's index in a (the block's place in the Model arrays, or its
-// copy in LDS).
-// FAST: the division by delta is a product with idelta, its hardware reciprocal.
-template <bool FAST, class T, class F, class I>
-__device__ __forceinline__ void grad_cell(T theta, T delta, T idelta, int x, int y, const F& a, const I& at, T& dadx,
-                                          T& dady) {
-    const T ai = a(at(x, y));
-    const T mx = minmod2(theta, a(at(x - 1, y)), ai, a(at(x + 1, y)));
-    const T my = minmod2(theta, a(at(x, y - 1)), ai, a(at(x, y + 1)));
-    dadx = FAST ? mx * idelta : mx / delta;
-    dady = FAST ? my * idelta : my / delta;
-}
-
-// Cell (x, y) of a block's 18x18 copy in LDS (x, y in [-1, 16]).
-__device__ __forceinline__ int lmem(int x, int y) { return (x + 1) + (y + 1) * MW; }
-
-// The block's slopes in LDS for its fluxes: x slopes at x in [-1, 16], y in
-// [0, 15] (index y * 18 + x + 1), y slopes at x in [0, 15], y in [-1, 16]
-// (index (y + 1) * 16 + x), each of h, zs, u, v (fields 0..3).
-constexpr int LGN = 18 * 16;
-__device__ __forceinline__ int lgx(int x, int y) { return y * 18 + x + 1; }
-__device__ __forceinline__ int lgy(int x, int y) { return (y + 1) * 16 + x; }
-// The block in LDS for its fluxes: its 18x18 cells of h, zb, u, v (lmem
-// order), its slopes, and the h and zb of the coarser neighbours' cells that
-// replace its own in the source terms of the faces of side s (sh[s], sz[s],
-// where son[s]: the neighbour on side s is coarser).
-template <class T> struct LdsGrad {
-    T gx[4][LGN];
-    T gy[4][LGN];
-    T h[BS], zb[BS], u[BS], v[BS];
-    T sh[4][BW], sz[4][BW];
-    int son[4];
-};
-
-// Block ib's cells (interior and halo: one contiguous run of the Model
-// arrays), two per thread and array, loaded into registers first so that the
-// loads are in flight together with the other loads of the launch's start.
-template <class T> struct TileRegs {
-    T h[2], zb[2], u[2], v[2];
-};
-template <class T>
-__device__ __forceinline__ void tile_load(const T* h, const T* u, const T* v, const T* zb, TileRegs<T>& R, int t,
-                                          int ib) {
-    const size_t o = (size_t)ib * BS;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int c = t + 256 * k;
-        if (c < BS) {
-            R.h[k] = h[o + c];
-            R.zb[k] = zb[o + c];
-            R.u[k] = u[o + c];
-            R.v[k] = v[o + c];
-        }
-    }
-}
-template <class T> __device__ __forceinline__ void tile_store(const TileRegs<T>& R, LdsGrad<T>& S, int t) {
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int c = t + 256 * k;
-        if (c < BS) {
-            S.h[c] = R.h[k];
-            S.zb[c] = R.zb[k];
-            S.u[c] = R.u[k];
-            S.v[c] = R.v[k];
-        }
-    }
-}
-
-// The slopes of h, zs, u, v of the block's cells, from its LDS copy.
-template <bool FAST, class T>
-__device__ __forceinline__ void amr_grad_lds(T theta, T delta, T idelta, LdsGrad<T>& S, int t) {
-    const int x = t & 15, y = t >> 4;
-    const int kx = lgx(x, y), ky = lgy(x, y);
-    const Fld<T, false> lh{S.h, S.zb}, lu{S.u, S.zb}, lv{S.v, S.zb};
-    const Fld<T, true> lzs{S.h, S.zb};
-    grad_cell<FAST>(theta, delta, idelta, x, y, lh, lmem, S.gx[0][kx], S.gy[0][ky]);
-    grad_cell<FAST>(theta, delta, idelta, x, y, lzs, lmem, S.gx[1][kx], S.gy[1][ky]);
-    grad_cell<FAST>(theta, delta, idelta, x, y, lu, lmem, S.gx[2][kx], S.gy[2][ky]);
-    grad_cell<FAST>(theta, delta, idelta, x, y, lv, lmem, S.gx[3][kx], S.gy[3][ky]);
-}
-
-// The slopes of h, zs, u, v normal to side s at the block's halo cell (s, j):
-// theta-minmod of the far value, the halo cell and the block's edge cell
-// (the left and bottom sides in that order, the right and top sides
-// reversed), from the block's halo and the neighbours' cells in the Model
-// arrays: every cell is loaded before the first slope is formed.
-template <bool FAST, class T>
-__device__ __forceinline__ void amr_grad_halo(const KParams& P, T theta, T delta, T idelta, const T* h, const T* u,
-                                              const T* v, const T* zb, LdsGrad<T>& S, int s, int j, int ib,
-                                              int lev) {
-    const Gather<T> far = far_recipe<T>(P, s, j, ib, lev);
-    const int i = edge_cell(s, -1, j, ib), e = edge_cell(s, 0, j, ib);
-    T fh[4], fz[4], fu[4], fv[4];
-    g_load(far, h, fh);
-    g_load(far, zb, fz);
-    g_load(far, u, fu);
-    g_load(far, v, fv);
-    const T hi = h[i], zi = zb[i], ui = u[i], vi = v[i];
-    const T he = h[e], ze = zb[e], ue = u[e], ve = v[e];
-    T fzs[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) fzs[m] = fz[m] + fh[m];
-    const bool lo = s == SL || s == SB;
-    auto slope = [&](T far_v, T halo_v, T own_v) {
-        const T m = lo ? minmod2(theta, far_v, halo_v, own_v) : minmod2(theta, own_v, halo_v, far_v);
-        return FAST ? m * idelta : m / delta;
-    };
-    const T g0 = slope(g_apply(far, fh), hi, he);
-    const T g1 = slope(g_apply(far, fzs), zi + hi, ze + he);
-    const T g2 = slope(g_apply(far, fu), ui, ue);
-    const T g3 = slope(g_apply(far, fv), vi, ve);
-    T(*g)[LGN] = s < 2 ? S.gx : S.gy;
-    const int k = s == SL ? lgx(-1, j) : s == SR ? lgx(BW, j) : s == SB ? lgy(j, -1) : lgy(j, BW);
-    g[0][k] = g0;
-    g[1][k] = g1;
-    g[2][k] = g2;
-    g[3][k] = g3;
 }
 
 // ----------------------------------------------------------- prolongation
@@ -547,8 +438,9 @@ template <class T> __device__ __forceinline__ HaloPt<T> pt_recipe(const KParams&
     }
     const int s = x < 0 ? SL : x >= BW ? SR : y < 0 ? SB : ST;
     const int j = s < 2 ? y : x;
-    r.g = fill_recipe<T>(P, s, j, C, levC);
-    r.wd = wetdry_recipe(P, s, j, C, levC);
+    const Side S = side_of(P, s, C);
+    r.g = fill_recipe<T>(P, S, s, j, C, levC);
+    r.wd = wetdry_recipe(P, S, s, j, C, levC);
     return r;
 }
 
@@ -598,13 +490,14 @@ template <class T> struct HaloVals {
 template <class T>
 __device__ __forceinline__ HaloVals<T> amr_halo_refine(const KParams& P, const T* h, const T* u, const T* v,
                                                        const T* zb, bool prolong, int s, int j, int ib, int lev) {
-    const int C = nb_first(P, s, ib), levC = lev_first(P, s, ib);
+    const Side S = side_of(P, s, ib);
+    const int C = S.n1, levC = S.l1;
     const bool coarse = levC < lev;
     const bool pro = coarse && prolong && levC == P.minlevel;
     HaloPt<T> pt[5];
     if (coarse) {
         const T fj = floor(T(j) * T(0.5));
-        const int jj = back_first(P, s, ib) ? ftoi(fj) : ftoi(fj + T(BW / 2));
+        const int jj = S.back ? ftoi(fj) : ftoi(fj + T(BW / 2));
         const int cx = s == SL ? BW - 1 : s == SR ? 0 : jj, cy = s == SB ? BW - 1 : s == ST ? 0 : jj;
         pt[0] = pt_recipe<T>(P, cx, cy, C, levC);
         pt[1] = pt_recipe<T>(P, cx - 1, cy, C, levC);
@@ -612,8 +505,8 @@ __device__ __forceinline__ HaloVals<T> amr_halo_refine(const KParams& P, const T
         pt[3] = pt_recipe<T>(P, cx, cy - 1, C, levC);
         pt[4] = pt_recipe<T>(P, cx, cy + 1, C, levC);
     } else {
-        pt[0].g = fill_recipe<T>(P, s, j, ib, lev);
-        pt[0].wd = wetdry_recipe(P, s, j, ib, lev);
+        pt[0].g = fill_recipe<T>(P, S, s, j, ib, lev);
+        pt[0].wd = wetdry_recipe(P, S, s, j, ib, lev);
 #pragma unroll
         for (int k = 1; k < 5; k++) pt[k].wd.on = 0;
     }
@@ -683,11 +576,12 @@ __device__ __forceinline__ void amr_prolong(const KParams& P, T* h, T* zb, const
     const int lev = P.level[ib];
     if (lev != level) return;
     const int s = (t >> 4) & 3, j = t & 15;
-    const int C = nb_first(P, s, ib);
-    if (!(lev > lev_first(P, s, ib))) return;
+    const Side S = side_of(P, s, ib);
+    const int C = S.n1;
+    if (!(lev > S.l1)) return;
     const T eps = T(P.eps);
     const T fj = floor(T(j) * T(0.5));
-    const int jp = back_first(P, s, ib) ? ftoi(fj) : ftoi(fj + T(BW / 2));
+    const int jp = S.back ? ftoi(fj) : ftoi(fj + T(BW / 2));
     const int cx = s == SL ? BW - 1 : s == SR ? 0 : jp;
     const int cy = s == SB ? BW - 1 : s == ST ? 0 : jp;
     // C's halo as the sequential reference sees it when it reaches this block
@@ -712,12 +606,90 @@ __global__ __launch_bounds__(256) void k_amr_prolong(KParams P, T* h, T* zb, con
 }
 
 // ----------------------------------------------------------------- fluxes
-// src/Kurganov.cu:1865-1911
-// FAST: hardware square roots and reciprocals for the IEEE ones.
-template <class T, bool FAST>
-__device__ __forceinline__ T kurg_solver(T g, T delta, T epsi, T CFL, T cm, T fm, T hp, T hm, T up, T um, T& fh,
-                                         T& fu) {
+template <class T> struct StageIn {
+    const T *h, *u, *v;
+};
+template <class T> struct FluxOut {
+    T *Fhu, *Fqux, *Su, *Fqvx, *Fhv, *Fqvy, *Sv, *Fquy;
+};
+
+// The block and what surrounds it in LDS: h, zs, u, v at x, y in [-2, 17]
+// (corners unused) and the slopes of the cells and of the halo ring; the
+// faces take the slopes' place once they are formed (a third of the memory
+// less, so four workgroups of the FP64 kernel share a CU instead of three),
+// and the coarse blocks' cells that the linear prolongation needs stand there
+// before the slopes are.  sh, sz: the h and zb of the coarser neighbours'
+// cells that replace their halo cells in the source terms of the shared faces
+// (src/Kurganov.cu:132-145).
+constexpr int NPT = 32;  // prolongation points per side: see stage_points
+template <class T> struct StageLds {
+    Q4<T> q[20 * TP];
+    union {
+        struct {
+            Q4<T> gx[16 * GXP];  // slopes along x of (h, zs, u, v)
+            Q4<T> gy[18 * GYP];  // slopes along y of (h, zs, v, u)
+        };
+        struct {
+            Q4<T> fx[16 * FP];   // X faces (Fhu, Fqux, Su, Fqvx)
+            Q4<T> fy[17 * FYP];  // Y faces (Fhv, Fqvy, Sv, Fquy)
+        };
+        T pt[4][4][NPT];         // h, u, v and the bed of the points
+    };
+    T sh[4][BW], sz[4][BW];
+    T red[4];
+};
+
+// theta-minmod of src/Util_CPU.cu:243-263 by selection, for any theta.
+template <class T> __device__ __forceinline__ T minmod2s(T theta, T s0, T s1, T s2) {
+    const T d1 = theta * (s1 - s0), d2 = (s2 - s0) * T(0.5), d3 = theta * (s2 - s1);
+    const bool up = s0 < s1 && s1 < s2, dn = s0 > s1 && s1 > s2;
+    const T mn = dmin(dmin(d1, d2), d3), mx = dmax(dmax(d1, d2), d3);
+    return up ? mn : dn ? mx : T(0.0);
+}
+// The slopes of a cell's four fields between its neighbours m and p.  FAST:
+// the division by delta is a product with idelta, its hardware reciprocal.
+template <bool FAST, class T>
+__device__ __forceinline__ Q4<T> slopes4(T theta, T delta, T idelta, const Q4<T>& m, const Q4<T>& c, const Q4<T>& p) {
+    auto one = [&](T a, T b, T d) {
+        const T g = minmod2s(theta, a, b, d);
+        return FAST ? g * idelta : g / delta;
+    };
+    return Q4<T>{one(m.a, c.a, p.a), one(m.b, c.b, p.b), one(m.c, c.c, p.c), one(m.d, c.d, p.d)};
+}
+
+// The h and zb of a coarser block's cell in the source term of a shared face;
+// on: the face has one.
+template <class T> struct SubVal {
+    T h, z;
+    bool on;
+};
+
+// One face between cell n (left or below) and cell i (src/Kurganov.cu:62-164,
+// 1865-1911), from their (h, zs, un, ut) and slopes; Y faces come with u and v
+// swapped.  FAST: hardware square roots and reciprocals for the IEEE ones.
+// Returns whether the face is wet; lim receives its wave speed (0: none), or
+// on spherical grids its CFL step.
+template <class T, bool SPH, bool FAST>
+__device__ __forceinline__ bool amr_face(T g, T CFL, T eps, T delta, T cm, T fm, const Q4<T>& qi, const Q4<T>& qn,
+                                         const Q4<T>& gi, const Q4<T>& gn, const SubVal<T>& si, const SubVal<T>& sn,
+                                         Q4<T>& F, T& lim) {
     using A = Ar<T, FAST>;
+    const T epsi = epsi_of<T>();
+    T hi = qi.a, hn = qn.a;
+    const bool wet = hi > eps || hn > eps;
+    const T dx = delta * T(0.5);
+    T zi = qi.b - hi;
+    const T zl = zi - dx * (gi.b - gi.a);
+    T zn = qn.b - hn;
+    const T zr = zn + dx * (gn.b - gn.a);
+    const T zlr = smax(zl, zr);
+    const T hl = hi - dx * gi.a;
+    const T up = qi.c - dx * gi.c;
+    const T hp = smax(T(0.0), hl + zl - zlr);
+    const T hr = hn + dx * gn.a;
+    const T um = qn.c + dx * gn.c;
+    const T hm = smax(T(0.0), hr + zr - zlr);
+    const T ga = g * T(0.5);
     const T cp = A::sqrt_(g * hp);
     const T cmo = A::sqrt_(g * hm);
     const T ap = smax(smax(up + cp, um + cmo), T(0.0));
@@ -728,97 +700,19 @@ __device__ __forceinline__ T kurg_solver(T g, T delta, T epsi, T CFL, T cm, T fm
     const T hm2 = hm * hm;
     const T hp2 = hp * hp;
     const T a = smax(ap, -am);
-    const T ga = g * T(0.5);
     const T apm = ap * am;
-    const T dlt = FAST ? delta * cm * A::rcp(fm) : delta * cm / fm;
-    if (a > epsi) {
-        fh = (ap * qm - am * qp + apm * (hp - hm)) * ad;
-        fu = (ap * (qm * um + ga * hm2) - am * (qp * up + ga * hp2) + apm * (qp - qm)) * ad;
-        return FAST ? CFL * dlt * A::rcp(a) : CFL * dlt / a;
+    const bool flow = a > epsi;
+    T fh = (ap * qm - am * qp + apm * (hp - hm)) * ad;
+    T fu = (ap * (qm * um + ga * hm2) - am * (qp * up + ga * hp2) + apm * (qp - qm)) * ad;
+    fh = flow ? fh : T(0.0);
+    fu = flow ? fu : T(0.0);
+    const T fv = (fh > T(0.0) ? qn.d + dx * gn.d : qi.d - dx * gi.d) * fh;
+    if (SPH) {
+        const T dlt = FAST ? delta * cm * A::rcp(fm) : delta * cm / fm;
+        lim = !flow ? T(1.0) / epsi : FAST ? CFL * dlt * A::rcp(a) : CFL * dlt / a;
+    } else {
+        lim = flow && wet ? a : T(0.0);
     }
-    fh = T(0.0);
-    fu = T(0.0);
-    return T(1.0) / epsi;
-}
-
-// The h and zb of the coarser block's cell that replace the block's own in the
-// source terms of a face shared with it (src/Kurganov.cu:132-145); on: the
-// face has one.
-template <class T> struct SubVal {
-    T h, z;
-    bool on;
-};
-// The substitution of face j of side s of block ib (lev its level): the cell of
-// the neighbour C next to the face, if C is coarser; stored in LDS for the
-// block's fluxes.
-template <class T>
-__device__ __forceinline__ void coarse_sub(const KParams& P, const T* gh, const T* gzb, int ib, int lev, int s, int j,
-                                           LdsGrad<T>& S) {
-    const int C = nb_first(P, s, ib);
-    const bool on = lev_first(P, s, ib) < lev;
-    if (on) {
-        const T f = floor(T(j) * T(0.5));
-        const int jj = back_first(P, s, ib) ? ftoi(f) : ftoi(f + T(BW / 2));
-        const int c = edge_cell(s ^ 1, 0, jj, C);
-        S.sh[s][j] = gh[c];
-        S.sz[s][j] = gzb[c];
-    }
-    if (j == 0) S.son[s] = on;
-}
-template <class T> __device__ __forceinline__ SubVal<T> sub_of(const LdsGrad<T>& S, int s, int j, bool here) {
-    SubVal<T> r{T(0), T(0), false};
-    if (here && S.son[s]) r = SubVal<T>{S.sh[s][j], S.sz[s][j], true};
-    return r;
-}
-
-template <class T> struct StageIn {
-    const T *h, *u, *v;
-};
-template <class T> struct FluxOut {
-    T *Fhu, *Fqux, *Su, *Fqvx, *Fhv, *Fqvy, *Sv, *Fquy;
-};
-
-// One face between cell n (left or below) and cell i.  Y faces swap the roles
-// of u and v.  si, sn: h and zb substituted into the source terms of cell i or
-// n at a face shared with a coarser block (src/Kurganov.cu:132-145).  The
-// slopes of cells i and n are at gi and gn of the slope arrays (the block's
-// LDS copies).  Returns whether the face is wet; dt receives the face's CFL step.
-template <class T, bool FAST>
-__device__ __forceinline__ bool kface(const KParams& P, T delta, T cm, T fm, const T* h, const T* zb, const T* un_,
-                                      const T* ut_, const T* dhd, const T* dzsd, const T* dund, const T* dutd, int gi,
-                                      int gn, int li, int ln, int i, const SubVal<T>& si, const SubVal<T>& sn,
-                                      T* F0, T* F1, T* F2, T* F3, T& dt) {
-    // h, zb, un_, ut_: the block's LDS copy at li, ln; F0..F3 at i.
-    const T g = T(P.g), CFL = T(P.CFL);
-    const T epsi = epsi_of<T>();
-    const T eps = T(P.eps) + epsi;
-    T hi = h[li], hn = h[ln];
-    if (!(hi > eps || hn > eps)) {
-        F0[i] = T(0.0);
-        F1[i] = T(0.0);
-        F2[i] = T(0.0);
-        F3[i] = T(0.0);
-        dt = T(1.0) / epsi;
-        return false;
-    }
-    const T dhdi = dhd[gi], dhdn = dhd[gn];
-    const T dx = delta * T(0.5);
-    T zi = (zb[li] + hi) - hi;
-    const T zl = zi - dx * (dzsd[gi] - dhdi);
-    T zn = (zb[ln] + hn) - hn;
-    const T zr = zn + dx * (dzsd[gn] - dhdn);
-    const T zlr = smax(zl, zr);
-    const T hl = hi - dx * dhdi;
-    const T up = un_[li] - dx * dund[gi];
-    const T hp = smax(T(0.0), hl + zl - zlr);
-    const T hr = hn + dx * dhdn;
-    const T um = un_[ln] + dx * dund[gn];
-    const T hm = smax(T(0.0), hr + zr - zlr);
-    const T ga = g * T(0.5);
-    T fh, fu, fv;
-    dt = kurg_solver<T, FAST>(g, delta, epsi, CFL, cm, fm, hp, hm, up, um, fh, fu);
-    if (fh > T(0.0)) fv = (ut_[ln] + dx * dutd[gn]) * fh;
-    else fv = (ut_[li] - dx * dutd[gi]) * fh;
     if (si.on) {
         hi = si.h;
         zi = si.z;
@@ -829,71 +723,35 @@ __device__ __forceinline__ bool kface(const KParams& P, T delta, T cm, T fm, con
     }
     const T sl = ga * (hp * hp - hl * hl + (hl + hi) * (zi - zl));
     const T sr = ga * (hm * hm - hr * hr + (hr + hn) * (zn - zr));
-    F0[i] = fm * fh;
-    F1[i] = fm * (fu - sl);
-    F2[i] = fm * (fu - sr);
-    F3[i] = fm * fv;
-    return true;
+    F.a = wet ? (SPH ? fm * fh : fh) : T(0.0);
+    F.b = wet ? (SPH ? fm * (fu - sl) : fu - sl) : T(0.0);
+    F.c = wet ? (SPH ? fm * (fu - sr) : fu - sr) : T(0.0);
+    F.d = wet ? (SPH ? fm * fv : fv) : T(0.0);
+    return wet;
 }
 
-// X face ix (0..16) of row iy (cm: the metric term of the row, fm = 1 on X
-// faces); Y face ix of row iy (0..16).  si, sn: the source substitutions.
-template <class T, bool FAST>
-__device__ __forceinline__ bool xface(const KParams& P, T delta, int ib, int ix, int iy, T cm, const SubVal<T>& si,
-                                      const SubVal<T>& sn, const LdsGrad<T>& G, const FluxOut<T>& F, T& dt) {
-    return kface<T, FAST>(P, delta, cm, T(1.0), G.h, G.zb, G.u, G.v, G.gx[0], G.gx[1], G.gx[2], G.gx[3], lgx(ix, iy),
-                 lgx(ix - 1, iy), lmem(ix, iy), lmem(ix - 1, iy), memloc(ix, iy, ib), si, sn, F.Fhu, F.Fqux, F.Su,
-                 F.Fqvx, dt);
-}
-template <class T, bool FAST>
-__device__ __forceinline__ bool yface(const KParams& P, T delta, int ib, int ix, int iy, T cm, T fm,
-                                      const SubVal<T>& si, const SubVal<T>& sn, const LdsGrad<T>& G,
-                                      const FluxOut<T>& F, T& dt) {
-    return kface<T, FAST>(P, delta, cm, fm, G.h, G.zb, G.v, G.u, G.gy[0], G.gy[1], G.gy[3], G.gy[2], lgy(ix, iy),
-                 lgy(ix, iy - 1), lmem(ix, iy), lmem(ix, iy - 1), memloc(ix, iy, ib), si, sn, F.Fhv, F.Fqvy, F.Sv,
-                 F.Fquy, dt);
+// Holds the end of a face's arithmetic in front of the next face's: the
+// compiler otherwise sinks it past the barrier to the stores, and the operands
+// of three faces outgrow the registers that the occupancy allows (83 VGPRs in
+// FP32 and 163 in FP64 against 60 and 110).
+template <class T> __device__ __forceinline__ void finish(Q4<T>& F) {
+    asm volatile("" : "+v"(F.a), "+v"(F.b), "+v"(F.c), "+v"(F.d));
 }
 
-// Metric terms of thread (x, y)'s faces: cm of its row's X faces, cm and fm of
-// its Y face and of the top face (y = 15 only); 1 on Cartesian grids.
+// Metric terms of the faces of row y: cm of its X faces, cm and fm of the Y
+// face below (y = 16: the top faces); 1 on Cartesian grids.
 template <class T> struct FaceMetric {
-    T cmx, cmy, fmy, cmt, fmt;
+    T cmx, cmy, fmy;
 };
 template <class T, bool SPH> __device__ __forceinline__ FaceMetric<T> face_metric(const KParams& P, int ib, int y) {
-    FaceMetric<T> M{T(1.0), T(1.0), T(1.0), T(1.0), T(1.0)};
+    FaceMetric<T> M{T(1.0), T(1.0), T(1.0)};
     if (SPH) {
         const T* m = (const T*)P.metric + (size_t)ib * METRIC_STRIDE;
-        M.cmx = m[MET_CMX + y];
+        M.cmx = m[MET_CMX + (y < BW ? y : BW - 1)];
         M.cmy = m[MET_CMY + y];
         M.fmy = m[MET_FMY + y];
-        if (y == BW - 1) {
-            M.cmt = m[MET_CMY + BW];
-            M.fmt = m[MET_FMY + BW];
-        }
     }
     return M;
-}
-
-template <class T, bool FAST>
-__device__ __forceinline__ void amr_flux(const KParams& P, T delta, int ib, const LdsGrad<T>& G, const FaceMetric<T>& M,
-                                         const FluxOut<T>& F, DevLoop* L, int corr, int t, int vb, T* red) {
-    const int x = t & 15, y = t >> 4;
-    const T inv_epsi = T(1.0) / epsi_of<T>();
-    const SubVal<T> none{T(0), T(0), false};
-    T d = tmax_of<T>(), dt;
-    // dtmax of the cell: its X face (left), then its Y face (bottom), each
-    // keeping the smaller step, a dry face resetting it to 1/epsi
-    if (xface<T, FAST>(P, delta, ib, x, y, M.cmx, none, sub_of(G, SL, y, x == 0), G, F, dt)) d = dt < d ? dt : d;
-    else d = inv_epsi;
-    if (yface<T, FAST>(P, delta, ib, x, y, M.cmy, M.fmy, none, sub_of(G, SB, x, y == 0), G, F, dt))
-        d = dt < d ? dt : d;
-    else d = inv_epsi;
-    if (x == BW - 1) (void)xface<T, FAST>(P, delta, ib, BW, y, M.cmx, sub_of(G, SR, y, true), none, G, F, dt);
-    if (y == BW - 1) (void)yface<T, FAST>(P, delta, ib, x, BW, M.cmt, M.fmt, sub_of(G, ST, x, true), none, G, F, dt);
-    if (!corr) {
-        const T m = block_min(d, red, t);
-        if (t == 0) slot_min(L, vb, m);
-    }
 }
 
 // Face position of side s at j: left and bottom faces are stored at the
@@ -910,8 +768,9 @@ __device__ __forceinline__ void amr_fluxfix_side(const KParams& P, const FluxOut
     const int lev = P.level[ib];
     T* const A[4] = {s < 2 ? F.Fhu : F.Fhv, s < 2 ? F.Fqux : F.Fqvy, s < 2 ? F.Su : F.Sv, s < 2 ? F.Fqvx : F.Fquy};
     // coarse face = mean of the two fine faces (src/Halo.cu:1441-1529, 1766-1862)
-    const int n = j < BW / 2 ? nb_first(P, s, ib) : nb_second(P, s, ib);
-    if ((j < BW / 2 ? lev_first(P, s, ib) : lev_second(P, s, ib)) > lev) {
+    const Side S = side_of(P, s, ib);
+    const int n = j < BW / 2 ? S.n1 : S.n2;
+    if ((j < BW / 2 ? S.l1 : S.l2) > lev) {
         const int jj = (j & (BW / 2 - 1)) * 2;
         const int i = face_at(s, j, ib), il = face_at(s ^ 1, jj, n), itl = face_at(s ^ 1, jj + 1, n);
 #pragma unroll
@@ -919,7 +778,7 @@ __device__ __forceinline__ void amr_fluxfix_side(const KParams& P, const FluxOut
     }
     // wall boundary (noslipbndQ, src/Boundary.cu:1887-1891): no mass flux through
     // the boundary face and no normal-momentum flux difference in the edge cell
-    if (nb_first(P, s, ib) != ib && nb_second(P, s, ib) != ib) return;
+    if (S.n1 != ib && S.n2 != ib) return;
     const int ty = blk_btype(P, ib);
     if (ty == 0 || ty >= 2) {
         const int i = face_at(s, j, ib);
@@ -931,10 +790,10 @@ __device__ __forceinline__ void amr_fluxfix_side(const KParams& P, const FluxOut
             const int in = s == SL ? memloc(1, j, ib) : s == SR ? memloc(BW - 1, j, ib) : s == SB ? memloc(j, 1, ib)
                                                                                           : memloc(j, BW - 1, ib);
             const double ts = corr ? L->tcorr : L->tpred;
-            const BSeg& S = P.seg[P.bseg[ib]];
+            const BSeg& G = P.seg[P.bseg[ib]];
             const int fx = s == SL ? 0 : s == SR ? BW : j, fy = s == SB ? 0 : s == ST ? BW : j;
             T q = A[0][i];
-            if (bnd_flux<T>(P, s, ty, seg_level<T>(P, S, ts, ib, fx, fy), bnd_taper<T>(P, S, ts), zb[i] + E0.h[i],
+            if (bnd_flux<T>(P, s, ty, seg_level<T>(P, G, ts, ib, fx, fy), bnd_taper<T>(P, G, ts), zb[i] + E0.h[i],
                             E0.h[i], zb[in] + E0.h[in], E0.h[in], (s < 2 ? E0.u : E0.v)[in], q)) {
                 A[0][i] = q;
                 return;
@@ -957,16 +816,19 @@ template <class T> struct AdvArgs {
     const T* cf;
 };
 
-// A cell's values that the advance reads besides the face fluxes (the
-// conditional ones too: the loads are issued before the face fix-up's barrier).
+// The tendencies of h, hu, hv of the blocks that do not wait for another
+// block's faces, interior cells only (BSI values per block), between the
+// predictor's stage and its advance.
+template <class T> struct Tend {
+    T *dh, *dhu, *dhv;
+};
+
+// A cell's values that the advance reads besides its tendencies.
 template <class T> struct AdvIn {
-    T h, u, v, hold, uold, vold, cf, zb;
+    T hold, uold, vold, cf, zb;
 };
 template <class T> __device__ __forceinline__ AdvIn<T> adv_load(const AdvArgs<T>& A, int i, int corr) {
     AdvIn<T> X;
-    X.h = A.h[i];
-    X.u = A.u[i];
-    X.v = A.v[i];
     X.hold = A.hold[i];
     X.uold = A.uold[i];
     X.vold = A.vold[i];
@@ -975,33 +837,42 @@ template <class T> __device__ __forceinline__ AdvIn<T> adv_load(const AdvArgs<T>
     return X;
 }
 
+// Tendencies of cell (x, y) of block ib (src/Advection.cu:160-254) from its
+// stage state and its left, right, bottom and top faces; spherical grids take
+// the row's metric terms.  The river discharges follow (AddRiverForcing after
+// updateEV, src/FlowCPU.cu:120-124).
 template <class T, bool SPH>
-__device__ __forceinline__ void amr_advance(const KParams& P, const AdvArgs<T>& A, const AdvIn<T>& X,
-                                            const FluxOut<T>& F, const DevLoop* L, int corr, int t, int ib) {
-    const int x = t & 15, y = t >> 4;
-    const int i = memloc(x, y, ib), iright = memloc(x + 1, y, ib), itop = memloc(x, y + 1, ib);
-    const T delta = calcres(T(P.delta0), P.level[ib]);
-    const T g = T(P.g);
-    // src/Advection.cu:160-254; spherical grids take the row's metric terms
+__device__ __forceinline__ void amr_tendencies(const KParams& P, T delta, T hi, T uui, T vvi, T Fhl, T Fhr, T Fhb,
+                                               T Fht, T Fql, T Sr, T Fqb, T St, T Ftb, T Ftt, T Ftl, T Ftr, int ib,
+                                               int x, int y, T& dh, T& dhu, T& dhv) {
     const T* met = (const T*)P.metric + (size_t)ib * METRIC_STRIDE;
-    const bool sph = SPH;
-    const T fc = sph ? met[MET_FC + y] : T(P.fc);
-    const T cm = sph ? met[MET_CME + y] : T(1.0), fmu = T(1.0), fmup = T(1.0);
-    const T fmv = sph ? met[MET_FMV + y] : T(1.0), fmvp = sph ? met[MET_FMVP + y] : T(1.0);
-    const T hi = X.h, uui = X.u, vvi = X.v;
+    const T fc = SPH ? met[MET_FC + y] : T(P.fc);
+    const T cm = SPH ? met[MET_CME + y] : T(1.0);
     const T cmdinv = T(1.0) / (cm * delta);
-    const T ga = T(0.5) * g;
-    // tendencies, then the river discharges (AddRiverForcing after updateEV, src/FlowCPU.cu:120-124)
-    const T dhi = river_inflow<T>(P, ib, x, y, T(-1.0) * (F.Fhu[iright] - F.Fhu[i] + F.Fhv[itop] - F.Fhv[i]) * cmdinv);
-    const T dmdl = (fmup - fmu) / (cm * delta);
-    const T dmdt = (fmvp - fmv) / (cm * delta);
-    const T fG = vvi * dmdl - uui * dmdt;
-    T dhu = (F.Fqux[i] + F.Fquy[i] - F.Su[iright] - F.Fquy[itop]) * cmdinv + fc * hi * vvi;
-    T dhv = (F.Fqvy[i] + F.Fqvx[i] - F.Sv[itop] - F.Fqvx[iright]) * cmdinv - fc * hi * uui;
-    dhu += hi * (ga * hi * dmdl + fG * vvi);
-    dhv += hi * (ga * hi * dmdt - fG * uui);
-    // src/Advection.cu:332-385; the drying limiter is evaluated in double
+    dh = river_inflow<T>(P, ib, x, y, T(-1.0) * (Fhr - Fhl + Fht - Fhb) * cmdinv);
+    dhu = (Fql + Ftb - Sr - Ftt) * cmdinv + fc * hi * vvi;
+    dhv = (Fqb + Ftl - St - Ftr) * cmdinv - fc * hi * uui;
+    if (SPH) {  // the metric differences, zero on Cartesian grids
+        const T fmu = T(1.0), fmup = T(1.0);
+        const T fmv = met[MET_FMV + y], fmvp = met[MET_FMVP + y];
+        const T ga = T(0.5) * T(P.g);
+        const T dmdl = (fmup - fmu) / (cm * delta);
+        const T dmdt = (fmvp - fmv) / (cm * delta);
+        const T fG = vvi * dmdl - uui * dmdt;
+        dhu += hi * (ga * hi * dmdl + fG * vvi);
+        dhv += hi * (ga * hi * dmdt - fG * uui);
+    }
+}
+
+// The update of a cell by its tendencies (src/Advection.cu:332-385; the drying
+// limiter in double), and in the corrector the bottom friction
+// (src/Friction.cu:89-148), cleanup and the implicit rain
+// (src/Updateforcing.cu:530-581).
+template <class T>
+__device__ __forceinline__ void amr_update(const KParams& P, const AdvArgs<T>& A, const AdvIn<T>& X, T dhi, T dhu,
+                                           T dhv, const DevLoop* L, int corr, int i, int ib, int x, int y) {
     const T dt = corr ? T(L->dt) : T(L->dt) * T(0.5);
+    const T g = T(P.g);
     const T eps = T(P.eps);
     const T hold = X.hold;
     T edt;
@@ -1062,24 +933,21 @@ __device__ __forceinline__ void amr_advance(const KParams& P, const AdvArgs<T>& 
     }
 }
 
-// Merged launches.  Within one launch a workgroup owns one block; a phase
-// that reads only its own block's output of the phase before it (and cells
-// of other blocks that neither phase writes) follows it in the same launch
-// after a workgroup barrier:
-//  - gradients, then fluxes: the fluxes read the block's own gradients (in
-//    LDS) and, at a face shared with a coarser block, that block's interior h
-//    and zb; the gradient halo reads neighbours' interior cells
-//    (src/Gradients.cu:2713-3294), which neither phase writes;
-//  - the face fix-up, then the advance: the fix-up reads the finer
-//    neighbours' faces on the shared side, which neither phase writes (a
-//    block's fix-up changes only faces beside a finer block or on the domain
-//    edge), and the block's own faces and step-start cells; the advance writes
-//    the block's interior cells only.  Both stages run them after the dt
-//    reduction; the predictor's boundary fluxes take the time the reduction
-//    recorded from the previous dt.
-// One wave per block, thread (side, j): the block's halo for the stage.  A
-// block writes its own halo only and reads other blocks' interior cells and
-// the bed halo cells that the prolongation leaves alone (beside a finer block).
+// Whether block ib's stage ends in the deferred fix-up (its faces stored,
+// restricted beside finer blocks and patched on open boundaries, then its
+// advance) instead of in the stage's own launch: it has a finer neighbour, or
+// a boundary side in a run with open segments, whose faces follow the dt
+// reduction.  info: any of the block's level words (REC_* flags).  The host's
+// list of these blocks (P.fix) follows the same rule.
+__device__ __forceinline__ bool fix_block(const KParams& P, int info) {
+    return P.fix_all || (info & REC_FINER) || (P.bopen && (info & REC_EDGE));
+}
+
+// One wave per block, thread (side, j): the block's halo for the stage, on
+// meshes of four levels and more, whose wet/dry prolongation runs level by
+// level (k_amr_prolong).  A block writes its own halo only and reads other
+// blocks' interior cells and the bed halo cells that the prolongation leaves
+// alone (beside a finer block).
 template <class T>
 __global__ __launch_bounds__(64) void k_amr_halo_refine(KParams P, T* h, T* u, T* v, T* zb, T* hsnap, DevLoop* L,
                                                         int corr) {
@@ -1096,97 +964,523 @@ __global__ __launch_bounds__(64) void k_amr_halo_refine(KParams P, T* h, T* u, T
     if (o.zbset) zb[w] = o.zb;
 }
 
-// Every global load of the block's state, its neighbours' cells and its
-// metric is issued before the stage flag is tested and before the first
-// barrier (they depend on the block only): the tile into registers, the halo
-// slopes (wave 0) and the source substitutions (wave 1) into LDS.  FAST:
-// hardware reciprocals and square roots in the slopes and the fluxes.
-template <class T, bool SPH, bool FAST>
-__global__ __launch_bounds__(256) void k_amr_grad_flux(KParams P, StageIn<T> E, const T* zb, FluxOut<T> F,
-                                                       DevLoop* L, int corr) {
-    __shared__ T red[4];
-    __shared__ LdsGrad<T> S;
-    const int t = threadIdx.x;
-    const int ib = P.active[blockIdx.x];
+// Tile position of depth d (-1 the halo, -2 beyond it) of side s at j.
+__device__ __forceinline__ int side_tix(int s, int d, int j) {
+    return s == SL ? tix(d, j) : s == SR ? tix(BW - 1 - d, j) : s == SB ? tix(j, d) : tix(j, BW - 1 - d);
+}
+
+// The coarse cells that the linear prolongation of side s (beside the coarser
+// block C) reads, one per lane k: a half side of C is eight edge cells, and
+// their neighbours make 26 points --
+//   0..9    C's edge cells from one before the half to one after it (an end
+//           beyond C's side is C's halo on the adjoining side),
+//   10..17  the cells behind them,
+//   18..25  C's halo in front of them;
+// 26..30 the five points (a cell of D and its four neighbours) behind C's
+//         halo at the end of its side, where the block D there is coarser than
+//         C,
+//   31    C's halo at that end, behind point 0 or 9.
+// The last six give C's halo at the end of the half as C's own halo stage
+// leaves it (end_halo), which the sequential reference's wet/dry prolongation
+// tests and the cells beyond the halo are interpolated from.
+// side_end gives that halo: side p of C, position je beside the shared side.
+struct SideEnd {
+    int p, je;
+    Side E;  // side p of C
+};
+__device__ __forceinline__ SideEnd side_end(const KParams& P, int s, const Side& S) {
+    SideEnd e;
+    const bool lo = S.back;
+    e.p = s < 2 ? (lo ? SB : ST) : (lo ? SL : SR);
+    e.je = (s == SL || s == SB) ? BW - 1 : 0;
+    e.E = side_of(P, e.p, S.n1);
+    return e;
+}
+// Cell of C at depth d from its side facing side s of the block, at position a.
+__device__ __forceinline__ void facing_cell(int s, int d, int a, int& x, int& y) {
+    const int n = (s == SL || s == SB) ? BW - 1 - d : d;
+    x = s < 2 ? n : a;
+    y = s < 2 ? a : n;
+}
+template <class T>
+__device__ __forceinline__ HaloPt<T> stage_point(const KParams& P, int s, int k, const Side& S) {
+    const int j0 = S.back ? 0 : BW / 2;
+    int x, y, b = S.n1, lev = S.l1;
+    if (k < 26 || k == 31) {
+        const int d = k < 10 ? 0 : k < 18 || k == 31 ? 1 : -1;
+        const int a = k < 10 ? j0 - 1 + k : k < 18 ? j0 + k - 10 : k < 26 ? j0 + k - 18 : S.back ? -1 : BW;
+        facing_cell(s, d, a, x, y);
+    } else {
+        const SideEnd e = side_end(P, s, S);
+        const Side& E = e.E;
+        if (!(E.l1 < S.l1)) {  // no coarser block there: any cell of C
+            facing_cell(s, 0, j0, x, y);
+        } else {
+            const int a = e.je / 2 + (E.back ? 0 : BW / 2);
+            facing_cell(e.p, 0, a, x, y);
+            const int m = k - 26;
+            x += m == 1 ? -1 : m == 2 ? 1 : 0;
+            y += m == 3 ? -1 : m == 4 ? 1 : 0;
+            b = E.n1;
+            lev = E.l1;
+        }
+    }
+    return pt_recipe<T>(P, x, y, b, lev);
+}
+
+// C's halo cell at the end of its half side, at depth d (0 or 1) from the
+// shared side, as C's halo stage leaves it: h, zs, u, v from the points pt
+// of the side.  Beside a coarser block D it is the linear reconstruction, or,
+// where the wet/dry prolongation applies, D's cell (both depths lie over one
+// cell of D); C's own workgroup may be writing the bed of that halo cell,
+// but only where it becomes the bed of D's cell, which is taken from D here.
+template <class T>
+__device__ __forceinline__ Q4<T> end_halo(const KParams& P, const T (*pt)[NPT], const SideEnd& e, const Side& S,
+                                          bool prolong, T eps, int d) {
+    const int k = d == 0 ? (S.back ? 0 : 9) : 31;
+    Q4<T> o{pt[0][k], pt[3][k], pt[1][k], pt[2][k]};
+    if (e.E.l1 < S.l1) {
+        const int je = e.je == 0 ? d : e.je - d;
+        T f[3][5];
+#pragma unroll
+        for (int n = 0; n < 3; n++)
+#pragma unroll
+            for (int m = 0; m < 5; m++) f[n][m] = pt[n][26 + m];
+        o.a = refine_from(P, e.p, je, S.l1, e.E.l1, f[0]);
+        o.c = refine_from(P, e.p, je, S.l1, e.E.l1, f[1]);
+        o.d = refine_from(P, e.p, je, S.l1, e.E.l1, f[2]);
+        if (prolong &&
+            !(f[0][0] > eps && f[0][1] > eps && f[0][2] > eps && f[0][4] > eps && f[0][3] > eps)) {
+            o.a = f[0][0];
+            o.b = pt[3][26];
+        }
+    }
+    o.b = o.b + o.a;
+    return o;
+}
+
+// A stage of a block in one workgroup: halo, slopes, faces, tendencies, and in
+// the corrector the advance.
+//
+// Wave s gathers side s: its halo cells (lanes 0-15, or beside a coarser block
+// the points of stage_point, lanes 0-31), the cells beyond the halo that the
+// limited slope at the halo reads (src/Gradients.cu:2713-3294, lanes 32-47)
+// and the source substitutions (lanes 48-63); the side's kind is uniform over
+// its wave.  Beside a coarser block a second pass forms the linear
+// reconstruction and the wet/dry prolongation (src/Halo.cu:1044-1405,
+// src/ConserveElevation.cu:80-205,451-482) from the points.  HALO: the halo
+// is formed here; otherwise it stands in the Model arrays (four levels and
+// more).  The slopes, faces and tendencies are those of the one-level tile.
+//
+// A block that needs no other block's faces has its tendencies stored (the
+// predictor, whose dt is not known yet) or is advanced here (the corrector:
+// it writes the state's interior cells, which no other block of the corrector
+// stage reads); beside a coarser block it leaves the shared faces in the face
+// arrays.  The others (fix_block) store all their faces for the fix-up.
+// Everything global is read before the stage flag is tested.
+template <class T, bool SPH, bool FAST, bool HALO, int corr>
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KParams P, AdvArgs<T> A, T* zb,
+                                                                           FluxOut<T> F, Tend<T> D, DevLoop* L) {
+    __shared__ StageLds<T> S;
+    const int t = threadIdx.x, x = t & 15, y = t >> 4;
+    const int ib = ldu(P.active, xcd_range(blockIdx.x % NXCD, P.nblk).start + blockIdx.x / NXCD);
     DevLoop* Lm = loop_of(P, L, ib);
-    const int lev = P.level[ib];
-    const T theta = T(P.theta);
+    const int lev = ldu(P.level, ib);
+    int nb[8], info[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        nb[k] = ldu(P.nbr, ib * NBR + k);
+        info[k] = ldu(P.nbr, ib * NBR + 8 + k);
+    }
+    bool cs[4];  // the side is beside a coarser block
+#pragma unroll
+    for (int k = 0; k < 4; k++) cs[k] = rec_level(info[2 * k]) < lev;
+    const bool fix = fix_block(P, info[0]);
+    const bool prolong = P.wetdryfix && P.maxlevel > P.minlevel;
+    const T theta = T(P.theta), eps = T(P.eps);
     const T delta = calcres(T(P.delta0), lev);
     const T idelta = Ar<T, FAST>::rcp(delta);
-    TileRegs<T> R;
-    tile_load(E.h, E.u, E.v, zb, R, t, ib);
-    const FaceMetric<T> M = face_metric<T, SPH>(P, ib, t >> 4);
-    if (t < 64) amr_grad_halo<FAST>(P, theta, delta, idelta, E.h, E.u, E.v, zb, S, t >> 4, t & 15, ib, lev);
-    else if (t < 128) coarse_sub(P, E.h, zb, ib, lev, (t >> 4) & 3, t & 15, S);
-    tile_store(R, S, t);
+
+    // the block's own cell
+    const int c = memloc(x, y, ib);
+    const T h0 = A.h[c], z0 = zb[c], u0 = A.u[c], v0 = A.v[c];
+    AdvIn<T> X;
+    if (corr && !fix) X = adv_load(A, c, 1);
+
+    // the wave's side
+    const int s = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63, j = l & 15;
+    const Side sd = side_of_uniform(P, s, ib);
+    const bool coarse = sd.l1 < lev;
+    const bool is_far = (l >> 4) == 2, is_sub = (l >> 4) == 3;
+    const int w = edge_cell(s, -1, j, ib);
+    Q4<T> r;  // the value of the lane's point: h, zs, u, v (halo cells: zs without the bed yet)
+    T zw = T(0), zown = T(0);  // the bed of the lane's point, and of the block's own halo cell
+    r.a = r.b = r.c = r.d = T(0);
+    const bool same = (sd.n1 == ib && sd.n2 == ib) || (sd.n1 != ib && sd.l1 == lev && sd.l2 == lev);
+    if (l < 16) zown = zw = zb[w];
+    if (same) {
+        if (l < 16 || is_far) {
+            const int i = sd.n1 == ib ? edge_cell(s, 0, j, ib) : edge_cell(s ^ 1, is_far ? 1 : 0, j, sd.n1);
+            r.a = A.h[i];
+            r.b = zb[i];
+            r.c = A.u[i];
+            r.d = A.v[i];
+            r.b = r.b + r.a;
+        }
+        if (!HALO && l < 16) {
+            r.a = A.h[w];
+            r.c = A.u[w];
+            r.d = A.v[w];
+        }
+    } else {
+        HaloPt<T> pt;
+        pt.wd.on = 0;
+        if (is_far) {
+            pt.g = far_recipe<T>(sd, s, j, ib, lev);
+        } else if (is_sub) {
+            // the coarse cell next to the face (where the side is coarse; read anyway)
+            int cx, cy;
+            facing_cell(s, 0, coarse ? j / 2 + (sd.back ? 0 : BW / 2) : 0, cx, cy);
+            pt.g = g_copy<T>(memloc(cx, cy, sd.n1));
+        } else if (!HALO) {
+            pt.g = g_copy<T>(w);
+        } else if (coarse) {
+            pt = stage_point<T>(P, s, l, sd);
+        } else {
+            pt.g = fill_recipe<T>(P, sd, s, j, ib, lev);
+            pt.wd = wetdry_recipe(P, sd, s, j, ib, lev);
+        }
+        T H[4], Z[4], U[4], V[4], WH[4], WZ[4];
+        g_load(pt.g, A.h, H);
+        g_load(pt.g, zb, Z);
+        g_load(pt.g, A.u, U);
+        g_load(pt.g, A.v, V);
+        if (pt.wd.on) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                WH[m] = A.h[pt.wd.i[m]];
+                WZ[m] = zb[pt.wd.i[m]];
+            }
+        }
+        if (HALO && coarse && l < 32) zw = zb[pt.wd.w];
+        r.a = g_apply(pt.g, H);
+        r.c = g_apply(pt.g, U);
+        r.d = g_apply(pt.g, V);
+        if (pt.wd.on) r.a = wetdry_apply(eps, WH, WZ, zw, r.a);
+        if (is_far) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) Z[m] = Z[m] + H[m];
+            r.b = g_apply(pt.g, Z);
+        } else {
+            r.b = Z[0];
+        }
+    }
     if (stage_off(Lm, corr)) return;  // the workgroup's one block: all threads leave together
+
+    const Q4<T> q{h0, z0 + h0, u0, v0};
+    S.q[tix(x, y)] = q;
+    if (is_far) S.q[side_tix(s, -2, j)] = r;
+    if (is_sub && coarse) {
+        S.sh[s][j] = r.a;
+        S.sz[s][j] = r.b;
+    }
+    if (HALO && coarse) {
+        if (l < 32) {
+            S.pt[s][0][l] = r.a;
+            S.pt[s][1][l] = r.c;
+            S.pt[s][2][l] = r.d;
+            S.pt[s][3][l] = zw;
+        }
+    } else if (l < 16) {
+        r.b = zw + r.a;
+        S.q[side_tix(s, -1, j)] = r;
+        // open boundaries take the step-start depth of the halo (amr_fluxfix_side: the right and top faces)
+        if (HALO && !corr && P.bopen && (sd.n1 == ib || sd.n2 == ib)) const_cast<T*>(A.h)[w] = r.a;
+    }
     __syncthreads();
-    amr_grad_lds<FAST>(theta, delta, idelta, S, t);
+    if (HALO && (cs[0] || cs[1] || cs[2] || cs[3])) {
+        if (coarse && l < 16) {
+            const int m = j / 2;
+            // the points of the coarse cell m of the half and of its neighbours in x and y
+            const int in = 10 + m, out = 18 + m, before = m, after = m + 2;
+            const bool lo = s == SL || s == SB;  // the side faces the neighbour's high end
+            const int xm = s < 2 ? (lo ? in : out) : before, xp = s < 2 ? (lo ? out : in) : after;
+            const int ym = s < 2 ? before : (lo ? in : out), yp = s < 2 ? after : (lo ? out : in);
+            T f[3][5];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                f[k][0] = S.pt[s][k][m + 1];
+                f[k][1] = S.pt[s][k][xm];
+                f[k][2] = S.pt[s][k][xp];
+                f[k][3] = S.pt[s][k][ym];
+                f[k][4] = S.pt[s][k][yp];
+            }
+            Q4<T> o;
+            o.a = refine_from(P, s, j, lev, sd.l1, f[0]);
+            o.c = refine_from(P, s, j, lev, sd.l1, f[1]);
+            o.d = refine_from(P, s, j, lev, sd.l1, f[2]);
+            T zo = zown;
+            if (prolong) {
+                if (m == (sd.back ? 0 : BW / 2 - 1)) {
+                    // C's halo at the end, prolonged if C comes before this block in the active list
+                    const SideEnd e = side_end(P, s, sd);
+                    f[0][s < 2 ? (sd.back ? 3 : 4) : (sd.back ? 1 : 2)] =
+                        end_halo<T>(P, S.pt[s], e, sd, P.inv[sd.n1] < P.inv[ib], eps, 0).a;
+                }
+                if (!(f[0][0] > eps && f[0][1] > eps && f[0][2] > eps && f[0][4] > eps && f[0][3] > eps)) {
+                    o.a = f[0][0];
+                    zo = S.sz[s][j];
+                    zb[w] = zo;
+                }
+            }
+            o.b = zo + o.a;
+            S.q[side_tix(s, -1, j)] = o;
+        }
+        if (coarse && is_far && j == (sd.back ? 0 : BW - 1)) {
+            // beyond the halo at the end of the half, two of the four cells are C's halo
+            const Gather<T> g = far_recipe<T>(sd, s, j, ib, lev);
+            const SideEnd e = side_end(P, s, sd);
+            T H[4], Z[4], U[4], V[4];
+            g_load(g, A.h, H);
+            g_load(g, zb, Z);
+            g_load(g, A.u, U);
+            g_load(g, A.v, V);
+            const Q4<T> e0 = end_halo<T>(P, S.pt[s], e, sd, prolong, eps, 0);
+            const Q4<T> e1 = end_halo<T>(P, S.pt[s], e, sd, prolong, eps, 1);
+            // C's cells at the end, at depths 0 and 1, as far_recipe indexes them
+            int x0, y0, x1, y1;
+            facing_cell(s, 0, sd.back ? -1 : BW, x0, y0);
+            facing_cell(s, 1, sd.back ? -1 : BW, x1, y1);
+            const int i0 = memloc(x0, y0, sd.n1), i1 = memloc(x1, y1, sd.n1);
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                Z[m] = Z[m] + H[m];
+                if (g.i[m] == i0 || g.i[m] == i1) {
+                    const Q4<T>& h = g.i[m] == i0 ? e0 : e1;
+                    H[m] = h.a;
+                    Z[m] = h.b;
+                    U[m] = h.c;
+                    V[m] = h.d;
+                }
+            }
+            S.q[side_tix(s, -2, j)] = Q4<T>{g_apply(g, H), g_apply(g, Z), g_apply(g, U), g_apply(g, V)};
+        }
+        __syncthreads();
+    }
+
+    // slopes: the thread's own cell, and the halo ring on wave 2 (lanes 0-31 along x, 32-63 along y)
+    const Q4<T> gxo = slopes4<FAST>(theta, delta, idelta, S.q[tix(x - 1, y)], q, S.q[tix(x + 1, y)]);
+    S.gx[gxi(x, y)] = gxo;
+    Q4<T> gyo = slopes4<FAST>(theta, delta, idelta, S.q[tix(x, y - 1)], q, S.q[tix(x, y + 1)]);
+    {
+        const T a = gyo.c;  // stored as (h, zs, v, u)
+        gyo.c = gyo.d;
+        gyo.d = a;
+        S.gy[gyi(x, y)] = gyo;
+    }
+    if (s == 2) {
+        const bool isx = l < 32;
+        const int o = (l & 16) ? BW : -1;
+        const int ci = isx ? tix(o, j) : tix(j, o), d = isx ? 1 : TP;
+        const Q4<T> g = slopes4<FAST>(theta, delta, idelta, S.q[ci - d], S.q[ci], S.q[ci + d]);
+        if (isx) S.gx[gxi(o, j)] = g;
+        else S.gy[gyi(j, o)] = Q4<T>{g.a, g.b, g.d, g.c};
+    }
     __syncthreads();
-    amr_flux<T, FAST>(P, delta, ib, S, M, F, Lm, corr, t, blockIdx.x, red);
+
+    // faces: the cell's left and bottom ones, and the seventeenth ones on wave 3 (lanes 0-15 X, 16-31 Y)
+    const T g = T(P.g), CFL = T(P.CFL), inv_epsi = T(1.0) / epsi_of<T>(), epsw = eps + epsi_of<T>();
+    const SubVal<T> none{T(0), T(0), false};
+    auto sub = [&](int k, int jj, bool here) {
+        return here && cs[k] ? SubVal<T>{S.sh[k][jj], S.sz[k][jj], true} : none;
+    };
+    auto swap_uv = [](const Q4<T>& a) { return Q4<T>{a.a, a.b, a.d, a.c}; };
+    const FaceMetric<T> M = face_metric<T, SPH>(P, ib, y);
+    Q4<T> Fl, Fb, Fe;
+    T lx, ly;
+    const bool wx = amr_face<T, SPH, FAST>(g, CFL, epsw, delta, M.cmx, T(1.0), q, S.q[tix(x - 1, y)], gxo,
+                                           S.gx[gxi(x - 1, y)], none, sub(SL, y, x == 0), Fl, lx);
+    finish(Fl);
+    const bool wy = amr_face<T, SPH, FAST>(g, CFL, epsw, delta, M.cmy, M.fmy, swap_uv(q), swap_uv(S.q[tix(x, y - 1)]),
+                                           gyo, S.gy[gyi(x, y - 1)], none, sub(SB, x, y == 0), Fb, ly);
+    finish(Fb);
+    const bool edge = s == 3 && l < 32, ex = l < 16;
+    if (edge) {
+        const FaceMetric<T> Me = face_metric<T, SPH>(P, ib, ex ? j : BW);
+        const int ci = ex ? tix(BW, j) : tix(j, BW);
+        Q4<T> qi = S.q[ci], qn = S.q[ci - (ex ? 1 : TP)];
+        if (!ex) {
+            qi = swap_uv(qi);
+            qn = swap_uv(qn);
+        }
+        const Q4<T> gi = ex ? S.gx[gxi(BW, j)] : S.gy[gyi(j, BW)], gn = ex ? S.gx[gxi(BW - 1, j)] : S.gy[gyi(j, BW - 1)];
+        SubVal<T> se = none;
+        if (ex ? cs[SR] : cs[ST]) se = SubVal<T>{S.sh[ex ? SR : ST][j], S.sz[ex ? SR : ST][j], true};
+        T le;
+        (void)amr_face<T, SPH, FAST>(g, CFL, epsw, delta, ex ? Me.cmx : Me.cmy, ex ? T(1.0) : Me.fmy, qi, qn, gi, gn, se,
+                                     none, Fe, le);
+    }
+    __syncthreads();  // the slopes are read: the faces take their place
+    S.fx[fxi(x, y)] = Fl;
+    S.fy[fyi(x, y)] = Fb;
+    if (edge) *(ex ? &S.fx[fxi(BW, j)] : &S.fy[fyi(j, BW)]) = Fe;
+    if (!corr) {
+        // dtmax of the cell: its X face, then its Y face, a dry face resetting it to 1/epsi
+        // (src/Kurganov.cu:1488-1491); off the sphere every face has the same cell size, so the block's
+        // largest wave speed gives its smallest step (the rounded division is monotone)
+        T d;
+        if (SPH) {
+            d = wx ? (lx < tmax_of<T>() ? lx : tmax_of<T>()) : inv_epsi;
+            d = wy ? (ly < d ? ly : d) : inv_epsi;
+        } else {
+            d = wy ? -smax(lx, ly) : T(0.0);
+        }
+        T m = block_min(d, S.red, t);
+        if (!SPH) {
+            m = -m > T(0.0) ? (FAST ? CFL * delta * Ar<T, FAST>::rcp(-m) : CFL * delta / -m) : inv_epsi;
+            m = m < inv_epsi ? m : inv_epsi;
+        }
+        if (t == 0) slot_min(Lm, blockIdx.x, m);
+    } else {
+        __syncthreads();
+    }
+
+    // faces that other launches read: all of a fix-up block's, else those beside a coarser block
+    auto put = [&](const Q4<T>& f, bool xface, int i) {
+        (xface ? F.Fhu : F.Fhv)[i] = f.a;
+        (xface ? F.Fqux : F.Fqvy)[i] = f.b;
+        (xface ? F.Su : F.Sv)[i] = f.c;
+        (xface ? F.Fqvx : F.Fquy)[i] = f.d;
+    };
+    if (fix || (cs[SL] && x == 0)) put(Fl, true, c);
+    if (fix || (cs[SB] && y == 0)) put(Fb, false, c);
+    if (edge && (fix || (ex ? cs[SR] : cs[ST]))) put(Fe, ex, ex ? memloc(BW, j, ib) : memloc(j, BW, ib));
+    if (fix) return;
+
+    const Q4<T> Fr = S.fx[fxi(x + 1, y)], Ft = S.fy[fyi(x, y + 1)];
+    T Fhl = Fl.a, Fhr = Fr.a, Fql = Fl.b, Sr = Fr.c;
+    T Fhb = Fb.a, Fht = Ft.a, Fqb = Fb.b, St = Ft.c;
+    if ((info[0] & REC_EDGE) && blk_btype(P, ib) == 0) {
+        // walls (noslipbndQ, src/Boundary.cu:1887-1891): no mass flux through the boundary face and no
+        // normal-momentum flux difference in the edge cell
+        if (x == 0 && (nb[0] == ib || nb[1] == ib)) { Fhl = T(0.0); Sr = Fql; }
+        if (x == BW - 1 && (nb[2] == ib || nb[3] == ib)) { Fhr = T(0.0); Fql = Sr; }
+        if (y == 0 && (nb[4] == ib || nb[5] == ib)) { Fhb = T(0.0); St = Fqb; }
+        if (y == BW - 1 && (nb[6] == ib || nb[7] == ib)) { Fht = T(0.0); Fqb = St; }
+    }
+    T dh, dhu, dhv;
+    amr_tendencies<T, SPH>(P, delta, h0, u0, v0, Fhl, Fhr, Fhb, Fht, Fql, Sr, Fqb, St, Fb.d, Ft.d, Fl.d, Fr.d, ib, x, y,
+                           dh, dhu, dhv);
+    if (corr) {
+        amr_update<T>(P, A, X, dh, dhu, dhv, Lm, 1, c, ib, x, y);
+    } else {
+        const int k = ib * BSI + t;
+        D.dh[k] = dh;
+        D.dhu[k] = dhu;
+        D.dhv[k] = dhv;
+    }
 }
 
-// The cell values besides the faces are loaded before the fix-up's barrier,
-// and before the run flag is known.
+// The fix-up of a block's stored faces (beside finer blocks: the finer
+// neighbours' faces, which no launch of this kernel writes; on the domain
+// edge), then its advance.
 template <class T, bool SPH>
-__global__ __launch_bounds__(256) void k_amr_fix_advance(KParams P, StageIn<T> E0, const T* zb, AdvArgs<T> A,
-                                                         FluxOut<T> F, DevLoop* L, int corr) {
-    const int ib = P.active[blockIdx.x];
+__device__ __forceinline__ void fix_advance(const KParams& P, const StageIn<T>& E0, const AdvArgs<T>& A,
+                                            const FluxOut<T>& F, const DevLoop* L, int corr, int t, int ib) {
+    const int x = t & 15, y = t >> 4;
+    const int i = memloc(x, y, ib), ir = memloc(x + 1, y, ib), it = memloc(x, y + 1, ib);
+    const AdvIn<T> X = adv_load(A, i, corr);
+    const T h = A.h[i], u = A.u[i], v = A.v[i];
+    if (!L->go) return;  // the workgroup's one block: all threads leave together
+    if (t < 64) amr_fluxfix_side<T>(P, F, E0, A.zb, L, corr, t >> 4, t & 15, ib);
+    __syncthreads();
+    T dh, dhu, dhv;
+    amr_tendencies<T, SPH>(P, calcres(T(P.delta0), P.level[ib]), h, u, v, F.Fhu[i], F.Fhu[ir], F.Fhv[i], F.Fhv[it],
+                           F.Fqux[i], F.Su[ir], F.Fqvy[i], F.Sv[it], F.Fquy[i], F.Fquy[it], F.Fqvx[i], F.Fqvx[ir], ib, x,
+                           y, dh, dhu, dhv);
+    amr_update<T>(P, A, X, dh, dhu, dhv, L, corr, i, ib, x, y);
+}
+
+// The predictor's advance, after the dt reduction: U* = U + dt/2 L(U) from the
+// stored tendencies, or from the fixed-up faces.
+template <class T, bool SPH>
+__global__ __launch_bounds__(256) void k_amr_advance(KParams P, StageIn<T> E0, AdvArgs<T> A, FluxOut<T> F, Tend<T> D,
+                                                     DevLoop* L) {
+    const int ib = ldu(P.active, xcd_range(blockIdx.x % NXCD, P.nblk).start + blockIdx.x / NXCD);
     const DevLoop* Lm = loop_of(P, L, ib);
     const int t = threadIdx.x;
-    const AdvIn<T> X = adv_load(A, memloc(t & 15, t >> 4, ib), corr);
-    if (!Lm->go) return;  // the workgroup's one block: all threads leave together
-    if (t < 64) amr_fluxfix_side<T>(P, F, E0, zb, Lm, corr, t >> 4, t & 15, ib);
-    __syncthreads();
-    amr_advance<T, SPH>(P, A, X, F, Lm, corr, t, ib);
+    if (fix_block(P, ldu(P.nbr, ib * NBR + 8))) {
+        fix_advance<T, SPH>(P, E0, A, F, Lm, 0, t, ib);
+        return;
+    }
+    const int i = memloc(t & 15, t >> 4, ib), k = ib * BSI + t;
+    const AdvIn<T> X = adv_load(A, i, 0);
+    const T dh = D.dh[k], dhu = D.dhu[k], dhv = D.dhv[k];
+    if (!Lm->go) return;
+    amr_update<T>(P, A, X, dh, dhu, dhv, Lm, 0, i, ib, t & 15, t >> 4);
 }
 
-template <class T, bool FAST>
-void stage(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int corr, hipStream_t st) {
-    const T* h = corr ? B.ho : B.h;
-    const T* u = corr ? B.uo : B.u;
-    const T* v = corr ? B.vo : B.v;
-    T* hw = const_cast<T*>(h);
-    T* uw = const_cast<T*>(u);
-    T* vw = const_cast<T*>(v);
+// The corrector's fix-up and advance of the blocks that the stage left out.
+template <class T, bool SPH>
+__global__ __launch_bounds__(256) void k_amr_fix_advance(KParams P, StageIn<T> E0, AdvArgs<T> A, FluxOut<T> F,
+                                                         DevLoop* L) {
+    const int ib = ldu(P.fix, blockIdx.x);
+    fix_advance<T, SPH>(P, E0, A, F, loop_of(P, L, ib), 1, threadIdx.x, ib);
+}
+
+template <class T, bool SPH, bool FAST, int corr>
+void stage(const KParams& P, const AmrBuffers<T>& B, const AdvArgs<T>& A, DevLoop* L, hipStream_t st) {
+    T* h = const_cast<T*>(A.h);
+    T* u = const_cast<T*>(A.u);
+    T* v = const_cast<T*>(A.v);
     const FluxOut<T> F{B.Fhu, B.Fqux, B.Su, B.Fqvx, B.Fhv, B.Fqvy, B.Sv, B.Fquy};
+    const Tend<T> D{B.dh, B.dhu, B.dhv};
     const dim3 quad((P.nblk + 3) / 4), blk(P.nblk), tpb(256);
-    const bool prolong = P.wetdryfix && P.maxlevel > P.minlevel;
-    hipLaunchKernelGGL(k_amr_halo_refine<T>, blk, dim3(64), 0, st, P, hw, uw, vw, B.zb,
-                       prolong ? B.hsnap : (T*)nullptr, L, corr);
-    // the wet/dry prolongation of the levels above minlevel + 1, coarsest first
-    if (prolong)
+    // With up to three levels the stage forms the halos itself: a block's prolongation depends on at
+    // most its coarse neighbour's, which it evaluates again.  With more levels that chain is longer:
+    // the halos are filled by a launch of their own and prolonged level by level, coarsest first.
+    if (P.wetdryfix && P.maxlevel - P.minlevel > 2) {
+        hipLaunchKernelGGL(k_amr_halo_refine<T>, blk, dim3(64), 0, st, P, h, u, v, B.zb, B.hsnap, L, corr);
         for (int lev = P.minlevel + 2; lev <= P.maxlevel; lev++)
-            hipLaunchKernelGGL(k_amr_prolong<T>, quad, tpb, 0, st, P, hw, B.zb, (const T*)B.hsnap, lev, L, corr);
-    const StageIn<T> E{h, u, v};
-    // Cartesian grids: the metric terms are the constant 1 and their divisions fold away
-    if (P.spherical)
-        hipLaunchKernelGGL((k_amr_grad_flux<T, true, FAST>), blk, tpb, 0, st, P, E, (const T*)B.zb, F, L, corr);
-    else hipLaunchKernelGGL((k_amr_grad_flux<T, false, FAST>), blk, tpb, 0, st, P, E, (const T*)B.zb, F, L, corr);
+            hipLaunchKernelGGL(k_amr_prolong<T>, quad, tpb, 0, st, P, h, B.zb, (const T*)B.hsnap, lev, L, corr);
+        hipLaunchKernelGGL((k_amr_stage<T, SPH, FAST, false, corr>), blk, tpb, 0, st, P, A, B.zb, F, D, L);
+    } else {
+        hipLaunchKernelGGL((k_amr_stage<T, SPH, FAST, true, corr>), blk, tpb, 0, st, P, A, B.zb, F, D, L);
+    }
 }
 
-template <class T, bool FAST>
+// Four launches and the dt reduction: the predictor's stage, its advance, the
+// corrector's stage with its advance, and the blocks whose faces wait for
+// their finer neighbours'.
+template <class T, bool SPH, bool FAST>
 void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int advance_time, hipStream_t st, hipEvent_t* ev) {
     const dim3 blk(P.nblk), tpb(256);
     const FluxOut<T> F{B.Fhu, B.Fqux, B.Su, B.Fqvx, B.Fhv, B.Fqvy, B.Sv, B.Fquy};
+    const Tend<T> D{B.dh, B.dhu, B.dhv};
+    // the face fix-ups read the step-start state in both stages
+    const StageIn<T> E0{B.h, B.u, B.v};
     if (!P.sid) launch_rain_now(P, L, st);  // batch members take no maps, rivers or level maps
     if (ev) (void)hipEventRecord(ev[0], st);
-    stage<T, FAST>(P, B, L, 0, st);
+    // predictor: evolv_o = evolv + dt/2 L(evolv)
+    const AdvArgs<T> a0{B.h, B.u, B.v, B.h, B.u, B.v, B.ho, B.uo, B.vo, B.zb, B.cf};
+    stage<T, SPH, FAST, 0>(P, B, a0, L, st);
     if (ev) (void)hipEventRecord(ev[1], st);
     launch_reduce_dt(sizeof(T) == 8 ? 0 : 1, L, P.sid ? P.nmember : 1, advance_time, st);
     if (ev) (void)hipEventRecord(ev[2], st);
-    // the face fix-ups read the step-start state in both stages
-    const StageIn<T> E0{B.h, B.u, B.v};
-    // predictor: evolv_o = evolv + dt/2 L(evolv)
-    AdvArgs<T> a0{B.h, B.u, B.v, B.h, B.u, B.v, B.ho, B.uo, B.vo, B.zb, B.cf};
-    if (P.spherical) hipLaunchKernelGGL((k_amr_fix_advance<T, true>), blk, tpb, 0, st, P, E0, (const T*)B.zb, a0, F, L, 0);
-    else hipLaunchKernelGGL((k_amr_fix_advance<T, false>), blk, tpb, 0, st, P, E0, (const T*)B.zb, a0, F, L, 0);
+    hipLaunchKernelGGL((k_amr_advance<T, SPH>), blk, tpb, 0, st, P, E0, a0, F, D, L);
     // corrector: evolv = friction(evolv + dt L(evolv_o)) + rain
-    stage<T, FAST>(P, B, L, 1, st);
-    AdvArgs<T> a1{B.ho, B.uo, B.vo, B.h, B.u, B.v, B.h, B.u, B.v, B.zb, B.cf};
-    if (P.spherical) hipLaunchKernelGGL((k_amr_fix_advance<T, true>), blk, tpb, 0, st, P, E0, (const T*)B.zb, a1, F, L, 1);
-    else hipLaunchKernelGGL((k_amr_fix_advance<T, false>), blk, tpb, 0, st, P, E0, (const T*)B.zb, a1, F, L, 1);
+    const AdvArgs<T> a1{B.ho, B.uo, B.vo, B.h, B.u, B.v, B.h, B.u, B.v, B.zb, B.cf};
+    stage<T, SPH, FAST, 1>(P, B, a1, L, st);
+    if (P.nfix > 0) hipLaunchKernelGGL((k_amr_fix_advance<T, SPH>), dim3(P.nfix), tpb, 0, st, P, E0, a1, F, L);
     if (ev) (void)hipEventRecord(ev[3], st);
+}
+
+template <class T, bool FAST>
+void amr_step(const KParams& P, const void* buffers, DevLoop* L, int advance_time, hipStream_t st, hipEvent_t* ev) {
+    const AmrBuffers<T>& B = *(const AmrBuffers<T>*)buffers;
+    // Cartesian grids: the metric terms are the constant 1 and their products fold away
+    if (P.spherical) amr_step<T, true, FAST>(P, B, L, advance_time, st, ev);
+    else amr_step<T, false, FAST>(P, B, L, advance_time, st, ev);
 }
 
 }  // namespace
@@ -1194,9 +1488,9 @@ void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int advance_
 void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLoop* L, int advance_time,
                      hipStream_t st, hipEvent_t* ev) {
     // BGF_FP32_FAST and BGF_FP32_COMP take the fast flux arithmetic (no compensated update here)
-    if (precision == 0) amr_step<double, false>(P, *(const AmrBuffers<double>*)buffers, L, advance_time, st, ev);
-    else if (precision == 1) amr_step<float, false>(P, *(const AmrBuffers<float>*)buffers, L, advance_time, st, ev);
-    else amr_step<float, true>(P, *(const AmrBuffers<float>*)buffers, L, advance_time, st, ev);
+    if (precision == 0) amr_step<double, false>(P, buffers, L, advance_time, st, ev);
+    else if (precision == 1) amr_step<float, false>(P, buffers, L, advance_time, st, ev);
+    else amr_step<float, true>(P, buffers, L, advance_time, st, ev);
 }
 
 __global__ __launch_bounds__(256) void k_amr_nbr(KParams P, int* nbr, int nbm) {
@@ -1206,14 +1500,17 @@ __global__ __launch_bounds__(256) void k_amr_nbr(KParams P, int* nbr, int nbm) {
                       P.BotLeft[b], P.BotRight[b], P.TopLeft[b], P.TopRight[b]};
     // the first-half neighbour arrays of the sides facing back: right, left, top, bottom
     const int* const back[4] = {P.RightBot, P.LeftBot, P.TopLeft, P.BotLeft};
-    int info[8];
+    int info[8], flags = 0;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
         const bool in = (unsigned)n[k] < (unsigned)nbm;  // unused slots may hold anything
         const int lev = in ? P.level[n[k]] : 0;
         const int bk = in && back[k >> 1][n[k]] == b ? 1 : 0;
-        info[k] = (lev & 0xff) | (bk << 8);
+        info[k] = (lev & 0xff) | (bk ? REC_BACK : 0);
+        flags |= (in && lev > P.level[b] ? REC_FINER : 0) | (n[k] == b ? REC_EDGE : 0);
     }
+#pragma unroll
+    for (int k = 0; k < 8; k++) info[k] |= flags;
     int4* r = (int4*)(nbr + NBR * (size_t)b);
     r[0] = make_int4(n[0], n[1], n[2], n[3]);
     r[1] = make_int4(n[4], n[5], n[6], n[7]);

@@ -37,6 +37,8 @@ struct Member {
     int nblkmem = 0;  // block slots
     std::vector<int> active;  // global block ids, in the member's own active order
     std::vector<int> order;   // global block ids, tiled processing order
+    std::vector<int> fix;     // multi-level: global ids of the blocks that wait for others' faces
+    bool fix_all = false;
     BlockXY xy;               // block coordinates (global ids), for re-tiling
     double rain = 0.0;
     std::vector<int> gauges;  // global cell indices
@@ -82,6 +84,7 @@ struct bgf_batch_s {
     bool amr = false;
     int* d_inv = nullptr;
     int* d_nbr = nullptr;
+    int* d_fix = nullptr;
     void* d_amr[11] = {nullptr};  // as a handle's: 2-9 face fluxes, 10 hsnap (0-1, remesh staging, unused)
     // the persistent kernels walk only the blocks of members still running:
     // their processing order, launch parameters, and the members it was built for
@@ -103,7 +106,7 @@ void free_batch(bgf_batch b) {
     F(b->d_zb); F(b->d_cf); F(b->d_dh); F(b->d_dhu); F(b->d_dhv); F(b->d_hmax); F(b->d_ch);
     F(b->d_volpart); F(b->d_volout); F(b->d_gcell); F(b->d_gval); F(b->d_loop);
     F(b->d_ring); F(b->d_tring);
-    F(b->d_inv); F(b->d_nbr);
+    F(b->d_inv); F(b->d_nbr); F(b->d_fix);
     for (int k = 0; k < 11; k++) F(b->d_amr[k]);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -169,7 +172,19 @@ bgf_status prepare_run(bgf_batch b) {
     b->krun = b->kp;
     b->krun.nblk = (int)order.size();
     b->krun.hmax = b->track_max ? (float*)b->d_hmax : nullptr;
-    if (b->amr) b->krun.active = b->d_order;  // the multi-level kernels walk the running members' active lists
+    if (b->amr) {
+        b->krun.active = b->d_order;  // the multi-level kernels walk the running members' active lists
+        bool all = false;
+        for (int m : running) all = all || b->members[m].fix_all;
+        std::vector<int> fix = all ? order : std::vector<int>();
+        for (int m : running)
+            if (!all) fix.insert(fix.end(), b->members[m].fix.begin(), b->members[m].fix.end());
+        if (!fix.empty())
+            HIPCHK(hipMemcpy(b->d_fix, fix.data(), sizeof(int) * fix.size(), hipMemcpyHostToDevice));
+        b->krun.fix = b->d_fix;
+        b->krun.nfix = (int)fix.size();
+        b->krun.fix_all = all ? 1 : 0;
+    }
     if (!order.empty() && !b->amr) {
         b->krun.grid_pred = bgf::persistent_grid(b->prec, 0, b->krun.nblk, b->wg_pred);
         b->krun.grid_corr = bgf::persistent_grid(b->prec, 1, b->krun.nblk, b->wg_corr);
@@ -216,6 +231,7 @@ template <class T> void fill_amr(bgf_batch b, bgf::AmrBuffers<T>* B) {
     T** f[8] = {&B->Fhu, &B->Fqux, &B->Su, &B->Fqvx, &B->Fhv, &B->Fqvy, &B->Sv, &B->Fquy};
     for (int k = 0; k < 8; k++) *f[k] = (T*)b->d_amr[2 + k];
     B->hsnap = (T*)b->d_amr[10];
+    B->dh = (T*)b->d_dh; B->dhu = (T*)b->d_dhu; B->dhv = (T*)b->d_dhv;
 }
 
 void enqueue_steps(bgf_batch b, int nsteps) {
@@ -308,7 +324,8 @@ bgf_status bgf_batch_create(const bgf_param* common, int max_blocks, int max_mem
          A((void**)&b->d_tring, sizeof(double) * NSAMP * max_members);
     b->amr = common->maxlevel > common->minlevel;
     if (b->amr) {
-        ok = ok && A((void**)&b->d_inv, sizeof(int) * max_blocks) && A((void**)&b->d_nbr, sizeof(int) * bgf::NBR * (size_t)max_blocks);
+        ok = ok && A((void**)&b->d_inv, sizeof(int) * max_blocks) && A((void**)&b->d_nbr, sizeof(int) * bgf::NBR * (size_t)max_blocks) &&
+             A((void**)&b->d_fix, sizeof(int) * (size_t)max_blocks);
         for (int k = 2; k < 11; k++) ok = ok && A(&b->d_amr[k], b->es * b->S);
     }
     if (!ok) {
@@ -425,6 +442,10 @@ bgf_status bgf_batch_add(bgf_batch b, const bgf_param* p, const bgf_blocks* blk,
     for (int k = 0; k < nblk; k++) M.active.push_back(off + blk->active[k]);
     if (b->amr) {
         M.order = M.active;  // the multi-level kernels keep the member's active order
+        const int* nbs[8] = {blk->LeftBot, blk->LeftTop, blk->RightBot, blk->RightTop,
+                             blk->TopLeft, blk->TopRight, blk->BotLeft, blk->BotRight};
+        M.fix = fix_blocks(blk->active, nblk, blk->level, nbs, false, M.fix_all);
+        for (int& ib : M.fix) ib += off;
     } else {
         M.xy = block_xy(blk, nblk, p->dx);
         for (int& ib : M.xy.id) ib += off;

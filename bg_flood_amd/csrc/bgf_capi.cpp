@@ -57,6 +57,7 @@ struct bgf_handle_s {
     bool cf_shared = false;  // the caller holds the cf device array
     int *d_nb[8] = {nullptr};  // LeftBot LeftTop RightBot RightTop TopLeft TopRight BotLeft BotRight
     int* d_nbr = nullptr;      // multi-level meshes: the neighbour record of each block slot (bgf::NBR ints)
+    int* d_fix = nullptr;      // and the blocks whose advance waits for other blocks' faces
     void *d_h[2] = {nullptr, nullptr}, *d_u[2] = {nullptr, nullptr}, *d_v[2] = {nullptr, nullptr};
     void *d_zb = nullptr, *d_cf = nullptr, *d_dh = nullptr, *d_dhu = nullptr, *d_dhv = nullptr;
     double *d_volpart = nullptr, *d_volout = nullptr;
@@ -136,7 +137,7 @@ void free_handle(bgf_handle h) {
     F(h->d_active); F(h->d_order); F(h->d_level); F(h->d_queue); F(h->d_rec);
     for (int k = 0; k < 15; k++) F(h->stats.a[k]);
     for (int k = 0; k < 8; k++) F(h->d_nb[k]);
-    F(h->d_nbr);
+    F(h->d_nbr); F(h->d_fix);
     for (int k = 0; k < 2; k++) { F(h->d_h[k]); F(h->d_u[k]); F(h->d_v[k]); }
     F(h->d_zb); F(h->d_cf); F(h->d_dh); F(h->d_dhu); F(h->d_dhv);
     F(h->d_volpart); F(h->d_volout); F(h->d_loop);
@@ -232,6 +233,7 @@ template <class T> void fill_amr_t(bgf_handle h, bgf::AmrBuffers<T>* B) {
     T** f[8] = {&B->Fhu, &B->Fqux, &B->Su, &B->Fqvx, &B->Fhv, &B->Fqvy, &B->Sv, &B->Fquy};
     for (int k = 0; k < 8; k++) *f[k] = (T*)h->d_amr[2 + k];
     B->hsnap = (T*)h->d_amr[10];
+    B->dh = (T*)h->d_dh; B->dhu = (T*)h->d_dhu; B->dhv = (T*)h->d_dhv;
 }
 
 void fill_amr_buffers(bgf_handle h, void* storage) {
@@ -393,6 +395,20 @@ bool upload_metric(bgf_handle h, const bgf_param* p, const bgf_blocks* b, int nb
     return hipMemcpy(h->d_metric, M.data(), sizeof(float) * M.size(), hipMemcpyHostToDevice) == hipSuccess;
 }
 
+// The blocks of the handle's current mesh that the multi-level step advances
+// after the others (fix_blocks), for the current boundary segments.
+bgf_status setup_fix(bgf_handle h) {
+    if (!h->amr) return BGF_OK;
+    bool all = false;
+    const std::vector<int> list =
+        fix_blocks(h->active.data(), h->nblk, h->h_level.data(), h->h_nb, h->kp.bopen != 0, all);
+    if (!list.empty()) HIPCHK(hipMemcpy(h->d_fix, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
+    h->kp.fix = h->d_fix;
+    h->kp.nfix = (int)list.size();
+    h->kp.fix_all = all ? 1 : 0;
+    return BGF_OK;
+}
+
 // The boundary segments on the handle's current mesh: the segment of each
 // boundary block (assign_segments; the side strips from the mesh's extent,
 // XParam.xmax = Param.xo + the right edge of the easternmost block as
@@ -412,7 +428,7 @@ bgf_status setup_segments(bgf_handle h) {
         (void)hipGraphExecDestroy(h->graph);
         h->graph = nullptr;
     }
-    if (h->segs.empty()) return BGF_OK;
+    if (h->segs.empty()) return setup_fix(h);
     const bgf_param& p = h->p;
     auto inT = [&](double v) { return h->prec == 0 ? v : (double)(float)v; };  // XBlock.xo is a T
     double xmax = -1e300, ymax = -1e300;
@@ -461,7 +477,7 @@ bgf_status setup_segments(bgf_handle h) {
     kp.bseg = h->d_bseg;
     kp.seg = h->d_seg;
     kp.nseg = (int)tab.size();
-    return BGF_OK;
+    return setup_fix(h);
 }
 
 // The rivers on the handle's current mesh (InitialConditions.cu:346-445):
@@ -602,6 +618,7 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     if (multilevel) {
         ok = ok && A((void**)&h->d_inv, sizeof(int) * cap);
         ok = ok && A((void**)&h->d_nbr, sizeof(int) * bgf::NBR * (size_t)cap);
+        ok = ok && A((void**)&h->d_fix, sizeof(int) * cap);
         for (int k = 0; k < 11; k++) ok = ok && A(&h->d_amr[k], h->es * SA);
     }
     if (!ok) {
@@ -676,6 +693,11 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     kp.byo = h->d_blkyo;
     kp.nbr = h->d_nbr;
     if (multilevel) bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->stream);
+    s = setup_fix(h);
+    if (s != BGF_OK) {
+        free_handle(h);
+        return s;
+    }
     bgf::launch_records(kp, h->d_rec, h->stream);
     if (hipGetLastError() != hipSuccess) {
         free_handle(h);
@@ -1618,8 +1640,10 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
     if (!h->segs.empty()) {
         HIPCHK(hipStreamSynchronize(h->stream));
         s = setup_segments(h);  // the boundary blocks of the new mesh
-        if (s != BGF_OK) return s;
+    } else {
+        s = setup_fix(h);
     }
+    if (s != BGF_OK) return s;
     // the bed's halo on the new mesh (src/InitialConditions.cu:135-147)
     bgf::launch_amr_fill(prec, kp, h->d_zb, h->stream);
     // the statistics restart on the new mesh

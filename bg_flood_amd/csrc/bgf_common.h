@@ -15,6 +15,62 @@ constexpr int BSI = BW * BW; // values per block of the interior-only tendency a
 // src/MemManagement.cu:37-40
 __device__ __forceinline__ int memloc(int i, int j, int ib) { return (i + 1) + (j + 1) * MW + ib * BS; }
 
+// LDS pitches.  128-bit accesses of 16-lane rows are free of bank conflicts
+// on gfx950 only at pitches of 16 or 32 entries (17 to 24 cost 4 conflict
+// cycles per read, measured with SQ_LDS_BANK_CONFLICT), so the arrays that are
+// only read by rows (y slopes, Y faces) are 16 wide; the others, which also
+// take column accesses (halo strips, the ring, the 17th faces), keep odd
+// pitches.
+constexpr int TP = 21;  // tile: x, y in [-2, 17]
+constexpr int GXP = 19; // x slopes: x in [-1, 16], y in [0, 15]
+constexpr int GYP = 16; // y slopes: x in [0, 15], y in [-1, 16]
+constexpr int FP = 17;  // X faces xf in [0, 16], y in [0, 15]
+constexpr int FYP = 16; // Y faces x in [0, 15], yf in [0, 16]
+
+__device__ __forceinline__ int tix(int x, int y) { return (y + 2) * TP + (x + 2); }
+__device__ __forceinline__ int gxi(int x, int y) { return y * GXP + (x + 1); }
+__device__ __forceinline__ int gyi(int x, int y) { return (y + 1) * GYP + x; }
+__device__ __forceinline__ int fxi(int xf, int y) { return y * FP + xf; }
+__device__ __forceinline__ int fyi(int x, int yf) { return yf * FYP + x; }
+
+// fmin/fmax (v_min/v_max, fused into v_min3/v_max3).  They differ from the
+// reference's std::min/std::max only for NaN operands and in the sign of a
+// zero result, neither of which changes any value of the step.
+__device__ __forceinline__ float dmax(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ float dmin(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ double dmax(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ double dmin(double a, double b) { return fmin(a, b); }
+
+// A cell's (h, zs, u, v), a cell's four gradients, or a face's four fluxes.
+template <class T> struct alignas(4 * sizeof(T)) Q4 {
+    T a, b, c, d;
+};
+
+// Block indices are workgroup-uniform: read them through the constant address
+// space so they become scalar loads, which do not wait behind the vector
+// loads of the prefetch.
+__device__ __forceinline__ int ldu(const int* p, int i) {
+    return ((const __attribute__((address_space(4))) int*)p)[i];
+}
+__device__ __forceinline__ double lds_f64(const double* p) {
+    return *(const __attribute__((address_space(4))) double*)p;
+}
+__device__ __forceinline__ float lds_f32(const float* p) {
+    return *(const __attribute__((address_space(4))) float*)p;
+}
+// The contiguous range of n positions that XCD xcd takes: workgroup b of a
+// launch of n workgroups runs on XCD b % NXCD and is the (b / NXCD)-th there.
+struct Range {
+    int start, end;
+};
+__device__ __forceinline__ Range xcd_range(int xcd, int n) {
+    const int per = n / NXCD, rem = n % NXCD;
+    Range R;
+    R.start = xcd * per + (xcd < rem ? xcd : rem);
+    R.end = R.start + per + (xcd < rem ? 1 : 0);
+    return R;
+}
+
 // Division and square root: IEEE in EXACT kernels, hardware approximations in FAST ones.
 template <class T, bool FAST> struct Ar {
     __device__ static __forceinline__ T rcp(T a) { return T(1.0) / a; }

@@ -297,6 +297,35 @@ inline bgf_status quadtree_neighbours(int n, const int* id, const int* lev, cons
     return BGF_OK;
 }
 
+// The blocks of a multi-level mesh whose advance waits for other blocks'
+// faces: those beside a finer block, and those on the domain edge when some
+// boundary segment is open (edges).  nb: the eight neighbour arrays in the
+// order LeftBot, LeftTop, RightBot, RightTop, TopLeft, TopRight, BotLeft,
+// BotRight.  The kernels leave a finer block's shared faces to its coarser
+// neighbour by what the finer block's own record says; a block list whose two
+// records disagree (all) has every block wait, with all its faces stored.
+template <class Nb>
+inline std::vector<int> fix_blocks(const int* active, int nblk, const int* level, const Nb& nb, bool edges, bool& all) {
+    static const int facing[8] = {2, 2, 0, 0, 6, 6, 4, 4};
+    std::vector<int> list;
+    all = false;
+    for (int k = 0; k < nblk; k++) {
+        const int ib = active[k];
+        bool wait = false;
+        for (int q = 0; q < 8; q++) {
+            const int n = nb[q][ib];
+            if (level[n] > level[ib]) {
+                wait = true;
+                if (nb[facing[q]][n] != ib || nb[facing[q] + 1][n] != ib) all = true;
+            }
+            if (edges && n == ib) wait = true;
+        }
+        if (wait) list.push_back(ib);
+    }
+    if (all) list.assign(active, active + nblk);
+    return list;
+}
+
 // ------------------------------------------------------------ boundary segments
 // A polygon (src/Input.h:107-111): closed vertex list and bounding box.
 struct Polygon {

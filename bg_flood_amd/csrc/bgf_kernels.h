@@ -98,7 +98,12 @@ struct KParams {
                           // neighbours LeftBot, LeftTop, RightBot, RightTop, BotLeft, BotRight,
                           // TopLeft, TopRight, then for each of them its level (low 8 bits, signed)
                           // and, in bit 8, whether the block is the first-half neighbour of the
-                          // neighbour's side facing it
+                          // neighbour's side facing it, and of the block itself, in every one of
+                          // them, whether it has a finer neighbour and a side on the domain edge
+    // multi-level meshes: the active blocks whose advance waits for other blocks' faces
+    // (nfix of them; fix_all: every block does)
+    const int* fix;
+    int nfix, fix_all;
     int minlevel, maxlevel;  // levels present among the active blocks
     // batches of domains: member of each block (DevLoop of that member), member count
     const int* sid;
@@ -216,7 +221,8 @@ template <class T> struct AmrBuffers {
     T* zb;            // its halo is written by the halo fill and the wet/dry prolongation
     const T* cf;
     T *Fhu, *Fqux, *Su, *Fqvx, *Fhv, *Fqvy, *Sv, *Fquy;  // face fluxes (no slope is stored)
-    T* hsnap;         // h before the wet/dry prolongation
+    T* hsnap;         // h before the wet/dry prolongation (meshes of four levels and more)
+    T *dh, *dhu, *dhv; // tendencies, interior cells only
 };
 // One step on a multi-level mesh: precision 0 FP64 and 1 FP32 in the reference
 // arithmetic; 2 and 3 (BGF_FP32_FAST, BGF_FP32_COMP) FP32 with hardware
@@ -226,6 +232,8 @@ void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLo
 // Fills nbr (NBR ints per block slot, nbm slots) from P's eight neighbour arrays
 // and the levels; slots whose neighbours are outside [0, nbm) get level 0.
 constexpr int NBR = 16;
+// Flags beside the level (low 8 bits) in a record's level words.
+enum { REC_BACK = 1 << 8, REC_FINER = 1 << 9, REC_EDGE = 1 << 10 };
 void launch_amr_nbr(const KParams& P, int* nbr, int nbm, hipStream_t st);
 // Halo of a static field (the bed) on a multi-level mesh, src/InitialConditions.cu:135-147.
 void launch_amr_fill(int precision, const KParams& P, void* z, hipStream_t st);

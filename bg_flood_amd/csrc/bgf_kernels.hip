@@ -53,38 +53,6 @@
 
 namespace bgf {
 
-// LDS pitches.  128-bit accesses of 16-lane rows are free of bank conflicts
-// on gfx950 only at pitches of 16 or 32 entries (17 to 24 cost 4 conflict
-// cycles per read, measured with SQ_LDS_BANK_CONFLICT), so the arrays that are
-// only read by rows (y slopes, Y faces) are 16 wide; the others, which also
-// take column accesses (halo strips, the ring, the 17th faces), keep odd
-// pitches.
-constexpr int TP = 21;  // tile: x, y in [-2, 17]
-constexpr int GXP = 19; // x slopes: x in [-1, 16], y in [0, 15]
-constexpr int GYP = 16; // y slopes: x in [0, 15], y in [-1, 16]
-constexpr int FP = 17;  // X faces xf in [0, 16], y in [0, 15]
-constexpr int FYP = 16; // Y faces x in [0, 15], yf in [0, 16]
-
-__device__ __forceinline__ int tix(int x, int y) { return (y + 2) * TP + (x + 2); }
-__device__ __forceinline__ int gxi(int x, int y) { return y * GXP + (x + 1); }
-__device__ __forceinline__ int gyi(int x, int y) { return (y + 1) * GYP + x; }
-__device__ __forceinline__ int fxi(int xf, int y) { return y * FP + xf; }
-__device__ __forceinline__ int fyi(int x, int yf) { return yf * FYP + x; }
-
-// fmin/fmax (v_min/v_max, fused into v_min3/v_max3).  They differ from the
-// reference's std::min/std::max only for NaN operands and in the sign of a
-// zero result, neither of which changes any value of the step.
-__device__ __forceinline__ float dmax(float a, float b) { return fmaxf(a, b); }
-__device__ __forceinline__ float dmin(float a, float b) { return fminf(a, b); }
-__device__ __forceinline__ double dmax(double a, double b) { return fmax(a, b); }
-__device__ __forceinline__ double dmin(double a, double b) { return fmin(a, b); }
-
-// A cell's (h, zs, u, v), a cell's four gradients, or a face's four fluxes.
-template <class T> struct alignas(4 * sizeof(T)) Q4 {
-    T a, b, c, d;
-};
-
-
 // src/Util_CPU.cu:243-263 without branches.  With d1 = theta*(s1-s0),
 // d2 = (s2-s0)/2, d3 = theta*(s2-s1): s0 < s1 < s2 holds exactly when
 // min(d1,d2,d3) > 0 (theta >= 1 and IEEE subtraction is zero only for equal
@@ -587,18 +555,6 @@ __device__ __forceinline__ void advance(const Cst<T>& C, int fmc, T dt, T hold, 
 // its own L2: the persistent kernels give each XCD a contiguous range of
 // blocks so a block's neighbours are mostly fetched into the same L2.
 
-// Block indices are workgroup-uniform: read them through the constant address
-// space so they become scalar loads, which do not wait behind the vector
-// loads of the prefetch.
-__device__ __forceinline__ int ldu(const int* p, int i) {
-    return ((const __attribute__((address_space(4))) int*)p)[i];
-}
-__device__ __forceinline__ double lds_f64(const double* p) {
-    return *(const __attribute__((address_space(4))) double*)p;
-}
-__device__ __forceinline__ float lds_f32(const float* p) {
-    return *(const __attribute__((address_space(4))) float*)p;
-}
 // Cell k of block ib of array a: the array base (a kernel argument, in scalar
 // registers for the whole launch) plus one 32-bit byte offset per thread that
 // carries both the block and the cell, boff(ib) + k * sizeof(T), so each load
@@ -695,16 +651,6 @@ template <class T, bool FAST> __device__ __forceinline__ void wave_flush(const C
 // own at zero: the first launch from the allocation, later ones from the
 // other kernel's launch in between (the zeroing comes before a kernel's
 // early return, and a launch that returns early takes no position).
-struct Range {
-    int start, end;
-};
-__device__ __forceinline__ Range xcd_range(int xcd, int n) {
-    const int per = n / NXCD, rem = n % NXCD;
-    Range R;
-    R.start = xcd * per + (xcd < rem ? xcd : rem);
-    R.end = R.start + per + (xcd < rem ? 1 : 0);
-    return R;
-}
 // Queue positions.  Each workgroup's positions increase (one thread's
 // atomics on one counter are ordered), so the first one past the range ends
 // the walk and no position is lost; the workgroup reads position j from slot
