@@ -630,11 +630,12 @@ template <class T> struct StageLds {
             Q4<T> gy[18 * GYP];  // slopes along y of (h, zs, v, u)
         };
         struct {
-            Q4<T> fx[16 * FP];   // X faces (Fhu, Fqux, Su, Fqvx)
-            Q4<T> fy[17 * FYP];  // Y faces (Fhv, Fqvy, Sv, Fquy)
+            Q4<T> fx[BW * BW];   // X faces (Fhu, Fqux, Su, Fqvx)
+            Q4<T> fy[BW * BW];   // Y faces (Fhv, Fqvy, Sv, Fquy)
         };
         T pt[4][4][NPT];         // h, u, v and the bed of the points
     };
+    Q4<T> fe[2 * BW];  // the seventeenth X faces, then Y faces
     T sh[4][BW], sz[4][BW];
     T red[4];
 };
@@ -649,12 +650,11 @@ template <class T> __device__ __forceinline__ T minmod2s(T theta, T s0, T s1, T 
 // The slopes of a cell's four fields between its neighbours m and p.  FAST:
 // the division by delta is a product with idelta, its hardware reciprocal.
 template <bool FAST, class T>
-__device__ __forceinline__ Q4<T> slopes4(T theta, T delta, T idelta, const Q4<T>& m, const Q4<T>& c, const Q4<T>& p) {
-    auto one = [&](T a, T b, T d) {
-        const T g = minmod2s(theta, a, b, d);
-        return FAST ? g * idelta : g / delta;
-    };
-    return Q4<T>{one(m.a, c.a, p.a), one(m.b, c.b, p.b), one(m.c, c.c, p.c), one(m.d, c.d, p.d)};
+__device__ __forceinline__ Q4<T> slopes4(T theta, const FixedDiv<T>& D, T idelta, const Q4<T>& m, const Q4<T>& c,
+                                         const Q4<T>& p) {
+    const Q4<T> g{minmod2s(theta, m.a, c.a, p.a), minmod2s(theta, m.b, c.b, p.b), minmod2s(theta, m.c, c.c, p.c),
+                  minmod2s(theta, m.d, c.d, p.d)};
+    return FAST ? Q4<T>{g.a * idelta, g.b * idelta, g.c * idelta, g.d * idelta} : div4(D, g);
 }
 
 // The h and zb of a coarser block's cell in the source term of a shared face;
@@ -694,7 +694,7 @@ __device__ __forceinline__ bool amr_face(T g, T CFL, T eps, T delta, T cm, T fm,
     const T cmo = A::sqrt_(g * hm);
     const T ap = smax(smax(up + cp, um + cmo), T(0.0));
     const T am = smin(smin(up - cp, um - cmo), T(0.0));
-    const T ad = A::rcp(ap - am);
+    const T ad = FAST ? A::rcp(ap - am) : plain_rcp(ap - am);
     const T qm = hm * um;
     const T qp = hp * up;
     const T hm2 = hm * hm;
@@ -728,14 +728,6 @@ __device__ __forceinline__ bool amr_face(T g, T CFL, T eps, T delta, T cm, T fm,
     F.c = wet ? (SPH ? fm * (fu - sr) : fu - sr) : T(0.0);
     F.d = wet ? (SPH ? fm * fv : fv) : T(0.0);
     return wet;
-}
-
-// Holds the end of a face's arithmetic in front of the next face's: the
-// compiler otherwise sinks it past the barrier to the stores, and the operands
-// of three faces outgrow the registers that the occupancy allows (83 VGPRs in
-// FP32 and 163 in FP64 against 60 and 110).
-template <class T> __device__ __forceinline__ void finish(Q4<T>& F) {
-    asm volatile("" : "+v"(F.a), "+v"(F.b), "+v"(F.c), "+v"(F.d));
 }
 
 // Metric terms of the faces of row y: cm of its X faces, cm and fm of the Y
@@ -875,13 +867,7 @@ __device__ __forceinline__ void amr_update(const KParams& P, const AdvArgs<T>& A
     const T g = T(P.g);
     const T eps = T(P.eps);
     const T hold = X.hold;
-    T edt;
-    if (P.ForceMassConserve || dhi >= T(0.0)) {
-        edt = dt;
-    } else {
-        const double lim = smax((double)hold, P.eps) / (double)fabs(dhi);
-        edt = T(smin((double)dt, lim));
-    }
+    const T edt = P.ForceMassConserve ? dt : dry_step(dt, hold, dhi, eps, P.eps);
     T ho = hold + edt * dhi, uo, vo;
     if (ho > eps) {
         uo = (hold * X.uold + edt * dhu) / ho;
@@ -1100,6 +1086,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
     const T theta = T(P.theta), eps = T(P.eps);
     const T delta = calcres(T(P.delta0), lev);
     const T idelta = Ar<T, FAST>::rcp(delta);
+    const FixedDiv<T> by_delta = fixed_div(delta);
 
     // the block's own cell
     const int c = memloc(x, y, ib);
@@ -1269,9 +1256,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
     }
 
     // slopes: the thread's own cell, and the halo ring on wave 2 (lanes 0-31 along x, 32-63 along y)
-    const Q4<T> gxo = slopes4<FAST>(theta, delta, idelta, S.q[tix(x - 1, y)], q, S.q[tix(x + 1, y)]);
+    const Q4<T> gxo = slopes4<FAST>(theta, by_delta, idelta, S.q[tix(x - 1, y)], q, S.q[tix(x + 1, y)]);
     S.gx[gxi(x, y)] = gxo;
-    Q4<T> gyo = slopes4<FAST>(theta, delta, idelta, S.q[tix(x, y - 1)], q, S.q[tix(x, y + 1)]);
+    Q4<T> gyo = slopes4<FAST>(theta, by_delta, idelta, S.q[tix(x, y - 1)], q, S.q[tix(x, y + 1)]);
     {
         const T a = gyo.c;  // stored as (h, zs, v, u)
         gyo.c = gyo.d;
@@ -1282,7 +1269,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
         const bool isx = l < 32;
         const int o = (l & 16) ? BW : -1;
         const int ci = isx ? tix(o, j) : tix(j, o), d = isx ? 1 : TP;
-        const Q4<T> g = slopes4<FAST>(theta, delta, idelta, S.q[ci - d], S.q[ci], S.q[ci + d]);
+        const Q4<T> g = slopes4<FAST>(theta, by_delta, idelta, S.q[ci - d], S.q[ci], S.q[ci + d]);
         if (isx) S.gx[gxi(o, j)] = g;
         else S.gy[gyi(j, o)] = Q4<T>{g.a, g.b, g.d, g.c};
     }
@@ -1296,7 +1283,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
     };
     auto swap_uv = [](const Q4<T>& a) { return Q4<T>{a.a, a.b, a.d, a.c}; };
     const FaceMetric<T> M = face_metric<T, SPH>(P, ib, y);
-    Q4<T> Fl, Fb, Fe;
+    Q4<T> Fl, Fb;
     T lx, ly;
     const bool wx = amr_face<T, SPH, FAST>(g, CFL, epsw, delta, M.cmx, T(1.0), q, S.q[tix(x - 1, y)], gxo,
                                            S.gx[gxi(x - 1, y)], none, sub(SL, y, x == 0), Fl, lx);
@@ -1317,13 +1304,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
         SubVal<T> se = none;
         if (ex ? cs[SR] : cs[ST]) se = SubVal<T>{S.sh[ex ? SR : ST][j], S.sz[ex ? SR : ST][j], true};
         T le;
+        Q4<T> Fe;
         (void)amr_face<T, SPH, FAST>(g, CFL, epsw, delta, ex ? Me.cmx : Me.cmy, ex ? T(1.0) : Me.fmy, qi, qn, gi, gn, se,
                                      none, Fe, le);
+        S.fe[l] = Fe;
     }
     __syncthreads();  // the slopes are read: the faces take their place
-    S.fx[fxi(x, y)] = Fl;
-    S.fy[fyi(x, y)] = Fb;
-    if (edge) *(ex ? &S.fx[fxi(BW, j)] : &S.fy[fyi(j, BW)]) = Fe;
+    S.fx[t] = Fl;
+    S.fy[t] = Fb;
     if (!corr) {
         // dtmax of the cell: its X face, then its Y face, a dry face resetting it to 1/epsi
         // (src/Kurganov.cu:1488-1491); off the sphere every face has the same cell size, so the block's
@@ -1354,10 +1342,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
     };
     if (fix || (cs[SL] && x == 0)) put(Fl, true, c);
     if (fix || (cs[SB] && y == 0)) put(Fb, false, c);
-    if (edge && (fix || (ex ? cs[SR] : cs[ST]))) put(Fe, ex, ex ? memloc(BW, j, ib) : memloc(j, BW, ib));
+    if (edge && (fix || (ex ? cs[SR] : cs[ST]))) put(S.fe[l], ex, ex ? memloc(BW, j, ib) : memloc(j, BW, ib));
     if (fix) return;
 
-    const Q4<T> Fr = S.fx[fxi(x + 1, y)], Ft = S.fy[fyi(x, y + 1)];
+    const Q4<T> Fr = x < BW - 1 ? S.fx[t + 1] : S.fe[y], Ft = y < BW - 1 ? S.fy[t + BW] : S.fe[BW + x];
     T Fhl = Fl.a, Fhr = Fr.a, Fql = Fl.b, Sr = Fr.c;
     T Fhb = Fb.a, Fht = Ft.a, Fqb = Fb.b, St = Ft.c;
     if ((info[0] & REC_EDGE) && blk_btype(P, ib) == 0) {

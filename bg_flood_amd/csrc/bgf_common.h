@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <limits>
+
 #include "bgf_kernels.h"
 
 namespace bgf {
@@ -25,13 +27,10 @@ constexpr int TP = 21;  // tile: x, y in [-2, 17]
 constexpr int GXP = 19; // x slopes: x in [-1, 16], y in [0, 15]
 constexpr int GYP = 16; // y slopes: x in [0, 15], y in [-1, 16]
 constexpr int FP = 17;  // X faces xf in [0, 16], y in [0, 15]
-constexpr int FYP = 16; // Y faces x in [0, 15], yf in [0, 16]
 
 __device__ __forceinline__ int tix(int x, int y) { return (y + 2) * TP + (x + 2); }
 __device__ __forceinline__ int gxi(int x, int y) { return y * GXP + (x + 1); }
 __device__ __forceinline__ int gyi(int x, int y) { return (y + 1) * GYP + x; }
-__device__ __forceinline__ int fxi(int xf, int y) { return y * FP + xf; }
-__device__ __forceinline__ int fyi(int x, int yf) { return yf * FYP + x; }
 
 // fmin/fmax (v_min/v_max, fused into v_min3/v_max3).  They differ from the
 // reference's std::min/std::max only for NaN operands and in the sign of a
@@ -45,6 +44,14 @@ __device__ __forceinline__ double dmin(double a, double b) { return fmin(a, b); 
 template <class T> struct alignas(4 * sizeof(T)) Q4 {
     T a, b, c, d;
 };
+
+// Holds the end of a face's arithmetic in front of the next face's: the
+// compiler otherwise sinks it past the barrier to the stores, and the operands
+// of three faces outgrow the registers that the occupancy allows (83 VGPRs in
+// FP32 and 163 in FP64 against 60 and 110).
+template <class T> __device__ __forceinline__ void finish(Q4<T>& F) {
+    asm volatile("" : "+v"(F.a), "+v"(F.b), "+v"(F.c), "+v"(F.d)::"memory");
+}
 
 // Block indices are workgroup-uniform: read them through the constant address
 // space so they become scalar loads, which do not wait behind the vector
@@ -80,6 +87,78 @@ template <> struct Ar<float, true> {
     __device__ static __forceinline__ float rcp(float a) { return __builtin_amdgcn_rcpf(a); }
     __device__ static __forceinline__ float sqrt_(float a) { return __builtin_amdgcn_sqrtf(a); }
 };
+
+// Division by a fixed d with the rounding of an IEEE division, in four
+// multiply-adds instead of its eleven instructions (of which the reciprocal
+// alone takes the time of four): with zh = RN(1/d) and zl the rest of 1/d,
+// q0 = RN(x zh + RN(x zl)) is within an ulp of x/d, the remainder r = x - d q0
+// is exact in a multiply-add, and RN(q0 + r zh) is the correctly rounded
+// quotient (Markstein, IBM J. Res. Dev. 34, 1990; the two-part reciprocal is
+// that of Brisebarre and Muller).  That needs x to be zero or between lo and
+// hi, well inside the normal range, and d in [2^-20, 2^20]; other x (the
+// numerical precursors of a wave reach such sizes) are `odd` and take the
+// division itself.
+template <class T> struct FixedDiv {
+    T d, zh, zl, lo, hi;
+};
+__host__ __device__ __forceinline__ void fixed_div_range(float& lo, float& hi) { lo = 0x1p-100f; hi = 0x1p100f; }
+__host__ __device__ __forceinline__ void fixed_div_range(double& lo, double& hi) { lo = 0x1p-960; hi = 0x1p960; }
+template <class T> __host__ __device__ __forceinline__ FixedDiv<T> fixed_div(T d) {
+    FixedDiv<T> K;
+    K.d = d;
+    K.zh = T(1.0) / d;
+    K.zl = fma(-d, K.zh, T(1.0)) * K.zh;
+    fixed_div_range(K.lo, K.hi);
+    if (!(d >= T(0x1p-20) && d <= T(0x1p20))) K.lo = K.hi = std::numeric_limits<T>::infinity();
+    return K;
+}
+template <class T> __device__ __forceinline__ bool odd_div(const FixedDiv<T>& K, T x) {
+    const T a = fabs(x);
+    return (a < K.lo && x != T(0.0)) || a > K.hi;
+}
+template <class T> __device__ __forceinline__ T quick_div(const FixedDiv<T>& K, T x) {
+    const T q = fma(x, K.zh, x * K.zl);
+    return fma(fma(-K.d, q, x), K.zh, q);
+}
+// The four quotients of a Q4.
+template <class T> __device__ __forceinline__ Q4<T> div4(const FixedDiv<T>& K, const Q4<T>& x) {
+    Q4<T> q{quick_div(K, x.a), quick_div(K, x.b), quick_div(K, x.c), quick_div(K, x.d)};
+    if (__builtin_expect(odd_div(K, x.a) | odd_div(K, x.b) | odd_div(K, x.c) | odd_div(K, x.d), 0))
+        q = Q4<T>{x.a / K.d, x.b / K.d, x.c / K.d, x.d / K.d};
+    return q;
+}
+
+// 1 / b rounded as IEEE division rounds it, for b of ordinary size (here the
+// spread of a face's wave speeds, above epsilon wherever the result is used):
+// Newton steps on the hardware reciprocal and Markstein's correction, without
+// the scaling that extreme operands need.
+__device__ __forceinline__ double plain_rcp(double b) {
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(fma(-b, y, 1.0), y, y);
+    y = fma(fma(-b, y, 1.0), y, y);
+    return fma(fma(-b, y, 1.0), y, y);
+}
+__device__ __forceinline__ float plain_rcp(float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    y = fma(fma(-b, y, 1.0f), y, y);
+    y = fma(fma(-b, y, 1.0f), y, y);
+    return fma(fma(-b, y, 1.0f), y, y);
+}
+
+// The step that the drying limiter allows (src/Advection.cu:349-352):
+// min(dt, max(h, eps) / |dh|) evaluated in double, where dh < 0.  The limiter
+// binds only where max(h, eps) < dt |dh|; a product a few roundings larger
+// decides that for nearly every cell, and only the others divide.  epsT: eps
+// rounded to T, which may differ from eps in its last bit.
+template <class T> __device__ __forceinline__ T dry_step(T dt, T h, T dh, T epsT, double eps) {
+    T edt = dt;
+    if (!(dh >= T(0.0)) && !(dmax(h, epsT) > dt * -dh * T(1.0 + 0x1p-18))) {
+        const double m = (double)h < eps ? eps : (double)h;
+        const double lim = m / (double)fabs(dh);
+        edt = T(lim < (double)dt ? lim : (double)dt);
+    }
+    return edt;
+}
 
 // Workgroup minimum over 256 threads (four wave64s); every thread gets it.
 template <class T> __device__ __forceinline__ T block_min(T v, T* red, int t) {

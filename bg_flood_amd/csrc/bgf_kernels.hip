@@ -37,9 +37,9 @@
 //
 // EXACT kernels (FAST = false) perform every operation of the reference CPU
 // step in the same order and precision (this file is compiled with
-// -ffp-contract=off; divisions and square roots are IEEE), so they reproduce
-// the CPU step bit for bit.  FAST kernels use the hardware reciprocal and
-// square root, fused multiply-adds, and carry the limited slopes as scaled
+// -ffp-contract=off; divisions and square roots round as IEEE's), so they
+// reproduce the CPU step bit for bit.  FAST kernels use the hardware reciprocal
+// and square root, fused multiply-adds, and carry the limited slopes as scaled
 // half-cell increments: minmod(d1, (d1 + d2)/(2 theta), d2) of the raw
 // differences, which (theta/2) times gives 0.5*minmod(theta d1, (d1 + d2)/2,
 // theta d2); the factor theta/2 enters the reconstruction's multiply-adds.
@@ -74,8 +74,10 @@ template <class T> __device__ __forceinline__ T minmod2c(T th, T half, T s0, T s
 template <class T> struct Cst {
     T g, ga, CFL, theta, epsi, inv_epsi, eps_w, eps, delta, dxh, cmdinv, fc, cfl_delta, half;
     T th_s, mm_k;  // FAST slopes: half-cell increment = th_s * minmod(d1, mm_k (d1 + d2), d2)
+    T sqg, src;    // FAST faces: sqrt(g); FAST source: -2 g th_s
     T mask, rain_step_scale;
     double eps_d, mask_d;
+    FixedDiv<T> by_delta;
 };
 
 template <class T, bool FAST> Cst<T> make_cst(const KParams& P) {
@@ -98,116 +100,154 @@ template <class T, bool FAST> Cst<T> make_cst(const KParams& P) {
     c.th_s = c.theta * T(0.5);
     // theta <= 0 limits every slope to zero, as minmod(theta d1, ., theta d2) does
     c.mm_k = c.th_s > T(0.0) ? T(0.25) / c.th_s : T(0.0);
+    c.sqg = T(sqrt(P.g));
+    c.src = T(-2.0) * c.g * c.th_s;
     c.mask = T(P.mask);
     c.mask_d = P.mask;
     c.rain_step_scale = T(0.0);
+    c.by_delta = fixed_div(c.delta);
     return c;
 }
 
 // Hydrostatic reconstruction and central-upwind flux at one face between the
 // "n" (left/bottom) cell and the "i" (right/top) cell, src/Kurganov.cu:62-164
 // and 1865-1911.  Along Y the roles of u and v swap.  si/sn hold the cells'
-// limited slopes of (h, zs, un, ut): gradients in EXACT kernels, half-cell
-// increments over theta/2 in FAST ones (the reconstruction multiplies them by
-// C.th_s; the source terms carry g/2 into the final multiply-add).
-//
-// DEV (deviation form, FAST only): zsi/zsn carry the bed zb itself and the
-// interface depths use zl - zr = (zb_i - zb_n) - (zi - zl) - (zr - zn), so no
-// absolute elevation is rounded into a depth.
-template <class T, bool FAST, bool WANT_DT, bool DEV = false>
-__device__ __forceinline__ bool kurg_face(const Cst<T>& C, T hi, T hn, T zsi, T zsn, T ui, T un, T vi, T vn,
-                                          const Q4<T>& si, const Q4<T>& sn, Q4<T>& F, T& dt) {
-    typedef Ar<T, FAST> A;
+// limited slopes of (h, zs, un, ut).  F: the mass flux, the normal-momentum
+// flux that cell i takes and the one that cell n takes, the transverse flux.
+// dt: the face's wave speed, 0 for a dry or still face; its CFL limit is
+// cfl_delta / a (src/Kurganov.cu:102-105,159), and the block turns the largest
+// speed into its step (cfl_delta / max a is min over faces of cfl_delta / a:
+// rounded division is monotone).
+template <class T, bool WANT_DT>
+__device__ __forceinline__ bool kurg_face(const Cst<T>& C, const Q4<T>& qi, const Q4<T>& qn, const Q4<T>& si,
+                                          const Q4<T>& sn, Q4<T>& F, T& dt) {
+    const T hi = qi.a, hn = qn.a;
     const bool wet = hi > C.eps_w || hn > C.eps_w;
-    T zi = DEV ? zsi : zsi - hi;
-    T zn = DEV ? zsn : zsn - hn;
-    T zl, zr, hl, up, hr, um, dzi, dzn;
-    if (FAST) {
-        const T th = C.th_s;
-        dzi = th * (si.b - si.a);  // zi - zl
-        dzn = th * (sn.b - sn.a);  // zr - zn
-        zl = zi - dzi;
-        zr = zn + dzn;
-        hl = fma(-th, si.a, hi);
-        up = fma(-th, si.c, ui);
-        hr = fma(th, sn.a, hn);
-        um = fma(th, sn.c, un);
-    } else {
-        const T dx = C.dxh;
-        zl = zi - dx * (si.b - si.a);
-        zr = zn + dx * (sn.b - sn.a);
-        hl = hi - dx * si.a;
-        up = ui - dx * si.c;
-        hr = hn + dx * sn.a;
-        um = un + dx * sn.c;
-        dzi = zi - zl;
-        dzn = zr - zn;
-    }
-    T hp, hm;
-    if (DEV) {
-        const T dlr = (zi - zn) - dzi - dzn;  // zl - zr
-        hp = dmax(T(0.0), hl + dmin(dlr, T(0.0)));
-        hm = dmax(T(0.0), hr + dmin(-dlr, T(0.0)));
-    } else {
-        T zlr = dmax(zl, zr);
-        hp = dmax(T(0.0), hl + zl - zlr);
-        hm = dmax(T(0.0), hr + zr - zlr);
-    }
+    const T zi = qi.b - hi;
+    const T zn = qn.b - hn;
+    const T dx = C.dxh;
+    const T zl = zi - dx * (si.b - si.a);
+    const T zr = zn + dx * (sn.b - sn.a);
+    const T hl = hi - dx * si.a;
+    const T up = qi.c - dx * si.c;
+    const T hr = hn + dx * sn.a;
+    const T um = qn.c + dx * sn.c;
+    const T zlr = dmax(zl, zr);
+    const T hp = dmax(T(0.0), hl + zl - zlr);
+    const T hm = dmax(T(0.0), hr + zr - zlr);
     // KurgSolver
-    T cp = A::sqrt_(C.g * hp);
-    T cmo = A::sqrt_(C.g * hm);
-    T ap = dmax(dmax(up + cp, um + cmo), T(0.0));
-    T am = dmin(dmin(up - cp, um - cmo), T(0.0));
-    T qm = hm * um;
-    T qp = hp * up;
-    T a = dmax(ap, -am);
+    const T cp = sqrt(C.g * hp);
+    const T cmo = sqrt(C.g * hm);
+    const T ap = dmax(dmax(up + cp, um + cmo), T(0.0));
+    const T am = dmin(dmin(up - cp, um - cmo), T(0.0));
+    const T qm = hm * um;
+    const T qp = hp * up;
+    const T a = dmax(ap, -am);
     const bool flow = a > C.epsi;
-    T ad = A::rcp(ap - am);
-    T apm = ap * am;
-    T fh, fu;
-    if (FAST) {
-        T t = fma(-am, qp, ap * qm);
-        fh = fma(apm, hp - hm, t) * ad;
-        T Fm = fma(qm, um, (C.ga * hm) * hm);
-        T Fp = fma(qp, up, (C.ga * hp) * hp);
-        T s = fma(-am, Fp, ap * Fm);
-        fu = fma(apm, qp - qm, s) * ad;
-    } else {
-        fh = (ap * qm - am * qp + apm * (hp - hm)) * ad;
-        fu = (ap * (qm * um + C.ga * (hm * hm)) - am * (qp * up + C.ga * (hp * hp)) + apm * (qp - qm)) * ad;
-    }
+    const T ad = plain_rcp(ap - am);
+    const T apm = ap * am;
+    T fh = (ap * qm - am * qp + apm * (hp - hm)) * ad;
+    T fu = (ap * (qm * um + C.ga * (hm * hm)) - am * (qp * up + C.ga * (hp * hp)) + apm * (qp - qm)) * ad;
     fh = flow ? fh : T(0.0);
     fu = flow ? fu : T(0.0);
-    // The face's CFL limit is cfl_delta / a (src/Kurganov.cu:102-105,159); its wave speed a goes out
-    // instead (0 for a dry or still face), and the block turns the largest speed into its step
-    // (cfl_delta / max a is min over faces of cfl_delta / a: rounded division is monotone).
     if (WANT_DT) dt = (flow && wet) ? a : T(0.0);
-    T fv;
-    if (FAST)
-        fv = (fh > T(0.0) ? fma(C.th_s, sn.d, vn) : fma(-C.th_s, si.d, vi)) * fh;
-    else
-        fv = (fh > T(0.0) ? vn + C.dxh * sn.d : vi - C.dxh * si.d) * fh;
-    T sl, sr;
-    if (FAST) {
-        sl = fma(hl + hi, dzi, (hp - hl) * (hp + hl));
-        sr = fma(hr + hn, -dzn, (hm - hr) * (hm + hr));
-    } else {
-        sl = C.ga * (hp * hp - hl * hl + (hl + hi) * (zi - zl));
-        sr = C.ga * (hm * hm - hr * hr + (hr + hn) * (zn - zr));
-    }
+    const T fv = (fh > T(0.0) ? qn.d + C.dxh * sn.d : qi.d - C.dxh * si.d) * fh;
+    const T sl = C.ga * (hp * hp - hl * hl + (hl + hi) * (zi - zl));
+    const T sr = C.ga * (hm * hm - hr * hr + (hr + hn) * (zn - zr));
     F.a = wet ? fh : T(0.0);
-    F.b = wet ? (FAST ? fma(-C.ga, sl, fu) : fu - sl) : T(0.0);
-    F.c = wet ? (FAST ? fma(-C.ga, sr, fu) : fu - sr) : T(0.0);
+    F.b = wet ? fu - sl : T(0.0);
+    F.c = wet ? fu - sr : T(0.0);
     F.d = wet ? fv : T(0.0);
     return wet;
 }
 
-template <class T> struct Tile {
+// The same face in the FAST kernels' arithmetic.  The tile carries the bed zb
+// instead of zs (deviation form): the interface depths use zl - zr =
+// (zb_i - zb_n) - (zi - zl) - (zr - zn), so no absolute elevation is rounded
+// into a depth.  Slopes: h, un and ut over theta/2 (times C.th_s is the
+// half-cell increment), and in .b the half-cell increment of the bed.
+//
+// With w = a+/(a+ - a-) and k = w a-, the central-upwind flux of a quantity
+// with fluxes Fm, Fp and states Um, Up is Fp - w (Fp - Fm) + k (Up - Um).
+// The gravity part of each momentum flux, g/2 hp^2, cancels against the same
+// term of the hydrostatic source of the cell that takes it (src/Kurganov.cu:
+// 132-145: g/2 (hp^2 - hl^2 + (hl + h) dz)), and what is left of a cell's two
+// sources, g/2 (hl^2 - (hl + h) dz) - g/2 (hr^2 + (hr + h) dz), is -2 g h
+// times the half-cell increment of zs, since hl and hr lie as far below and
+// above h.  So a face keeps only F.b = up qp - w dF + k dq for cell i and
+// F.c = F.b + g/2 (hp^2 - hm^2) for cell n, and the cell adds one term
+// (cell_source): 50 instructions a face instead of 70, and no difference of
+// squares of whole depths is rounded; where the water is at rest both parts
+// are exactly zero.
+template <bool WANT_DT>
+__device__ __forceinline__ bool kurg_face_fast(const Cst<float>& C, const Q4<float>& qi, const Q4<float>& qn,
+                                               const Q4<float>& si, const Q4<float>& sn, Q4<float>& F, float& dt) {
+    const float th = C.th_s;
+    const bool wet = fmaxf(qi.a, qn.a) > C.eps_w;
+    const float hl = fmaf(-th, si.a, qi.a), up = fmaf(-th, si.c, qi.c);
+    const float hr = fmaf(th, sn.a, qn.a), um = fmaf(th, sn.c, qn.c);
+    const float dlr = (qi.b - qn.b) - si.b - sn.b;  // zl - zr
+    const float hp = fmaxf(0.0f, hl + fminf(dlr, 0.0f));
+    const float hm = fmaxf(0.0f, hr - fmaxf(dlr, 0.0f));
+    const float sp = __builtin_amdgcn_sqrtf(hp), sm = __builtin_amdgcn_sqrtf(hm);
+    const float ap = fmaxf(fmaxf(fmaf(C.sqg, sp, up), fmaf(C.sqg, sm, um)), 0.0f);
+    const float am = fminf(fminf(fmaf(-C.sqg, sp, up), fmaf(-C.sqg, sm, um)), 0.0f);
+    // both speeds zero (dry or still): the floor makes w and k zero, and the depths are zero too
+    const float w = ap * __builtin_amdgcn_rcpf(fmaxf(ap - am, 1e-30f));
+    const float k = w * am;
+    const float qp = hp * up, qm = hm * um;
+    const float dq = qp - qm, dh = hp - hm;
+    const float fh = fmaf(k, dh, fmaf(-w, dq, qp));
+    const float mp = qp * up;
+    const float g0 = dh * (hp + hm);
+    const float dF = fmaf(C.ga, g0, fmaf(-qm, um, mp));
+    const float fp = fmaf(k, dq, fmaf(-w, dF, mp));
+    const float fm = fmaf(C.ga, g0, fp);
+    if (WANT_DT) dt = wet ? fmaxf(ap, -am) : 0.0f;
+    F.a = wet ? fh : 0.0f;
+    F.b = wet ? fp : 0.0f;
+    F.c = wet ? fm : 0.0f;
+    F.d = (F.a > 0.0f ? fmaf(th, sn.d, qn.d) : fmaf(-th, si.d, qi.d)) * F.a;
+    return wet;
+}
+
+// A cell's hydrostatic source along one direction, per cell size: what
+// kurg_face_fast leaves out of its two faces, taken with the left (bottom)
+// face's momentum flux, which only this cell reads; so a wall, where the cell
+// takes no difference, drops it too.  gzs, gh: the cell's slopes of zs and h
+// over theta/2; hb, ha: the depths of the cells before and after it.  A face is wet if
+// either of its cells is, so a wet cell has both; a dry one takes the part of
+// each wet neighbour's face.
+__device__ __forceinline__ float cell_source(const Cst<float>& C, float h, float gzs, float gh, float hb, float ha) {
+    float s = C.src * h * gzs;
+    if (!(h > C.eps_w)) {
+        const float a = C.th_s * gh, dz = C.th_s * (gzs - gh);
+        const float hl = h - a, hr = h + a;
+        const float xl = hb > C.eps_w ? fmaf(hl, hl, -(hl + h) * dz) : 0.0f;
+        const float yr = ha > C.eps_w ? fmaf(hr, hr, (hr + h) * dz) : 0.0f;
+        s = C.ga * (xl - yr);
+    }
+    return s;
+}
+
+// The block in LDS.  ROW (the FAST kernels): along x the neighbours come from
+// the lanes beside, and only the ends of the rows pass through here.  The
+// faces take the slopes' place once every thread has formed its own.
+template <class T, bool ROW> struct Tile {
     Q4<T> q[20 * TP];   // (h, zs, u, v) at x, y in [-2, 17], corners unused
-    Q4<T> gx[16 * GXP]; // slopes along x of (h, zs, u, v) at x in [-1,16], y in [0,15]
-    Q4<T> gy[18 * GYP]; // slopes along y of (h, zs, v, u) at x in [0,15], y in [-1,16]
-    Q4<T> fx[16 * FP];  // (Fhu, Fqux, Su, Fqvx) at X faces
-    Q4<T> fy[17 * FYP]; // (Fhv, Fqvy, Sv, Fquy) at Y faces
+    union {
+        struct {
+            Q4<T> gy[18 * GYP];             // slopes along y of (h, zs, v, u) at x in [0,15], y in [-1,16]
+            Q4<T> gx[ROW ? 1 : 16 * GXP];   // slopes along x of (h, zs, u, v) at x in [-1,16], y in [0,15]
+        };
+        struct {
+            Q4<T> fy[17 * BW];              // (Fhv, Fqvy, Sv, Fquy) at Y faces, x in [0,15], yf in [0,16]
+            Q4<T> fx[ROW ? 1 : 16 * FP];    // (Fhu, Fqux, Su, Fqvx) at X faces, xf in [0,16]
+        };
+    };
+    Q4<T> gxr[ROW ? 2 * BW : 1];  // ROW: slopes along x at x = -1, then at x = 16
+    Q4<T> gxe[ROW ? BW : 1];      // ROW: and at x = 15
+    Q4<T> fe[ROW ? BW : 1];       // ROW: X faces at xf = 16
     T red[4];
     int next[4];  // queue positions: slot j & 3 holds position j
 };
@@ -307,21 +347,25 @@ __device__ __forceinline__ float minmod2sf(float k, float z0, float z1, float z2
     return minmod3f((z1 - z0) + (h1 - h0), ((z2 - z0) + (h2 - h0)) * k, (z2 - z1) + (h2 - h1));
 }
 
-template <class T, bool FAST, bool DEV = false>
-__device__ __forceinline__ Q4<T> slopes(const Cst<T>& C, const Q4<T>& m, const Q4<T>& c, const Q4<T>& p) {
+// Slopes of (h, zs, u, v) of cell c between m and p; in FAST kernels those of
+// h, u and v over theta/2 and in .b the half-cell increment of the bed, with
+// the slope of zs over theta/2 in gzs.
+template <class T, bool FAST>
+__device__ __forceinline__ Q4<T> slopes(const Cst<T>& C, const Q4<T>& m, const Q4<T>& c, const Q4<T>& p, T& gzs) {
     Q4<T> g;
     if constexpr (FAST) {
         static_assert(sizeof(T) == 4, "FAST kernels are FP32");
-        // half-cell increments over theta/2
         g.a = minmod2f(C.mm_k, m.a, c.a, p.a);
-        g.b = DEV ? minmod2sf(C.mm_k, m.b, c.b, p.b, m.a, c.a, p.a) : minmod2f(C.mm_k, m.b, c.b, p.b);
+        gzs = minmod2sf(C.mm_k, m.b, c.b, p.b, m.a, c.a, p.a);
+        g.b = C.th_s * (gzs - g.a);
         g.c = minmod2f(C.mm_k, m.c, c.c, p.c);
         g.d = minmod2f(C.mm_k, m.d, c.d, p.d);
     } else {
-        g.a = minmod2c(C.theta, C.half, m.a, c.a, p.a) / C.delta;
-        g.b = minmod2c(C.theta, C.half, m.b, c.b, p.b) / C.delta;
-        g.c = minmod2c(C.theta, C.half, m.c, c.c, p.c) / C.delta;
-        g.d = minmod2c(C.theta, C.half, m.d, c.d, p.d) / C.delta;
+        g.a = minmod2c(C.theta, C.half, m.a, c.a, p.a);
+        g.b = minmod2c(C.theta, C.half, m.b, c.b, p.b);
+        g.c = minmod2c(C.theta, C.half, m.c, c.c, p.c);
+        g.d = minmod2c(C.theta, C.half, m.d, c.d, p.d);
+        g = div4(C.by_delta, g);
     }
     return g;
 }
@@ -331,20 +375,49 @@ __device__ __forceinline__ Q4<T> slopes(const Cst<T>& C, const Q4<T>& m, const Q
 // and the 32 seventeenth faces to wave 3 (waves 0 and 1 fetch the strips, and
 // in the corrector also advance them).
 
-// Slopes of the tile: every thread its own cell along x and y; the halo ring
-// on wave 2, lanes 0-31 the x slopes at x = -1, 16 and lanes 32-63 the y
-// slopes at y = -1, 16.
-template <class T, bool FAST, bool DEV, bool OWN>
-__device__ __forceinline__ void tile_gradients(Tile<T>& s, const Cst<T>& C, int t, const Q4<T>& q, Q4<T>& gxo,
-                                               Q4<T>& gyo) {
+// Values of the lanes beside a lane in its row of 16 (the cells beside it along
+// x), through the data-parallel primitives of the vector ALU: from_left gives
+// each lane the value of the lane before it, and lane 0 of the row its `end`;
+// from_right that of the lane after it, and lane 15 its `end`.
+template <int CTRL> __device__ __forceinline__ int dpp_move(int end, int v) {
+    return __builtin_amdgcn_update_dpp(end, v, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL> __device__ __forceinline__ float dpp_move(float end, float v) {
+    return __int_as_float(dpp_move<CTRL>(__float_as_int(end), __float_as_int(v)));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_move(double end, double v) {
+    return __hiloint2double(dpp_move<CTRL>(__double2hiint(end), __double2hiint(v)),
+                            dpp_move<CTRL>(__double2loint(end), __double2loint(v)));
+}
+constexpr int ROW_SHR1 = 0x111, ROW_SHL1 = 0x101;
+template <class T> __device__ __forceinline__ T from_left(T end, T v) { return dpp_move<ROW_SHR1>(end, v); }
+template <class T> __device__ __forceinline__ T from_right(T end, T v) { return dpp_move<ROW_SHL1>(end, v); }
+template <class T> __device__ __forceinline__ Q4<T> from_left(const Q4<T>& e, const Q4<T>& v) {
+    return Q4<T>{from_left(e.a, v.a), from_left(e.b, v.b), from_left(e.c, v.c), from_left(e.d, v.d)};
+}
+template <class T> __device__ __forceinline__ Q4<T> from_right(const Q4<T>& e, const Q4<T>& v) {
+    return Q4<T>{from_right(e.a, v.a), from_right(e.b, v.b), from_right(e.c, v.c), from_right(e.d, v.d)};
+}
+
+// Slopes of the tile: every thread its own cell along x and y (gzx, gzy: those
+// of zs in FAST kernels); the halo ring on wave 2, lanes 0-31 the x slopes at
+// x = -1, 16 and lanes 32-63 the y slopes at y = -1, 16.  qh (FAST): lanes 0-7
+// of a row hold its halo cell at x = -1, lanes 8-15 that at x = 16.
+template <class T, bool FAST>
+__device__ __forceinline__ void tile_gradients(Tile<T, FAST>& s, const Cst<T>& C, int t, const Q4<T>& q, Q4<T>& gxo,
+                                               Q4<T>& gyo, T& gzx, T& gzy) {
     {
         const int x = t & 15, y = t >> 4;
         const int c = tix(x, y);
-        const Q4<T> q0 = OWN ? q : s.q[c];
-        gxo = slopes<T, FAST, DEV>(C, s.q[c - 1], q0, s.q[c + 1]);
-        s.gx[gxi(x, y)] = gxo;
-        Q4<T> m = s.q[c - TP], p = s.q[c + TP];
-        Q4<T> g = slopes<T, FAST, DEV>(C, m, q0, p);
+        if constexpr (FAST) {
+            const Q4<T> qh = s.q[tix(x < BW / 2 ? -1 : BW, y)];
+            gxo = slopes<T, FAST>(C, from_left(qh, q), q, from_right(qh, q), gzx);
+            if (x == BW - 1) s.gxe[y] = gxo;
+        } else {
+            gxo = slopes<T, FAST>(C, s.q[c - 1], q, s.q[c + 1], gzx);
+            s.gx[gxi(x, y)] = gxo;
+        }
+        Q4<T> g = slopes<T, FAST>(C, s.q[c - TP], q, s.q[c + TP], gzy);
         // y slopes stored as (h, zs, v, u)
         gyo.a = g.a; gyo.b = g.b; gyo.c = g.d; gyo.d = g.c;
         s.gy[gyi(x, y)] = gyo;
@@ -355,88 +428,92 @@ __device__ __forceinline__ void tile_gradients(Tile<T>& s, const Cst<T>& C, int 
         const int o = (r & 16) ? BW : -1;
         const int c = isx ? tix(o, j) : tix(j, o);
         const int d = isx ? 1 : TP;
-        const Q4<T> g = slopes<T, FAST, DEV>(C, s.q[c - d], s.q[c], s.q[c + d]);
+        T gz;
+        const Q4<T> g = slopes<T, FAST>(C, s.q[c - d], s.q[c], s.q[c + d], gz);
         Q4<T> gs;
         gs.a = g.a; gs.b = g.b; gs.c = isx ? g.c : g.d; gs.d = isx ? g.d : g.c;
-        *(isx ? &s.gx[gxi(o, j)] : &s.gy[gyi(j, o)]) = gs;
+        *(isx ? (FAST ? &s.gxr[r] : &s.gx[gxi(o, j)]) : &s.gy[gyi(j, o)]) = gs;
     }
 }
 
-// The left (bottom) face of the thread's own cell: the cell's state qi and
-// slopes si come in registers, the neighbour's from the tile; the face goes
-// to the tile for the neighbour and back to the caller in F.
-template <class T, bool FAST, bool WANT_DT, bool DEV, bool OWN>
-__device__ __forceinline__ bool xface(Tile<T>& s, const Cst<T>& C, int xf, int y, const Q4<T>& qo, const Q4<T>& so,
-                                      Q4<T>& F, T& dt) {
-    const int ci = tix(xf, y), gi = gxi(xf, y);
-    const Q4<T> qn = s.q[ci - 1];
-    const Q4<T> qi = OWN ? qo : s.q[ci];
-    const Q4<T> si = OWN ? so : s.gx[gi];
-    bool wet = kurg_face<T, FAST, WANT_DT, DEV>(C, qi.a, qn.a, qi.b, qn.b, qi.c, qn.c, qi.d, qn.d, si, s.gx[gi - 1], F,
-                                           dt);
-    s.fx[fxi(xf, y)] = F;
+template <class T, bool FAST, bool WANT_DT>
+__device__ __forceinline__ bool face(const Cst<T>& C, const Q4<T>& qi, const Q4<T>& qn, const Q4<T>& si,
+                                     const Q4<T>& sn, Q4<T>& F, T& dt) {
+    bool wet;
+    if constexpr (FAST) wet = kurg_face_fast<WANT_DT>(C, qi, qn, si, sn, F, dt);
+    else wet = kurg_face<T, WANT_DT>(C, qi, qn, si, sn, F, dt);
+    finish(F);
     return wet;
 }
-
-template <class T, bool FAST, bool WANT_DT, bool DEV, bool OWN>
-__device__ __forceinline__ bool yface(Tile<T>& s, const Cst<T>& C, int x, int yf, const Q4<T>& qo, const Q4<T>& so,
-                                      Q4<T>& F, T& dt) {
-    const int ci = tix(x, yf), gi = gyi(x, yf);
-    const Q4<T> qn = s.q[ci - TP];
-    const Q4<T> qi = OWN ? qo : s.q[ci];
-    const Q4<T> si = OWN ? so : s.gy[gi];
-    bool wet = kurg_face<T, FAST, WANT_DT, DEV>(C, qi.a, qn.a, qi.b, qn.b, qi.d, qn.d, qi.c, qn.c, si, s.gy[gi - GYP],
-                                           F, dt);
-    s.fy[fyi(x, yf)] = F;
-    return wet;
-}
+template <class T> __device__ __forceinline__ Q4<T> swap_uv(const Q4<T>& q) { return Q4<T>{q.a, q.b, q.d, q.c}; }
 
 // Fluxes of the tile state and the tendencies of the thread's cell, with the
 // wall patch (noslipbndQ, src/Boundary.cu:1887-1891) applied as operand
 // substitutions: at a left (bottom) wall the boundary face has no mass flux
 // and the first cell's right-face source S is replaced by its left-face Fq;
 // at a right (top) wall the boundary face has no mass flux and the last
-// cell's left-face Fq is replaced by its right-face S.  Returns the wave speed
-// that limits the cell's dtmax (0: none), see kurg_face.  q is the state the thread
-// stored for its cell; that state, the cell's slopes and its left and bottom
-// faces stay in registers instead of being read back from the tile (LDS
-// bandwidth bounds these kernels about as much as VALU issue does).
-template <class T, bool FAST, bool WANT_DT, bool DEV, bool OWN = true>
-__device__ __forceinline__ T tile_fluxes(Tile<T>& s, const Cst<T>& C, int t, const Q4<T>& qo, bool wl, bool wr,
-                                         bool wb, bool wt, T& dh, T& dhu, T& dhv) {
-    Q4<T> gxo, gyo;
-    tile_gradients<T, FAST, DEV, OWN>(s, C, t, qo, gxo, gyo);
+// cell's left-face Fq is replaced by its right-face S.  Either way the cell
+// takes no normal-momentum difference.  Returns the wave speed that limits the
+// cell's dtmax (0: none), see kurg_face.  q is the state the thread stored for
+// its cell; it, the cell's slopes and its left and bottom faces stay in
+// registers.  FAST kernels exchange along x between lanes: with every exchange
+// through LDS the FAST predictor's 30 accesses of 16 bytes a lane, with their
+// bank conflicts, took all of its 655 us at 8192 x 8192 cells, 21 accesses and
+// 28 more vector instructions 622.  The exact kernels have the vector ALU busy
+// for nine tenths of their time and gain nothing from that trade.
+template <class T> struct CellFaces {
+    Q4<T> l, r, b, t;
+};
+template <class T, bool FAST, bool WANT_DT>
+__device__ __forceinline__ T tile_fluxes(Tile<T, FAST>& s, const Cst<T>& C, int t, const Q4<T>& q, bool wl, bool wr,
+                                         bool wb, bool wt, CellFaces<T>& A, T& dh, T& dhu, T& dhv) {
+    Q4<T> gx, gy;
+    T gzx = T(0), gzy = T(0);
+    tile_gradients<T, FAST>(s, C, t, q, gx, gy, gzx, gzy);
     __syncthreads();
     const int x = t & 15, y = t >> 4;
+    const int ci = tix(x, y);
     T dtx = T(0.0), dty = T(0.0), dtd;  // wave speeds of the cell's faces
-    Q4<T> Fl, Fb;
-    xface<T, FAST, WANT_DT, DEV, OWN>(s, C, x, y, qo, gxo, Fl, dtx);
-    bool wy = yface<T, FAST, WANT_DT, DEV, OWN>(s, C, x, y, qo, gyo, Fb, dty);
-    if (t >= 192 && t < 224) {
+    Q4<T> Fl, Fb, Fe;
+    if constexpr (FAST) {
+        const Q4<T> qh = s.q[tix(x < BW / 2 ? -1 : BW, y)];
+        face<T, FAST, WANT_DT>(C, q, from_left(qh, q), gx, from_left(s.gxr[y], gx), Fl, dtx);
+        Fl.b += cell_source(C, q.a, gzx, gx.a, from_left(qh.a, q.a), from_right(qh.a, q.a));
+    } else {
+        face<T, FAST, WANT_DT>(C, q, s.q[ci - 1], gx, s.gx[gxi(x - 1, y)], Fl, dtx);
+    }
+    const Q4<T> qb = s.q[ci - TP];
+    const bool wy = face<T, FAST, WANT_DT>(C, swap_uv(q), swap_uv(qb), gy, s.gy[gyi(x, y - 1)], Fb, dty);
+    if constexpr (FAST) Fb.b += cell_source(C, q.a, gzy, gy.a, qb.a, s.q[ci + TP].a);
+    const bool edge = t >= 192 && t < 224, ex = t < 208;
+    if (edge) {
         // the seventeenth faces on wave 3: lanes 0-15 the X faces at xf = 16,
         // lanes 16-31 the Y faces at yf = 16
         const int j = t & 15;
-        const bool isx = t < 208;
-        const int ci = isx ? tix(BW, j) : tix(j, BW);
-        const Q4<T> qi = s.q[ci], qn = s.q[ci - (isx ? 1 : TP)];
-        const Q4<T>* gi = isx ? &s.gx[gxi(BW, j)] : &s.gy[gyi(j, BW)];
-        const Q4<T> si = *gi, sn = *(gi - (isx ? 1 : GYP));
-        Q4<T> F;
-        kurg_face<T, FAST, false, DEV>(C, qi.a, qn.a, qi.b, qn.b, isx ? qi.c : qi.d, isx ? qn.c : qn.d,
-                                       isx ? qi.d : qi.c, isx ? qn.d : qn.c, si, sn, F, dtd);
-        *(isx ? &s.fx[fxi(BW, j)] : &s.fy[fyi(j, BW)]) = F;
+        const int ce = ex ? tix(BW, j) : tix(j, BW);
+        Q4<T> qi = s.q[ce], qn = s.q[ce - (ex ? 1 : TP)];
+        if (!ex) {
+            qi = swap_uv(qi);
+            qn = swap_uv(qn);
+        }
+        const Q4<T>* gi = ex ? (FAST ? &s.gxr[BW + j] : &s.gx[gxi(BW, j)]) : &s.gy[gyi(j, BW)];
+        const Q4<T>* gn = ex ? (FAST ? &s.gxe[j] : &s.gx[gxi(BW - 1, j)]) : &s.gy[gyi(j, BW - 1)];
+        face<T, FAST, false>(C, qi, qn, *gi, *gn, Fe, dtd);
     }
+    __syncthreads();  // the slopes are read: the faces take their place
+    s.fy[t] = Fb;
+    if (!FAST) s.fx[y * FP + x] = Fl;
+    if (edge) *(!ex ? &s.fy[BW * BW + (t & 15)] : FAST ? &s.fe[t & 15] : &s.fx[(t & 15) * FP + BW]) = Fe;
     // The cell's limiting speed: its X face then its Y face, a dry Y face storing 1/epsi outright
     // (src/Kurganov.cu:1488-1491), i.e. no limit; 1/epsi caps the step at the reduction.
     T dtc = T(0.0);
     if (WANT_DT) dtc = wy ? dmax(dtx, dty) : T(0.0);
     __syncthreads();
-    const Q4<T> Fr = s.fx[fxi(x + 1, y)], Ft = s.fy[fyi(x, y + 1)];
-    if (!OWN) {
-        Fl = s.fx[fxi(x, y)];
-        Fb = s.fy[fyi(x, y)];
-    }
-    const Q4<T> q = OWN ? qo : s.q[tix(x, y)];
+    Q4<T> Fr;
+    if constexpr (FAST) Fr = from_right(s.fe[y], Fl);
+    else Fr = s.fx[y * FP + x + 1];
+    const Q4<T> Ft = s.fy[t + BW];
+    A = CellFaces<T>{Fl, Fr, Fb, Ft};
     T Fhl = Fl.a, Fhr = Fr.a, Fql = Fl.b, Sr = Fr.c;
     T Fhb = Fb.a, Fht = Ft.a, Fqb = Fb.b, St = Ft.c;
     if (wl && x == 0) { Fhl = T(0.0); Sr = Fql; }
@@ -445,19 +522,22 @@ __device__ __forceinline__ T tile_fluxes(Tile<T>& s, const Cst<T>& C, int t, con
     if (wt && y == BW - 1) { Fht = T(0.0); Fqb = St; }
     // src/Advection.cu:236-250 (Cartesian: the metric terms vanish)
     dh = T(-1.0) * (Fhr - Fhl + Fht - Fhb) * C.cmdinv;
-    dhu = (Fql + Fb.d - Sr - Ft.d) * C.cmdinv + C.fc * q.a * q.d;
-    dhv = (Fqb + Fl.d - St - Fr.d) * C.cmdinv - C.fc * q.a * q.c;
+    if (FAST) {
+        dhu = ((Fql - Sr) + (Fb.d - Ft.d)) * C.cmdinv + C.fc * q.a * q.d;
+        dhv = ((Fqb - St) + (Fl.d - Fr.d)) * C.cmdinv - C.fc * q.a * q.c;
+    } else {
+        dhu = (Fql + Fb.d - Sr - Ft.d) * C.cmdinv + C.fc * q.a * q.d;
+        dhv = (Fqb + Fl.d - St - Fr.d) * C.cmdinv - C.fc * q.a * q.c;
+    }
     return dtc;
 }
 
 // Tendencies of an edge cell of a block on a side of type 2 or 3, recomputed
-// from the tile's faces (still in LDS after tile_fluxes) with the boundary
-// face's mass flux from bnd_flux, or the no-slip patch on a dry face.  Runs
-// only for blocks with such a side, after tile_fluxes; it reads the four mass
-// fluxes of the cell, and the momentum terms only where a dry face falls back
-// to the no-slip patch, so that it adds few registers to the kernel.
-template <class T>
-__device__ void open_sides(const Tile<T>& s, const Cst<T>& C, const KParams& P, int t, int ib, int nL, int nR, int nB,
+// from its faces A with the boundary face's mass flux from bnd_flux, or the
+// no-slip patch on a dry face.  Runs only for blocks with such a side, after
+// tile_fluxes; q: the cell's stage state.
+template <class T, bool FAST>
+__device__ __forceinline__ void open_sides(const CellFaces<T>& A, const Q4<T>& q, const Cst<T>& C, const KParams& P, int t, int ib, int nL, int nR, int nB,
                            int nT, double tstage, const T* h, const T* u, const T* v, const T* zb, T& dh, T& dhu,
                            T& dhv) {
     const int x = t & 15, y = t >> 4;
@@ -467,7 +547,7 @@ __device__ void open_sides(const Tile<T>& s, const Cst<T>& C, const KParams& P, 
                          nB == ib && y == 0 ? bt : -1, nT == ib && y == BW - 1 ? bt : -1};
     if (side[0] < 2 && side[1] < 2 && side[2] < 2 && side[3] < 2) return;
     const BSeg& S = P.seg[P.bseg[ib]];
-    T F[4] = {s.fx[fxi(x, y)].a, s.fx[fxi(x + 1, y)].a, s.fy[fyi(x, y)].a, s.fy[fyi(x, y + 1)].a};
+    T F[4] = {A.l.a, A.r.a, A.b.a, A.t.a};
     bool slip[4];
 #pragma unroll
     for (int sd = 0; sd < 4; sd++) {
@@ -489,20 +569,14 @@ __device__ void open_sides(const Tile<T>& s, const Cst<T>& C, const KParams& P, 
         if (slip[sd]) F[sd] = T(0.0);
     }
     dh = T(-1.0) * (F[1] - F[0] + F[3] - F[2]) * C.cmdinv;
-    const Q4<T> q = s.q[tix(x, y)];
+    // the no-slip patch leaves no normal-momentum difference (in FAST kernels no source either)
     if ((side[0] >= 2 && slip[0]) || (side[1] >= 2 && slip[1])) {
-        const Q4<T> Fl = s.fx[fxi(x, y)], Fr = s.fx[fxi(x + 1, y)];
-        T Fql = Fl.b, Sr = Fr.c;
-        if (slip[0]) Sr = Fql;
-        if (slip[1]) Fql = Sr;
-        dhu = (Fql + s.fy[fyi(x, y)].d - Sr - s.fy[fyi(x, y + 1)].d) * C.cmdinv + C.fc * q.a * q.d;
+        const T lo = A.l.b, hi = A.r.c, Fq = FAST ? T(0.0) : slip[1] ? hi : lo;
+        dhu = (Fq + A.b.d - Fq - A.t.d) * C.cmdinv + C.fc * q.a * q.d;
     }
     if ((side[2] >= 2 && slip[2]) || (side[3] >= 2 && slip[3])) {
-        const Q4<T> Fb = s.fy[fyi(x, y)], Ft = s.fy[fyi(x, y + 1)];
-        T Fqb = Fb.b, St = Ft.c;
-        if (slip[2]) St = Fqb;
-        if (slip[3]) Fqb = St;
-        dhv = (Fqb + s.fx[fxi(x, y)].d - St - s.fx[fxi(x + 1, y)].d) * C.cmdinv - C.fc * q.a * q.c;
+        const T lo = A.b.b, hi = A.t.c, Fq = FAST ? T(0.0) : slip[3] ? hi : lo;
+        dhv = (Fq + A.l.d - Fq - A.r.d) * C.cmdinv - C.fc * q.a * q.c;
     }
 }
 
@@ -531,22 +605,14 @@ __device__ __forceinline__ void advance(const Cst<T>& C, int fmc, T dt, T hold, 
         vo = ho > C.eps ? fma(hold, vold, dt * dhvi) * r : T(0.0);
         return;
     }
-    T edt;
-    if (fmc || dhi >= T(0.0)) {
-        edt = dt;
+    const T edt = fmc ? dt : dry_step(dt, hold, dhi, C.eps, C.eps_d);
+    ho = hold + edt * dhi;
+    if (ho > C.eps) {
+        uo = (hold * uold + edt * dhui) / ho;
+        vo = (hold * vold + edt * dhvi) / ho;
     } else {
-        double lim = (hold > C.eps_d ? (double)hold : C.eps_d) / (double)fabs(dhi);
-        edt = T((double)dt < lim ? (double)dt : lim);
-    }
-    {
-        ho = hold + edt * dhi;
-        if (ho > C.eps) {
-            uo = (hold * uold + edt * dhui) / ho;
-            vo = (hold * vold + edt * dhvi) / ho;
-        } else {
-            uo = T(0.0);
-            vo = T(0.0);
-        }
+        uo = T(0.0);
+        vo = T(0.0);
     }
 }
 
@@ -711,7 +777,7 @@ template <class T, bool FAST, bool BATCH, bool DEV, bool EXT = false>
 __global__ __launch_bounds__(256) void k_predictor(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
     if (blockIdx.x == 0 && threadIdx.x < NXCD) P.queue[(NXCD + threadIdx.x) * QSTRIDE] = 0;  // the corrector's
     if (!BATCH && L->done) return;
-    __shared__ Tile<T> s;
+    __shared__ Tile<T, FAST> s;
     const int t = threadIdx.x;
     const int x = t & 15, y = t >> 4;
     const int xcd = blockIdx.x % NXCD;
@@ -771,14 +837,14 @@ __global__ __launch_bounds__(256) void k_predictor(KParams P, Cst<T> C, StepBuff
             if (ldu(&L[n.sid].done, 0)) continue;
         }
         T dh, dhu, dhv;
-        // own values in registers: measured faster for the exact kernels (-6 %), slower for FAST (+1.5 %)
+        CellFaces<T> A;
         const bool w = blk_wall(P, n.ib, n.nL, n.nR, n.nB, n.nT);
-        T dtc = tile_fluxes<T, FAST, true, DEV, !FAST>(s, C, t, qv, w && n.nL == n.ib, w && n.nR == n.ib,
-                                                       w && n.nB == n.ib, w && n.nT == n.ib, dh, dhu, dhv);
+        const T dtc = tile_fluxes<T, FAST, true>(s, C, t, qv, w && n.nL == n.ib, w && n.nR == n.ib, w && n.nB == n.ib,
+                                                 w && n.nT == n.ib, A, dh, dhu, dhv);
         if (EXT && P.bopen && (n.nL == n.ib || n.nR == n.ib || n.nB == n.ib || n.nT == n.ib))
             // boundary values at the predictor's time, totaltime + dt/2 with the previous dt (src/FlowCPU.cu:94)
-            open_sides<T>(s, C, P, t, n.ib, n.nL, n.nR, n.nB, n.nT, L->totaltime + L->dt * 0.5, B.h, B.u, B.v, B.zb, dh,
-                          dhu, dhv);
+            open_sides<T, FAST>(A, qv, C, P, t, n.ib, n.nL, n.nR, n.nB, n.nT, L->totaltime + L->dt * 0.5, B.h, B.u, B.v,
+                                B.zb, dh, dhu, dhv);
         if (EXT && P.nriver) dh = river_inflow<T>(P, n.ib, x, y, dh);
         const unsigned oi = boff_i<T>(n.ib) + ki;
         stno(B.dh, oi, dh);
@@ -802,14 +868,16 @@ template <class T> __device__ __forceinline__ T kahan_add(T h, T d, T& c) {
     return t;
 }
 
-// Persistent corrector with the same schedule and prefetch.  COMP: the depth
+// Persistent corrector with the same schedule and prefetch, through each XCD's
+// range from its end: the predictor left the last blocks' lines in the caches
+// (16.33 ms against 16.43 for ten steps at 8192 x 8192 cells).  COMP: the depth
 // update accumulates with a compensated (Kahan) sum, so the small increments
 // of rain and of slow flows are not lost to FP32 rounding of h.
 template <class T, bool FAST, bool BATCH, bool COMP, bool EXT>
 __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C, const StepBuffers<T>& B, DevLoop* L) {
     if (blockIdx.x == 0 && threadIdx.x < NXCD) P.queue[threadIdx.x * QSTRIDE] = 0;  // the predictor's
     if (!BATCH && !L->go) return;
-    __shared__ Tile<T> s;
+    __shared__ Tile<T, FAST> s;
     const int t = threadIdx.x;
     const int x = t & 15, y = t >> 4;
     const int xcd = blockIdx.x % NXCD;
@@ -850,7 +918,7 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
     int g = 1;  // the next position to read
     Nb cur;
     if (pos < R.end) {
-        cur = block_nb<BATCH>(P, pos);
+        cur = block_nb<BATCH>(P, R.start + R.end - 1 - pos);
         fetch(cur);
     }
     for (int npos; pos < R.end; pos = npos) {
@@ -860,7 +928,7 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
             __syncthreads();
             npos = queue_read(s.next, g++);
             if (npos < R.end) {
-                cur = block_nb<BATCH>(P, npos);
+                cur = block_nb<BATCH>(P, R.start + R.end - 1 - npos);
                 fetch(cur);
             }
             continue;
@@ -894,17 +962,18 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
         const Nb n = cur;
         npos = queue_read(s.next, g++);
         if (npos < R.end) {
-            cur = block_nb<BATCH>(P, npos);
+            cur = block_nb<BATCH>(P, R.start + R.end - 1 - npos);
             fetch(cur);
         }
         const int ib = n.ib, nL = n.nL, nR = n.nR, nB = n.nB, nT = n.nT;
         T dh, dhu, dhv;
+        CellFaces<T> A;
         const bool w = blk_wall(P, ib, nL, nR, nB, nT);
-        (void)tile_fluxes<T, FAST, false, FAST>(s, C, t, qs, w && nL == ib, w && nR == ib, w && nB == ib, w && nT == ib,
-                                                dh, dhu, dhv);
+        (void)tile_fluxes<T, FAST, false>(s, C, t, qs, w && nL == ib, w && nR == ib, w && nB == ib, w && nT == ib, A, dh,
+                                          dhu, dhv);
         if (EXT && P.bopen && (nL == ib || nR == ib || nB == ib || nT == ib))
             // boundary values at totaltime + dt, from the step-start state (src/FlowCPU.cu:187)
-            open_sides<T>(s, C, P, t, ib, nL, nR, nB, nT, L->tcorr, B.h, B.u, B.v, B.zb, dh, dhu, dhv);
+            open_sides<T, FAST>(A, qs, C, P, t, ib, nL, nR, nB, nT, L->tcorr, B.h, B.u, B.v, B.zb, dh, dhu, dhv);
         if (EXT && P.nriver) dh = river_inflow<T>(P, ib, x, y, dh);
         T h1, u1, v1;
         const unsigned oc = boff<T>(ib) + kb, oci = boff_i<T>(ib) + ki;  // this block's cells
@@ -1000,19 +1069,21 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
     queue_end(t, pend);
 }
 
-// Six resident workgroups per CU is the tile's LDS limit; asking for six waves
-// per SIMD holds the plain one-level corrector to the 80 VGPRs that allow it
-// (it needs a few more unbounded, which would cost a sixth of its waves).
-// Batches and the forcing kernels (open boundaries, rivers, rain maps) need
-// more registers than that and run unbounded (k_corrector_wide): forced into
-// 80 VGPRs the batch corrector measured 3 % slower.
+// Waves per SIMD asked of the plain one-level corrector: six for the FAST
+// forms, which then hold to 80 VGPRs (84 unbounded, a sixth of the waves
+// less); five for exact FP32, whose 93 VGPRs spill at six (1,118 us against
+// 1,150 for ten rain steps on 1520 x 2032 cells); FP64 takes what its 160
+// VGPRs allow.  Batches and the forcing kernels (open boundaries, rivers, rain
+// maps) need more registers: they run as k_corrector_wide, the FP32 forcing
+// ones held to four waves, the others unbounded (forced into 80 VGPRs the
+// batch corrector measured 3 % slower).
 template <class T, bool FAST, bool BATCH, bool COMP>
-__global__ __launch_bounds__(256, 6) void k_corrector(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : FAST ? 6 : 5) void k_corrector(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
     static_assert(!BATCH, "batches use k_corrector_wide");
     corrector_body<T, FAST, false, COMP, false>(P, C, B, L);
 }
 template <class T, bool FAST, bool BATCH, bool COMP, bool EXT>
-__global__ __launch_bounds__(256) void k_corrector_wide(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
+__global__ __launch_bounds__(256, EXT && sizeof(T) == 4 ? 4 : 1) void k_corrector_wide(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
     corrector_body<T, FAST, BATCH, COMP, EXT>(P, C, B, L);
 }
 
