@@ -23,7 +23,7 @@
 //                    (src/Advection.cu:160-254), all in LDS; zs = zb + h
 //                    (src/Halo.cu:72-107) is formed where it is read.  The
 //                    block's largest wave speed goes to the dt slots.
-//   k_amr_advance    after the dt reduction, U* = U + dt/2 L(U)
+//   k_amr_advance    the dt reduction and U* = U + dt/2 L(U)
 //                    (src/Advection.cu:332-385).  A block beside a finer one
 //                    takes its shared faces as the means of the finer faces
 //                    first (src/Halo.cu:1441-1862), a block on an open
@@ -756,7 +756,7 @@ __device__ __forceinline__ int face_at(int s, int j, int b) {
 // neighbour and the boundary patch.
 template <class T>
 __device__ __forceinline__ void amr_fluxfix_side(const KParams& P, const FluxOut<T>& F, const StageIn<T>& E0,
-                                                 const T* zb, const DevLoop* L, int corr, int s, int j, int ib) {
+                                                 const T* zb, const LoopState& L, int corr, int s, int j, int ib) {
     const int lev = P.level[ib];
     T* const A[4] = {s < 2 ? F.Fhu : F.Fhv, s < 2 ? F.Fqux : F.Fqvy, s < 2 ? F.Su : F.Sv, s < 2 ? F.Fqvx : F.Fquy};
     // coarse face = mean of the two fine faces (src/Halo.cu:1441-1529, 1766-1862)
@@ -781,7 +781,7 @@ __device__ __forceinline__ void amr_fluxfix_side(const KParams& P, const FluxOut
             // reduction recorded them
             const int in = s == SL ? memloc(1, j, ib) : s == SR ? memloc(BW - 1, j, ib) : s == SB ? memloc(j, 1, ib)
                                                                                           : memloc(j, BW - 1, ib);
-            const double ts = corr ? L->tcorr : L->tpred;
+            const double ts = corr ? L.tcorr : L.tpred;
             const BSeg& G = P.seg[P.bseg[ib]];
             const int fx = s == SL ? 0 : s == SR ? BW : j, fy = s == SB ? 0 : s == ST ? BW : j;
             T q = A[0][i];
@@ -835,13 +835,13 @@ template <class T> __device__ __forceinline__ AdvIn<T> adv_load(const AdvArgs<T>
 // updateEV, src/FlowCPU.cu:120-124).
 template <class T, bool SPH>
 __device__ __forceinline__ void amr_tendencies(const KParams& P, T delta, T hi, T uui, T vvi, T Fhl, T Fhr, T Fhb,
-                                               T Fht, T Fql, T Sr, T Fqb, T St, T Ftb, T Ftt, T Ftl, T Ftr, int ib,
-                                               int x, int y, T& dh, T& dhu, T& dhv) {
+                                               T Fht, T Fql, T Sr, T Fqb, T St, T Ftb, T Ftt, T Ftl, T Ftr,
+                                               double tstart, int ib, int x, int y, T& dh, T& dhu, T& dhv) {
     const T* met = (const T*)P.metric + (size_t)ib * METRIC_STRIDE;
     const T fc = SPH ? met[MET_FC + y] : T(P.fc);
     const T cm = SPH ? met[MET_CME + y] : T(1.0);
     const T cmdinv = T(1.0) / (cm * delta);
-    dh = river_inflow<T>(P, ib, x, y, T(-1.0) * (Fhr - Fhl + Fht - Fhb) * cmdinv);
+    dh = river_inflow<T>(P, ib, x, y, tstart, T(-1.0) * (Fhr - Fhl + Fht - Fhb) * cmdinv);
     dhu = (Fql + Ftb - Sr - Ftt) * cmdinv + fc * hi * vvi;
     dhv = (Fqb + Ftl - St - Ftr) * cmdinv - fc * hi * uui;
     if (SPH) {  // the metric differences, zero on Cartesian grids
@@ -862,8 +862,8 @@ __device__ __forceinline__ void amr_tendencies(const KParams& P, T delta, T hi, 
 // (src/Updateforcing.cu:530-581).
 template <class T>
 __device__ __forceinline__ void amr_update(const KParams& P, const AdvArgs<T>& A, const AdvIn<T>& X, T dhi, T dhu,
-                                           T dhv, const DevLoop* L, int corr, int i, int ib, int x, int y) {
-    const T dt = corr ? T(L->dt) : T(L->dt) * T(0.5);
+                                           T dhv, const LoopState& L, int corr, int i, int ib, int x, int y) {
+    const T dt = corr ? T(L.dt) : T(L.dt) * T(0.5);
     const T g = T(P.g);
     const T eps = T(P.eps);
     const T hold = X.hold;
@@ -900,7 +900,7 @@ __device__ __forceinline__ void amr_update(const KParams& P, const AdvArgs<T>& A
         // cleanup then implicit uniform rain, src/Updateforcing.cu:530-581
         if (P.rain_on) {
             const T act = (double)X.zb < P.mask ? T(1.0) : T(0.0);
-            T rainhh = rain_depth<T>(P, L, ib, x, y, T(L->dt)) * act;
+            T rainhh = rain_depth<T>(P, L, ib, x, y, T(L.dt)) * act;
             const T qvol = ho / (ho + rainhh);
             const bool wet = (double)ho > P.eps;
             ho = ho + rainhh;
@@ -1357,10 +1357,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
         if (y == BW - 1 && (nb[6] == ib || nb[7] == ib)) { Fht = T(0.0); Fqb = St; }
     }
     T dh, dhu, dhv;
-    amr_tendencies<T, SPH>(P, delta, h0, u0, v0, Fhl, Fhr, Fhb, Fht, Fql, Sr, Fqb, St, Fb.d, Ft.d, Fl.d, Fr.d, ib, x, y,
-                           dh, dhu, dhv);
+    amr_tendencies<T, SPH>(P, delta, h0, u0, v0, Fhl, Fhr, Fhb, Fht, Fql, Sr, Fqb, St, Fb.d, Ft.d, Fl.d, Fr.d,
+                           corr ? Lm->tstart : Lm->totaltime, ib, x, y, dh, dhu, dhv);
     if (corr) {
-        amr_update<T>(P, A, X, dh, dhu, dhv, Lm, 1, c, ib, x, y);
+        amr_update<T>(P, A, X, dh, dhu, dhv, *Lm, 1, c, ib, x, y);
     } else {
         const int k = ib * BSI + t;
         D.dh[k] = dh;
@@ -1374,38 +1374,49 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
 // edge), then its advance.
 template <class T, bool SPH>
 __device__ __forceinline__ void fix_advance(const KParams& P, const StageIn<T>& E0, const AdvArgs<T>& A,
-                                            const FluxOut<T>& F, const DevLoop* L, int corr, int t, int ib) {
+                                            const FluxOut<T>& F, const LoopState& L, int corr, int t, int ib) {
     const int x = t & 15, y = t >> 4;
     const int i = memloc(x, y, ib), ir = memloc(x + 1, y, ib), it = memloc(x, y + 1, ib);
     const AdvIn<T> X = adv_load(A, i, corr);
     const T h = A.h[i], u = A.u[i], v = A.v[i];
-    if (!L->go) return;  // the workgroup's one block: all threads leave together
+    if (!L.go) return;  // the workgroup's one block: all threads leave together
     if (t < 64) amr_fluxfix_side<T>(P, F, E0, A.zb, L, corr, t >> 4, t & 15, ib);
     __syncthreads();
     T dh, dhu, dhv;
     amr_tendencies<T, SPH>(P, calcres(T(P.delta0), P.level[ib]), h, u, v, F.Fhu[i], F.Fhu[ir], F.Fhv[i], F.Fhv[it],
-                           F.Fqux[i], F.Su[ir], F.Fqvy[i], F.Sv[it], F.Fquy[i], F.Fquy[it], F.Fqvx[i], F.Fqvx[ir], ib, x,
-                           y, dh, dhu, dhv);
+                           F.Fqux[i], F.Su[ir], F.Fqvy[i], F.Sv[it], F.Fquy[i], F.Fquy[it], F.Fqvx[i], F.Fqvx[ir],
+                           L.tstart, ib, x, y, dh, dhu, dhv);
     amr_update<T>(P, A, X, dh, dhu, dhv, L, corr, i, ib, x, y);
 }
 
-// The predictor's advance, after the dt reduction: U* = U + dt/2 L(U) from the
-// stored tendencies, or from the fixed-up faces.
-template <class T, bool SPH>
+// The predictor's advance: U* = U + dt/2 L(U) from the stored tendencies, or
+// from the fixed-up faces, with the step's dt.  REDUCED: the reduction was a
+// launch before (a block of a batch finds its member's state in L); otherwise
+// every workgroup works it out from the slots (step_state).
+template <class T, bool SPH, bool REDUCED>
 __global__ __launch_bounds__(256) void k_amr_advance(KParams P, StageIn<T> E0, AdvArgs<T> A, FluxOut<T> F, Tend<T> D,
-                                                     DevLoop* L) {
+                                                     DevLoop* L, DevLoop* Lnext, int mode) {
     const int ib = ldu(P.active, xcd_range(blockIdx.x % NXCD, P.nblk).start + blockIdx.x / NXCD);
-    const DevLoop* Lm = loop_of(P, L, ib);
     const int t = threadIdx.x;
-    if (fix_block(P, ldu(P.nbr, ib * NBR + 8))) {
-        fix_advance<T, SPH>(P, E0, A, F, Lm, 0, t, ib);
+    const int i = memloc(t & 15, t >> 4, ib), k = ib * BSI + t;
+    const bool fix = fix_block(P, ldu(P.nbr, ib * NBR + 8));
+    AdvIn<T> X;
+    T dh = T(0), dhu = T(0), dhv = T(0);
+    if (!fix) {
+        X = adv_load(A, i, 0);
+        dh = D.dh[k];
+        dhu = D.dhu[k];
+        dhv = D.dhv[k];
+    }
+    LoopState S;
+    if (REDUCED) S = *loop_of(P, L, ib);
+    else S = step_state<T>(L, Lnext, mode);
+    if (fix) {
+        fix_advance<T, SPH>(P, E0, A, F, S, 0, t, ib);
         return;
     }
-    const int i = memloc(t & 15, t >> 4, ib), k = ib * BSI + t;
-    const AdvIn<T> X = adv_load(A, i, 0);
-    const T dh = D.dh[k], dhu = D.dhu[k], dhv = D.dhv[k];
-    if (!Lm->go) return;
-    amr_update<T>(P, A, X, dh, dhu, dhv, Lm, 0, i, ib, t & 15, t >> 4);
+    if (!S.go) return;
+    amr_update<T>(P, A, X, dh, dhu, dhv, S, 0, i, ib, t & 15, t >> 4);
 }
 
 // The corrector's fix-up and advance of the blocks that the stage left out.
@@ -1413,7 +1424,7 @@ template <class T, bool SPH>
 __global__ __launch_bounds__(256) void k_amr_fix_advance(KParams P, StageIn<T> E0, AdvArgs<T> A, FluxOut<T> F,
                                                          DevLoop* L) {
     const int ib = ldu(P.fix, blockIdx.x);
-    fix_advance<T, SPH>(P, E0, A, F, loop_of(P, L, ib), 1, threadIdx.x, ib);
+    fix_advance<T, SPH>(P, E0, A, F, *loop_of(P, L, ib), 1, threadIdx.x, ib);
 }
 
 template <class T, bool SPH, bool FAST, int corr>
@@ -1437,11 +1448,17 @@ void stage(const KParams& P, const AmrBuffers<T>& B, const AdvArgs<T>& A, DevLoo
     }
 }
 
-// Four launches and the dt reduction: the predictor's stage, its advance, the
-// corrector's stage with its advance, and the blocks whose faces wait for
-// their finer neighbours'.
+// Meshes of up to so many blocks have each workgroup of the predictor's advance
+// work out the time step itself; larger ones, whose thousands of workgroups
+// would repeat it, and batches, whose blocks are of many members, have it done
+// by a launch in between.
+constexpr int SELF_REDUCE = 4096;
+
+// Four launches: the predictor's stage, its advance, the corrector's stage with
+// its advance, and the blocks whose faces wait for their finer neighbours'.
 template <class T, bool SPH, bool FAST>
-void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int advance_time, hipStream_t st, hipEvent_t* ev) {
+void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, DevLoop* Lnext, int advance_time, hipStream_t st,
+              hipEvent_t* ev) {
     const dim3 blk(P.nblk), tpb(256);
     const FluxOut<T> F{B.Fhu, B.Fqux, B.Su, B.Fqvx, B.Fhv, B.Fqvy, B.Sv, B.Fquy};
     const Tend<T> D{B.dh, B.dhu, B.dhv};
@@ -1453,9 +1470,17 @@ void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int advance_
     const AdvArgs<T> a0{B.h, B.u, B.v, B.h, B.u, B.v, B.ho, B.uo, B.vo, B.zb, B.cf};
     stage<T, SPH, FAST, 0>(P, B, a0, L, st);
     if (ev) (void)hipEventRecord(ev[1], st);
-    launch_reduce_dt(sizeof(T) == 8 ? 0 : 1, L, P.sid ? P.nmember : 1, advance_time, st);
+    const bool reduce = P.sid || P.nblk > SELF_REDUCE;
+    if (reduce) {
+        if (P.sid) Lnext = L;
+        launch_reduce_dt(sizeof(T) == 8 ? 0 : 1, L, Lnext, P.sid ? P.nmember : 1, advance_time, st);
+    }
     if (ev) (void)hipEventRecord(ev[2], st);
-    hipLaunchKernelGGL((k_amr_advance<T, SPH>), blk, tpb, 0, st, P, E0, a0, F, D, L);
+    if (reduce)
+        hipLaunchKernelGGL((k_amr_advance<T, SPH, true>), blk, tpb, 0, st, P, E0, a0, F, D, Lnext, Lnext, advance_time);
+    else
+        hipLaunchKernelGGL((k_amr_advance<T, SPH, false>), blk, tpb, 0, st, P, E0, a0, F, D, L, Lnext, advance_time);
+    L = Lnext;  // the state past the reduction
     // corrector: evolv = friction(evolv + dt L(evolv_o)) + rain
     const AdvArgs<T> a1{B.ho, B.uo, B.vo, B.h, B.u, B.v, B.h, B.u, B.v, B.zb, B.cf};
     stage<T, SPH, FAST, 1>(P, B, a1, L, st);
@@ -1464,21 +1489,22 @@ void amr_step(const KParams& P, const AmrBuffers<T>& B, DevLoop* L, int advance_
 }
 
 template <class T, bool FAST>
-void amr_step(const KParams& P, const void* buffers, DevLoop* L, int advance_time, hipStream_t st, hipEvent_t* ev) {
+void amr_step(const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext, int advance_time, hipStream_t st,
+              hipEvent_t* ev) {
     const AmrBuffers<T>& B = *(const AmrBuffers<T>*)buffers;
     // Cartesian grids: the metric terms are the constant 1 and their products fold away
-    if (P.spherical) amr_step<T, true, FAST>(P, B, L, advance_time, st, ev);
-    else amr_step<T, false, FAST>(P, B, L, advance_time, st, ev);
+    if (P.spherical) amr_step<T, true, FAST>(P, B, L, Lnext, advance_time, st, ev);
+    else amr_step<T, false, FAST>(P, B, L, Lnext, advance_time, st, ev);
 }
 
 }  // namespace
 
-void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLoop* L, int advance_time,
-                     hipStream_t st, hipEvent_t* ev) {
+void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext,
+                     int advance_time, hipStream_t st, hipEvent_t* ev) {
     // BGF_FP32_FAST and BGF_FP32_COMP take the fast flux arithmetic (no compensated update here)
-    if (precision == 0) amr_step<double, false>(P, buffers, L, advance_time, st, ev);
-    else if (precision == 1) amr_step<float, false>(P, buffers, L, advance_time, st, ev);
-    else amr_step<float, true>(P, buffers, L, advance_time, st, ev);
+    if (precision == 0) amr_step<double, false>(P, buffers, L, Lnext, advance_time, st, ev);
+    else if (precision == 1) amr_step<float, false>(P, buffers, L, Lnext, advance_time, st, ev);
+    else amr_step<float, true>(P, buffers, L, Lnext, advance_time, st, ev);
 }
 
 __global__ __launch_bounds__(256) void k_amr_nbr(KParams P, int* nbr, int nbm) {

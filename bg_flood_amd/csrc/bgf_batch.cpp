@@ -243,7 +243,7 @@ void enqueue_steps(bgf_batch b, int nsteps) {
         if (b->prec == 0) fill_amr(b, (bgf::AmrBuffers<double>*)storage);
         else fill_amr(b, (bgf::AmrBuffers<float>*)storage);
         for (int k = 0; k < nsteps; k++) {
-            bgf::launch_amr_step(b->prec, b->krun, storage, b->d_loop, 1, b->stream, nullptr);
+            bgf::launch_amr_step(b->prec, b->krun, storage, b->d_loop, nullptr, 1, b->stream, nullptr);
             if (b->gauges_on)
                 bgf::launch_gauge_step(b->prec, b->d_h[0], b->d_gcell, b->d_loop, b->cap_members, NSAMP, b->d_ring,
                                        b->d_tring, b->stream);
@@ -263,7 +263,7 @@ void enqueue_steps(bgf_batch b, int nsteps) {
                   (float*)b->d_h[out], (float*)b->d_u[out], (float*)b->d_v[out], (const float*)b->d_zb,
                   (const float*)b->d_cf, (float*)b->d_dh, (float*)b->d_dhu, (float*)b->d_dhv, (float*)b->d_ch};
         }
-        bgf::launch_step(b->prec, b->krun, storage, b->d_loop, 1, b->stream, nullptr);
+        bgf::launch_step(b->prec, b->krun, storage, b->d_loop, nullptr, 1, b->stream, nullptr);
         if (b->gauges_on)
             bgf::launch_gauge_step(b->prec, b->d_h[out], b->d_gcell, b->d_loop, b->cap_members, NSAMP, b->d_ring,
                                    b->d_tring, b->stream);

@@ -61,7 +61,8 @@ struct bgf_handle_s {
     void *d_h[2] = {nullptr, nullptr}, *d_u[2] = {nullptr, nullptr}, *d_v[2] = {nullptr, nullptr};
     void *d_zb = nullptr, *d_cf = nullptr, *d_dh = nullptr, *d_dhu = nullptr, *d_dhv = nullptr;
     double *d_volpart = nullptr, *d_volout = nullptr;
-    bgf::DevLoop* d_loop = nullptr;
+    bgf::DevLoop* d_loop = nullptr;  // two loop states: a step takes one and leaves the next in the other
+    int loop_at = 0;                 // the one that the enqueued work leaves last
     bgf::KParams kp;
     hipStream_t stream = nullptr;
     bool timing = false;
@@ -115,8 +116,8 @@ struct bgf_handle_s {
     std::vector<double> h_xo, h_yo;
     std::vector<double> riv_box, riv_t, riv_q;
     std::vector<int> riv_n;
-    // rivers on the device: boxes, series, offsets, areas, block flags, rates
-    double *d_rbox = nullptr, *d_rt = nullptr, *d_rq = nullptr, *d_rarea = nullptr, *d_rrate = nullptr;
+    // rivers on the device: boxes, series, offsets, areas, block flags
+    double *d_rbox = nullptr, *d_rt = nullptr, *d_rq = nullptr, *d_rarea = nullptr;
     int* d_roff = nullptr;
     unsigned char* d_rblk = nullptr;
     int bed_nx = 0, bed_ny = 0;
@@ -147,7 +148,7 @@ void free_handle(bgf_handle h) {
     F(h->d_bed);
     for (HostSeg& g : h->segs) free_seg(g);
     F(h->d_bseg); F(h->d_seg);
-    F(h->d_rbox); F(h->d_rt); F(h->d_rq); F(h->d_rarea); F(h->d_rrate); F(h->d_roff); F(h->d_rblk);
+    F(h->d_rbox); F(h->d_rt); F(h->d_rq); F(h->d_rarea); F(h->d_roff); F(h->d_rblk);
     F(h->d_blkxo); F(h->d_blkyo); F(h->d_rain_t); F(h->d_rain_v); F(h->d_rframes); F(h->d_rnow);
     for (int k = 0; k < 11; k++) F(h->d_mesh2[k]);
     F(h->d_remap); F(h->d_bxo); F(h->d_byo); F(h->d_flags);
@@ -182,11 +183,12 @@ bgf_status upload_loop(bgf_handle h, const bgf_loop* loop, double endtime) {
     }
     HIPCHK(hipMemcpyAsync(h->d_loop, &L, sizeof(L), hipMemcpyHostToDevice, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    h->loop_at = 0;
     return BGF_OK;
 }
 
 bgf_status download_loop(bgf_handle h, bgf::DevLoop* L) {
-    HIPCHK(hipMemcpyAsync(L, h->d_loop, sizeof(*L), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipMemcpyAsync(L, h->d_loop + h->loop_at, sizeof(*L), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     h->stats_n = L->stats_n;
     h->nstep = L->nstep;
@@ -195,16 +197,18 @@ bgf_status download_loop(bgf_handle h, bgf::DevLoop* L) {
 
 constexpr int GAUGE_CAP = 2048;  // gauge samples kept per gauge
 
-// Output statistics and gauge samples of the state after a step: one-level
-// steps end in buffer `out`, multi-level steps in buffer 0.
-void enqueue_stats(bgf_handle h, int out, int advanced) {
+// Output statistics and gauge samples of the state after a step of parity k,
+// which leaves its loop state in 1 - k: one-level steps end in buffer 1 - k,
+// multi-level steps in buffer 0.
+void enqueue_stats(bgf_handle h, int k, int advanced) {
+    const int b = h->amr ? 0 : 1 - k;
+    const bgf::DevLoop* L = h->d_loop + (1 - k);
     if (h->gevery > 0)
-        bgf::launch_gauge_step(h->prec == 0 ? 0 : 1, h->d_h[h->amr ? 0 : out], h->d_gcell, h->d_loop, 1, GAUGE_CAP,
-                               h->d_gring, h->d_gtring, h->stream);
+        bgf::launch_gauge_step(h->prec == 0 ? 0 : 1, h->d_h[b], h->d_gcell, L, 1, GAUGE_CAP, h->d_gring, h->d_gtring,
+                               h->stream);
     if (!h->stats.mask) return;
-    const int b = h->amr ? 0 : out;
-    bgf::launch_stats(h->prec == 0 ? 0 : 1, h->kp, h->stats, h->d_h[b], h->d_u[b], h->d_v[b], h->d_zb, h->d_loop,
-                      advanced, h->stream);
+    bgf::launch_stats(h->prec == 0 ? 0 : 1, h->kp, h->stats, h->d_h[b], h->d_u[b], h->d_v[b], h->d_zb, L, advanced,
+                      h->stream);
 }
 
 void fill_buffers(bgf_handle h, int in, void* out_storage) {
@@ -241,27 +245,23 @@ void fill_amr_buffers(bgf_handle h, void* storage) {
     else fill_amr_t<float>(h, (bgf::AmrBuffers<float>*)storage);
 }
 
-// One multi-level step: the per-phase launches.
-void enqueue_amr_step(bgf_handle h, const void* storage, int advance_time, hipEvent_t* ev) {
-    bgf::launch_amr_step(h->prec, h->kp, storage, h->d_loop, advance_time, h->stream, ev);
-}
-
-// Enqueues `period` steps (one AMR step, or an even/odd pair of one-level
-// steps) starting at buffer parity 0.
-void enqueue_period(bgf_handle h, int advance_time) {
+// One step of parity k: from loop state k to 1 - k, and on one-level meshes
+// from buffer k to 1 - k.
+void enqueue_step(bgf_handle h, int k, int advance_time, hipEvent_t* ev) {
     alignas(16) unsigned char storage[sizeof(bgf::AmrBuffers<double>)];
+    bgf::DevLoop *L = h->d_loop + k, *Lnext = h->d_loop + (1 - k);
     if (h->amr) {
         fill_amr_buffers(h, storage);
-        bgf::launch_amr_step(h->prec, h->kp, storage, h->d_loop, advance_time, h->stream, nullptr);
-        enqueue_stats(h, 0, advance_time);
-        return;
-    }
-    for (int k = 0; k < 2; k++) {
+        bgf::launch_amr_step(h->prec, h->kp, storage, L, Lnext, advance_time, h->stream, ev);
+    } else {
         fill_buffers(h, k, storage);
-        bgf::launch_step(h->prec, h->kp, storage, h->d_loop, advance_time, h->stream, nullptr);
-        enqueue_stats(h, 1 - k, advance_time);
+        bgf::launch_step(h->prec, h->kp, storage, L, Lnext, advance_time, h->stream, ev);
     }
+    enqueue_stats(h, k, advance_time);
 }
+
+// Steps of a captured graph: an even and an odd one.
+constexpr int PERIOD = 2;
 
 // Runs of many steps replay a captured HIP graph of one period instead of
 // relaunching every kernel (the step is launch-bound on small domains and
@@ -270,7 +270,7 @@ bgf_status graph_steps(bgf_handle h, int nperiods) {
     if (!h->graph) {
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_period(h, 1);
+        for (int k = 0; k < PERIOD; k++) enqueue_step(h, k, 1, nullptr);
         HIPCHK(hipStreamEndCapture(h->stream, &g));
         hipError_t e = hipGraphInstantiate(&h->graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -284,24 +284,14 @@ bgf_status graph_steps(bgf_handle h, int nperiods) {
 }
 
 bgf_status enqueue_steps(bgf_handle h, int nsteps, int advance_time) {
-    const int period = h->amr ? 1 : 2;
-    if (advance_time == 1 && !h->timing && h->use_graph && nsteps >= 2 * period) {
-        bgf_status s = graph_steps(h, nsteps / period);
+    h->loop_at = nsteps & 1;
+    if (advance_time == 1 && !h->timing && h->use_graph && nsteps >= 2 * PERIOD) {
+        bgf_status s = graph_steps(h, nsteps / PERIOD);
         if (s != BGF_OK) return s;
-        nsteps %= period;  // at most one step left, at parity 0
+        nsteps %= PERIOD;  // at most one step left, at parity 0
     }
-    alignas(16) unsigned char storage[sizeof(bgf::AmrBuffers<double>)];
-    if (h->amr) fill_amr_buffers(h, storage);
     for (int k = 0; k < nsteps; k++) {
-        if (h->amr) {
-            enqueue_amr_step(h, storage, advance_time, h->timing ? h->ev : nullptr);
-            enqueue_stats(h, 0, advance_time);
-        } else {
-            fill_buffers(h, k & 1, storage);
-            bgf::launch_step(h->prec, h->kp, storage, h->d_loop, advance_time, h->stream,
-                             h->timing ? h->ev : nullptr);
-            enqueue_stats(h, 1 - (k & 1), advance_time);
-        }
+        enqueue_step(h, k & 1, advance_time, h->timing ? h->ev : nullptr);
         if (h->timing) {
             HIPCHK(hipEventSynchronize(h->ev[3]));
             float a = 0, b = 0, c = 0;
@@ -320,7 +310,7 @@ bgf_status settle(bgf_handle h, int steps_done) {
     if (!h->amr && (steps_done & 1)) {
         const void* src[3] = {h->d_h[1], h->d_u[1], h->d_v[1]};
         void* dst[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};
-        bgf::launch_settle(h->prec, h->kp, src, dst, h->d_loop, h->stream);
+        bgf::launch_settle(h->prec, h->kp, src, dst, h->d_loop + h->loop_at, h->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(h->stream));
     }
@@ -487,11 +477,10 @@ bgf_status setup_segments(bgf_handle h) {
 // discharge cell of any river are flagged.  Uploads everything the kernels read.
 bgf_status setup_rivers(bgf_handle h) {
     auto F = [](auto*& p) { if (p) (void)hipFree(p); p = nullptr; };
-    F(h->d_rbox); F(h->d_rt); F(h->d_rq); F(h->d_rarea); F(h->d_rrate); F(h->d_roff); F(h->d_rblk);
+    F(h->d_rbox); F(h->d_rt); F(h->d_rq); F(h->d_rarea); F(h->d_roff); F(h->d_rblk);
     bgf::KParams& kp = h->kp;
     kp.nriver = 0;
     kp.rbox = kp.rt = kp.rq = kp.rarea = nullptr;
-    kp.rrate = nullptr;
     kp.roff = nullptr;
     kp.rblk = nullptr;
     const int nr = (int)h->riv_n.size();
@@ -539,7 +528,6 @@ bgf_status setup_rivers(bgf_handle h) {
               hipMalloc((void**)&h->d_rt, sizeof(double) * tt.size()) == hipSuccess &&
               hipMalloc((void**)&h->d_rq, sizeof(double) * qq.size()) == hipSuccess &&
               hipMalloc((void**)&h->d_rarea, sizeof(double) * nk) == hipSuccess &&
-              hipMalloc((void**)&h->d_rrate, sizeof(double) * 2 * nk) == hipSuccess &&
               hipMalloc((void**)&h->d_roff, sizeof(int) * (nk + 1)) == hipSuccess &&
               hipMalloc((void**)&h->d_rblk, h->cap) == hipSuccess;
     ok = ok && hipMemcpy(h->d_rbox, box.data(), sizeof(double) * box.size(), hipMemcpyHostToDevice) == hipSuccess &&
@@ -547,11 +535,10 @@ bgf_status setup_rivers(bgf_handle h) {
          hipMemcpy(h->d_rq, qq.data(), sizeof(double) * qq.size(), hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(h->d_rarea, area.data(), sizeof(double) * nk, hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(h->d_roff, off.data(), sizeof(int) * (nk + 1), hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(h->d_rblk, blk.data(), h->cap, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemset(h->d_rrate, 0, sizeof(double) * 2 * nk) == hipSuccess;
+         hipMemcpy(h->d_rblk, blk.data(), h->cap, hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) return fail(BGF_ERR_HIP, "river upload failed");
     kp.nriver = nk;
-    kp.rbox = h->d_rbox; kp.rt = h->d_rt; kp.rq = h->d_rq; kp.rarea = h->d_rarea; kp.rrate = h->d_rrate;
+    kp.rbox = h->d_rbox; kp.rt = h->d_rt; kp.rq = h->d_rq; kp.rarea = h->d_rarea;
     kp.roff = h->d_roff; kp.rblk = h->d_rblk;
     return BGF_OK;
 }
@@ -610,7 +597,7 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     ok = ok && A(&h->d_zb, h->es * SA) && A(&h->d_cf, h->es * SA);
     ok = ok && A(&h->d_dh, h->es * SA) && A(&h->d_dhu, h->es * SA) && A(&h->d_dhv, h->es * SA);
     ok = ok && A((void**)&h->d_volpart, sizeof(double) * cap) && A((void**)&h->d_volout, sizeof(double));
-    ok = ok && A((void**)&h->d_loop, sizeof(bgf::DevLoop));
+    ok = ok && A((void**)&h->d_loop, 2 * sizeof(bgf::DevLoop));
     ok = ok && A((void**)&h->d_blkxo, sizeof(double) * cap) && A((void**)&h->d_blkyo, sizeof(double) * cap);
     h->amr = multilevel;
     if (p->precision == BGF_FP32_COMP && !multilevel) ok = ok && A(&h->d_ch, h->es * SA);
@@ -948,8 +935,9 @@ bgf_status bgf_step_device(bgf_handle h, void* hh, void* zs, void* u, void* v, c
             auto* B = (bgf::StepBuffers<float>*)storage;
             B->h = (const float*)hh; B->u = (const float*)u; B->v = (const float*)v;
         }
-        bgf::launch_step(h->prec, h->kp, storage, h->d_loop, 0, h->stream, nullptr);
-        enqueue_stats(h, 1, 0);
+        bgf::launch_step(h->prec, h->kp, storage, h->d_loop, h->d_loop + 1, 0, h->stream, nullptr);
+        enqueue_stats(h, 0, 0);
+        h->loop_at = 1;
         const void* res[3] = {h->d_h[1], h->d_u[1], h->d_v[1]};
         void* out[4] = {hh, zs, u, v};
         void* keep[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};

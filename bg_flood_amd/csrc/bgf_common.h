@@ -183,70 +183,93 @@ __device__ __forceinline__ void slot_min(DevLoop* L, int k, double v) {
     atomicMin(&L->slot64[k & (NSLOT - 1)], (unsigned long long)__double_as_longlong(v));
 }
 
-// One wave (threads 0-63) per loop state: min of the 64 block-minimum slots and 1/epsi
-// (slots reset for the next step), then the clamp and the output-time landing
-// of CalctimestepCPU in FP64.  mode 0: a step that leaves totaltime to the
-// caller; 1: a step followed by totaltime += dt; 2: the initial dt only.
-template <class T> __device__ __forceinline__ void reduce_dt_wave(DevLoop* L, int mode) {
-    const int t = threadIdx.x;
-    if (L->done) {
-        if (t == 0) L->go = 0;
+// Minimum of a loop state's slots, by a whole wave.
+template <class T> __device__ __forceinline__ T slots_min(const DevLoop* L) {
+    const int l = threadIdx.x & 63;
+    T m = sizeof(T) == 8 ? (T)__longlong_as_double((long long)L->slot64[l]) : (T)__uint_as_float(L->slot32[l]);
+    for (int off = 32; off > 0; off >>= 1) {
+        const T o = __shfl_xor(m, off, 64);
+        m = o < m ? o : m;
+    }
+    return m;
+}
+__device__ __forceinline__ void slots_empty(DevLoop* L) {
+    const int l = threadIdx.x & 63;
+    L->slot32[l] = 0x7f800000u;
+    L->slot64[l] = 0x7ff0000000000000ull;
+}
+
+// A loop state past the dt reduction of its step, from the slots' minimum m:
+// the smaller of m and 1/epsi, the clamp and the output-time landing of
+// CalctimestepCPU in FP64.  mode 0: a step that leaves totaltime to the caller;
+// 1: a step followed by totaltime += dt; 2: the initial dt only.
+template <class T> __device__ __forceinline__ void advance_loop(LoopState& L, T m, int mode) {
+    if (L.done) {
+        L.go = 0;
         return;
     }
     const T epsi = sizeof(T) == 8 ? T(2.220446049250313e-16) : T(1.1920928955078125e-07);
-    T m;
-    if (sizeof(T) == 8) {
-        unsigned long long b = L->slot64[t];
-        m = (T)__longlong_as_double((long long)b);
-        L->slot64[t] = 0x7ff0000000000000ull;
-    } else {
-        unsigned int b = L->slot32[t];
-        m = (T)__uint_as_float(b);
-        L->slot32[t] = 0x7f800000u;
+    if (L.rain_n > 0) {
+        // the uniform rain of this step, at its start (Forcingthisstep,
+        // src/Updateforcing.cu:45-60, interptime src/Util_CPU.cu:107-110)
+        const double tt = L.totaltime;
+        int k = 1;
+        while (k < L.rain_n - 1 && L.rain_t[k] - tt < 0.0) k++;
+        const double prev = L.rain_v[k - 1];
+        const double now = prev + (tt - L.rain_t[k - 1]) / (L.rain_t[k] - L.rain_t[k - 1]) * (L.rain_v[k] - prev);
+        L.rain = now;
+        L.rate64 = now / 1000.0 / 3600.0;
+        L.rate32 = (float)now / 1000.0f / 3600.0f;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        T o = __shfl_xor(m, off, 64);
-        m = o < m ? o : m;
+    L.tstart = L.totaltime;
+    L.tpred = L.totaltime + L.dt * 0.5;
+    T dt = T(1.0) / epsi;
+    dt = m < dt ? m : dt;
+    if ((double)dt > 1.5 * L.dtmax) dt = T(1.5 * L.dtmax);
+    double rem = L.nextoutputtime - L.totaltime;
+    if (ceil(rem / (double)dt) > 0.0) dt = T(rem / ceil(rem / (double)dt));
+    L.dt = (double)dt;
+    L.dtmax = (double)dt;
+    L.tcorr = L.totaltime + L.dt;
+    if (!isfinite((double)dt) || dt <= T(0)) L.bad |= 1;
+    if (mode != 2) {
+        L.go = 1;
+        L.steps_done = L.steps_done + 1;
+        L.nstep = L.nstep + 1;
+        L.stats_n = L.stats_n + 1;
     }
-    if (t == 0) {
-        if (L->rain_n > 0) {
-            // the uniform rain of this step, at its start (Forcingthisstep,
-            // src/Updateforcing.cu:45-60, interptime src/Util_CPU.cu:107-110)
-            const double tt = L->totaltime;
-            int k = 1;
-            while (k < L->rain_n - 1 && L->rain_t[k] - tt < 0.0) k++;
-            const double prev = L->rain_v[k - 1];
-            const double now = prev + (tt - L->rain_t[k - 1]) / (L->rain_t[k] - L->rain_t[k - 1]) * (L->rain_v[k] - prev);
-            L->rain = now;
-            L->rate64 = now / 1000.0 / 3600.0;
-            L->rate32 = (float)now / 1000.0f / 3600.0f;
-        }
-        L->tpred = L->totaltime + L->dt * 0.5;
-        T dt = T(1.0) / epsi;
-        dt = m < dt ? m : dt;
-        if ((double)dt > 1.5 * L->dtmax) dt = T(1.5 * L->dtmax);
-        double rem = L->nextoutputtime - L->totaltime;
-        if (ceil(rem / (double)dt) > 0.0) dt = T(rem / ceil(rem / (double)dt));
-        L->dt = (double)dt;
-        L->dtmax = (double)dt;
-        L->tcorr = L->totaltime + L->dt;
-        if (!isfinite((double)dt) || dt <= T(0)) L->bad |= 1;
-        if (mode != 2) {
-            L->go = 1;
-            L->steps_done = L->steps_done + 1;
-            L->nstep = L->nstep + 1;
-            L->stats_n = L->stats_n + 1;
-        }
-        if (mode == 1) {
-            L->totaltime = L->totaltime + L->dt;
-            if (L->totaltime >= L->endtime) L->done = 1;
-            // CrashDetection (src/Mainloop.cu:648-660): after the step that advanced the time
-            if (L->dt < L->dtmin && L->totaltime < L->endtime) {
-                L->crashed = 1;
-                L->done = 1;
-            }
+    if (mode == 1) {
+        L.totaltime = L.totaltime + L.dt;
+        if (L.totaltime >= L.endtime) L.done = 1;
+        // CrashDetection (src/Mainloop.cu:648-660): after the step that advanced the time
+        if (L.dt < L.dtmin && L.totaltime < L.endtime) {
+            L.crashed = 1;
+            L.done = 1;
         }
     }
+}
+
+// The reduction as a launch of its own, one wave per loop state: L's state past
+// it goes to Lnext (L itself for batches), with empty slots.
+template <class T> __device__ __forceinline__ void reduce_dt_wave(const DevLoop* L, DevLoop* Lnext, int mode) {
+    LoopState S = *L;
+    advance_loop<T>(S, slots_min<T>(L), mode);
+    slots_empty(Lnext);
+    if (threadIdx.x == 0) *(LoopState*)Lnext = S;
+}
+
+// The state of a step past its dt reduction, worked out by every wave of the
+// launch that follows the predictor from the predictor's state L; the first
+// wave of workgroup 0 leaves it in Lnext.  A reduction launch of its own took
+// 4.7 us a step, a third of what a small domain's other two launches need.
+template <class T> __device__ __forceinline__ LoopState step_state(const DevLoop* L, DevLoop* Lnext, int mode) {
+    LoopState S = *L;
+    advance_loop<T>(S, slots_min<T>(L), mode);
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        if (threadIdx.x == 0) *(LoopState*)Lnext = S;
+        slots_empty(Lnext);
+    }
+    return S;
 }
 
 // calcres (src/Util_CPU.cu:194-198): cell size of a level.
@@ -281,10 +304,11 @@ template <class T> __device__ __forceinline__ T rain_map_rate(const KParams& P, 
 // The per-step rain depth of a cell, m: max(rate / 1000 / 3600 * dt, 0)
 // (src/Updateforcing.cu:560) from the rain map, or from the loop's uniform
 // rate (precomputed as rate64 / rate32).
-template <class T> __device__ __forceinline__ T rain_depth(const KParams& P, const DevLoop* L, int ib, int ix, int iy, T dt) {
+template <class T>
+__device__ __forceinline__ T rain_depth(const KParams& P, const LoopState& L, int ib, int ix, int iy, T dt) {
     T a;
     if (P.rnow) a = rain_map_rate<T>(P, ib, ix, iy) / T(1000.0) / T(3600.0) * dt;
-    else a = (sizeof(T) == 8 ? T(L->rate64) : T(L->rate32)) * dt;
+    else a = (sizeof(T) == 8 ? T(L.rate64) : T(L.rate32)) * dt;
     return a < T(0.0) ? T(0.0) : a;  // std::max(a, 0)
 }
 
@@ -383,8 +407,13 @@ __device__ __forceinline__ bool bnd_flux(const KParams& P, int s, int type, floa
 // by river (InjectRiverCPU, src/Updateforcing.cu:314-363): a cell receives a
 // river's rate when its box, formed in T, overlaps the river's (OBBdetect,
 // src/Util_CPU.cu:286-296); only blocks that held a discharge cell when the
-// rivers were set (or the mesh last changed) are visited.
-template <class T> __device__ __forceinline__ T river_inflow(const KParams& P, int ib, int ix, int iy, T dh) {
+// rivers were set (or the mesh last changed) are visited.  The rate is the
+// flow at tt, the step's start, over the discharge area (AddRiverForcing,
+// src/Updateforcing.cu:146-165): interpolated between the first entry later
+// than tt and the one before, where it is used (a launch of its own for it
+// took 4.6 us a step).
+template <class T>
+__device__ __forceinline__ T river_inflow(const KParams& P, int ib, int ix, int iy, double tt, T dh) {
     if (!P.nriver || !P.rblk[ib]) return dh;
     const T levdx = calcres(T(P.dx), P.level[ib]);
     const T xllo = T(P.xo + P.bxo[ib]), yllo = T(P.yo + P.byo[ib]);
@@ -394,7 +423,17 @@ template <class T> __device__ __forceinline__ T river_inflow(const KParams& P, i
         const double* b = P.rbox + 4 * r;
         const bool tx = T(b[0]) <= xr && T(b[1]) >= xl;
         const bool ty = T(b[2]) <= yt && T(b[3]) >= yb;
-        if (tx && ty) dh += sizeof(T) == 8 ? T(P.rrate[2 * r]) : T(P.rrate[2 * r + 1]);
+        if (tx && ty) {
+            const double* t = P.rt + P.roff[r];
+            const double* q = P.rq + P.roff[r];
+            const int n = P.roff[r + 1] - P.roff[r];
+            int e = 0;
+            while (e < n - 1 && t[e] - tt <= 0.0) e++;  // the reference does not stop at the end
+            const int a = e - 1 > 0 ? e - 1 : 0;
+            const double flow = q[a] + (tt - t[a]) / (t[e] - t[a]) * (q[e] - q[a]);
+            // the reference's array of rates is a T
+            dh += sizeof(T) == 8 ? T(flow / P.rarea[r]) : T((double)(float)flow / P.rarea[r]);
+        }
     }
     return dh;
 }

@@ -6,45 +6,50 @@ namespace bgf {
 
 constexpr int NSLOT = 64;  // block-minimum dt slots (atomic min, spread to avoid contention)
 
-// Device-resident Loop<T> time keeping (src/Arrays.h:358-366), run flags and
-// the dt reduction slots (bit patterns of positive floats; +inf when empty).
-struct DevLoop;
-// Sets a loop state's rain rate and its per-second depth rates.
-inline void set_rain(DevLoop& L, double rain_mmh);
-
-struct DevLoop {
+// Device-resident Loop<T> time keeping (src/Arrays.h:358-366) and run flags.
+struct LoopState {
     double nextoutputtime;
     double dt;
     double dtmax;
     double totaltime;
     double endtime;  // the run stops once totaltime reaches it
     double rain;     // uniform rain rate, mm/h (Rain.nowvalue)
-    double rate64;   // T(rain) / T(1000) / T(3600) in FP64 and FP32: the depth rate in m/s
-    float rate32;    // (src/Updateforcing.cu:559), formed once per loop instead of per cell
+    double rate64;   // T(rain) / T(1000) / T(3600) in FP64, and rate32 in FP32: the depth rate in m/s
+                     // (src/Updateforcing.cu:559), formed once per loop instead of per cell
+    double tcorr;    // time of the corrector's boundary values: the step's start + dt (set by the dt reduction)
+    double tpred;    // time of the predictor's boundary fluxes: the step's start + half the previous dt (set
+                     // by the dt reduction before it replaces dt; multi-level kernels read it after it)
+    double tstart;   // time at the step's start (set by the dt reduction)
+    double cf_value; // batch member: the roughness where cf_uniform is set
+    double dtmin;    // Param.dtmin: a run stops after a step with dt < dtmin before its end time (0: never)
+    // uniform rain as a time series (rain_n > 0): the rate of each step is
+    // interpolated at its start by the dt reduction, which sets rate64/rate32
+    const double* rain_t;
+    const double* rain_v;
+    int rain_n;
+    float rate32;
     int done;        // totaltime reached the end time: later steps are no-ops
     int bad;         // a non-finite or non-positive dt was produced
     int steps_done;  // steps executed since the loop was uploaded
     int go;          // set by the dt reduction: the corrector half of this step runs
     int nstep;       // steps since the domain started (gauge sampling counts these)
     int gevery;      // gauge sampling period in steps (batch members)
-    // uniform rain as a time series (rain_n > 0): the rate of each step is
-    // interpolated at its start by the dt reduction, which sets rate64/rate32
-    const double* rain_t;
-    const double* rain_v;
-    int rain_n;
-    double tcorr;    // time of the corrector's boundary values: the step's start + dt (set by the dt reduction)
-    double tpred;    // time of the predictor's boundary fluxes: the step's start + half the previous dt (set
-                     // by the dt reduction before it replaces dt; multi-level kernels read it after it)
     int stats_n;     // steps since the output statistics' means were reset (Loop.nstep of Calcmeanmax)
     int cf_uniform;  // batch member: every active cell has roughness cf_value (the corrector skips the cf array)
-    double cf_value;
-    double dtmin;    // Param.dtmin: a run stops after a step with dt < dtmin before its end time (0: never)
     int crashed;     // the run stopped on dtmin (CrashDetection, src/Mainloop.cu:648-660)
+    int unused;      // keeps the size a multiple of eight, so copies leave no padding behind
+};
+// A loop state with the dt reduction's slots (bit patterns of positive floats; +inf when empty).
+// A single domain has two: a step's predictor fills the slots of the first, its later launches
+// each work the new state out from them, and one workgroup leaves it, with empty slots, in the
+// second, which the next step takes as its first.  A batch has one per member, reduced in place.
+struct DevLoop : LoopState {
     unsigned int slot32[NSLOT];
     unsigned long long slot64[NSLOT];
 };
 
-inline void set_rain(DevLoop& L, double rain_mmh) {
+// Sets a loop state's rain rate and its per-second depth rates.
+inline void set_rain(LoopState& L, double rain_mmh) {
     L.rain = rain_mmh;
     L.rate64 = rain_mmh / 1000.0 / 3600.0;
     volatile float r = (float)rain_mmh;  // each division rounded to float, as on the device
@@ -137,8 +142,7 @@ struct KParams {
     double bzsoffset, btaper, binittime;
     // river discharges (nriver > 0): each river's box (xstart, xend, ystart,
     // yend), flow series (time rt, flow rq from roff[r] to roff[r+1]), its
-    // discharge area, the blocks that may receive water, and the rates of the
-    // step (rrate[2r] in FP64, rrate[2r+1] the FP32 value), set at its start
+    // discharge area, and the blocks that may receive water
     int nriver;
     const double* rbox;
     const double* rt;
@@ -146,7 +150,6 @@ struct KParams {
     const int* roff;
     const double* rarea;
     const unsigned char* rblk;
-    double* rrate;
 };
 
 // Layout of a block's metric terms (spherical grids, src/Spherical.cu:15-64):
@@ -174,10 +177,11 @@ template <class T> struct StepBuffers {
 };
 
 // ev (optional): four events recorded before the predictor, after it, after
-// the reduction and after the corrector.  With P.sid set, the block list packs
-// P.nmember domains and L holds one loop state per member.
-void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* L, int advance_time,
-                 hipStream_t st, hipEvent_t* ev);
+// the reduction and after the corrector.  L: the step's loop state, Lnext: the
+// next step's.  With P.sid set, the block list packs P.nmember domains, L holds
+// one loop state per member, and Lnext is not used.
+void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext,
+                 int advance_time, hipStream_t st, hipEvent_t* ev);
 // Workgroups of a persistent launch; wg_per_cu > 0 caps the resident workgroups per CU.
 int persistent_grid(int precision, int corrector, int nblk, int wg_per_cu);
 void launch_init_dt(int precision, const KParams& P, const void* h, DevLoop* L, hipStream_t st);
@@ -211,8 +215,9 @@ void launch_export(int precision, const KParams& P, const void* const* src, cons
 void launch_refine_flags(int precision, const KParams& P, const void* a, const void* b, int mode, double lo,
                          double hi, unsigned char* flags, hipStream_t st);
 
-// dt reduction of the block-minimum slots, clamp and output landing (one wave).
-void launch_reduce_dt(int precision, DevLoop* L, int nloop, int advance_time, hipStream_t st);
+// dt reduction of the block-minimum slots, clamp and output landing (one wave per loop state), from
+// L to Lnext (which may be L).
+void launch_reduce_dt(int precision, DevLoop* L, DevLoop* Lnext, int nloop, int advance_time, hipStream_t st);
 
 // Arrays of the multi-level step (the reference's Model<T> layout).
 template <class T> struct AmrBuffers {
@@ -227,8 +232,8 @@ template <class T> struct AmrBuffers {
 // One step on a multi-level mesh: precision 0 FP64 and 1 FP32 in the reference
 // arithmetic; 2 and 3 (BGF_FP32_FAST, BGF_FP32_COMP) FP32 with hardware
 // reciprocals and square roots in the slopes and the fluxes.
-void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLoop* L, int advance_time,
-                     hipStream_t st, hipEvent_t* ev);
+void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext,
+                     int advance_time, hipStream_t st, hipEvent_t* ev);
 // Fills nbr (NBR ints per block slot, nbm slots) from P's eight neighbour arrays
 // and the levels; slots whose neighbours are outside [0, nbm) get level 0.
 constexpr int NBR = 16;
@@ -237,8 +242,8 @@ enum { REC_BACK = 1 << 8, REC_FINER = 1 << 9, REC_EDGE = 1 << 10 };
 void launch_amr_nbr(const KParams& P, int* nbr, int nbm, hipStream_t st);
 // Halo of a static field (the bed) on a multi-level mesh, src/InitialConditions.cu:135-147.
 void launch_amr_fill(int precision, const KParams& P, void* z, hipStream_t st);
-// The rain map of the coming step from the rain frames (nothing without frames),
-// and the river discharge rates of the coming step (nothing without rivers).
+// The rain map of the coming step from the rain frames, and the boundary level
+// maps of the coming step (nothing without frames).
 void launch_rain_now(const KParams& P, const DevLoop* L, hipStream_t st);
 // The step's halo fill of h, u, v on a multi-level mesh (src/Halo.cu:586-616) by itself.
 void launch_amr_halo(int precision, const KParams& P, void* h, void* u, void* v, const void* zb, hipStream_t st);

@@ -16,11 +16,12 @@
 //                (src/Advection.cu:160-254, src/Boundary.cu:587-760), and the
 //                block's minimum CFL step (src/Advection.cu:470-498), which
 //                it merges into one of 64 device slots with an atomic min.
-//   k_reduce_dt  one wave: minimum of the slots and 1/epsi, the 1.5x growth
-//                clamp and the output-time landing in FP64
-//                (src/Advection.cu:511-535), then totaltime += dt
-//                (src/Mainloop.cu:60), all on the GPU.
-//   k_corrector  rebuilds U* = U + dt/2 L(U) (src/Advection.cu:332-385) on
+//   k_corrector  works out dt from the slots (step_state: their minimum and
+//                1/epsi, the 1.5x growth clamp and the output-time landing in
+//                FP64, src/Advection.cu:511-535, then totaltime += dt,
+//                src/Mainloop.cu:60; batches, whose blocks are of many members,
+//                have k_reduce_dt do it once per member);
+//                rebuilds U* = U + dt/2 L(U) (src/Advection.cu:332-385) on
 //                its own 20x20 tile from U and the predictor tendencies, so
 //                no U* array is written; forms the corrector fluxes of U*,
 //                advances U^{n+1} = U + dt L(U*), applies bottom friction
@@ -621,6 +622,14 @@ __device__ __forceinline__ void advance(const Cst<T>& C, int fmc, T dt, T hold, 
 // its own L2: the persistent kernels give each XCD a contiguous range of
 // blocks so a block's neighbours are mostly fetched into the same L2.
 
+// A value that every lane holds, kept in scalar registers.
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ double uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
 // Cell k of block ib of array a: the array base (a kernel argument, in scalar
 // registers for the whole launch) plus one 32-bit byte offset per thread that
 // carries both the block and the cell, boff(ib) + k * sizeof(T), so each load
@@ -717,6 +726,10 @@ template <class T, bool FAST> __device__ __forceinline__ void wave_flush(const C
 // own at zero: the first launch from the allocation, later ones from the
 // other kernel's launch in between (the zeroing comes before a kernel's
 // early return, and a launch that returns early takes no position).
+// A workgroup's first position is its rank on the XCD, and the queue hands out
+// those after the workgroups' first ones; where the XCD's range has no more
+// (more false: a domain of up to about 1,500 blocks) nothing is taken.
+//
 // Queue positions.  Each workgroup's positions increase (one thread's
 // atomics on one counter are ordered), so the first one past the range ends
 // the walk and no position is lost; the workgroup reads position j from slot
@@ -742,13 +755,6 @@ __device__ __forceinline__ int queue_take(int* q) {
     int z = 0;
     asm volatile("" : "+v"(z));
     return __hip_atomic_fetch_add(q + z, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void queue_start(int* q, int start, int* next, int t, int& pend) {
-    if (t == 0) {
-        const int p0 = queue_take(q);
-        pend = queue_take(q);
-        next[0] = start + p0;
-    }
 }
 __device__ __forceinline__ void queue_publish(int* q, int start, int* next, int j, int t, int& pend) {
     if (t == 0) {
@@ -799,16 +805,16 @@ __global__ __launch_bounds__(256) void k_predictor(KParams P, Cst<T> C, StepBuff
             sh = ldo(B.h, so); sz = ldo(B.zb, so); su = ldo(B.u, so); sv = ldo(B.v, so);
         }
     };
-    queue_take_now(qc, R.start, s.next, 0, t);
-    queue_take_now(qc, R.start, s.next, 1, t);
-    __syncthreads();
-    int pos = queue_read(s.next, 0);
+    const int nwg = gridDim.x / NXCD, first = R.start + nwg;
+    const bool more = R.end > first;
+    int pos = R.start + blockIdx.x / NXCD;
     int g = 1;  // the next position to read
     Nb cur;
     if (pos < R.end) {
         cur = block_nb<BATCH>(P, pos);
         fetch(cur);
     }
+    if (more) queue_take_now(qc, first, s.next, 1, t);
     for (int npos; pos < R.end; pos = npos) {
         Q4<T> qv;
         qv.a = ph; qv.b = DEV ? pz : pz + ph; qv.c = pu; qv.d = pv;
@@ -820,10 +826,10 @@ __global__ __launch_bounds__(256) void k_predictor(KParams P, Cst<T> C, StepBuff
                 s.q[cs] = r;
             }
         }
-        queue_take_now(qc, R.start, s.next, g + 1, t);
+        if (more) queue_take_now(qc, first, s.next, g + 1, t);
         __syncthreads();
         const Nb n = cur;
-        npos = queue_read(s.next, g++);
+        npos = more ? queue_read(s.next, g++) : R.end;
         if (npos < R.end) {
             cur = block_nb<BATCH>(P, npos);
             fetch(cur);
@@ -845,7 +851,7 @@ __global__ __launch_bounds__(256) void k_predictor(KParams P, Cst<T> C, StepBuff
             // boundary values at the predictor's time, totaltime + dt/2 with the previous dt (src/FlowCPU.cu:94)
             open_sides<T, FAST>(A, qv, C, P, t, n.ib, n.nL, n.nR, n.nB, n.nT, L->totaltime + L->dt * 0.5, B.h, B.u, B.v,
                                 B.zb, dh, dhu, dhv);
-        if (EXT && P.nriver) dh = river_inflow<T>(P, n.ib, x, y, dh);
+        if (EXT && P.nriver) dh = river_inflow<T>(P, n.ib, x, y, L->totaltime, dh);
         const unsigned oi = boff_i<T>(n.ib) + ki;
         stno(B.dh, oi, dh);
         stno(B.dhu, oi, dhu);
@@ -874,9 +880,12 @@ template <class T> __device__ __forceinline__ T kahan_add(T h, T d, T& c) {
 // update accumulates with a compensated (Kahan) sum, so the small increments
 // of rain and of slow flows are not lost to FP32 rounding of h.
 template <class T, bool FAST, bool BATCH, bool COMP, bool EXT>
-__device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C, const StepBuffers<T>& B, DevLoop* L) {
+__device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C, const StepBuffers<T>& B, DevLoop* L,
+                                               DevLoop* Lnext, int mode) {
+    LoopState S;
+    if (!BATCH) S = step_state<T>(L, Lnext, mode);
     if (blockIdx.x == 0 && threadIdx.x < NXCD) P.queue[threadIdx.x * QSTRIDE] = 0;  // the predictor's
-    if (!BATCH && !L->go) return;
+    if (!BATCH && !S.go) return;
     __shared__ Tile<T, FAST> s;
     const int t = threadIdx.x;
     const int x = t & 15, y = t >> 4;
@@ -908,13 +917,14 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
             sz = ldo(B.zb, so);
         }
     };
-    // The step's dt and rain rate are uniform over a launch (one domain): read once with scalar loads.
-    const T dt_one = BATCH ? T(0) : T(lds_f64(&L->dt));
-    const T rate_one = BATCH ? T(0) : (sizeof(T) == 8 ? T(lds_f64(&L->rate64)) : T(lds_f32(&L->rate32)));
+    // The step's dt and rain rate are uniform over a launch (one domain).
+    const T dt_one = BATCH ? T(0) : uniform(T(S.dt));
+    const T rate_one = BATCH ? T(0) : uniform(sizeof(T) == 8 ? T(S.rate64) : T(S.rate32));
+    const int nwg = gridDim.x / NXCD, first_pos = R.start + nwg;
+    const bool more = R.end > first_pos;
     int pend = 0;
-    queue_start(qc, R.start, s.next, t, pend);
-    __syncthreads();
-    int pos = queue_read(s.next, 0);
+    if (more && t == 0) pend = queue_take(qc);
+    int pos = R.start + blockIdx.x / NXCD;
     int g = 1;  // the next position to read
     Nb cur;
     if (pos < R.end) {
@@ -922,11 +932,11 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
         fetch(cur);
     }
     for (int npos; pos < R.end; pos = npos) {
-        const DevLoop* Lm = L + cur.sid;
+        const DevLoop* Lm = L + (BATCH ? cur.sid : 0);
         if (BATCH && !ldu(&Lm->go, 0)) {
-            queue_publish(qc, R.start, s.next, g, t, pend);
+            if (more) queue_publish(qc, first_pos, s.next, g, t, pend);
             __syncthreads();
-            npos = queue_read(s.next, g++);
+            npos = more ? queue_read(s.next, g++) : R.end;
             if (npos < R.end) {
                 cur = block_nb<BATCH>(P, R.start + R.end - 1 - npos);
                 fetch(cur);
@@ -957,10 +967,10 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
                 s.q[cs] = r;
             }
         }
-        queue_publish(qc, R.start, s.next, g, t, pend);
+        if (more) queue_publish(qc, first_pos, s.next, g, t, pend);
         __syncthreads();
         const Nb n = cur;
-        npos = queue_read(s.next, g++);
+        npos = more ? queue_read(s.next, g++) : R.end;
         if (npos < R.end) {
             cur = block_nb<BATCH>(P, R.start + R.end - 1 - npos);
             fetch(cur);
@@ -973,8 +983,8 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
                                           dhu, dhv);
         if (EXT && P.bopen && (nL == ib || nR == ib || nB == ib || nT == ib))
             // boundary values at totaltime + dt, from the step-start state (src/FlowCPU.cu:187)
-            open_sides<T, FAST>(A, qs, C, P, t, ib, nL, nR, nB, nT, L->tcorr, B.h, B.u, B.v, B.zb, dh, dhu, dhv);
-        if (EXT && P.nriver) dh = river_inflow<T>(P, ib, x, y, dh);
+            open_sides<T, FAST>(A, qs, C, P, t, ib, nL, nR, nB, nT, S.tcorr, B.h, B.u, B.v, B.zb, dh, dhu, dhv);
+        if (EXT && P.nriver) dh = river_inflow<T>(P, ib, x, y, S.tstart, dh);
         T h1, u1, v1;
         const unsigned oc = boff<T>(ib) + kb, oci = boff_i<T>(ib) + ki;  // this block's cells
         if (COMP) {
@@ -993,7 +1003,7 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
         if (P.rain_on) {
             T act = (double)zb0 < C.mask_d ? T(1.0) : T(0.0);
             if (EXT) {
-                rainhh = rain_depth<T>(P, Lm, ib, x, y, dt) * act;
+                rainhh = rain_depth<T>(P, S, ib, x, y, dt) * act;
             } else {
                 const T rate = BATCH ? (sizeof(T) == 8 ? T(lds_f64(&Lm->rate64)) : T(lds_f32(&Lm->rate32))) : rate_one;
                 const T a = rate * dt;
@@ -1078,18 +1088,18 @@ __device__ __forceinline__ void corrector_body(const KParams& P, const Cst<T>& C
 // ones held to four waves, the others unbounded (forced into 80 VGPRs the
 // batch corrector measured 3 % slower).
 template <class T, bool FAST, bool BATCH, bool COMP>
-__global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : FAST ? 6 : 5) void k_corrector(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : FAST ? 6 : 5) void k_corrector(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L, DevLoop* Lnext, int mode) {
     static_assert(!BATCH, "batches use k_corrector_wide");
-    corrector_body<T, FAST, false, COMP, false>(P, C, B, L);
+    corrector_body<T, FAST, false, COMP, false>(P, C, B, L, Lnext, mode);
 }
 template <class T, bool FAST, bool BATCH, bool COMP, bool EXT>
-__global__ __launch_bounds__(256, EXT && sizeof(T) == 4 ? 4 : 1) void k_corrector_wide(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L) {
-    corrector_body<T, FAST, BATCH, COMP, EXT>(P, C, B, L);
+__global__ __launch_bounds__(256, EXT && sizeof(T) == 4 ? 4 : 1) void k_corrector_wide(KParams P, Cst<T> C, StepBuffers<T> B, DevLoop* L, DevLoop* Lnext, int mode) {
+    corrector_body<T, FAST, BATCH, COMP, EXT>(P, C, B, L, Lnext, mode);
 }
 
 // One wave per loop state: reduce_dt_wave (the slots' minimum, clamp, landing, time keeping).
-template <class T> __global__ __launch_bounds__(64) void k_reduce_dt(DevLoop* L, int mode) {
-    reduce_dt_wave<T>(L + blockIdx.x, mode);
+template <class T> __global__ __launch_bounds__(64) void k_reduce_dt(DevLoop* L, DevLoop* Lnext, int mode) {
+    reduce_dt_wave<T>(L + blockIdx.x, Lnext + blockIdx.x, mode);
 }
 
 // Output statistics after a step (Calcmeanmax, src/Meanmax.cu:15-112), all
@@ -1173,24 +1183,6 @@ __global__ __launch_bounds__(256) void k_rain_now(KParams P, const DevLoop* L) {
     P.rnow[i] = (float)((double)uo + (tt - P.rdtf * k) * (double)(un - uo) / P.rdtf);
 }
 
-// River discharge rates of a step, at its start (AddRiverForcing,
-// src/Updateforcing.cu:146-165): the flow interpolated at totaltime between the
-// first entry later than it and the one before, over the discharge area.
-__global__ void k_river_rates(KParams P, const DevLoop* L) {
-    const int r = threadIdx.x;
-    if (r >= P.nriver || L->done) return;
-    const double* t = P.rt + P.roff[r];
-    const double* q = P.rq + P.roff[r];
-    const int n = P.roff[r + 1] - P.roff[r];
-    const double tt = L->totaltime;
-    int b = 0;
-    while (b < n - 1 && t[b] - tt <= 0.0) b++;  // the reference does not stop at the end
-    const int a = b - 1 > 0 ? b - 1 : 0;
-    const double flow = q[a] + (tt - t[a]) / (t[b] - t[a]) * (q[b] - q[a]);
-    P.rrate[2 * r] = (double)(flow / P.rarea[r]);
-    P.rrate[2 * r + 1] = (double)(float)((double)(float)flow / P.rarea[r]);
-}
-
 // Level maps of the boundary segments at the step's start (Forcingthisstep on
 // each segment's WLmap, src/Updateforcing.cu:29-35, 83-126): InterpstepCPU
 // (src/GridManip.cu:602-622) between the frames bracketing totaltime, with its
@@ -1207,7 +1199,6 @@ __global__ __launch_bounds__(256) void k_bnd_now(KParams P, const DevLoop* L) {
 }
 
 void launch_rain_now(const KParams& P, const DevLoop* L, hipStream_t st) {
-    if (P.nriver > 0) hipLaunchKernelGGL(k_river_rates, dim3(1), dim3(64), 0, st, P, L);
     if (P.bmapmax > 0)
         hipLaunchKernelGGL(k_bnd_now, dim3((P.bmapmax + 255) / 256, P.nseg), dim3(256), 0, st, P, L);
     if (!P.rframes || P.rnframes < 2) return;
@@ -1372,8 +1363,8 @@ inline int fit_grid(int grid, int resident) {
 }
 
 template <class T, bool FAST, bool BATCH, bool COMP>
-void launch_step_t(const KParams& P, const StepBuffers<T>& B, DevLoop* L, int advance_time, hipStream_t st,
-                   hipEvent_t* ev) {
+void launch_step_t(const KParams& P, const StepBuffers<T>& B, DevLoop* L, DevLoop* Lnext, int advance_time,
+                   hipStream_t st, hipEvent_t* ev) {
     if (!BATCH) launch_rain_now(P, L, st);
     if (ev) (void)hipEventRecord(ev[0], st);
     const Cst<T> C = make_cst<T, FAST>(P);
@@ -1390,34 +1381,34 @@ void launch_step_t(const KParams& P, const StepBuffers<T>& B, DevLoop* L, int ad
     if (ext) hipLaunchKernelGGL((k_predictor<T, FAST, BATCH, FAST, EXT_OK>), dim3(gp), dim3(256), 0, st, P, C, B, L);
     else hipLaunchKernelGGL((k_predictor<T, FAST, BATCH, FAST>), dim3(gp), dim3(256), 0, st, P, C, B, L);
     if (ev) (void)hipEventRecord(ev[1], st);
-    hipLaunchKernelGGL((k_reduce_dt<T>), dim3(BATCH ? P.nmember : 1), dim3(64), 0, st, L, advance_time);
+    if (BATCH) hipLaunchKernelGGL((k_reduce_dt<T>), dim3(P.nmember), dim3(64), 0, st, L, L, advance_time);
     if (ev) (void)hipEventRecord(ev[2], st);
     if constexpr (BATCH)
-        hipLaunchKernelGGL((k_corrector_wide<T, FAST, true, COMP, false>), dim3(gc), dim3(256), 0, st, P, C, B, L);
+        hipLaunchKernelGGL((k_corrector_wide<T, FAST, true, COMP, false>), dim3(gc), dim3(256), 0, st, P, C, B, L, Lnext,
+                           advance_time);
     else if (ext)
-        hipLaunchKernelGGL((k_corrector_wide<T, FAST, false, COMP, true>), dim3(gc), dim3(256), 0, st, P, C, B, L);
+        hipLaunchKernelGGL((k_corrector_wide<T, FAST, false, COMP, true>), dim3(gc), dim3(256), 0, st, P, C, B, L, Lnext,
+                           advance_time);
     else
-        hipLaunchKernelGGL((k_corrector<T, FAST, false, COMP>), dim3(gc), dim3(256), 0, st, P, C, B, L);
+        hipLaunchKernelGGL((k_corrector<T, FAST, false, COMP>), dim3(gc), dim3(256), 0, st, P, C, B, L, Lnext,
+                           advance_time);
     if (ev) (void)hipEventRecord(ev[3], st);
 }
 
 template <class T, bool FAST, bool COMP>
-void launch_step_b(const KParams& P, const StepBuffers<T>& B, DevLoop* L, int advance_time, hipStream_t st,
+void launch_step_b(const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext, int advance_time, hipStream_t st,
                    hipEvent_t* ev) {
-    if (P.sid) launch_step_t<T, FAST, true, COMP>(P, B, L, advance_time, st, ev);
-    else launch_step_t<T, FAST, false, COMP>(P, B, L, advance_time, st, ev);
+    const StepBuffers<T>& B = *(const StepBuffers<T>*)buffers;
+    if (P.sid) launch_step_t<T, FAST, true, COMP>(P, B, L, Lnext, advance_time, st, ev);
+    else launch_step_t<T, FAST, false, COMP>(P, B, L, Lnext, advance_time, st, ev);
 }
 
-void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* L, int advance_time, hipStream_t st,
-                 hipEvent_t* ev) {
-    if (precision == 0)
-        launch_step_b<double, false, false>(P, *(const StepBuffers<double>*)buffers, L, advance_time, st, ev);
-    else if (precision == 1)
-        launch_step_b<float, false, false>(P, *(const StepBuffers<float>*)buffers, L, advance_time, st, ev);
-    else if (precision == 2)
-        launch_step_b<float, true, false>(P, *(const StepBuffers<float>*)buffers, L, advance_time, st, ev);
-    else
-        launch_step_b<float, true, true>(P, *(const StepBuffers<float>*)buffers, L, advance_time, st, ev);
+void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* L, DevLoop* Lnext, int advance_time,
+                 hipStream_t st, hipEvent_t* ev) {
+    if (precision == 0) launch_step_b<double, false, false>(P, buffers, L, Lnext, advance_time, st, ev);
+    else if (precision == 1) launch_step_b<float, false, false>(P, buffers, L, Lnext, advance_time, st, ev);
+    else if (precision == 2) launch_step_b<float, true, false>(P, buffers, L, Lnext, advance_time, st, ev);
+    else launch_step_b<float, true, true>(P, buffers, L, Lnext, advance_time, st, ev);
 }
 
 // Persistent grid: all workgroups resident at once (CUs x occupancy), a
@@ -1454,20 +1445,20 @@ int persistent_grid(int precision, int corrector, int nblk, int wg_per_cu) {
 void launch_init_dt(int precision, const KParams& P, const void* h, DevLoop* L, hipStream_t st) {
     if (precision == 0) {
         hipLaunchKernelGGL(k_init_dt<double>, dim3(P.nblk), dim3(256), 0, st, P, (const double*)h, L);
-        hipLaunchKernelGGL(k_reduce_dt<double>, dim3(P.sid ? P.nmember : 1), dim3(64), 0, st, L, 2);
+        hipLaunchKernelGGL(k_reduce_dt<double>, dim3(P.sid ? P.nmember : 1), dim3(64), 0, st, L, L, 2);
     } else {
         hipLaunchKernelGGL(k_init_dt<float>, dim3(P.nblk), dim3(256), 0, st, P, (const float*)h, L);
-        hipLaunchKernelGGL(k_reduce_dt<float>, dim3(P.sid ? P.nmember : 1), dim3(64), 0, st, L, 2);
+        hipLaunchKernelGGL(k_reduce_dt<float>, dim3(P.sid ? P.nmember : 1), dim3(64), 0, st, L, L, 2);
     }
 }
 
 void launch_init_dt_member(int precision, const KParams& P, const void* h, DevLoop* L, int member, hipStream_t st) {
     if (precision == 0) {
         hipLaunchKernelGGL(k_init_dt<double>, dim3(P.nblk), dim3(256), 0, st, P, (const double*)h, L);
-        hipLaunchKernelGGL(k_reduce_dt<double>, dim3(1), dim3(64), 0, st, L + member, 2);
+        hipLaunchKernelGGL(k_reduce_dt<double>, dim3(1), dim3(64), 0, st, L + member, L + member, 2);
     } else {
         hipLaunchKernelGGL(k_init_dt<float>, dim3(P.nblk), dim3(256), 0, st, P, (const float*)h, L);
-        hipLaunchKernelGGL(k_reduce_dt<float>, dim3(1), dim3(64), 0, st, L + member, 2);
+        hipLaunchKernelGGL(k_reduce_dt<float>, dim3(1), dim3(64), 0, st, L + member, L + member, 2);
     }
 }
 
@@ -1500,9 +1491,10 @@ void launch_refine_flags(int precision, const KParams& P, const void* a, const v
                            (const float*)b, mode, (float)lo, (float)hi, flags);
 }
 
-void launch_reduce_dt(int precision, DevLoop* L, int nloop, int advance_time, hipStream_t st) {
-    if (precision == 0) hipLaunchKernelGGL(k_reduce_dt<double>, dim3(nloop), dim3(64), 0, st, L, advance_time);
-    else hipLaunchKernelGGL(k_reduce_dt<float>, dim3(nloop), dim3(64), 0, st, L, advance_time);
+void launch_reduce_dt(int precision, DevLoop* L, DevLoop* Lnext, int nloop, int advance_time, hipStream_t st) {
+    if (precision == 0)
+        hipLaunchKernelGGL(k_reduce_dt<double>, dim3(nloop), dim3(64), 0, st, L, Lnext, advance_time);
+    else hipLaunchKernelGGL(k_reduce_dt<float>, dim3(nloop), dim3(64), 0, st, L, Lnext, advance_time);
 }
 
 void launch_volume(int precision, const KParams& P, const void* h, double* part, double* out, hipStream_t st) {

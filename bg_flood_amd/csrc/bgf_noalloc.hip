@@ -46,7 +46,7 @@ inline size_t up256(size_t n) { return (n + 255) / 256 * 256; }
 Layout layout(long long nblk, size_t es) {
     Layout L;
     L.loop = 0;
-    L.queue = up256(sizeof(bgf::DevLoop));
+    L.queue = up256(2 * sizeof(bgf::DevLoop));  // the step's loop state and the one that it leaves
     L.rec = L.queue + up256(sizeof(int) * 2 * bgf::NXCD * bgf::QSTRIDE);
     const size_t tend = up256((size_t)nblk * BSI * es);
     L.dh = L.rec + up256((size_t)nblk * 8 * sizeof(int));
@@ -97,11 +97,13 @@ __global__ void k_loop_state(bgf::DevLoop* L, double nextoutputtime, double dt, 
         L->rain_n = 0;
         L->tcorr = 0.0;
         L->tpred = 0.0;
+        L->tstart = 0.0;
         L->stats_n = 0;
         L->cf_uniform = 0;
         L->cf_value = 0.0;
         L->dtmin = dtmin;
         L->crashed = 0;
+        L->unused = 0;
     }
     if (t < bgf::NSLOT) {
         L->slot32[t] = 0x7f800000u;
@@ -215,10 +217,10 @@ extern "C" bgf_status bgf_step_noalloc(const bgf_param* p, const bgf_blocks* d_b
         B->dh = (float*)(base + Lo.dh); B->dhu = (float*)(base + Lo.dhu); B->dhv = (float*)(base + Lo.dhv);
         B->ch = nullptr;
     }
-    bgf::launch_step(p->precision, kp, storage, dL, 0, st, nullptr);
+    bgf::launch_step(p->precision, kp, storage, dL, dL + 1, 0, st, nullptr);
     HIPCHK(hipGetLastError());
     bgf::DevLoop D;
-    HIPCHK(hipMemcpyAsync(&D, dL, sizeof(D), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(&D, dL + 1, sizeof(D), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     loop->dt = D.dt;
     loop->dtmax = D.dtmax;
