@@ -78,7 +78,7 @@ struct bgf_batch_s {
     int wg_pred = 0, wg_corr = 0;
     int tile_x = TILE_X, tile_y = TILE_Y;
     bool use_graph = true;
-    hipGraphExec_t graph = nullptr;  // an even/odd pair of batch steps; rebuilt after membership changes
+    hipGraphExec_t graph = nullptr;  // PERIOD batch steps; rebuilt after membership changes
     // multi-level members: position of each block slot in the packed active
     // list, the neighbour records, and the gradient / face / snapshot arrays
     bool amr = false;
@@ -95,6 +95,8 @@ struct bgf_batch_s {
 
 namespace {
 
+// Steps of a captured graph, as a handle's: even, and used by runs of twice as many and more.
+constexpr int PERIOD = 8;
 constexpr int NGAUGE = 16;
 constexpr int NSAMP = 2048;  // gauge samples kept per member
 
@@ -552,11 +554,11 @@ bgf_status bgf_batch_run_async(bgf_batch b, int nsteps) {
     HIPCHK(hipMemcpyAsync(b->d_loop, b->loops.data(), sizeof(bgf::DevLoop) * b->cap_members, hipMemcpyHostToDevice,
                           b->stream));
     if (b->krun.nblk > 0) {
-        if (b->use_graph && nsteps >= 4) {
+        if (b->use_graph && nsteps >= 2 * PERIOD) {
             if (!b->graph) {
                 hipGraph_t g = nullptr;
                 HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-                enqueue_steps(b, 2);
+                enqueue_steps(b, PERIOD);
                 HIPCHK(hipStreamEndCapture(b->stream, &g));
                 hipError_t e = hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
@@ -565,8 +567,8 @@ bgf_status bgf_batch_run_async(bgf_batch b, int nsteps) {
                     return fail(BGF_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
                 }
             }
-            for (int k = 0; k < nsteps / 2; k++) HIPCHK(hipGraphLaunch(b->graph, b->stream));
-            nsteps &= 1;
+            for (int k = 0; k < nsteps / PERIOD; k++) HIPCHK(hipGraphLaunch(b->graph, b->stream));
+            nsteps %= PERIOD;
         }
         enqueue_steps(b, nsteps);
     }

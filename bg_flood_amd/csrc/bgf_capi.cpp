@@ -83,7 +83,7 @@ struct bgf_handle_s {
     void* d_ch = nullptr;          // compensation of h (BGF_FP32_COMP)
     void* d_metric = nullptr;      // spherical metric terms per block
     bool use_graph = true;
-    hipGraphExec_t graph = nullptr;  // one period of steps, captured on first use
+    hipGraphExec_t graph = nullptr;  // PERIOD steps, captured on first use
     int last_steps = 0;              // steps taken by the last bgf_run / bgf_sync
     // launch schedule of the persistent one-level kernels
     BlockXY xy;
@@ -260,17 +260,22 @@ void enqueue_step(bgf_handle h, int k, int advance_time, hipEvent_t* ev) {
     enqueue_stats(h, k, advance_time);
 }
 
-// Steps of a captured graph: an even and an odd one.
-constexpr int PERIOD = 2;
+// Steps of a captured graph (even: the last leaves the state where the first
+// found it).  Shorter runs than two of them launch their kernels directly:
+// replaying a graph of two steps was slower than that (1.55 against 1.43 ms
+// for 100 steps of 256 x 256 cells), one of eight is faster (1.36 ms), since a
+// replay starts about 3 us after the last, and what its capture costs comes
+// back only in longer runs.
+constexpr int PERIOD = 8;
 
-// Runs of many steps replay a captured HIP graph of one period instead of
+// Runs of many steps replay a captured HIP graph of PERIOD steps instead of
 // relaunching every kernel (the step is launch-bound on small domains and
 // multi-level meshes).  The graph holds kernel launches only.
 bgf_status graph_steps(bgf_handle h, int nperiods) {
     if (!h->graph) {
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < PERIOD; k++) enqueue_step(h, k, 1, nullptr);
+        for (int k = 0; k < PERIOD; k++) enqueue_step(h, k & 1, 1, nullptr);
         HIPCHK(hipStreamEndCapture(h->stream, &g));
         hipError_t e = hipGraphInstantiate(&h->graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -288,7 +293,7 @@ bgf_status enqueue_steps(bgf_handle h, int nsteps, int advance_time) {
     if (advance_time == 1 && !h->timing && h->use_graph && nsteps >= 2 * PERIOD) {
         bgf_status s = graph_steps(h, nsteps / PERIOD);
         if (s != BGF_OK) return s;
-        nsteps %= PERIOD;  // at most one step left, at parity 0
+        nsteps %= PERIOD;
     }
     for (int k = 0; k < nsteps; k++) {
         enqueue_step(h, k & 1, advance_time, h->timing ? h->ev : nullptr);
