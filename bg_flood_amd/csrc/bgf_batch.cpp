@@ -91,6 +91,7 @@ struct bgf_batch_s {
     bgf::KParams krun;
     std::vector<int> run_members;
     bool run_valid = false;
+    std::unique_ptr<ReadBack> back{new ReadBack};
 };
 
 namespace {
@@ -619,39 +620,9 @@ bgf_status bgf_batch_get_state(bgf_batch b, int m, void* zs, void* hh, void* u, 
     bgf_status s = check_member(b, m);
     if (s != BGF_OK) return s;
     const Member& M = b->members[m];
-    const size_t n = (size_t)M.nblkmem * BS, bytes = b->es * n, o = b->es * (size_t)M.off * BS;
-    std::vector<unsigned char> t(bytes), tz;
-    auto down = [&](const void* src, void* dst) -> bool {
-        if (hipMemcpy(t.data(), (const char*)src + o, bytes, hipMemcpyDeviceToHost) != hipSuccess) return false;
-        for (int ib : M.active) {
-            const int lb = ib - M.off;
-            for (int j = 0; j < BW; j++) {
-                const size_t c = (size_t)memloc(0, j, lb) * b->es;
-                std::memcpy((char*)dst + c, t.data() + c, BW * b->es);
-            }
-        }
-        return true;
-    };
-    if (u && !down(b->d_u[0], u)) return fail(BGF_ERR_HIP, "download failed");
-    if (v && !down(b->d_v[0], v)) return fail(BGF_ERR_HIP, "download failed");
-    if (hh && !down(b->d_h[0], hh)) return fail(BGF_ERR_HIP, "download failed");
-    if (zs) {
-        if (hipMemcpy(t.data(), (const char*)b->d_h[0] + o, bytes, hipMemcpyDeviceToHost) != hipSuccess)
-            return fail(BGF_ERR_HIP, "download failed");
-        tz.resize(bytes);
-        if (hipMemcpy(tz.data(), (const char*)b->d_zb + o, bytes, hipMemcpyDeviceToHost) != hipSuccess)
-            return fail(BGF_ERR_HIP, "download failed");
-        for (int ib : M.active) {
-            const int lb = ib - M.off;
-            for (int j = 0; j < BW; j++)
-                for (int i = 0; i < BW; i++) {
-                    const size_t c = memloc(i, j, lb);
-                    if (b->prec == 0) ((double*)zs)[c] = ((double*)tz.data())[c] + ((double*)t.data())[c];
-                    else ((float*)zs)[c] = ((float*)tz.data())[c] + ((float*)t.data())[c];
-                }
-        }
-    }
-    return BGF_OK;
+    void* const dst[4] = {zs, hh, u, v};
+    return read_back(*b->back, b->prec, M.active, M.off, b->d_active + active_offset(b, m), b->d_zb, b->d_h[0],
+                     b->d_u[0], b->d_v[0], dst, b->stream);
 }
 
 bgf_status bgf_batch_volume(bgf_batch b, int m, double* volume) {

@@ -65,6 +65,7 @@ struct bgf_handle_s {
     int loop_at = 0;                 // the one that the enqueued work leaves last
     bgf::KParams kp;
     hipStream_t stream = nullptr;
+    std::unique_ptr<ReadBack> back{new ReadBack};
     bool timing = false;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     double t_pred = 0, t_red = 0, t_corr = 0;
@@ -764,37 +765,9 @@ bgf_status bgf_set_state(bgf_handle h, const void* zb, const void* hh, const voi
 bgf_status bgf_get_state(bgf_handle h, void* zs, void* hh, void* u, void* v) {
     if (!h) return fail(BGF_ERR_INVALID_ARG, "null handle");
     if (h->pending_steps) return fail(BGF_ERR_STATE, "bgf_run_async pending: call bgf_sync first");
-    size_t bytes = h->es * h->S;
-    std::vector<unsigned char> tmp(bytes), tzb;
-    auto scatter = [&](void* dst) {
-        for (int ibl = 0; ibl < h->nblk; ibl++) {
-            int ib = h->active[ibl];
-            for (int j = 0; j < BW; j++) {
-                size_t off = (size_t)memloc(0, j, ib) * h->es;
-                std::memcpy((unsigned char*)dst + off, tmp.data() + off, BW * h->es);
-            }
-        }
-    };
-    if (hh || zs) {
-        HIPCHK(hipMemcpy(tmp.data(), h->d_h[0], bytes, hipMemcpyDeviceToHost));
-        if (hh) scatter(hh);
-        if (zs) {
-            tzb.resize(bytes);
-            HIPCHK(hipMemcpy(tzb.data(), h->d_zb, bytes, hipMemcpyDeviceToHost));
-            for (int ibl = 0; ibl < h->nblk; ibl++) {
-                int ib = h->active[ibl];
-                for (int j = 0; j < BW; j++)
-                    for (int i = 0; i < BW; i++) {
-                        size_t n = memloc(i, j, ib);
-                        if (h->prec == 0) ((double*)zs)[n] = ((double*)tzb.data())[n] + ((double*)tmp.data())[n];
-                        else ((float*)zs)[n] = ((float*)tzb.data())[n] + ((float*)tmp.data())[n];
-                    }
-            }
-        }
-    }
-    if (u) { HIPCHK(hipMemcpy(tmp.data(), h->d_u[0], bytes, hipMemcpyDeviceToHost)); scatter(u); }
-    if (v) { HIPCHK(hipMemcpy(tmp.data(), h->d_v[0], bytes, hipMemcpyDeviceToHost)); scatter(v); }
-    return BGF_OK;
+    void* const dst[4] = {zs, hh, u, v};
+    return read_back(*h->back, h->prec, h->active, 0, h->d_active, h->d_zb, h->d_h[0], h->d_u[0], h->d_v[0], dst,
+                     h->stream);
 }
 
 bgf_status bgf_init_dt(bgf_handle h, double dtinit, bgf_loop* loop) {

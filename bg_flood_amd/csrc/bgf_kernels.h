@@ -209,6 +209,11 @@ void launch_import(int precision, const KParams& P, const void* const* src, void
 void launch_export(int precision, const KParams& P, const void* const* src, const void* zb, void* const* dst,
                    void* const* keep, hipStream_t st);
 
+// Interior cells of the n blocks active[0..n) to out (host memory the GPU can write): block by block
+// the fields whose bit is set in fields (0 zs = zb + h, 1 h, 2 u, 3 v), 256 values each.
+void launch_pack_state(int precision, const int* active, int n, const void* zb, const void* h, const void* u,
+                       const void* v, int fields, void* out, hipStream_t st);
+
 // Refinement criteria (src/AdaptCriteria.cu:62-160) per active block of P:
 // flags[ib] = any interior cell of a (plus b when b is not null: zs = zb + h)
 // exceeds lo (mode 0) or lies in [lo, hi] (mode 1).

@@ -1542,4 +1542,27 @@ void launch_export(int precision, const KParams& P, const void* const* src, cons
                            keep ? (float*)keep[1] : nullptr, keep ? (float*)keep[2] : nullptr);
 }
 
+// Interior cells of n blocks, field by field of each (zs = zb + h, h, u, v
+// where asked), BSI values apiece, to host memory that the GPU can reach.
+template <class T>
+__global__ __launch_bounds__(256) void k_pack_state(const int* active, const T* zb, const T* h, const T* u, const T* v,
+                                                    int fields, T* out) {
+    const int t = threadIdx.x, c = memloc(t & 15, t >> 4, ldu(active, blockIdx.x));
+    T* o = out + (size_t)blockIdx.x * __builtin_popcount(fields) * BSI + t;
+    if (fields & 1) { *o = zb[c] + h[c]; o += BSI; }
+    if (fields & 2) { *o = h[c]; o += BSI; }
+    if (fields & 4) { *o = u[c]; o += BSI; }
+    if (fields & 8) *o = v[c];
+}
+
+void launch_pack_state(int precision, const int* active, int n, const void* zb, const void* h, const void* u,
+                       const void* v, int fields, void* out, hipStream_t st) {
+    if (precision == 0)
+        hipLaunchKernelGGL(k_pack_state<double>, dim3(n), dim3(256), 0, st, active, (const double*)zb, (const double*)h,
+                           (const double*)u, (const double*)v, fields, (double*)out);
+    else
+        hipLaunchKernelGGL(k_pack_state<float>, dim3(n), dim3(256), 0, st, active, (const float*)zb, (const float*)h,
+                           (const float*)u, (const float*)v, fields, (float*)out);
+}
+
 }  // namespace bgf
