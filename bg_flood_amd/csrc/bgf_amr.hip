@@ -37,7 +37,8 @@
 // fix-up and advance, two of each, with eight face arrays between them: 103 us
 // a step on a mesh of 1,607 blocks in FP32 and 2.01 ms on 39,348 blocks in
 // FP64; with the stage in one launch and faces stored only where another
-// block reads them 66 us and 0.98 ms.
+// block reads them 66 us and 0.98 ms; with the mesh's gather recipes formed
+// beforehand (k_amr_recipes) 48 us and 0.94 ms.
 //
 // On meshes of four levels and more the halos are filled by a launch of their
 // own (k_amr_halo_refine) and prolonged level by level (k_amr_prolong).
@@ -149,12 +150,29 @@ template <class T> struct Gather {
     int kind;
     int i[4];  // cells; unused places repeat i[0]
     T a, b, c; // G_W3: the weights of i[0..2]; G_BILIN: the point (a, b)
+    int set;   // G_W3: which weights (w3_weights)
 };
 template <class T> __device__ __forceinline__ Gather<T> g_copy(int c) {
-    return Gather<T>{G_COPY, {c, c, c, c}, T(0), T(0), T(0)};
+    return Gather<T>{G_COPY, {c, c, c, c}, T(0), T(0), T(0), 0};
 }
 template <class T> __device__ __forceinline__ Gather<T> g_mean4(int c0, int c1, int c2, int c3) {
-    return Gather<T>{G_MEAN4, {c0, c1, c2, c3}, T(0), T(0), T(0)};
+    return Gather<T>{G_MEAN4, {c0, c1, c2, c3}, T(0), T(0), T(0), 0};
+}
+// The weights of a halo cell beside a coarser block: of the own edge cell and
+// of the coarse cells after and before it (src/Halo.cu:2083-2286): W3_UP, W3_DOWN
+// the nearer one counts more; at the end of a side, by the block beside the
+// coarse one: W3_SAME none, W3_AFTER and W3_BEFORE a coarser one (beyond the
+// side's first and last cell), W3_FINE a finer one.
+enum { W3_UP = 0, W3_DOWN = 1, W3_SAME = 2, W3_AFTER = 3, W3_BEFORE = 4, W3_FINE = 5 };
+template <class T> __device__ __forceinline__ void w3_weights(int set, T& a, T& b, T& c) {
+    a = T(1.0 / 3.0);
+    // T(0.5*(1.0-w1)) and T(0.5)*(T(1.0)-w1) round to the same float
+    const T half = T(0.5 * (1.0 - (double)T(1.0 / 3.0)));
+    b = set == W3_UP ? T(1.0 / 6.0) : set == W3_SAME ? half : T(0.5);
+    c = set == W3_UP ? T(0.5) : set == W3_SAME ? half : T(1.0 / 6.0);
+    if (set == W3_AFTER) { a = T(4.0 / 10.0); b = T(5.0 / 10.0); c = T(1.0 / 10.0); }
+    if (set == W3_BEFORE) { a = T(4.0 / 10.0); b = T(1.0 / 10.0); c = T(5.0 / 10.0); }
+    if (set == W3_FINE) { a = T(1.0 / 4.0); b = T(1.0 / 2.0); c = T(1.0 / 4.0); }
 }
 
 // src/Util_CPU.cu:129-144 on the unit square.
@@ -208,9 +226,7 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, const Side& S
     const T cj = ceil(T(j) * T(0.5));
     const int jjc = first ? ftoi(cj) : ftoi(cj + T(BW / 2));
     const bool up = cj * T(2) > T(j);
-    T w1 = T(1.0 / 3.0);
-    T w2 = up ? T(1.0 / 6.0) : T(0.5);
-    T w3 = up ? T(0.5) : T(1.0 / 6.0);
+    int set = up ? W3_UP : W3_DOWN;
     const int ii = edge_cell(s, 0, j, ib);
     int ir = edge_cell(os, 0, jjc, C);
     int it = edge_cell(os, 0, jjc - 1, C);
@@ -219,14 +235,12 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, const Side& S
             int ln;
             const int n = corner_lo(P, s, C, ln);
             if (n == C) {
-                // T(0.5*(1.0-w1)) and T(0.5)*(T(1.0)-w1) round to the same float
-                w3 = T(0.5 * (1.0 - (double)w1));
-                w2 = w3;
+                set = W3_SAME;
                 it = ir;
             } else {
                 it = edge_cell(os, 0, BW - 1, n);
-                if (ln < l1) { w1 = T(4.0 / 10.0); w2 = T(5.0 / 10.0); w3 = T(1.0 / 10.0); }
-                else if (ln > l1) { w1 = T(1.0 / 4.0); w2 = T(1.0 / 2.0); w3 = T(1.0 / 4.0); }
+                if (ln < l1) set = W3_AFTER;
+                else if (ln > l1) set = W3_FINE;
             }
         }
     } else if (j == BW - 1) {
@@ -234,16 +248,17 @@ __device__ __forceinline__ Gather<T> fill_recipe(const KParams& P, const Side& S
         int ln;
         const int n = corner_hi(P, s, C2, ln);
         if (n == C2) {
-            w3 = T(0.5 * (1.0 - (double)w1));
-            w2 = w3;
+            set = W3_SAME;
             ir = it;
         } else {
             ir = edge_cell(os, 0, 0, n);
-            if (ln < l2) { w1 = T(4.0 / 10.0); w2 = T(1.0 / 10.0); w3 = T(5.0 / 10.0); }
-            else if (ln > l2) { w1 = T(1.0 / 4.0); w2 = T(1.0 / 2.0); w3 = T(1.0 / 4.0); }
+            if (ln < l2) set = W3_BEFORE;
+            else if (ln > l2) set = W3_FINE;
         }
     }
-    return Gather<T>{G_W3, {ii, ir, it, ii}, w1, w2, w3};
+    Gather<T> g{G_W3, {ii, ir, it, ii}, T(0), T(0), T(0), set};
+    w3_weights(set, g.a, g.b, g.c);
+    return g;
 }
 template <class T> __device__ __forceinline__ T fill_value(const KParams& P, int s, int j, int ib, const T* z) {
     const Gather<T> g = fill_recipe<T>(P, side_of(P, s, ib), s, j, ib, P.level[ib]);
@@ -413,10 +428,10 @@ template <class T> __device__ __forceinline__ Gather<T> far_recipe(const Side& S
     const int q0 = edge_cell(os, 0, jj - 1, C), q1 = edge_cell(os, 1, jj - 1, C);
     // bilinear(q11, q12, q21, q22, x, y) with the side's corner order
     switch (s) {
-        case SL: return Gather<T>{G_BILIN, {q1, p1, q0, p0}, T(0.75), jr, T(0)};
-        case SR: return Gather<T>{G_BILIN, {q0, p0, q1, p1}, T(0.25), jr, T(0)};
-        case SB: return Gather<T>{G_BILIN, {q1, q0, p1, p0}, jr, T(0.75), T(0)};
-        default: return Gather<T>{G_BILIN, {q0, q1, p0, p1}, jr, T(0.25), T(0)};
+        case SL: return Gather<T>{G_BILIN, {q1, p1, q0, p0}, T(0.75), jr, T(0), 0};
+        case SR: return Gather<T>{G_BILIN, {q0, p0, q1, p1}, T(0.25), jr, T(0), 0};
+        case SB: return Gather<T>{G_BILIN, {q1, q0, p1, p0}, jr, T(0.75), T(0), 0};
+        default: return Gather<T>{G_BILIN, {q0, q1, p0, p1}, jr, T(0.25), T(0), 0};
     }
 }
 
@@ -621,7 +636,7 @@ template <class T> struct FluxOut {
 // before the slopes are.  sh, sz: the h and zb of the coarser neighbours'
 // cells that replace their halo cells in the source terms of the shared faces
 // (src/Kurganov.cu:132-145).
-constexpr int NPT = 32;  // prolongation points per side: see stage_points
+constexpr int NPT = 33;  // prolongation points per side: see stage_point
 template <class T> struct StageLds {
     Q4<T> q[20 * TP];
     union {
@@ -635,7 +650,7 @@ template <class T> struct StageLds {
         };
         T pt[4][4][NPT];         // h, u, v and the bed of the points
     };
-    Q4<T> fe[2 * BW];  // the seventeenth X faces, then Y faces
+    Q4<T> fe[2 * BW];  // the seventeenth X faces, then Y faces (before that: four of each side's, see EndHalo)
     T sh[4][BW], sz[4][BW];
     T red[4];
 };
@@ -965,20 +980,23 @@ __device__ __forceinline__ int side_tix(int s, int d, int j) {
 // 26..30 the five points (a cell of D and its four neighbours) behind C's
 //         halo at the end of its side, where the block D there is coarser than
 //         C,
-//   31    C's halo at that end, behind point 0 or 9.
-// The last six give C's halo at the end of the half as C's own halo stage
-// leaves it (end_halo), which the sequential reference's wet/dry prolongation
-// tests and the cells beyond the halo are interpolated from.
+//   31    C's halo at that end, behind point 0 or 9,
+//   32    C's cell behind the edge cell at the other end of the half.
+// 26..31 give C's halo at the end of the half as C's own halo stage leaves it
+// (k_amr_stage), which the sequential reference's wet/dry prolongation tests
+// and the cells beyond the halo are interpolated from.
 // side_end gives that halo: side p of C, position je beside the shared side.
 struct SideEnd {
     int p, je;
     Side E;  // side p of C
 };
+__device__ __forceinline__ void side_end(int s, bool lo, int& p, int& je) {
+    p = s < 2 ? (lo ? SB : ST) : (lo ? SL : SR);
+    je = (s == SL || s == SB) ? BW - 1 : 0;
+}
 __device__ __forceinline__ SideEnd side_end(const KParams& P, int s, const Side& S) {
     SideEnd e;
-    const bool lo = S.back;
-    e.p = s < 2 ? (lo ? SB : ST) : (lo ? SL : SR);
-    e.je = (s == SL || s == SB) ? BW - 1 : 0;
+    side_end(s, S.back, e.p, e.je);
     e.E = side_of(P, e.p, S.n1);
     return e;
 }
@@ -992,9 +1010,13 @@ template <class T>
 __device__ __forceinline__ HaloPt<T> stage_point(const KParams& P, int s, int k, const Side& S) {
     const int j0 = S.back ? 0 : BW / 2;
     int x, y, b = S.n1, lev = S.l1;
-    if (k < 26 || k == 31) {
-        const int d = k < 10 ? 0 : k < 18 || k == 31 ? 1 : -1;
-        const int a = k < 10 ? j0 - 1 + k : k < 18 ? j0 + k - 10 : k < 26 ? j0 + k - 18 : S.back ? -1 : BW;
+    if (k < 26 || k > 30) {
+        const int d = k < 10 ? 0 : k < 18 || k > 30 ? 1 : -1;
+        const int a = k < 10   ? j0 - 1 + k
+                      : k < 18 ? j0 + k - 10
+                      : k < 26 ? j0 + k - 18
+                      : k < 32 ? (S.back ? -1 : BW)
+                               : (S.back ? BW / 2 : BW / 2 - 1);
         facing_cell(s, d, a, x, y);
     } else {
         const SideEnd e = side_end(P, s, S);
@@ -1014,49 +1036,77 @@ __device__ __forceinline__ HaloPt<T> stage_point(const KParams& P, int s, int k,
     return pt_recipe<T>(P, x, y, b, lev);
 }
 
-// C's halo cell at the end of its half side, at depth d (0 or 1) from the
-// shared side, as C's halo stage leaves it: h, zs, u, v from the points pt
-// of the side.  Beside a coarser block D it is the linear reconstruction, or,
-// where the wet/dry prolongation applies, D's cell (both depths lie over one
-// cell of D); C's own workgroup may be writing the bed of that halo cell,
-// but only where it becomes the bed of D's cell, which is taken from D here.
-template <class T>
-__device__ __forceinline__ Q4<T> end_halo(const KParams& P, const T (*pt)[NPT], const SideEnd& e, const Side& S,
-                                          bool prolong, T eps, int d) {
-    const int k = d == 0 ? (S.back ? 0 : 9) : 31;
-    Q4<T> o{pt[0][k], pt[3][k], pt[1][k], pt[2][k]};
-    if (e.E.l1 < S.l1) {
-        const int je = e.je == 0 ? d : e.je - d;
-        T f[3][5];
-#pragma unroll
-        for (int n = 0; n < 3; n++)
-#pragma unroll
-            for (int m = 0; m < 5; m++) f[n][m] = pt[n][26 + m];
-        o.a = refine_from(P, e.p, je, S.l1, e.E.l1, f[0]);
-        o.c = refine_from(P, e.p, je, S.l1, e.E.l1, f[1]);
-        o.d = refine_from(P, e.p, je, S.l1, e.E.l1, f[2]);
-        if (prolong &&
-            !(f[0][0] > eps && f[0][1] > eps && f[0][2] > eps && f[0][4] > eps && f[0][3] > eps)) {
-            o.a = f[0][0];
-            o.b = pt[3][26];
-        }
+// The recipes of the sides that are not beside blocks of the block's own
+// level: NPT entries a side, of a coarse side its points, of another the halo
+// cells (0..15) and the cells beyond them (16..31).  They depend on the mesh
+// only and are formed once for it: to form them in every stage again took a
+// chain of dependent loads through the neighbours' records and half of the
+// stage's 44 to 53 KB of code, more for the two stages than the instruction
+// cache holds (1,607 blocks in FP32: 23 us a stage, now 17; the same blocks
+// taken as all of one level, wrongly, 13).  An entry is four cells (P.rcell) and a code with
+// the cell of the bed (P.rmeta).
+enum {
+    RC_KIND = 3, RC_SET = 2, RC_WD = 1 << 5, RC_SIDE = 6,  // G_* kind; w3 set; wet/dry restriction; its side
+    RC_FIRST = 1 << 8,                                     // coarse sides: C comes before the block in the active list
+    RC_END = 16                                            // and the level of the block at the end of the half
+};
+static_assert(4 * NPT == RECIPES, "");
+__global__ __launch_bounds__(192) void k_amr_recipes(KParams P, int4* rcell, int2* rmeta) {
+    const int t = threadIdx.x, ib = P.active[blockIdx.x], s = t / NPT, k = t % NPT;
+    if (s > 3) return;
+    const int lev = P.level[ib];
+    const Side S = side_of(P, s, ib);
+    const bool coarse = S.l1 < lev;
+    if (!coarse && k >= 32) return;
+    HaloPt<float> r;
+    int code = 0;
+    if (coarse) {
+        r = stage_point<float>(P, s, k, S);
+        const SideEnd e = side_end(P, s, S);
+        code = (P.inv[S.n1] < P.inv[ib] ? RC_FIRST : 0) | (e.E.l1 & 0xff) << RC_END;
+    } else if (k < 16) {
+        r.g = fill_recipe<float>(P, S, s, k, ib, lev);
+        r.wd = wetdry_recipe(P, S, s, k, ib, lev);
+    } else {
+        r.g = far_recipe<float>(S, s, k - 16, ib, lev);
+        r.wd.on = 0;
+        r.wd.w = r.g.i[0];
     }
-    o.b = o.b + o.a;
-    return o;
+    // the side whose patch a restriction reads: the mean's cells are that patch's, in its side's order
+    int rs = s;
+    if (coarse) {
+        const int x = r.wd.w % BS % MW, y = r.wd.w % BS / MW;
+        rs = x == 0 ? SL : x == MW - 1 ? SR : y == 0 ? SB : ST;
+    }
+    const size_t e = ((size_t)ib * 4 + s) * NPT + k;
+    rcell[e] = make_int4(r.g.i[0], r.g.i[1], r.g.i[2], r.g.i[3]);
+    rmeta[e] = make_int2(code | r.g.kind | r.g.set << RC_SET | (r.wd.on ? RC_WD : 0) | rs << RC_SIDE, r.wd.w);
+}
+
+// What a wave keeps of C's halo at the end of its half side: the cell beside the
+// shared side as this block's prolongation sees it, as C's own stage leaves it,
+// and the cell behind that.
+enum { EH_SEEN = 0, EH_FACING = 1, EH_BEHIND = 2, EH_N = 3 };
+
+// Orders a wave's LDS writes before its lanes' reads of one another's.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // A stage of a block in one workgroup: halo, slopes, faces, tendencies, and in
 // the corrector the advance.
 //
-// Wave s gathers side s: its halo cells (lanes 0-15, or beside a coarser block
-// the points of stage_point, lanes 0-31), the cells beyond the halo that the
-// limited slope at the halo reads (src/Gradients.cu:2713-3294, lanes 32-47)
-// and the source substitutions (lanes 48-63); the side's kind is uniform over
-// its wave.  Beside a coarser block a second pass forms the linear
+// Wave s gathers side s: its halo cells (lanes 0-15) and the cells beyond the
+// halo that the limited slope at the halo reads (src/Gradients.cu:2713-3294,
+// lanes 32-47), by the mesh's recipes where the neighbours are of another
+// level; the side's kind is uniform over its wave.  Beside a coarser block it
+// gathers the points of stage_point (lanes 0-32) and forms from them the linear
 // reconstruction and the wet/dry prolongation (src/Halo.cu:1044-1405,
-// src/ConserveElevation.cu:80-205,451-482) from the points.  HALO: the halo
-// is formed here; otherwise it stands in the Model arrays (four levels and
-// more).  The slopes, faces and tendencies are those of the one-level tile.
+// src/ConserveElevation.cu:80-205,451-482), the cells beyond and the source
+// substitutions (lanes 48-63).  HALO: the halo is formed here; otherwise it
+// stands in the Model arrays (four levels and more).  The slopes, faces and
+// tendencies are those of the one-level tile.
 //
 // A block that needs no other block's faces has its tendencies stored (the
 // predictor, whose dt is not known yet) or is advanced here (the corrector:
@@ -1102,6 +1152,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
     const int w = edge_cell(s, -1, j, ib);
     Q4<T> r;  // the value of the lane's point: h, zs, u, v (halo cells: zs without the bed yet)
     T zw = T(0), zown = T(0);  // the bed of the lane's point, and of the block's own halo cell
+    int ends = 0;              // the coarse side's code
     r.a = r.b = r.c = r.d = T(0);
     const bool same = (sd.n1 == ib && sd.n2 == ib) || (sd.n1 != ib && sd.l1 == lev && sd.l2 == lev);
     if (l < 16) zown = zw = zb[w];
@@ -1119,45 +1170,87 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
             r.c = A.u[w];
             r.d = A.v[w];
         }
+    } else if (HALO) {
+        const int e = (ib * 4 + s) * NPT;
+        if (coarse) ends = ldu((const int*)P.rmeta, 2 * e);
+        if (coarse ? l < NPT : l < 16 || is_far) {
+            const int k = e + (coarse || l < 16 ? l : l - 16);
+            const int4 n = P.rcell[k];
+            const int2 m = P.rmeta[k];
+            const int kind = m.x & RC_KIND;
+            T H[4], Z[4], U[4], V[4];
+            auto load = [&](int q, int c) {
+                H[q] = A.h[c];
+                Z[q] = zb[c];
+                U[q] = A.u[c];
+                V[q] = A.v[c];
+            };
+            load(0, n.x);
+            if (coarse) zw = zb[m.y];
+            if (kind != G_COPY) {
+                load(1, n.y);
+                load(2, n.z);
+                load(3, n.w);
+            }
+            r = Q4<T>{H[0], Z[0] + H[0], U[0], V[0]};
+            if (kind == G_MEAN4) {
+                auto mean = [](const T* z) { return T(0.25) * (z[0] + z[1] + z[2] + z[3]); };
+                r.a = mean(H);
+                r.c = mean(U);
+                r.d = mean(V);
+                if (is_far) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) Z[q] = Z[q] + H[q];
+                    r.b = mean(Z);
+                }
+                if ((m.x & RC_WD) && P.wetdryfix) {
+                    // the patch's cells in the restriction's order (lower left, right, top, top right)
+                    const int rs = (m.x >> RC_SIDE) & 3;
+                    const bool lo = rs == SL || rs == SB, xs = rs < 2;
+                    auto patch = [&](const T* z, T* o) {
+                        o[0] = lo ? z[1] : z[0];
+                        o[1] = xs ? (lo ? z[0] : z[1]) : (lo ? z[3] : z[2]);
+                        o[2] = xs ? (lo ? z[3] : z[2]) : (lo ? z[0] : z[1]);
+                        o[3] = lo ? z[2] : z[3];
+                    };
+                    T hh[4], zz[4];
+                    patch(H, hh);
+                    patch(Z, zz);
+                    r.a = wetdry_apply(eps, hh, zz, zw, r.a);
+                }
+            } else if (kind == G_W3) {
+                T a, b, c;
+                w3_weights((m.x >> RC_SET) & 7, a, b, c);
+                auto w3 = [&](const T* z) { return a * z[0] + b * z[1] + c * z[2]; };
+                r.a = w3(H);
+                r.c = w3(U);
+                r.d = w3(V);
+            }
+        }
     } else {
-        HaloPt<T> pt;
-        pt.wd.on = 0;
+        Gather<T> g;
         if (is_far) {
-            pt.g = far_recipe<T>(sd, s, j, ib, lev);
+            g = far_recipe<T>(sd, s, j, ib, lev);
         } else if (is_sub) {
             // the coarse cell next to the face (where the side is coarse; read anyway)
             int cx, cy;
             facing_cell(s, 0, coarse ? j / 2 + (sd.back ? 0 : BW / 2) : 0, cx, cy);
-            pt.g = g_copy<T>(memloc(cx, cy, sd.n1));
-        } else if (!HALO) {
-            pt.g = g_copy<T>(w);
-        } else if (coarse) {
-            pt = stage_point<T>(P, s, l, sd);
+            g = g_copy<T>(memloc(cx, cy, sd.n1));
         } else {
-            pt.g = fill_recipe<T>(P, sd, s, j, ib, lev);
-            pt.wd = wetdry_recipe(P, sd, s, j, ib, lev);
+            g = g_copy<T>(w);
         }
-        T H[4], Z[4], U[4], V[4], WH[4], WZ[4];
-        g_load(pt.g, A.h, H);
-        g_load(pt.g, zb, Z);
-        g_load(pt.g, A.u, U);
-        g_load(pt.g, A.v, V);
-        if (pt.wd.on) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                WH[m] = A.h[pt.wd.i[m]];
-                WZ[m] = zb[pt.wd.i[m]];
-            }
-        }
-        if (HALO && coarse && l < 32) zw = zb[pt.wd.w];
-        r.a = g_apply(pt.g, H);
-        r.c = g_apply(pt.g, U);
-        r.d = g_apply(pt.g, V);
-        if (pt.wd.on) r.a = wetdry_apply(eps, WH, WZ, zw, r.a);
+        T H[4], Z[4], U[4], V[4];
+        g_load(g, A.h, H);
+        g_load(g, zb, Z);
+        g_load(g, A.u, U);
+        g_load(g, A.v, V);
+        r.a = g_apply(g, H);
+        r.c = g_apply(g, U);
+        r.d = g_apply(g, V);
         if (is_far) {
 #pragma unroll
             for (int m = 0; m < 4; m++) Z[m] = Z[m] + H[m];
-            r.b = g_apply(pt.g, Z);
+            r.b = g_apply(g, Z);
         } else {
             r.b = Z[0];
         }
@@ -1166,94 +1259,131 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
 
     const Q4<T> q{h0, z0 + h0, u0, v0};
     S.q[tix(x, y)] = q;
-    if (is_far) S.q[side_tix(s, -2, j)] = r;
-    if (is_sub && coarse) {
-        S.sh[s][j] = r.a;
-        S.sz[s][j] = r.b;
-    }
     if (HALO && coarse) {
-        if (l < 32) {
+        // the side's own wave passes its points through LDS: in order within a wave, no barrier
+        if (l < NPT) {
             S.pt[s][0][l] = r.a;
             S.pt[s][1][l] = r.c;
             S.pt[s][2][l] = r.d;
             S.pt[s][3][l] = zw;
         }
-    } else if (l < 16) {
-        r.b = zw + r.a;
-        S.q[side_tix(s, -1, j)] = r;
-        // open boundaries take the step-start depth of the halo (amr_fluxfix_side: the right and top faces)
-        if (HALO && !corr && P.bopen && (sd.n1 == ib || sd.n2 == ib)) const_cast<T*>(A.h)[w] = r.a;
-    }
-    __syncthreads();
-    if (HALO && (cs[0] || cs[1] || cs[2] || cs[3])) {
-        if (coarse && l < 16) {
-            const int m = j / 2;
-            // the points of the coarse cell m of the half and of its neighbours in x and y
-            const int in = 10 + m, out = 18 + m, before = m, after = m + 2;
-            const bool lo = s == SL || s == SB;  // the side faces the neighbour's high end
-            const int xm = s < 2 ? (lo ? in : out) : before, xp = s < 2 ? (lo ? out : in) : after;
-            const int ym = s < 2 ? before : (lo ? in : out), yp = s < 2 ? after : (lo ? out : in);
-            T f[3][5];
+        wave_sync();
+        // the linear reconstructions: lanes 0-15 of the halo cells, lanes 48-50 of C's halo at the end of
+        // the half (EndHalo)
+        int p = s, jr = j;
+        const int m = j / 2, lend = (int)(signed char)(ends >> RC_END);
+        const bool lo = s == SL || s == SB;  // the side faces the neighbour's high end
+        const int kend = l == 48 + EH_BEHIND ? 31 : sd.back ? 0 : 9;
+        Q4<T> o{T(0), T(0), T(0), T(0)};
+        T f0[5];
+        if (l < 16 || (is_sub && j < EH_N)) {
+            int k[5], lv = lev, lc = sd.l1;
+            if (l < 16) {
+                // the points of the coarse cell m of the half and of its neighbours in x and y
+                const int in = 10 + m, out = 18 + m, before = m, after = m + 2;
+                k[0] = m + 1;
+                k[1] = s < 2 ? (lo ? in : out) : before;
+                k[2] = s < 2 ? (lo ? out : in) : after;
+                k[3] = s < 2 ? before : (lo ? in : out);
+                k[4] = s < 2 ? after : (lo ? out : in);
+            } else {
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                f[k][0] = S.pt[s][k][m + 1];
-                f[k][1] = S.pt[s][k][xm];
-                f[k][2] = S.pt[s][k][xp];
-                f[k][3] = S.pt[s][k][ym];
-                f[k][4] = S.pt[s][k][yp];
+                for (int n = 0; n < 5; n++) k[n] = 26 + n;
+                side_end(s, sd.back, p, jr);
+                if (j == EH_BEHIND) jr += jr == 0 ? 1 : -1;
+                lv = sd.l1;
+                lc = lend;
             }
-            Q4<T> o;
-            o.a = refine_from(P, s, j, lev, sd.l1, f[0]);
-            o.c = refine_from(P, s, j, lev, sd.l1, f[1]);
-            o.d = refine_from(P, s, j, lev, sd.l1, f[2]);
+            T f[2][5];
+#pragma unroll
+            for (int n = 0; n < 5; n++) {
+                f0[n] = S.pt[s][0][k[n]];
+                f[0][n] = S.pt[s][1][k[n]];
+                f[1][n] = S.pt[s][2][k[n]];
+            }
+            o.a = refine_from(P, p, jr, lv, lc, f0);
+            o.c = refine_from(P, p, jr, lv, lc, f[0]);
+            o.d = refine_from(P, p, jr, lv, lc, f[1]);
+        }
+        auto dry = [&]() { return !(f0[0] > eps && f0[1] > eps && f0[2] > eps && f0[4] > eps && f0[3] > eps); };
+        if (is_sub) {
+            S.sh[s][j] = S.pt[s][0][m + 1];
+            S.sz[s][j] = S.pt[s][3][m + 1];
+            if (j < EH_N) {
+                // Beside a coarser block D it is the linear reconstruction, or, where the wet/dry
+                // prolongation applies, D's cell (both depths lie over one cell of D); C's own workgroup
+                // may be writing the bed of that halo cell, but only where it becomes the bed of D's cell,
+                // which is taken from D here.
+                if (!(lend < sd.l1)) o = Q4<T>{S.pt[s][0][kend], T(0), S.pt[s][1][kend], S.pt[s][2][kend]};
+                o.b = S.pt[s][3][kend];
+                if (lend < sd.l1 && prolong && (j != EH_SEEN || (ends & RC_FIRST)) && dry()) {
+                    o.a = f0[0];
+                    o.b = S.pt[s][3][26];
+                }
+                o.b = o.b + o.a;
+                S.fe[4 * s + j] = o;
+            }
+        }
+        wave_sync();
+        if (l < 16) {
             T zo = zown;
             if (prolong) {
+                // C's halo at the end, prolonged if C comes before this block in the active list
                 if (m == (sd.back ? 0 : BW / 2 - 1)) {
-                    // C's halo at the end, prolonged if C comes before this block in the active list
-                    const SideEnd e = side_end(P, s, sd);
-                    f[0][s < 2 ? (sd.back ? 3 : 4) : (sd.back ? 1 : 2)] =
-                        end_halo<T>(P, S.pt[s], e, sd, P.inv[sd.n1] < P.inv[ib], eps, 0).a;
+                    const T ha = S.fe[4 * s + EH_SEEN].a;
+                    if (s < 2) (sd.back ? f0[3] : f0[4]) = ha;
+                    else (sd.back ? f0[1] : f0[2]) = ha;
                 }
-                if (!(f[0][0] > eps && f[0][1] > eps && f[0][2] > eps && f[0][4] > eps && f[0][3] > eps)) {
-                    o.a = f[0][0];
-                    zo = S.sz[s][j];
+                if (dry()) {
+                    o.a = f0[0];
+                    zo = S.pt[s][3][m + 1];
                     zb[w] = zo;
                 }
             }
             o.b = zo + o.a;
             S.q[side_tix(s, -1, j)] = o;
-        }
-        if (coarse && is_far && j == (sd.back ? 0 : BW - 1)) {
-            // beyond the halo at the end of the half, two of the four cells are C's halo
-            const Gather<T> g = far_recipe<T>(sd, s, j, ib, lev);
-            const SideEnd e = side_end(P, s, sd);
-            T H[4], Z[4], U[4], V[4];
-            g_load(g, A.h, H);
-            g_load(g, zb, Z);
-            g_load(g, A.u, U);
-            g_load(g, A.v, V);
-            const Q4<T> e0 = end_halo<T>(P, S.pt[s], e, sd, prolong, eps, 0);
-            const Q4<T> e1 = end_halo<T>(P, S.pt[s], e, sd, prolong, eps, 1);
-            // C's cells at the end, at depths 0 and 1, as far_recipe indexes them
-            int x0, y0, x1, y1;
-            facing_cell(s, 0, sd.back ? -1 : BW, x0, y0);
-            facing_cell(s, 1, sd.back ? -1 : BW, x1, y1);
-            const int i0 = memloc(x0, y0, sd.n1), i1 = memloc(x1, y1, sd.n1);
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                Z[m] = Z[m] + H[m];
-                if (g.i[m] == i0 || g.i[m] == i1) {
-                    const Q4<T>& h = g.i[m] == i0 ? e0 : e1;
-                    H[m] = h.a;
-                    Z[m] = h.b;
-                    U[m] = h.c;
-                    V[m] = h.d;
-                }
+        } else if (is_far) {
+            // the cells beyond the halo: bilinear from C's cells at depths 0 and 1 (far_recipe), at the
+            // end of the half C's halo
+            const int cj = (j + 1) / 2;
+            const T b = cj * 2 > j ? T(0.25) : T(0.75);
+            auto at = [&](int k) {
+                const T h = S.pt[s][0][k];
+                return Q4<T>{h, S.pt[s][3][k] + h, S.pt[s][1][k], S.pt[s][2][k]};
+            };
+            Q4<T> p0 = at(cj + 1), q0 = at(cj), p1 = at(cj < BW / 2 ? 10 + cj : sd.back ? 32 : 31),
+                  q1 = at(cj > 0 ? 9 + cj : sd.back ? 31 : 32);
+            if (sd.back && cj == 0) {
+                q0 = S.fe[4 * s + EH_FACING];
+                q1 = S.fe[4 * s + EH_BEHIND];
             }
-            S.q[side_tix(s, -2, j)] = Q4<T>{g_apply(g, H), g_apply(g, Z), g_apply(g, U), g_apply(g, V)};
+            if (!sd.back && cj == BW / 2) {
+                p0 = S.fe[4 * s + EH_FACING];
+                p1 = S.fe[4 * s + EH_BEHIND];
+            }
+            // bilinear(q11, q12, q21, q22, x, y) with the side's corner order
+            const Q4<T> c12 = s < 2 ? (lo ? p1 : p0) : (lo ? q0 : q1), c21 = s < 2 ? (lo ? q0 : q1) : (lo ? p1 : p0);
+            const Q4<T> c11 = lo ? q1 : q0, c22 = lo ? p0 : p1;
+            const T a = lo ? T(0.75) : T(0.25), bx = s < 2 ? a : b, by = s < 2 ? b : a;
+            S.q[side_tix(s, -2, j)] = Q4<T>{bilinear(c11.a, c12.a, c21.a, c22.a, bx, by),
+                                            bilinear(c11.b, c12.b, c21.b, c22.b, bx, by),
+                                            bilinear(c11.c, c12.c, c21.c, c22.c, bx, by),
+                                            bilinear(c11.d, c12.d, c21.d, c22.d, bx, by)};
         }
-        __syncthreads();
+    } else {
+        if (is_far) S.q[side_tix(s, -2, j)] = r;
+        if (is_sub && coarse) {
+            S.sh[s][j] = r.a;
+            S.sz[s][j] = r.b;
+        }
+        if (l < 16) {
+            r.b = zw + r.a;
+            S.q[side_tix(s, -1, j)] = r;
+            // open boundaries take the step-start depth of the halo (amr_fluxfix_side: the right and top faces)
+            if (HALO && !corr && P.bopen && (sd.n1 == ib || sd.n2 == ib)) const_cast<T*>(A.h)[w] = r.a;
+        }
     }
+    __syncthreads();
 
     // slopes: the thread's own cell, and the halo ring on wave 2 (lanes 0-31 along x, 32-63 along y)
     const Q4<T> gxo = slopes4<FAST>(theta, by_delta, idelta, S.q[tix(x - 1, y)], q, S.q[tix(x + 1, y)]);
@@ -1438,9 +1568,13 @@ void stage(const KParams& P, const AmrBuffers<T>& B, const AdvArgs<T>& A, DevLoo
     // With up to three levels the stage forms the halos itself: a block's prolongation depends on at
     // most its coarse neighbour's, which it evaluates again.  With more levels that chain is longer:
     // the halos are filled by a launch of their own and prolonged level by level, coarsest first.
-    if (P.wetdryfix && P.maxlevel - P.minlevel > 2) {
-        hipLaunchKernelGGL(k_amr_halo_refine<T>, blk, dim3(64), 0, st, P, h, u, v, B.zb, B.hsnap, L, corr);
-        for (int lev = P.minlevel + 2; lev <= P.maxlevel; lev++)
+    // So are they on meshes whose sides are no quadtree's (P.odd), which the recipes do not cover.
+    const bool levels = P.wetdryfix && P.maxlevel - P.minlevel > 2;
+    if (levels || P.odd) {
+        const bool prolong = P.wetdryfix && P.maxlevel > P.minlevel;
+        hipLaunchKernelGGL(k_amr_halo_refine<T>, blk, dim3(64), 0, st, P, h, u, v, B.zb, prolong ? B.hsnap : (T*)nullptr,
+                           L, corr);
+        for (int lev = P.minlevel + 2; prolong && lev <= P.maxlevel; lev++)
             hipLaunchKernelGGL(k_amr_prolong<T>, quad, tpb, 0, st, P, h, B.zb, (const T*)B.hsnap, lev, L, corr);
         hipLaunchKernelGGL((k_amr_stage<T, SPH, FAST, false, corr>), blk, tpb, 0, st, P, A, B.zb, F, D, L);
     } else {
@@ -1532,8 +1666,9 @@ __global__ __launch_bounds__(256) void k_amr_nbr(KParams P, int* nbr, int nbm) {
     r[3] = make_int4(info[4], info[5], info[6], info[7]);
 }
 
-void launch_amr_nbr(const KParams& P, int* nbr, int nbm, hipStream_t st) {
+void launch_amr_nbr(const KParams& P, int* nbr, int nbm, int4* rcell, int2* rmeta, hipStream_t st) {
     if (nbm > 0) hipLaunchKernelGGL(k_amr_nbr, dim3((nbm + 255) / 256), dim3(256), 0, st, P, nbr, nbm);
+    if (P.nblk > 0) hipLaunchKernelGGL(k_amr_recipes, dim3(P.nblk), dim3(192), 0, st, P, rcell, rmeta);
 }
 
 void launch_amr_fill(int precision, const KParams& P, void* z, hipStream_t st) {

@@ -38,7 +38,7 @@ struct Member {
     std::vector<int> active;  // global block ids, in the member's own active order
     std::vector<int> order;   // global block ids, tiled processing order
     std::vector<int> fix;     // multi-level: global ids of the blocks that wait for others' faces
-    bool fix_all = false;
+    bool fix_all = false, odd = false;
     BlockXY xy;               // block coordinates (global ids), for re-tiling
     double rain = 0.0;
     std::vector<int> gauges;  // global cell indices
@@ -85,6 +85,8 @@ struct bgf_batch_s {
     int* d_inv = nullptr;
     int* d_nbr = nullptr;
     int* d_fix = nullptr;
+    int4* d_rcell = nullptr;
+    int2* d_rmeta = nullptr;
     void* d_amr[11] = {nullptr};  // as a handle's: 2-9 face fluxes, 10 hsnap (0-1, remesh staging, unused)
     // the persistent kernels walk only the blocks of members still running:
     // their processing order, launch parameters, and the members it was built for
@@ -109,7 +111,7 @@ void free_batch(bgf_batch b) {
     F(b->d_zb); F(b->d_cf); F(b->d_dh); F(b->d_dhu); F(b->d_dhv); F(b->d_hmax); F(b->d_ch);
     F(b->d_volpart); F(b->d_volout); F(b->d_gcell); F(b->d_gval); F(b->d_loop);
     F(b->d_ring); F(b->d_tring);
-    F(b->d_inv); F(b->d_nbr); F(b->d_fix);
+    F(b->d_inv); F(b->d_nbr); F(b->d_fix); F(b->d_rcell); F(b->d_rmeta);
     for (int k = 0; k < 11; k++) F(b->d_amr[k]);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -154,7 +156,7 @@ bgf_status rebuild(bgf_batch b) {
         std::vector<int> inv(b->cap_blocks, -1);
         for (size_t k = 0; k < active.size(); k++) inv[active[k]] = (int)k;
         HIPCHK(hipMemcpy(b->d_inv, inv.data(), sizeof(int) * inv.size(), hipMemcpyHostToDevice));
-        bgf::launch_amr_nbr(b->kp, b->d_nbr, b->cap_blocks, b->stream);
+        bgf::launch_amr_nbr(b->kp, b->d_nbr, b->cap_blocks, b->d_rcell, b->d_rmeta, b->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(b->stream));
     }
@@ -177,8 +179,11 @@ bgf_status prepare_run(bgf_batch b) {
     b->krun.hmax = b->track_max ? (float*)b->d_hmax : nullptr;
     if (b->amr) {
         b->krun.active = b->d_order;  // the multi-level kernels walk the running members' active lists
-        bool all = false;
-        for (int m : running) all = all || b->members[m].fix_all;
+        bool all = false, odd = false;
+        for (int m : running) {
+            all = all || b->members[m].fix_all;
+            odd = odd || b->members[m].odd;
+        }
         std::vector<int> fix = all ? order : std::vector<int>();
         for (int m : running)
             if (!all) fix.insert(fix.end(), b->members[m].fix.begin(), b->members[m].fix.end());
@@ -187,6 +192,7 @@ bgf_status prepare_run(bgf_batch b) {
         b->krun.fix = b->d_fix;
         b->krun.nfix = (int)fix.size();
         b->krun.fix_all = all ? 1 : 0;
+        b->krun.odd = odd ? 1 : 0;
     }
     if (!order.empty() && !b->amr) {
         b->krun.grid_pred = bgf::persistent_grid(b->prec, 0, b->krun.nblk, b->wg_pred);
@@ -328,7 +334,9 @@ bgf_status bgf_batch_create(const bgf_param* common, int max_blocks, int max_mem
     b->amr = common->maxlevel > common->minlevel;
     if (b->amr) {
         ok = ok && A((void**)&b->d_inv, sizeof(int) * max_blocks) && A((void**)&b->d_nbr, sizeof(int) * bgf::NBR * (size_t)max_blocks) &&
-             A((void**)&b->d_fix, sizeof(int) * (size_t)max_blocks);
+             A((void**)&b->d_fix, sizeof(int) * (size_t)max_blocks) &&
+             hipMalloc((void**)&b->d_rcell, sizeof(int4) * bgf::RECIPES * (size_t)max_blocks) == hipSuccess &&
+             hipMalloc((void**)&b->d_rmeta, sizeof(int2) * bgf::RECIPES * (size_t)max_blocks) == hipSuccess;
         for (int k = 2; k < 11; k++) ok = ok && A(&b->d_amr[k], b->es * b->S);
     }
     if (!ok) {
@@ -348,6 +356,8 @@ bgf_status bgf_batch_create(const bgf_param* common, int max_blocks, int max_mem
     kp.maxlevel = b->amr ? common->maxlevel : 0;
     kp.inv = b->d_inv;
     kp.nbr = b->d_nbr;
+    kp.rcell = b->d_rcell;
+    kp.rmeta = b->d_rmeta;
     kp.fc = p.precision == 0 ? coriolis<double>(p.lat) : coriolis<float>(p.lat);
     kp.mask = p.mask;
     kp.frictionmodel = p.frictionmodel;
@@ -447,7 +457,7 @@ bgf_status bgf_batch_add(bgf_batch b, const bgf_param* p, const bgf_blocks* blk,
         M.order = M.active;  // the multi-level kernels keep the member's active order
         const int* nbs[8] = {blk->LeftBot, blk->LeftTop, blk->RightBot, blk->RightTop,
                              blk->TopLeft, blk->TopRight, blk->BotLeft, blk->BotRight};
-        M.fix = fix_blocks(blk->active, nblk, blk->level, nbs, false, M.fix_all);
+        M.fix = fix_blocks(blk->active, nblk, blk->level, nbs, false, M.fix_all, M.odd);
         for (int& ib : M.fix) ib += off;
     } else {
         M.xy = block_xy(blk, nblk, p->dx);

@@ -57,6 +57,8 @@ struct bgf_handle_s {
     bool cf_shared = false;  // the caller holds the cf device array
     int *d_nb[8] = {nullptr};  // LeftBot LeftTop RightBot RightTop TopLeft TopRight BotLeft BotRight
     int* d_nbr = nullptr;      // multi-level meshes: the neighbour record of each block slot (bgf::NBR ints)
+    int4* d_rcell = nullptr;   // their gather recipes (bgf::RECIPES per slot)
+    int2* d_rmeta = nullptr;
     int* d_fix = nullptr;      // and the blocks whose advance waits for other blocks' faces
     void *d_h[2] = {nullptr, nullptr}, *d_u[2] = {nullptr, nullptr}, *d_v[2] = {nullptr, nullptr};
     void *d_zb = nullptr, *d_cf = nullptr, *d_dh = nullptr, *d_dhu = nullptr, *d_dhv = nullptr;
@@ -139,7 +141,7 @@ void free_handle(bgf_handle h) {
     F(h->d_active); F(h->d_order); F(h->d_level); F(h->d_queue); F(h->d_rec);
     for (int k = 0; k < 15; k++) F(h->stats.a[k]);
     for (int k = 0; k < 8; k++) F(h->d_nb[k]);
-    F(h->d_nbr); F(h->d_fix);
+    F(h->d_nbr); F(h->d_rcell); F(h->d_rmeta); F(h->d_fix);
     for (int k = 0; k < 2; k++) { F(h->d_h[k]); F(h->d_u[k]); F(h->d_v[k]); }
     F(h->d_zb); F(h->d_cf); F(h->d_dh); F(h->d_dhu); F(h->d_dhv);
     F(h->d_volpart); F(h->d_volout); F(h->d_loop);
@@ -395,13 +397,14 @@ bool upload_metric(bgf_handle h, const bgf_param* p, const bgf_blocks* b, int nb
 // after the others (fix_blocks), for the current boundary segments.
 bgf_status setup_fix(bgf_handle h) {
     if (!h->amr) return BGF_OK;
-    bool all = false;
+    bool all = false, odd = false;
     const std::vector<int> list =
-        fix_blocks(h->active.data(), h->nblk, h->h_level.data(), h->h_nb, h->kp.bopen != 0, all);
+        fix_blocks(h->active.data(), h->nblk, h->h_level.data(), h->h_nb, h->kp.bopen != 0, all, odd);
     if (!list.empty()) HIPCHK(hipMemcpy(h->d_fix, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
     h->kp.fix = h->d_fix;
     h->kp.nfix = (int)list.size();
     h->kp.fix_all = all ? 1 : 0;
+    h->kp.odd = odd ? 1 : 0;
     return BGF_OK;
 }
 
@@ -611,6 +614,8 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     if (multilevel) {
         ok = ok && A((void**)&h->d_inv, sizeof(int) * cap);
         ok = ok && A((void**)&h->d_nbr, sizeof(int) * bgf::NBR * (size_t)cap);
+        ok = ok && hipMalloc((void**)&h->d_rcell, sizeof(int4) * bgf::RECIPES * (size_t)cap) == hipSuccess &&
+             hipMalloc((void**)&h->d_rmeta, sizeof(int2) * bgf::RECIPES * (size_t)cap) == hipSuccess;
         ok = ok && A((void**)&h->d_fix, sizeof(int) * cap);
         for (int k = 0; k < 11; k++) ok = ok && A(&h->d_amr[k], h->es * SA);
     }
@@ -685,7 +690,9 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     kp.bxo = h->d_blkxo;
     kp.byo = h->d_blkyo;
     kp.nbr = h->d_nbr;
-    if (multilevel) bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->stream);
+    kp.rcell = h->d_rcell;
+    kp.rmeta = h->d_rmeta;
+    if (multilevel) bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->d_rcell, h->d_rmeta, h->stream);
     s = setup_fix(h);
     if (s != BGF_OK) {
         free_handle(h);
@@ -1583,7 +1590,7 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
     kp.inv = h->d_inv;
     kp.bxo = h->d_blkxo;
     kp.byo = h->d_blkyo;
-    bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->stream);
+    bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->d_rcell, h->d_rmeta, h->stream);
     // the processing order and its block records serve the one-level kernels only,
     // which a multi-level handle never runs: they are not rebuilt here
     ok = hipGetLastError() == hipSuccess;

@@ -381,10 +381,11 @@ inline bgf_status quadtree_neighbours(int n, const int* id, const int* lev, cons
 // neighbour by what the finer block's own record says; a block list whose two
 // records disagree (all) has every block wait, with all its faces stored.
 template <class Nb>
-inline std::vector<int> fix_blocks(const int* active, int nblk, const int* level, const Nb& nb, bool edges, bool& all) {
+inline std::vector<int> fix_blocks(const int* active, int nblk, const int* level, const Nb& nb, bool edges, bool& all,
+                                   bool& odd) {
     static const int facing[8] = {2, 2, 0, 0, 6, 6, 4, 4};
     std::vector<int> list;
-    all = false;
+    all = odd = false;
     for (int k = 0; k < nblk; k++) {
         const int ib = active[k];
         bool wait = false;
@@ -395,6 +396,8 @@ inline std::vector<int> fix_blocks(const int* active, int nblk, const int* level
                 if (nb[facing[q]][n] != ib || nb[facing[q] + 1][n] != ib) all = true;
             }
             if (edges && n == ib) wait = true;
+            const int n1 = nb[q & ~1][ib];
+            if ((q & 1) && n1 != ib && level[n1] <= level[ib] && level[n] > level[ib]) odd = true;
         }
         if (wait) list.push_back(ib);
     }

@@ -108,6 +108,9 @@ struct KParams {
     // multi-level meshes: the active blocks whose advance waits for other blocks' faces
     // (nfix of them; fix_all: every block does)
     const int* fix;
+    const int4* rcell;    // RECIPES per block slot: the cells a stage gathers (multi-level meshes; launch_amr_nbr)
+    const int2* rmeta;    // and how it combines them
+    int odd;              // a side's first neighbour is not finer than the block and its second is: no quadtree
     int nfix, fix_all;
     int minlevel, maxlevel;  // levels present among the active blocks
     // batches of domains: member of each block (DevLoop of that member), member count
@@ -244,7 +247,9 @@ void launch_amr_step(int precision, const KParams& P, const void* buffers, DevLo
 constexpr int NBR = 16;
 // Flags beside the level (low 8 bits) in a record's level words.
 enum { REC_BACK = 1 << 8, REC_FINER = 1 << 9, REC_EDGE = 1 << 10 };
-void launch_amr_nbr(const KParams& P, int* nbr, int nbm, hipStream_t st);
+// and then the gather recipes of P's active blocks (RECIPES entries of cells and codes per block slot).
+constexpr int RECIPES = 132;
+void launch_amr_nbr(const KParams& P, int* nbr, int nbm, int4* rcell, int2* rmeta, hipStream_t st);
 // Halo of a static field (the bed) on a multi-level mesh, src/InitialConditions.cu:135-147.
 void launch_amr_fill(int precision, const KParams& P, void* z, hipStream_t st);
 // The rain map of the coming step from the rain frames, and the boundary level
