@@ -598,7 +598,7 @@ bgf_status bgf_batch_sync(bgf_batch b) {
     if (b->nactive_blocks > 0 && !b->amr) {  // multi-level members end every step in buffer 0
         const void* src[3] = {b->d_h[1], b->d_u[1], b->d_v[1]};
         void* dst[3] = {b->d_h[0], b->d_u[0], b->d_v[0]};
-        bgf::launch_settle(b->prec, b->kp, src, dst, b->d_loop, b->stream);
+        bgf::launch_settle(b->prec, b->kp, src, dst, b->d_loop, nullptr, b->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(b->stream));
     }

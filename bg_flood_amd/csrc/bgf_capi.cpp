@@ -74,7 +74,7 @@ struct bgf_handle_s {
     int t_n = 0;
     int pending_steps = 0;  // steps enqueued by bgf_run_async
     bool state_set = false;
-    bgf::DevLoop loop_host;  // staging copy of the loop state for uploads
+    bgf::LoopState* loop_host = nullptr;  // pinned: the loop state after the enqueued work
     // output statistics (Calcmeanmax): enabled set, arrays, steps since the means were reset
     bgf::StatsLaunch stats{};
     int stats_n = 0;
@@ -160,11 +160,12 @@ void free_handle(bgf_handle h) {
     for (int k = 0; k < 4; k++) if (h->ev[k]) (void)hipEventDestroy(h->ev[k]);
     if (h->graph) (void)hipGraphExecDestroy(h->graph);
     if (h->stream) (void)hipStreamDestroy(h->stream);
+    if (h->loop_host) (void)hipHostFree(h->loop_host);
     delete h;
 }
 
 bgf_status upload_loop(bgf_handle h, const bgf_loop* loop, double endtime) {
-    bgf::DevLoop& L = h->loop_host;
+    bgf::LoopState L;
     std::memset(&L, 0, sizeof(L));
     L.nextoutputtime = loop->nextoutputtime;
     L.dt = loop->dt;
@@ -180,22 +181,43 @@ bgf_status upload_loop(bgf_handle h, const bgf_loop* loop, double endtime) {
     L.nstep = h->nstep;
     L.gevery = h->gevery;
     L.stats_n = h->stats_n;
-    for (int k = 0; k < bgf::NSLOT; k++) {
-        L.slot32[k] = 0x7f800000u;
-        L.slot64[k] = 0x7ff0000000000000ull;
-    }
-    HIPCHK(hipMemcpyAsync(h->d_loop, &L, sizeof(L), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
+    bgf::launch_set_loop(L, h->d_loop, h->stream);
+    HIPCHK(hipGetLastError());
     h->loop_at = 0;
     return BGF_OK;
 }
 
-bgf_status download_loop(bgf_handle h, bgf::DevLoop* L) {
-    HIPCHK(hipMemcpyAsync(L, h->d_loop + h->loop_at, sizeof(*L), hipMemcpyDeviceToHost, h->stream));
+// Brings the state back to buffer 0 where it ended in buffer 1 (one-level
+// meshes after an odd number of steps); out: see launch_settle.
+void enqueue_settle(bgf_handle h, bgf::LoopState* out) {
+    const void* src[3] = {h->d_h[1], h->d_u[1], h->d_v[1]};
+    void* dst[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};
+    bgf::launch_settle(h->prec, h->kp, src, dst, h->d_loop + h->loop_at, out, h->stream);
+}
+
+// Waits for the enqueued work, whose last launch wrote the loop state out.
+bgf_status finish_loop(bgf_handle h, bgf::LoopState* L) {
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(h->stream));
+    *L = *h->loop_host;
     h->stats_n = L->stats_n;
     h->nstep = L->nstep;
     return BGF_OK;
+}
+
+// The loop state after `steps` enqueued steps, the state of the domain back in
+// buffer 0.
+bgf_status download_loop(bgf_handle h, int steps, bgf::LoopState* L) {
+    const bool one = !h->amr, odd = one && (steps & 1);
+    if (odd) enqueue_settle(h, h->loop_host);
+    else bgf::launch_loop_out(h->d_loop + h->loop_at, h->loop_host, h->stream);
+    bgf_status s = finish_loop(h, L);
+    if (s == BGF_OK && one && !odd && (L->steps_done & 1)) {  // stopped early, after an odd step
+        enqueue_settle(h, nullptr);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(h->stream));
+    }
+    return s;
 }
 
 constexpr int GAUGE_CAP = 2048;  // gauge samples kept per gauge
@@ -310,18 +332,6 @@ bgf_status enqueue_steps(bgf_handle h, int nsteps, int advance_time) {
         }
     }
     HIPCHK(hipGetLastError());
-    return BGF_OK;
-}
-
-// After a run, bring the state back to buffer 0 if it ended in buffer 1.
-bgf_status settle(bgf_handle h, int steps_done) {
-    if (!h->amr && (steps_done & 1)) {
-        const void* src[3] = {h->d_h[1], h->d_u[1], h->d_v[1]};
-        void* dst[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};
-        bgf::launch_settle(h->prec, h->kp, src, dst, h->d_loop + h->loop_at, h->stream);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(h->stream));
-    }
     return BGF_OK;
 }
 
@@ -607,6 +617,7 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     ok = ok && A(&h->d_dh, h->es * SA) && A(&h->d_dhu, h->es * SA) && A(&h->d_dhv, h->es * SA);
     ok = ok && A((void**)&h->d_volpart, sizeof(double) * cap) && A((void**)&h->d_volout, sizeof(double));
     ok = ok && A((void**)&h->d_loop, 2 * sizeof(bgf::DevLoop));
+    ok = ok && hipHostMalloc((void**)&h->loop_host, sizeof(bgf::LoopState), hipHostMallocDefault) == hipSuccess;
     ok = ok && A((void**)&h->d_blkxo, sizeof(double) * cap) && A((void**)&h->d_blkyo, sizeof(double) * cap);
     h->amr = multilevel;
     if (p->precision == BGF_FP32_COMP && !multilevel) ok = ok && A(&h->d_ch, h->es * SA);
@@ -789,8 +800,8 @@ bgf_status bgf_init_dt(bgf_handle h, double dtinit, bgf_loop* loop) {
     if (s != BGF_OK) return s;
     bgf::launch_init_dt(h->prec, h->kp, h->d_h[0], h->d_loop, h->stream);
     HIPCHK(hipGetLastError());
-    bgf::DevLoop D;
-    s = download_loop(h, &D);
+    bgf::LoopState D;
+    s = download_loop(h, 0, &D);
     if (s != BGF_OK) return s;
     loop->dtmax = D.dt;
     return BGF_OK;
@@ -804,10 +815,8 @@ bgf_status bgf_step(bgf_handle h, bgf_loop* loop) {
     if (s != BGF_OK) return s;
     s = enqueue_steps(h, 1, 0);
     if (s != BGF_OK) return s;
-    bgf::DevLoop D;
-    s = download_loop(h, &D);
-    if (s != BGF_OK) return s;
-    s = settle(h, 1);  // cleanup: evolv_o -> evolv (src/FlowGPU.cu:282)
+    bgf::LoopState D;
+    s = download_loop(h, 1, &D);  // cleanup: evolv_o -> evolv (src/FlowGPU.cu:282)
     if (s != BGF_OK) return s;
     loop->dt = D.dt;
     loop->dtmax = D.dtmax;
@@ -830,11 +839,10 @@ bgf_status bgf_run_async(bgf_handle h, const bgf_loop* loop, int nsteps, double 
 bgf_status bgf_sync(bgf_handle h, bgf_loop* loop) {
     if (!h) return fail(BGF_ERR_INVALID_ARG, "null handle");
     if (!h->pending_steps) return fail(BGF_ERR_STATE, "nothing pending");
-    bgf::DevLoop D;
+    bgf::LoopState D;
+    const int steps = h->pending_steps > 0 ? h->pending_steps : 0;
     h->pending_steps = 0;
-    bgf_status s = download_loop(h, &D);
-    if (s != BGF_OK) return s;
-    s = settle(h, D.steps_done);
+    bgf_status s = download_loop(h, steps, &D);
     if (s != BGF_OK) return s;
     h->last_steps = D.steps_done;
     if (loop) {
@@ -905,7 +913,7 @@ bgf_status bgf_step_device(bgf_handle h, void* hh, void* zs, void* u, void* v, c
         if (s != BGF_OK) return s;
         const void* res[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};
         void* out[4] = {hh, zs, u, v};
-        bgf::launch_export(pr, h->kp, res, h->d_zb, out, nullptr, h->stream);
+        bgf::launch_export(pr, h->kp, res, h->d_zb, out, nullptr, h->d_loop + h->loop_at, h->loop_host, h->stream);
     } else {
         // the one-level kernels read the step-start state straight from the caller's arrays and
         // write U^{n+1} into the handle's second buffer, which then goes back to the caller (the
@@ -926,11 +934,10 @@ bgf_status bgf_step_device(bgf_handle h, void* hh, void* zs, void* u, void* v, c
         const void* res[3] = {h->d_h[1], h->d_u[1], h->d_v[1]};
         void* out[4] = {hh, zs, u, v};
         void* keep[3] = {h->d_h[0], h->d_u[0], h->d_v[0]};
-        bgf::launch_export(pr, h->kp, res, h->d_zb, out, keep, h->stream);
+        bgf::launch_export(pr, h->kp, res, h->d_zb, out, keep, h->d_loop + h->loop_at, h->loop_host, h->stream);
     }
-    HIPCHK(hipGetLastError());
-    bgf::DevLoop D;
-    s = download_loop(h, &D);
+    bgf::LoopState D;
+    s = finish_loop(h, &D);
     if (s != BGF_OK) return s;
     loop->dt = D.dt;
     loop->dtmax = D.dtmax;

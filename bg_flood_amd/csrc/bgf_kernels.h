@@ -204,13 +204,17 @@ void launch_gauge_step(int precision, const void* h, const int* cell, const DevL
 void launch_volume(int precision, const KParams& P, const void* h, double* part, double* out, hipStream_t st);
 // Copies h, u, v from src to dst for the blocks whose member ran an odd number of steps.
 void launch_settle(int precision, const KParams& P, const void* const* src, void* const* dst, const DevLoop* L,
-                   hipStream_t st);
+                   LoopState* out, hipStream_t st);
+// The loop state S to L, with empty slots; and L's state to out, host memory the GPU can write, which
+// launch_settle and launch_export do as well where out is not null.
+void launch_set_loop(const LoopState& S, DevLoop* L, hipStream_t st);
+void launch_loop_out(const DevLoop* L, LoopState* out, hipStream_t st);
 
 // Interior cells of the active blocks: dst[0..2] = src[0..2] (h, u, v).
 void launch_import(int precision, const KParams& P, const void* const* src, void* const* dst, hipStream_t st);
 // Interior cells: dst = (h, zb + h, u, v) of src = (h, u, v); keep (may be null) receives h, u, v too.
 void launch_export(int precision, const KParams& P, const void* const* src, const void* zb, void* const* dst,
-                   void* const* keep, hipStream_t st);
+                   void* const* keep, const DevLoop* L, LoopState* lout, hipStream_t st);
 
 // Interior cells of the n blocks active[0..n) to out (host memory the GPU can write): block by block
 // the fields whose bit is set in fields (0 zs = zb + h, 1 h, 2 u, 3 v), 256 values each.

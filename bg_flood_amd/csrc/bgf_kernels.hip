@@ -1298,13 +1298,29 @@ __global__ __launch_bounds__(1024) void k_sum(const double* __restrict__ part, i
     }
 }
 
+// The loop state enters a run in the arguments of a launch and leaves it in
+// host memory that the last launch writes (out, may be null), both in stream
+// order: with a copy and a wait at either end, and a third wait for the settled
+// state, a step called by itself took 64 us on 256 x 256 cells in FP64.
+__global__ __launch_bounds__(64) void k_set_loop(LoopState S, DevLoop* L) {
+    slots_empty(L);
+    if (threadIdx.x == 0) *(LoopState*)L = S;
+}
+static_assert(sizeof(LoopState) % 4 == 0 && sizeof(LoopState) <= 256, "a lane copies a word");
+__device__ __forceinline__ void loop_out(const DevLoop* L, LoopState* out) {
+    if (out && blockIdx.x == 0 && threadIdx.x < sizeof(LoopState) / 4)
+        ((int*)out)[threadIdx.x] = ((const int*)(const LoopState*)L)[threadIdx.x];
+}
+__global__ __launch_bounds__(64) void k_loop_out(const DevLoop* L, LoopState* out) { loop_out(L, out); }
+
 // cleanupGPU semantics (src/Advection.cu:399-417): copy interior h, u, v of
 // the blocks whose state ended in the second buffer (odd step count).
 template <class T>
 __global__ __launch_bounds__(256) void k_settle(KParams P, const T* __restrict__ h, const T* __restrict__ u,
                                                 const T* __restrict__ v, T* __restrict__ ho, T* __restrict__ uo,
-                                                T* __restrict__ vo, const DevLoop* L) {
+                                                T* __restrict__ vo, const DevLoop* L, LoopState* out) {
     const int t = threadIdx.x;
+    loop_out(L, out);
     const int ib = P.active[blockIdx.x];
     if (!(L[P.sid ? P.sid[ib] : 0].steps_done & 1)) return;
     const int i = memloc(t & 15, t >> 4, ib);
@@ -1331,7 +1347,9 @@ template <class T>
 __global__ __launch_bounds__(256) void k_export(KParams P, const T* __restrict__ h, const T* __restrict__ u,
                                                 const T* __restrict__ v, const T* __restrict__ zb, T* __restrict__ ho,
                                                 T* __restrict__ zso, T* __restrict__ uo, T* __restrict__ vo,
-                                                T* __restrict__ hk, T* __restrict__ uk, T* __restrict__ vk) {
+                                                T* __restrict__ hk, T* __restrict__ uk, T* __restrict__ vk,
+                                                const DevLoop* L, LoopState* out) {
+    loop_out(L, out);
     const int i = memloc(threadIdx.x & 15, threadIdx.x >> 4, P.active[blockIdx.x]);
     const T hh = h[i], uu = u[i], vv = v[i];
     ho[i] = hh;
@@ -1503,16 +1521,24 @@ void launch_volume(int precision, const KParams& P, const void* h, double* part,
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, st, part, P.nblk, out);
 }
 
+void launch_set_loop(const LoopState& S, DevLoop* L, hipStream_t st) {
+    hipLaunchKernelGGL(k_set_loop, dim3(1), dim3(64), 0, st, S, L);
+}
+
+void launch_loop_out(const DevLoop* L, LoopState* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_loop_out, dim3(1), dim3(64), 0, st, L, out);
+}
+
 void launch_settle(int precision, const KParams& P, const void* const* src, void* const* dst, const DevLoop* L,
-                   hipStream_t st) {
+                   LoopState* out, hipStream_t st) {
     if (precision == 0)
         hipLaunchKernelGGL(k_settle<double>, dim3(P.nblk), dim3(256), 0, st, P, (const double*)src[0],
                            (const double*)src[1], (const double*)src[2], (double*)dst[0], (double*)dst[1],
-                           (double*)dst[2], L);
+                           (double*)dst[2], L, out);
     else
         hipLaunchKernelGGL(k_settle<float>, dim3(P.nblk), dim3(256), 0, st, P, (const float*)src[0],
                            (const float*)src[1], (const float*)src[2], (float*)dst[0], (float*)dst[1],
-                           (float*)dst[2], L);
+                           (float*)dst[2], L, out);
 }
 
 void launch_import(int precision, const KParams& P, const void* const* src, void* const* dst, hipStream_t st) {
@@ -1528,18 +1554,18 @@ void launch_import(int precision, const KParams& P, const void* const* src, void
 }
 
 void launch_export(int precision, const KParams& P, const void* const* src, const void* zb, void* const* dst,
-                   void* const* keep, hipStream_t st) {
+                   void* const* keep, const DevLoop* L, LoopState* lout, hipStream_t st) {
     if (P.nblk <= 0) return;
     if (precision == 0)
         hipLaunchKernelGGL(k_export<double>, dim3(P.nblk), dim3(256), 0, st, P, (const double*)src[0],
                            (const double*)src[1], (const double*)src[2], (const double*)zb, (double*)dst[0],
                            (double*)dst[1], (double*)dst[2], (double*)dst[3], keep ? (double*)keep[0] : nullptr,
-                           keep ? (double*)keep[1] : nullptr, keep ? (double*)keep[2] : nullptr);
+                           keep ? (double*)keep[1] : nullptr, keep ? (double*)keep[2] : nullptr, L, lout);
     else
         hipLaunchKernelGGL(k_export<float>, dim3(P.nblk), dim3(256), 0, st, P, (const float*)src[0],
                            (const float*)src[1], (const float*)src[2], (const float*)zb, (float*)dst[0],
                            (float*)dst[1], (float*)dst[2], (float*)dst[3], keep ? (float*)keep[0] : nullptr,
-                           keep ? (float*)keep[1] : nullptr, keep ? (float*)keep[2] : nullptr);
+                           keep ? (float*)keep[1] : nullptr, keep ? (float*)keep[2] : nullptr, L, lout);
 }
 
 // Interior cells of n blocks, field by field of each (zs = zb + h, h, u, v
