@@ -84,9 +84,9 @@ struct bgf_batch_s {
     bool amr = false;
     int* d_inv = nullptr;
     int* d_nbr = nullptr;
-    int* d_fix = nullptr;
-    int4* d_rcell = nullptr;
+    int4* d_rcell = nullptr;  // with d_rmeta and d_fix behind it
     int2* d_rmeta = nullptr;
+    int* d_fix = nullptr;
     void* d_amr[11] = {nullptr};  // as a handle's: 2-9 face fluxes, 10 hsnap (0-1, remesh staging, unused)
     // the persistent kernels walk only the blocks of members still running:
     // their processing order, launch parameters, and the members it was built for
@@ -111,7 +111,7 @@ void free_batch(bgf_batch b) {
     F(b->d_zb); F(b->d_cf); F(b->d_dh); F(b->d_dhu); F(b->d_dhv); F(b->d_hmax); F(b->d_ch);
     F(b->d_volpart); F(b->d_volout); F(b->d_gcell); F(b->d_gval); F(b->d_loop);
     F(b->d_ring); F(b->d_tring);
-    F(b->d_inv); F(b->d_nbr); F(b->d_fix); F(b->d_rcell); F(b->d_rmeta);
+    F(b->d_inv); F(b->d_nbr); F(b->d_rcell);
     for (int k = 0; k < 11; k++) F(b->d_amr[k]);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -334,9 +334,7 @@ bgf_status bgf_batch_create(const bgf_param* common, int max_blocks, int max_mem
     b->amr = common->maxlevel > common->minlevel;
     if (b->amr) {
         ok = ok && A((void**)&b->d_inv, sizeof(int) * max_blocks) && A((void**)&b->d_nbr, sizeof(int) * bgf::NBR * (size_t)max_blocks) &&
-             A((void**)&b->d_fix, sizeof(int) * (size_t)max_blocks) &&
-             hipMalloc((void**)&b->d_rcell, sizeof(int4) * bgf::RECIPES * (size_t)max_blocks) == hipSuccess &&
-             hipMalloc((void**)&b->d_rmeta, sizeof(int2) * bgf::RECIPES * (size_t)max_blocks) == hipSuccess;
+             mesh_tables((size_t)max_blocks, &b->d_rcell, &b->d_rmeta, &b->d_fix);
         for (int k = 2; k < 11; k++) ok = ok && A(&b->d_amr[k], b->es * b->S);
     }
     if (!ok) {

@@ -57,7 +57,7 @@ struct bgf_handle_s {
     bool cf_shared = false;  // the caller holds the cf device array
     int *d_nb[8] = {nullptr};  // LeftBot LeftTop RightBot RightTop TopLeft TopRight BotLeft BotRight
     int* d_nbr = nullptr;      // multi-level meshes: the neighbour record of each block slot (bgf::NBR ints)
-    int4* d_rcell = nullptr;   // their gather recipes (bgf::RECIPES per slot)
+    int4* d_rcell = nullptr;   // their gather recipes (bgf::RECIPES per slot), with d_rmeta and d_fix behind them
     int2* d_rmeta = nullptr;
     int* d_fix = nullptr;      // and the blocks whose advance waits for other blocks' faces
     void *d_h[2] = {nullptr, nullptr}, *d_u[2] = {nullptr, nullptr}, *d_v[2] = {nullptr, nullptr};
@@ -141,7 +141,7 @@ void free_handle(bgf_handle h) {
     F(h->d_active); F(h->d_order); F(h->d_level); F(h->d_queue); F(h->d_rec);
     for (int k = 0; k < 15; k++) F(h->stats.a[k]);
     for (int k = 0; k < 8; k++) F(h->d_nb[k]);
-    F(h->d_nbr); F(h->d_rcell); F(h->d_rmeta); F(h->d_fix);
+    F(h->d_nbr); F(h->d_rcell);
     for (int k = 0; k < 2; k++) { F(h->d_h[k]); F(h->d_u[k]); F(h->d_v[k]); }
     F(h->d_zb); F(h->d_cf); F(h->d_dh); F(h->d_dhu); F(h->d_dhv);
     F(h->d_volpart); F(h->d_volout); F(h->d_loop);
@@ -625,9 +625,7 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     if (multilevel) {
         ok = ok && A((void**)&h->d_inv, sizeof(int) * cap);
         ok = ok && A((void**)&h->d_nbr, sizeof(int) * bgf::NBR * (size_t)cap);
-        ok = ok && hipMalloc((void**)&h->d_rcell, sizeof(int4) * bgf::RECIPES * (size_t)cap) == hipSuccess &&
-             hipMalloc((void**)&h->d_rmeta, sizeof(int2) * bgf::RECIPES * (size_t)cap) == hipSuccess;
-        ok = ok && A((void**)&h->d_fix, sizeof(int) * cap);
+        ok = ok && mesh_tables(cap, &h->d_rcell, &h->d_rmeta, &h->d_fix);
         for (int k = 0; k < 11; k++) ok = ok && A(&h->d_amr[k], h->es * SA);
     }
     if (!ok) {
