@@ -46,6 +46,8 @@
 // theta d2); the factor theta/2 enters the reconstruction's multiply-adds.
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <stdint.h>
 
 #include <limits>
@@ -1430,13 +1432,21 @@ void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* 
 }
 
 // Persistent grid: all workgroups resident at once (CUs x occupancy), a
-// multiple of NXCD, and no more than the blocks need.
-template <class K> int grid_for(K kernel, int nblk, int wg_per_cu) {
+// multiple of NXCD, and no more than the blocks need.  most: workgroups per CU
+// that a grid not asked for by wg_per_cu takes at the most.  The FP32
+// predictors fit seven by their registers, but the seventh starts late (its
+// first block waits for another workgroup's end, and the launch for it) and
+// more of them only lengthen the tail; six of the exact one and five of the
+// FAST one are as fast or faster at every size.  Ten steps, exact FP32: 720 x
+// 640 cells 392 -> 317 us, 1024 x 1024 557 -> 511, 2048 x 2048 1471 -> 1419,
+// 4096 x 4096 4763 -> 4786 (run to run: 1 %); FAST: 344 -> 262, 445 -> 378,
+// 1065 -> 1029, 3681 -> 3654.
+template <class K> int grid_for(K kernel, int nblk, int wg_per_cu, int most = 8) {
     int dev = 0, ncu = 0, occ = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, 256, 0) != hipSuccess) return 0;
-    if (wg_per_cu > 0 && wg_per_cu < occ) occ = wg_per_cu;
+    occ = std::min(occ, wg_per_cu > 0 ? wg_per_cu : most);
     if (occ < 1) occ = 1;
     long nwg = (long)ncu * occ;
     long need = ((long)nblk + NXCD - 1) / NXCD * NXCD;
@@ -1452,12 +1462,12 @@ int persistent_grid(int precision, int corrector, int nblk, int wg_per_cu) {
                          : grid_for(k_predictor<double, false, false, false>, nblk, w);
     if (precision == 1)
         return corrector ? grid_for(k_corrector<float, false, false, false>, nblk, w)
-                         : grid_for(k_predictor<float, false, false, false>, nblk, w);
+                         : grid_for(k_predictor<float, false, false, false>, nblk, w, 6);
     if (precision == 2)
         return corrector ? grid_for(k_corrector<float, true, false, false>, nblk, w)
-                         : grid_for(k_predictor<float, true, false, true>, nblk, w);
+                         : grid_for(k_predictor<float, true, false, true>, nblk, w, 5);
     return corrector ? grid_for(k_corrector<float, true, false, true>, nblk, w)
-                     : grid_for(k_predictor<float, true, false, true>, nblk, w);
+                     : grid_for(k_predictor<float, true, false, true>, nblk, w, 5);
 }
 
 void launch_init_dt(int precision, const KParams& P, const void* h, DevLoop* L, hipStream_t st) {
