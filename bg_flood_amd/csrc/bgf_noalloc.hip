@@ -20,10 +20,12 @@
 // streams in flight) race on the array.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "bgf_host.h"
 #include "bgf_kernels.h"
@@ -37,30 +39,32 @@ constexpr int MAX_DEVICES = 64;
 
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
-// Byte offsets of the scratch regions for nblk blocks of values of es bytes,
-// each region 256-byte aligned.
+// Byte offsets of the scratch regions for nblk blocks in `slots` block slots
+// and values of es bytes, each region 256-byte aligned.  The block records go
+// by position in the block list, the tendencies by block slot: the kernels
+// address every cell array with the slot, and a list may leave slots unused.
 struct Layout {
     size_t loop, queue, rec, dh, dhu, dhv, end;
 };
 inline size_t up256(size_t n) { return (n + 255) / 256 * 256; }
-Layout layout(long long nblk, size_t es) {
+Layout layout(long long nblk, long long slots, size_t es) {
     Layout L;
     L.loop = 0;
     L.queue = up256(2 * sizeof(bgf::DevLoop));  // the step's loop state and the one that it leaves
     L.rec = L.queue + up256(sizeof(int) * 2 * bgf::NXCD * bgf::QSTRIDE);
-    const size_t tend = up256((size_t)nblk * BSI * es);
+    const size_t tend = up256((size_t)slots * BSI * es);
     L.dh = L.rec + up256((size_t)nblk * 8 * sizeof(int));
     L.dhu = L.dh + tend;
     L.dhv = L.dhu + tend;
     L.end = L.dhv + tend;
     return L;
 }
-// The largest block count whose regions fit the array.
+// The largest count of blocks, without unused slots, whose regions fit the array.
 long long max_blocks(size_t es) {
     long long lo = 0, hi = (long long)(SCRATCH_BYTES / (BSI * es)) + 1;
     while (hi - lo > 1) {
         const long long mid = (lo + hi) / 2;
-        (layout(mid, es).end <= SCRATCH_BYTES ? lo : hi) = mid;
+        (layout(mid, mid, es).end <= SCRATCH_BYTES ? lo : hi) = mid;
     }
     return lo;
 }
@@ -124,7 +128,7 @@ bgf_status scratch_on_device(int dev, hipStream_t st, unsigned char** out) {
         const hipError_t e = hipGetSymbolAddress((void**)&ptr, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !ptr)
             return fail(BGF_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        const Layout L = layout(0, 4);
+        const Layout L = layout(0, 0, 4);
         const int nq = 2 * bgf::NXCD * bgf::QSTRIDE;
         hipLaunchKernelGGL(k_zero_ints, dim3((nq + 255) / 256), dim3(256), 0, st, (int*)(ptr + L.queue), nq);
         HIPCHK(hipGetLastError());
@@ -165,7 +169,19 @@ extern "C" bgf_status bgf_step_noalloc(const bgf_param* p, const bgf_blocks* d_b
     unsigned char* base = nullptr;
     s = scratch_on_device(dev, st, &base);
     if (s != BGF_OK) return s;
-    const Layout Lo = layout(p->nblk, es);
+    long long slots = p->nblkmem;
+    if (layout(p->nblk, slots, es).end > SCRATCH_BYTES) {
+        // the list may still use low slots only: those up to the greatest in it are needed
+        std::vector<int> act(p->nblk);
+        HIPCHK(hipMemcpyAsync(act.data(), d_blocks->active, sizeof(int) * act.size(), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        slots = *std::max_element(act.begin(), act.end()) + 1LL;
+        if (layout(p->nblk, slots, es).end > SCRATCH_BYTES)
+            return fail(BGF_ERR_INVALID_ARG, "a block in slot " + std::to_string(slots - 1) + ": the 64 MiB scratch "
+                                             "array does not hold " + std::to_string(slots) +
+                                             " block slots at this precision");
+    }
+    const Layout Lo = layout(p->nblk, slots, es);
     bgf::DevLoop* dL = (bgf::DevLoop*)(base + Lo.loop);
 
     bgf::KParams kp;

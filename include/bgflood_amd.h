@@ -187,7 +187,8 @@ bgf_status bgf_step_device(bgf_handle h, void* hh, void* zs, void* u, void* v, c
  * the call waits for it.  The step's scratch (tendencies, block records, loop
  * state, work-queue counters) is one 64 MiB device array per GPU, held until
  * the process ends: at most 21,618 blocks (FP32 forms) or 10,865 blocks (FP64),
- * BGF_ERR_INVALID_ARG beyond.  Calls on one GPU share that array: calls that
+ * and as many block slots up to the greatest in the list (somewhat more where
+ * the list is shorter), BGF_ERR_INVALID_ARG beyond.  Calls on one GPU share that array: calls that
  * overlap on one GPU (other threads, other streams) race. */
 bgf_status bgf_step_noalloc(const bgf_param* p, const bgf_blocks* d_blocks, const void* zb, const void* cf,
                             const void* hh, const void* u, const void* v, void* ho, void* uo, void* vo,

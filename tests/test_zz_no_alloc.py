@@ -115,3 +115,68 @@ def test_noalloc_refuses_what_it_cannot_hold():
     big64 = bgf._param_struct(dict(dd.param, precision="fp64", nblk=10866, nblkmem=10866))
     rc = L.bgf_step_noalloc(ctypes.byref(big64), ctypes.byref(dd.B), *args, ctypes.byref(loop), None)
     assert rc == 1 and b"10865" in L.bgf_last_error()
+
+
+def _spread(sc, slots, seed):
+    """The scenario with its blocks in random slots of `slots` ones, in another order of the list."""
+    p, b = sc["param"], sc["blocks"]
+    n = p["nblk"]
+    rng = np.random.default_rng(seed)
+    at = np.full(p["nblkmem"], -1)
+    at[b["active"][:n]] = np.append(rng.permutation(slots - 1)[:n - 1], slots - 1)
+    out = dict(sc, param=dict(p, nblkmem=slots))
+    blocks = {}
+    for k, v in b.items():
+        v = np.asarray(v)
+        if k == "active":
+            w = rng.permutation(at[v[:n]]).astype(v.dtype)
+        else:
+            w = np.zeros(slots, v.dtype)
+            w[at[b["active"][:n]]] = at[v[b["active"][:n]]] if k not in ("level", "xo", "yo") else v[b["active"][:n]]
+        blocks[k] = w
+    out["blocks"] = blocks
+    for k in ("zb", "h", "u", "v", "cf"):
+        a = np.zeros((slots, 324), np.asarray(sc[k]).dtype)
+        a[at[b["active"][:n]]] = np.asarray(sc[k]).reshape(-1, 324)[b["active"][:n]]
+        out[k] = a.reshape(-1)
+    return out, at
+
+
+# slots as many as the blocks, a few unused, and more than the scratch holds at the top of the arrays with all
+# used ones below (the declared count alone does not decide)
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("slots,declared", [(64, 64), (97, 97), (1500, 1500), (97, 30000)])
+def test_noalloc_with_unused_slots(slots, declared, prec):
+    L = _lib()
+    print("case no-alloc step: %s, 64 blocks in %d of %d slots" % (prec, slots, declared), flush=True)
+    sc = _scenario(128, prec)
+    sp, at = _spread(sc, slots, slots)
+    d = domain_for(sc, precision=prec)
+    lg = bgf.Loop(nextoutputtime=1e9, dt=0, dtmax=0, totaltime=0)
+    d.init_dt(lg)
+    dd = DeviceDomain(sp, prec)
+    dd.P.nblkmem = declared
+    ln = bgf.Loop(nextoutputtime=1e9, dt=lg.dt, dtmax=lg.dtmax, totaltime=0)
+    for _ in range(2):
+        d.step(lg)
+        dd.step(L, ln)
+        assert ln.dt == lg.dt and ln.dtmax == lg.dtmax
+    ref, got = d.get_state(), dd.state()
+    n = sc["param"]["nblk"]
+    act = sc["blocks"]["active"][:n]
+    for k in ("h", "u", "v"):
+        a, b = ref[k].reshape(-1, 18, 18)[act, 1:-1, 1:-1], got[k].reshape(-1, 18, 18)[at[act], 1:-1, 1:-1]
+        assert np.array_equal(a, b), k
+    d.close()
+
+
+def test_noalloc_refuses_slots_it_cannot_hold():
+    L = _lib()
+    sc = _scenario(128, "fp32")
+    sp, _ = _spread(sc, 22000, 1)
+    dd = DeviceDomain(sp, "fp32")
+    loop = bgf.Loop(nextoutputtime=1e9, dt=1.0, dtmax=1.0, totaltime=0)
+    a = dd.a
+    rc = L.bgf_step_noalloc(ctypes.byref(dd.P), ctypes.byref(dd.B), a["zb"].ptr, a["cf"].ptr, a["h"].ptr, a["u"].ptr,
+                            a["v"].ptr, a["ho"].ptr, a["uo"].ptr, a["vo"].ptr, ctypes.byref(loop), None)
+    assert rc == 1 and b"21999" in L.bgf_last_error()
