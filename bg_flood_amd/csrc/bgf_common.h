@@ -5,6 +5,7 @@
 
 #include <limits>
 
+#include "bgf_arith.h"
 #include "bgf_kernels.h"
 
 namespace bgf {
@@ -88,38 +89,6 @@ template <> struct Ar<float, true> {
     __device__ static __forceinline__ float sqrt_(float a) { return __builtin_amdgcn_sqrtf(a); }
 };
 
-// Division by a fixed d with the rounding of an IEEE division, in four
-// multiply-adds instead of its eleven instructions (of which the reciprocal
-// alone takes the time of four): with zh = RN(1/d) and zl the rest of 1/d,
-// q0 = RN(x zh + RN(x zl)) is within an ulp of x/d, the remainder r = x - d q0
-// is exact in a multiply-add, and RN(q0 + r zh) is the correctly rounded
-// quotient (Markstein, IBM J. Res. Dev. 34, 1990; the two-part reciprocal is
-// that of Brisebarre and Muller).  That needs x to be zero or between lo and
-// hi, well inside the normal range, and d in [2^-20, 2^20]; other x (the
-// numerical precursors of a wave reach such sizes) are `odd` and take the
-// division itself.
-template <class T> struct FixedDiv {
-    T d, zh, zl, lo, hi;
-};
-__host__ __device__ __forceinline__ void fixed_div_range(float& lo, float& hi) { lo = 0x1p-100f; hi = 0x1p100f; }
-__host__ __device__ __forceinline__ void fixed_div_range(double& lo, double& hi) { lo = 0x1p-960; hi = 0x1p960; }
-template <class T> __host__ __device__ __forceinline__ FixedDiv<T> fixed_div(T d) {
-    FixedDiv<T> K;
-    K.d = d;
-    K.zh = T(1.0) / d;
-    K.zl = fma(-d, K.zh, T(1.0)) * K.zh;
-    fixed_div_range(K.lo, K.hi);
-    if (!(d >= T(0x1p-20) && d <= T(0x1p20))) K.lo = K.hi = std::numeric_limits<T>::infinity();
-    return K;
-}
-template <class T> __device__ __forceinline__ bool odd_div(const FixedDiv<T>& K, T x) {
-    const T a = fabs(x);
-    return (a < K.lo && x != T(0.0)) || a > K.hi;
-}
-template <class T> __device__ __forceinline__ T quick_div(const FixedDiv<T>& K, T x) {
-    const T q = fma(x, K.zh, x * K.zl);
-    return fma(fma(-K.d, q, x), K.zh, q);
-}
 // The four quotients of a Q4.
 template <class T> __device__ __forceinline__ Q4<T> div4(const FixedDiv<T>& K, const Q4<T>& x) {
     Q4<T> q{quick_div(K, x.a), quick_div(K, x.b), quick_div(K, x.c), quick_div(K, x.d)};
@@ -128,22 +97,10 @@ template <class T> __device__ __forceinline__ Q4<T> div4(const FixedDiv<T>& K, c
     return q;
 }
 
-// 1 / b rounded as IEEE division rounds it, for b of ordinary size (here the
-// spread of a face's wave speeds, above epsilon wherever the result is used):
-// Newton steps on the hardware reciprocal and Markstein's correction, without
-// the scaling that extreme operands need.
-__device__ __forceinline__ double plain_rcp(double b) {
-    double y = __builtin_amdgcn_rcp(b);
-    y = fma(fma(-b, y, 1.0), y, y);
-    y = fma(fma(-b, y, 1.0), y, y);
-    return fma(fma(-b, y, 1.0), y, y);
-}
-__device__ __forceinline__ float plain_rcp(float b) {
-    float y = __builtin_amdgcn_rcpf(b);
-    y = fma(fma(-b, y, 1.0f), y, y);
-    y = fma(fma(-b, y, 1.0f), y, y);
-    return fma(fma(-b, y, 1.0f), y, y);
-}
+// 1 / b rounded as IEEE division rounds it (rounded_rcp), from the hardware's
+// reciprocal.
+__device__ __forceinline__ double plain_rcp(double b) { return rounded_rcp(b, __builtin_amdgcn_rcp(b)); }
+__device__ __forceinline__ float plain_rcp(float b) { return rounded_rcp(b, __builtin_amdgcn_rcpf(b)); }
 
 // The step that the drying limiter allows (src/Advection.cu:349-352):
 // min(dt, max(h, eps) / |dh|) evaluated in double, where dh < 0.  The limiter
