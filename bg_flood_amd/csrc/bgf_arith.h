@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <limits>
 
 namespace bgf {
 
@@ -31,7 +30,7 @@ template <class T> __host__ __device__ inline FixedDiv<T> fixed_div(T d) {
     K.zh = T(1.0) / d;
     K.zl = fma(-d, K.zh, T(1.0)) * K.zh;
     fixed_div_range(K.lo, K.hi);
-    if (!(d >= T(0x1p-20) && d <= T(0x1p20))) K.lo = K.hi = std::numeric_limits<T>::infinity();
+    if (!(d >= T(0x1p-20) && d <= T(0x1p20))) K.hi = T(-1.0);  // every x is odd
     return K;
 }
 template <class T> __host__ __device__ inline bool odd_div(const FixedDiv<T>& K, T x) {

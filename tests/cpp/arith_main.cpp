@@ -3,6 +3,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <random>
 #include <vector>
 
@@ -61,7 +62,8 @@ template <class T> T any(std::mt19937_64& rng) {
 template <class T> void fixed_divisions() {
     std::mt19937_64 rng(6);
     const T one = 1, ones = std::nextafter(T(2), one), inf = std::numeric_limits<T>::infinity();
-    std::vector<T> ds = {one / 3, 10, T(9.99), 40, 20, ones, std::nextafter(one, T(2)), T(0x1p-20), T(0x1p20)};
+    std::vector<T> ds = {one / 3, 10, T(9.99), 40, 20, ones, std::nextafter(one, T(2)), T(0x1p-20), T(0x1p20), T(0x1p-21), T(3e6), T(1e-4),
+                         T(0x1p-60)};
     for (T d : ds) {
         const bgf::FixedDiv<T> K = bgf::fixed_div(d);
         auto check = [&](T x) {
