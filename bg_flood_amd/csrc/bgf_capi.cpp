@@ -51,13 +51,16 @@ struct bgf_handle_s {
     int nblk, nblkmem;
     size_t S;   // elements per array
     std::vector<int> active;
+    // one allocation that holds the mesh's arrays and the loop state, and on multi-level meshes the
+    // cells' arrays and the staging of bgf_remesh as well (device_room)
+    void* arena = nullptr;
     int *d_active = nullptr, *d_order = nullptr, *d_level = nullptr;
     int* d_queue = nullptr;  // work-queue counters of the persistent kernels
     int* d_rec = nullptr;    // per-position block records of the processing order
     bool cf_shared = false;  // the caller holds the cf device array
     int *d_nb[8] = {nullptr};  // LeftBot LeftTop RightBot RightTop TopLeft TopRight BotLeft BotRight
     int* d_nbr = nullptr;      // multi-level meshes: the neighbour record of each block slot (bgf::NBR ints)
-    int4* d_rcell = nullptr;   // their gather recipes (bgf::RECIPES per slot), with d_rmeta and d_fix behind them
+    int4* d_rcell = nullptr;   // their gather recipes (bgf::RECIPES per slot)
     int2* d_rmeta = nullptr;
     int* d_fix = nullptr;      // and the blocks whose advance waits for other blocks' faces
     void *d_h[2] = {nullptr, nullptr}, *d_u[2] = {nullptr, nullptr}, *d_v[2] = {nullptr, nullptr};
@@ -138,30 +141,32 @@ namespace {
 
 void free_handle(bgf_handle h) {
     auto F = [](void* p) { if (p) (void)hipFree(p); };
-    F(h->d_active); F(h->d_order); F(h->d_level); F(h->d_queue); F(h->d_rec);
+    F(h->arena);
+    if (!h->amr) {
+        for (int k = 0; k < 2; k++) { F(h->d_h[k]); F(h->d_u[k]); F(h->d_v[k]); }
+        F(h->d_zb); F(h->d_cf); F(h->d_dh); F(h->d_dhu); F(h->d_dhv); F(h->d_ch);
+    }
     for (int k = 0; k < 15; k++) F(h->stats.a[k]);
-    for (int k = 0; k < 8; k++) F(h->d_nb[k]);
-    F(h->d_nbr); F(h->d_rcell);
-    for (int k = 0; k < 2; k++) { F(h->d_h[k]); F(h->d_u[k]); F(h->d_v[k]); }
-    F(h->d_zb); F(h->d_cf); F(h->d_dh); F(h->d_dhu); F(h->d_dhv);
-    F(h->d_volpart); F(h->d_volout); F(h->d_loop);
-    F(h->d_inv);
-    F(h->d_ch);
-    F(h->d_metric);
     F(h->d_bed);
     for (HostSeg& g : h->segs) free_seg(g);
     F(h->d_bseg); F(h->d_seg);
     F(h->d_rbox); F(h->d_rt); F(h->d_rq); F(h->d_rarea); F(h->d_roff); F(h->d_rblk);
-    F(h->d_blkxo); F(h->d_blkyo); F(h->d_rain_t); F(h->d_rain_v); F(h->d_rframes); F(h->d_rnow);
-    for (int k = 0; k < 11; k++) F(h->d_mesh2[k]);
-    F(h->d_remap); F(h->d_bxo); F(h->d_byo); F(h->d_flags);
+    F(h->d_rain_t); F(h->d_rain_v); F(h->d_rframes); F(h->d_rnow);
+    F(h->d_flags);
     F(h->d_gcell); F(h->d_gring); F(h->d_gtring);
-    for (int k = 0; k < 11; k++) F(h->d_amr[k]);
     for (int k = 0; k < 4; k++) if (h->ev[k]) (void)hipEventDestroy(h->ev[k]);
     if (h->graph) (void)hipGraphExecDestroy(h->graph);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     if (h->loop_host) (void)hipHostFree(h->loop_host);
     delete h;
+}
+
+// What a handle keeps besides its mesh's buffers: stream, events, pinned memory.
+void swap_host_side(bgf_handle a, bgf_handle b) {
+    std::swap(a->stream, b->stream);
+    std::swap(a->ev, b->ev);
+    std::swap(a->loop_host, b->loop_host);
+    std::swap(a->back, b->back);
 }
 
 bgf_status upload_loop(bgf_handle h, const bgf_loop* loop, double endtime) {
@@ -562,8 +567,67 @@ bgf_status setup_rivers(bgf_handle h) {
     return BGF_OK;
 }
 
-// bgf_create with device arrays for cap >= nblkmem block slots.
-bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_handle* out) {
+// The device arrays of a new handle for h->cap block slots, cleared.  What is
+// small goes into one allocation, and on multi-level meshes everything: such a
+// handle grows with its mesh (bgf_remesh re-creates it), and an allocation of a
+// cells' array takes 0.28 ms and its release 0.26 ms (5 MB each) wherever the
+// runtime has no freed piece of its size at hand, so that a growth of 22 of
+// them took from 3.8 to 6.8 ms as it came.
+bool device_room(bgf_handle h) {
+    const size_t cap = h->cap, cells = h->es * cap * BS;
+    const bool all = h->amr;
+    std::vector<std::pair<void**, size_t>> parts, own;
+    auto put = [&](auto*& ptr, size_t bytes) { parts.push_back({(void**)&ptr, bytes}); };
+    auto put_cells = [&](void*& ptr) { (all ? parts : own).push_back({&ptr, cells}); };
+    put(h->d_active, sizeof(int) * cap);
+    put(h->d_level, sizeof(int) * cap);
+    for (int k = 0; k < 8; k++) put(h->d_nb[k], sizeof(int) * cap);
+    put(h->d_volpart, sizeof(double) * cap);
+    put(h->d_volout, sizeof(double));
+    put(h->d_loop, 2 * sizeof(bgf::DevLoop));
+    put(h->d_blkxo, sizeof(double) * cap);
+    put(h->d_blkyo, sizeof(double) * cap);
+    for (int k = 0; k < 2; k++) {
+        put_cells(h->d_h[k]);
+        put_cells(h->d_u[k]);
+        put_cells(h->d_v[k]);
+    }
+    for (void** a : {&h->d_zb, &h->d_cf, &h->d_dh, &h->d_dhu, &h->d_dhv}) put_cells(*a);
+    if (h->p.spherical) put(h->d_metric, h->es * cap * bgf::METRIC_STRIDE);
+    if (all) {
+        put(h->d_inv, sizeof(int) * cap);
+        put(h->d_nbr, sizeof(int) * bgf::NBR * cap);
+        put(h->d_rcell, sizeof(int4) * bgf::RECIPES * cap);
+        put(h->d_rmeta, sizeof(int2) * bgf::RECIPES * cap);
+        put(h->d_fix, sizeof(int) * cap);
+        for (int k = 0; k < 11; k++) put_cells(h->d_amr[k]);
+        for (int k = 0; k < 11; k++) put(h->d_mesh2[k], sizeof(int) * cap);
+        put(h->d_remap, sizeof(int) * 5 * cap);
+        put(h->d_bxo, sizeof(double) * cap);
+        put(h->d_byo, sizeof(double) * cap);
+    } else {  // the persistent kernels' order, records and queues
+        put(h->d_order, sizeof(int) * cap);
+        put(h->d_rec, sizeof(int) * 8 * cap);
+        put(h->d_queue, sizeof(int) * 2 * bgf::NXCD * bgf::QSTRIDE);
+        if (h->prec == BGF_FP32_COMP) put_cells(h->d_ch);
+    }
+    auto up = [](size_t n) { return (n + 4095) / 4096 * 4096; };  // as allocations of their own are aligned
+    size_t bytes = 0;
+    for (auto& q : parts) bytes += up(q.second);
+    own.push_back({&h->arena, bytes});
+    for (auto& q : own)
+        if (hipMalloc(q.first, q.second) != hipSuccess || hipMemset(*q.first, 0, q.second) != hipSuccess) return false;
+    unsigned char* at = (unsigned char*)h->arena;
+    for (auto& q : parts) {
+        *q.first = at;
+        at += up(q.second);
+    }
+    return true;
+}
+
+// bgf_create with device arrays for cap >= nblkmem block slots.  from: a handle
+// that the new one replaces, whose stream, events and pinned memory it takes.
+bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_handle* out, bgf_handle from = nullptr) {
     if (!out || !b) return fail(BGF_ERR_INVALID_ARG, "null argument");
     *out = nullptr;
     bgf_status s = check_param(p);
@@ -581,6 +645,12 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     const int minlev = mi.minlev, maxlev = mi.maxlev;
     std::vector<int>& inv = mi.inv;
     auto* h = new bgf_handle_s();
+    if (from) swap_host_side(h, from);
+    auto drop = [&](bgf_status e) {
+        if (from) swap_host_side(h, from);
+        free_handle(h);
+        return e;
+    };
     h->p = *p;
     h->prec = p->precision;
     h->es = p->precision == 0 ? sizeof(double) : sizeof(float);
@@ -597,47 +667,21 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
         const int* nb[8] = {b->LeftBot, b->LeftTop, b->RightBot, b->RightTop, b->TopLeft, b->TopRight, b->BotLeft, b->BotRight};
         for (int k = 0; k < 8; k++) h->h_nb[k].assign(nb[k], nb[k] + nbm);
     }
-    auto A = [&](void** ptr, size_t bytes) -> bool {
-        if (hipMalloc(ptr, bytes) != hipSuccess) return false;
-        return hipMemset(*ptr, 0, bytes) == hipSuccess;
-    };
-    bool ok = true;
-    ok = ok && A((void**)&h->d_active, sizeof(int) * cap);
-    ok = ok && A((void**)&h->d_order, sizeof(int) * cap);
-    ok = ok && A((void**)&h->d_rec, sizeof(int) * 8 * (size_t)cap);
-    ok = ok && A((void**)&h->d_queue, sizeof(int) * 2 * bgf::NXCD * bgf::QSTRIDE);
-    ok = ok && A((void**)&h->d_level, sizeof(int) * cap);
-    for (int k = 0; k < 8; k++) ok = ok && A((void**)&h->d_nb[k], sizeof(int) * cap);
-    for (int k = 0; k < 2; k++) {
-        ok = ok && A(&h->d_h[k], h->es * SA);
-        ok = ok && A(&h->d_u[k], h->es * SA);
-        ok = ok && A(&h->d_v[k], h->es * SA);
-    }
-    ok = ok && A(&h->d_zb, h->es * SA) && A(&h->d_cf, h->es * SA);
-    ok = ok && A(&h->d_dh, h->es * SA) && A(&h->d_dhu, h->es * SA) && A(&h->d_dhv, h->es * SA);
-    ok = ok && A((void**)&h->d_volpart, sizeof(double) * cap) && A((void**)&h->d_volout, sizeof(double));
-    ok = ok && A((void**)&h->d_loop, 2 * sizeof(bgf::DevLoop));
-    ok = ok && hipHostMalloc((void**)&h->loop_host, sizeof(bgf::LoopState), hipHostMallocDefault) == hipSuccess;
-    ok = ok && A((void**)&h->d_blkxo, sizeof(double) * cap) && A((void**)&h->d_blkyo, sizeof(double) * cap);
     h->amr = multilevel;
-    if (p->precision == BGF_FP32_COMP && !multilevel) ok = ok && A(&h->d_ch, h->es * SA);
-    if (p->spherical) ok = ok && A(&h->d_metric, h->es * (size_t)cap * bgf::METRIC_STRIDE);
-    if (multilevel) {
-        ok = ok && A((void**)&h->d_inv, sizeof(int) * cap);
-        ok = ok && A((void**)&h->d_nbr, sizeof(int) * bgf::NBR * (size_t)cap);
-        ok = ok && mesh_tables(cap, &h->d_rcell, &h->d_rmeta, &h->d_fix);
-        for (int k = 0; k < 11; k++) ok = ok && A(&h->d_amr[k], h->es * SA);
-    }
+    bool ok = device_room(h);
+    if (!h->loop_host)
+        ok = ok && hipHostMalloc((void**)&h->loop_host, sizeof(bgf::LoopState), hipHostMallocDefault) == hipSuccess;
     if (!ok) {
-        free_handle(h);
         (void)hipGetLastError();
-        return fail(BGF_ERR_OOM, "device allocation failed");
+        return drop(fail(BGF_ERR_OOM, "device allocation failed"));
     }
     const int* nbs[8] = {b->LeftBot, b->LeftTop, b->RightBot, b->RightTop, b->TopLeft, b->TopRight, b->BotLeft, b->BotRight};
     h->xy = block_xy(b, nblk, p->dx);
-    std::vector<int> order = processing_order(h->xy);
     bool cp = hipMemcpy(h->d_active, b->active, sizeof(int) * nblk, hipMemcpyHostToDevice) == hipSuccess;
-    cp = cp && hipMemcpy(h->d_order, order.data(), sizeof(int) * nblk, hipMemcpyHostToDevice) == hipSuccess;
+    if (!multilevel) {
+        std::vector<int> order = processing_order(h->xy);
+        cp = cp && hipMemcpy(h->d_order, order.data(), sizeof(int) * nblk, hipMemcpyHostToDevice) == hipSuccess;
+    }
     cp = cp && hipMemcpy(h->d_level, b->level, sizeof(int) * nbm, hipMemcpyHostToDevice) == hipSuccess;
     cp = cp && hipMemcpy(h->d_blkxo, b->xo, sizeof(double) * nbm, hipMemcpyHostToDevice) == hipSuccess;
     cp = cp && hipMemcpy(h->d_blkyo, b->yo, sizeof(double) * nbm, hipMemcpyHostToDevice) == hipSuccess;
@@ -646,12 +690,11 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     if (multilevel) {
         cp = cp && hipMemcpy(h->d_inv, inv.data(), sizeof(int) * nbm, hipMemcpyHostToDevice) == hipSuccess;
     }
-    cp = cp && hipStreamCreate(&h->stream) == hipSuccess;
-    for (int k = 0; k < 4; k++) cp = cp && hipEventCreate(&h->ev[k]) == hipSuccess;
-    if (!cp) {
-        free_handle(h);
-        return fail(BGF_ERR_HIP, "device upload failed");
+    if (!from) {
+        cp = cp && hipStreamCreate(&h->stream) == hipSuccess;
+        for (int k = 0; k < 4; k++) cp = cp && hipEventCreate(&h->ev[k]) == hipSuccess;
     }
+    if (!cp) return drop(fail(BGF_ERR_HIP, "device upload failed"));
     bgf::KParams& kp = h->kp;
     kp.g = p->g; kp.eps = p->eps; kp.CFL = p->CFL; kp.theta = p->theta;
     kp.delta0 = p->delta;
@@ -673,10 +716,7 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     if (const char* e = std::getenv("BGF_GRAPH")) h->use_graph = std::atoi(e) != 0;
     kp.grid_pred = bgf::persistent_grid(h->prec, 0, nblk, h->wg_pred);
     kp.grid_corr = bgf::persistent_grid(h->prec, 1, nblk, h->wg_corr);
-    if (kp.grid_pred <= 0 || kp.grid_corr <= 0) {
-        free_handle(h);
-        return fail(BGF_ERR_HIP, "occupancy query failed");
-    }
+    if (kp.grid_pred <= 0 || kp.grid_corr <= 0) return drop(fail(BGF_ERR_HIP, "occupancy query failed"));
     kp.active = h->d_active;
     kp.order = h->d_order;
     kp.rec = h->d_rec;
@@ -702,16 +742,10 @@ bgf_status create_handle(const bgf_param* p, const bgf_blocks* b, int cap, bgf_h
     kp.rcell = h->d_rcell;
     kp.rmeta = h->d_rmeta;
     if (multilevel) bgf::launch_amr_nbr(kp, h->d_nbr, nbm, h->d_rcell, h->d_rmeta, h->stream);
+    else bgf::launch_records(kp, h->d_rec, h->stream);
+    if (hipGetLastError() != hipSuccess) return drop(fail(BGF_ERR_HIP, "block records launch failed"));
     s = setup_fix(h);
-    if (s != BGF_OK) {
-        free_handle(h);
-        return s;
-    }
-    bgf::launch_records(kp, h->d_rec, h->stream);
-    if (hipGetLastError() != hipSuccess) {
-        free_handle(h);
-        return fail(BGF_ERR_HIP, "block records launch failed");
-    }
+    if (s != BGF_OK) return drop(s);
     *out = h;
     g_err.clear();
     return BGF_OK;
@@ -1456,38 +1490,29 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
         s = create_handle(&q, b,
                           (int)std::min<long long>(std::min<long long>(2LL * nbm, kMaxBlocks),
                                                    max_blocks_for(q.precision)),
-                          &nh);
+                          &nh, h);
         if (s != BGF_OK) return s;
-        bool ok = hipMalloc((void**)&nh->d_remap, sizeof(int) * 5 * (size_t)nh->cap) == hipSuccess &&
-                  hipMalloc((void**)&nh->d_bxo, sizeof(double) * nh->cap) == hipSuccess &&
-                  hipMalloc((void**)&nh->d_byo, sizeof(double) * nh->cap) == hipSuccess;
-        ok = ok && hipMemcpy(nh->d_remap, remap, sizeof(int) * 5 * (size_t)nbm, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(nh->d_bxo, b->xo, sizeof(double) * nbm, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(nh->d_byo, b->yo, sizeof(double) * nbm, hipMemcpyHostToDevice) == hipSuccess;
-        if (!ok) {
-            bgf_destroy(nh);
-            return fail(BGF_ERR_HIP, "remesh: upload failed");
-        }
-        bgf::launch_amr_halo(prec, h->kp, h->d_h[0], h->d_u[0], h->d_v[0], h->d_zb, h->stream);
+        auto undo = [&](bgf_status e) {
+            (void)hipStreamSynchronize(nh->stream);
+            swap_host_side(nh, h);
+            free_handle(nh);
+            return e;
+        };
+        if (hipMemcpy(nh->d_remap, remap, sizeof(int) * 5 * (size_t)nbm, hipMemcpyHostToDevice) != hipSuccess)
+            return undo(fail(BGF_ERR_HIP, "remesh: upload failed"));
+        bgf::launch_amr_halo(prec, h->kp, h->d_h[0], h->d_u[0], h->d_v[0], h->d_zb, nh->stream);
         bgf::RemeshLaunch R;
         R.nblk = q.nblk;
         R.h = h->d_h[0]; R.u = h->d_u[0]; R.v = h->d_v[0]; R.zb = h->d_zb; R.cf = h->d_cf;
-        R.active = nh->d_active; R.level = nh->d_level; R.xo = nh->d_bxo; R.yo = nh->d_byo; R.remap = nh->d_remap;
+        R.active = nh->d_active; R.level = nh->d_level; R.xo = nh->d_blkxo; R.yo = nh->d_blkyo; R.remap = nh->d_remap;
         R.nh = nh->d_h[0]; R.nu = nh->d_u[0]; R.nv = nh->d_v[0]; R.nzb = nh->d_zb; R.ncf = nh->d_cf;
         R.bed = h->d_bed; R.bnx = h->bed_nx; R.bny = h->bed_ny; R.bxo = h->bed_xo; R.byo = h->bed_yo;
         R.bdx = h->bed_dx; R.pxo = q.xo; R.pyo = q.yo; R.dx = q.dx; R.eps = q.eps;
-        bgf::launch_remesh(prec, h->kp, R, h->stream);
+        bgf::launch_remesh(prec, h->kp, R, nh->stream);
+        bgf::launch_amr_fill(prec, nh->kp, nh->d_zb, nh->stream);  // the bed's halo (src/InitialConditions.cu:135-147)
         hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        if (e == hipSuccess) {
-            bgf::launch_amr_fill(prec, nh->kp, nh->d_zb, nh->stream);  // the bed's halo (src/InitialConditions.cu:135-147)
-            e = hipGetLastError();
-            if (e == hipSuccess) e = hipStreamSynchronize(nh->stream);
-        }
-        if (e != hipSuccess) {
-            bgf_destroy(nh);
-            return fail(BGF_ERR_HIP, std::string("remesh: ") + hipGetErrorString(e));
-        }
+        if (e == hipSuccess) e = hipStreamSynchronize(nh->stream);
+        if (e != hipSuccess) return undo(fail(BGF_ERR_HIP, std::string("remesh: ") + hipGetErrorString(e)));
         nh->state_set = true;
         nh->timing = h->timing;
         nh->use_graph = h->use_graph;
@@ -1521,7 +1546,7 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
         std::swap(*h, *nh);  // h takes the new mesh; nh (the old one) is freed
         const int smask = nh->stats.mask;
         const double sthr = nh->stats.wet_threshold;
-        bgf_destroy(nh);
+        free_handle(nh);
         if (smask) {  // the statistics restart on the new mesh
             s = bgf_set_stats(h, smask, sthr);
             if (s != BGF_OK) return s;
@@ -1538,17 +1563,9 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
     // in place: the new mesh goes to the staging arrays, the new state to the
     // scratch buffers (buffer 1 of h, u, v; two of the stage arrays for the bed
     // and the roughness), then the pointers are exchanged
-    const int cap = h->cap;
-    bool ok = true;
-    for (int k = 0; k < 11; k++)
-        if (!h->d_mesh2[k]) ok = ok && hipMalloc((void**)&h->d_mesh2[k], sizeof(int) * cap) == hipSuccess;
-    if (!h->d_remap) ok = ok && hipMalloc((void**)&h->d_remap, sizeof(int) * 5 * (size_t)cap) == hipSuccess;
-    if (!h->d_bxo) ok = ok && hipMalloc((void**)&h->d_bxo, sizeof(double) * cap) == hipSuccess;
-    if (!h->d_byo) ok = ok && hipMalloc((void**)&h->d_byo, sizeof(double) * cap) == hipSuccess;
-    if (!ok) return fail(BGF_ERR_OOM, "remesh: staging allocation failed");
     const int* src[10] = {b->level, b->LeftBot, b->LeftTop, b->RightBot, b->RightTop,
                           b->TopLeft, b->TopRight, b->BotLeft, b->BotRight, mi.inv.data()};
-    ok = hipMemcpy(h->d_mesh2[0], b->active, sizeof(int) * q.nblk, hipMemcpyHostToDevice) == hipSuccess;
+    bool ok = hipMemcpy(h->d_mesh2[0], b->active, sizeof(int) * q.nblk, hipMemcpyHostToDevice) == hipSuccess;
     for (int k = 0; k < 10; k++)
         ok = ok && hipMemcpy(h->d_mesh2[1 + k], src[k], sizeof(int) * nbm, hipMemcpyHostToDevice) == hipSuccess;
     ok = ok && hipMemcpy(h->d_remap, remap, sizeof(int) * 5 * (size_t)nbm, hipMemcpyHostToDevice) == hipSuccess &&
@@ -1692,11 +1709,13 @@ bgf_status bgf_set_schedule(bgf_handle h, int tile_x, int tile_y, int wg_pred, i
         return fail(BGF_ERR_INVALID_ARG, "schedule out of range");
     const int tx = tile_x ? tile_x : h->tile_x, ty = tile_y ? tile_y : h->tile_y;
     if (tx != h->tile_x || ty != h->tile_y) {
-        std::vector<int> order = processing_order(h->xy, tx, ty);
-        HIPCHK(hipStreamSynchronize(h->stream));
-        HIPCHK(hipMemcpy(h->d_order, order.data(), sizeof(int) * h->nblk, hipMemcpyHostToDevice));
-        bgf::launch_records(h->kp, h->d_rec, h->stream);
-        HIPCHK(hipGetLastError());
+        if (!h->amr) {  // multi-level meshes have no processing order
+            std::vector<int> order = processing_order(h->xy, tx, ty);
+            HIPCHK(hipStreamSynchronize(h->stream));
+            HIPCHK(hipMemcpy(h->d_order, order.data(), sizeof(int) * h->nblk, hipMemcpyHostToDevice));
+            bgf::launch_records(h->kp, h->d_rec, h->stream);
+            HIPCHK(hipGetLastError());
+        }
         h->tile_x = tx;
         h->tile_y = ty;
     }

@@ -114,3 +114,46 @@ def test_adapt_helper_keeps_the_lake_at_rest_away_from_the_shore():
     assert deep.sum() > 1000
     assert np.max(np.abs(st["zs"][m][deep])) < 1e-12
     assert np.all(st["u"][m] == 0) and np.all(st["v"][m] == 0)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_growth_twice_keeps_the_handle(prec):
+    """Refinement beyond the handle's slots, twice, and back within them: the state read, run (replayed and
+    launched) and timed before and after, the stream, events and pinned memory being those of the first mesh."""
+    sc = scenario(prec)
+    d, o = domain_for(sc, precision=prec), oracle_for(sc, precision=prec)
+    d.set_timing(False)
+    lg = bgf.Loop(nextoutputtime=1e9, dt=0, dtmax=0, totaltime=0)
+    lo = po.OrcLoop(nextoutputtime=1e9, dt=0, dtmax=0, totaltime=0)
+    d.init_dt(lg)
+    o.init_loop(lo)
+    rng = np.random.default_rng(3)
+    room = d.nblkmem  # slots that the handle has: twice the need after each growth
+    grown = 0
+    for cycle, share in enumerate((0.0, 1.0, 0.9, 0.4)):
+        ref = np.zeros(d.nblkmem, np.uint8)
+        ref[d.active] = rng.random(d.nblk) < share
+        co = np.zeros(d.nblkmem, np.uint8)
+        co[d.active] = 1 - ref[d.active]
+        blocks, nb, nm, remap = bgf.adapt_mesh(d.param, d.blocks, ref, co if share < 0.5 else None, NBX, NBY)
+        print("case growth %s cycle=%d nblk=%d -> %d, slots %d of %d" % (prec, cycle, d.nblk, nb, nm, room), flush=True)
+        if nm > room:
+            room, grown = 2 * nm, grown + 1
+        d.remesh(blocks, nb, nm, remap)
+        o.remesh(orc_param_with(o.p, nblk=nb, nblkmem=nm), blocks, remap, bed=None)
+        assert_same_state(d, o)
+        for n in (19, 3):  # replays of the captured steps with some left over, and launches
+            d.run(lg, n)
+            o.run(lo, n)
+            assert (lg.dt, lg.totaltime) == (lo.dt, lo.totaltime)
+            assert_same_state(d, o)
+        d.set_timing(True)
+        d.run(lg, 1)
+        o.run(lo, 1)
+        t = d.kernel_times()
+        d.set_timing(False)
+        assert t["k_predictor"] > 0 and t["k_corrector"] > 0
+        d.set_schedule(8 + cycle, 8)  # accepted, without effect on a multi-level mesh
+    assert grown == 2
+    assert_same_state(d, o)
+    d.close()
