@@ -28,10 +28,12 @@ import numpy as np
 from . import BS, Batch, BgfError, Domain, Loop, interior_mask
 
 # HBM bytes of one block slot in the batch (h, u, v twice, zb, cf, dh, dhu, dhv, max depth,
-# compensation) and of one block of a multi-level domain (those arrays without the compensation,
-# the eight face-flux arrays and the pre-prolongation copy of h, with a margin).
+# compensation) and of one block slot of a multi-level domain or batch: the cells' arrays (those
+# without the compensation, the eight face-flux arrays, the pre-prolongation copy of h, and in a
+# domain the remesh staging of the bed and the roughness instead of the max depth), the gather
+# recipes (132 entries of 24 bytes), the neighbour record (64) and the block lists and tables.
 BATCH_BYTES_PER_BLOCK = 13 * BS * 4
-AMR_BYTES_PER_BLOCK = 22 * BS * 4
+AMR_BYTES_PER_BLOCK = 22 * BS * 4 + 132 * 24 + 64 + 160
 
 
 class Request:

@@ -1,10 +1,14 @@
 """Continuous batching on the GPU: requests that arrive while others run are admitted as slots free
 up, run overlapped, and each result (maximum depth, gauge series) is bit-identical to the same
 request served alone."""
+import ctypes
+
 import numpy as np
 import pytest
 
+import bg_flood_amd as bgf
 from bg_flood_amd import scenarios, serving
+from tests._util import hip
 
 pytestmark = pytest.mark.gpu
 
@@ -155,3 +159,29 @@ def test_admission_is_first_fit():
     assert [r.rid for r in srv.waiting] == [0]
     assert any(r is small for r in srv.members.values())
     srv.close()
+
+
+def _device_bytes_free():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("kind", ["domain", "batch"])
+def test_admission_counts_the_memory_of_a_multi_level_slot(kind):
+    """A multi-level domain's and batch's device memory for many block slots against what admission
+    counts for them: no more than counted (allocations are rounded up: 2 %), and most of it used."""
+    slots = 100000
+    sc = scenarios.amr_basin(precision="fp32")
+    print("case memory of %d slots, %s" % (slots, kind), flush=True)
+    small = dict(sc["param"])
+    bgf.Domain(small, sc["blocks"]).close()  # the runtime's own first allocations
+    before = _device_bytes_free()
+    if kind == "domain":
+        x = bgf.Domain(dict(small, nblkmem=slots), sc["blocks"])
+    else:
+        x = bgf.Batch(small, slots, 8)
+    used = before - _device_bytes_free()
+    x.close()
+    counted = serving.AMR_BYTES_PER_BLOCK * slots
+    assert 0.9 * counted < used < 1.02 * counted, (used, counted)
