@@ -156,6 +156,21 @@ __device__ __forceinline__ void slots_empty(DevLoop* L) {
     L->slot64[l] = 0x7ff0000000000000ull;
 }
 
+// The first entry k from lo on of a series of increasing times t with
+// t[k] > tt (or >= tt where AT), or its last entry n - 1.  By halves: the
+// entries are read one after the other, and a series by the minute over days
+// has thousands.
+template <bool AT> __device__ __forceinline__ int series_entry(const double* t, int lo, int n, double tt) {
+    int hi = n - 1;
+    while (lo < hi) {
+        const int m = (lo + hi) >> 1;
+        const double d = t[m] - tt;
+        if (AT ? d < 0.0 : d <= 0.0) lo = m + 1;
+        else hi = m;
+    }
+    return lo;
+}
+
 // A loop state past the dt reduction of its step, from the slots' minimum m:
 // the smaller of m and 1/epsi, the clamp and the output-time landing of
 // CalctimestepCPU in FP64.  mode 0: a step that leaves totaltime to the caller;
@@ -170,8 +185,7 @@ template <class T> __device__ __forceinline__ void advance_loop(LoopState& L, T 
         // the uniform rain of this step, at its start (Forcingthisstep,
         // src/Updateforcing.cu:45-60, interptime src/Util_CPU.cu:107-110)
         const double tt = L.totaltime;
-        int k = 1;
-        while (k < L.rain_n - 1 && L.rain_t[k] - tt < 0.0) k++;
+        const int k = series_entry<true>(L.rain_t, 1, L.rain_n, tt);
         const double prev = L.rain_v[k - 1];
         const double now = prev + (tt - L.rain_t[k - 1]) / (L.rain_t[k] - L.rain_t[k - 1]) * (L.rain_v[k] - prev);
         L.rain = now;
@@ -384,8 +398,7 @@ __device__ __forceinline__ T river_inflow(const KParams& P, int ib, int ix, int 
             const double* t = P.rt + P.roff[r];
             const double* q = P.rq + P.roff[r];
             const int n = P.roff[r + 1] - P.roff[r];
-            int e = 0;
-            while (e < n - 1 && t[e] - tt <= 0.0) e++;  // the reference does not stop at the end
+            const int e = series_entry<false>(t, 0, n, tt);  // the reference does not stop at the end
             const int a = e - 1 > 0 ? e - 1 : 0;
             const double flow = q[a] + (tt - t[a]) / (t[e] - t[a]) * (q[e] - q[a]);
             // the reference's array of rates is a T
