@@ -8,10 +8,10 @@ keep the L2 working set small).  Results do not depend on either (every block is
 way and the time step is a minimum), so the tuner only times.
 
 The search is coordinate-wise: tiles at the default workgroup counts, then the predictor's
-workgroups per CU, then the corrector's, each candidate warmed up (first run captures its graph) and
-timed as the best of a few repeats of `steps` steps.  Tuning advances the state it runs on, so it runs
-on a scratch Domain or Batch (autotune_domain and autotune_batch build one from the caller's inputs
-and free it).  Chosen schedules can be kept in a JSON cache keyed by the workload.
+workgroups per CU, then the corrector's, each candidate warmed up (the first run of its length captures
+its graph) and timed as the best of a few repeats of `steps` steps.  Tuning advances the state it runs
+on, so it runs on a scratch Domain or Batch (autotune_domain and autotune_batch build one from the
+caller's inputs and free it).  Chosen schedules can be kept in a JSON cache keyed by the workload.
 """
 import json
 import os
@@ -22,7 +22,7 @@ MAX_WG = 8
 
 
 def _time(run, steps, repeats):
-    run(max(2, steps // 4))  # warm-up: captures the candidate's graph
+    run(steps)  # warm-up: a run of this length captures the candidate's graph if the timed ones replay one
     best = float("inf")
     for _ in range(repeats):
         t0 = time.perf_counter()

@@ -40,6 +40,25 @@ def test_tune_finds_the_coordinate_minimum(monkeypatch):
         assert abs(t["s_per_step"] - cost(t["tile_x"], t["tile_y"], t["wg_pred"], t["wg_corr"])) < 1e-12
 
 
+def test_tune_times_no_capture(monkeypatch):
+    """Runs of sixteen steps and more replay a graph, which the first of them with a schedule captures:
+    that first one is not among the timed runs, however few they are."""
+    class Capturing(FakeStep):
+        captured = None
+
+        def run(self, n):
+            super().run(n)
+            if n >= 16 and self.captured != self.s:
+                self.captured = self.s
+                self.clock += 100.0
+
+    for steps in (8, 16, 40):
+        f = Capturing(lambda *s: 1.0)
+        monkeypatch.setattr(autotune.time, "perf_counter", lambda: f.clock)
+        _, trials = autotune.tune(f, f.run, steps=steps, repeats=1, max_wg=2)
+        assert all(t["s_per_step"] == 1.0 for t in trials)
+
+
 def test_tune_keeps_the_default_on_ties(monkeypatch):
     f = FakeStep(lambda *s: 1.0)
     monkeypatch.setattr(autotune.time, "perf_counter", lambda: f.clock)
