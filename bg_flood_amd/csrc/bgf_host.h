@@ -58,10 +58,13 @@ inline bool device_accessible(const void* p) {
 // rows over the caller's arrays (whose other cells stay as they are); one piece
 // is written while the one before is spread, so the pinned memory stays small.
 // Copying whole arrays, with their halos and the bed, through pageable memory
-// took 3.48 ms for the eight members (25.6 MB of arrays) of an ensemble.
+// took 3.48 ms for the eight members (25.6 MB of arrays) of an ensemble.  The
+// pieces are no larger than what was read through them needs, and one that
+// suffices has no second: a domain of one block takes 8 KB, not 2 MB.
 struct ReadBack {
-    static constexpr size_t PIECE = 1024 * 1024;  // bytes of one of the two pieces
+    static constexpr size_t PIECE = 1024 * 1024;  // bytes of one of the two pieces at the most, a power of two
     unsigned char* mem[2] = {nullptr, nullptr};
+    size_t size[2] = {0, 0};
     hipEvent_t ev[2] = {nullptr, nullptr};
     std::mutex busy;  // several threads may read the states of one batch
     ~ReadBack() {
@@ -99,14 +102,21 @@ inline bgf_status read_back(ReadBack& R, int prec, const std::vector<int>& activ
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? hipEventRecord(R.ev[k & 1], st) : e;
     };
-    for (int k = 0; k < 2; k++) {
+    for (int k = 0; k < std::min(2, pieces); k++) {
         if (!R.ev[k]) HIPCHK(hipEventCreateWithFlags(&R.ev[k], hipEventDisableTiming));
+        size_t need = 4096;  // doubled: at most eight times for a handle
+        while (need < (size_t)std::min(per, n) * nf * BSI * es) need *= 2;
+        if (R.size[k] >= need) continue;
+        if (R.mem[k]) (void)hipHostFree(R.mem[k]);
+        R.mem[k] = nullptr;
+        R.size[k] = 0;
         void* p = nullptr;
-        if (!R.mem[k] && hipHostMalloc(&p, ReadBack::PIECE, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc(&p, need, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             return fail(BGF_ERR_OOM, "host allocation failed");
         }
-        if (p) R.mem[k] = (unsigned char*)p;
+        R.mem[k] = (unsigned char*)p;
+        R.size[k] = need;
     }
     HIPCHK(fetch(0));
     for (int k = 0; k < pieces; k++) {

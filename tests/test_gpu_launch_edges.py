@@ -122,3 +122,34 @@ def test_multi_level_reduction(part, above):
     print("case multi-level reduction, %d blocks" % n, flush=True)
     assert (n > 4096) == above
     against_oracle(sc, "fp32", 3)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_read_back_grows_with_the_members(prec):
+    """Members of one batch read in turn, from one block to more than a piece of the pinned memory holds and
+    back, all fields and some: the pieces grow from read to read."""
+    T = np.float64 if prec == "fp64" else np.float32
+    sides = [(1, 1), (3, 1), (17, 2), (40, 9), (2, 1)]
+    parts = [scenarios.uniform(16 * nx, 16 * ny, 1.0, prec)[:2] for nx, ny in sides]
+    rng = np.random.default_rng(2)
+    b = bgf.Batch(parts[0][0], sum(p["nblkmem"] for p, _ in parts), len(parts))
+    held = []
+    for p, blocks in parts:
+        n = p["nblkmem"] * 324
+        a = [(1.0 + rng.random(n)).astype(T) for _ in range(5)]
+        held.append((b.add(p, blocks, *a, endtime=1e9), p, blocks, a))
+    for order in (range(len(held)), reversed(range(len(held)))):
+        for k in order:
+            mid, p, blocks, (zb, h, u, v, _) = held[k]
+            print("case read-back of member %d, %d blocks, %s" % (k, p["nblk"], prec), flush=True)
+            m = bgf.interior_mask(p["nblkmem"], blocks["active"][:p["nblk"]])
+            n = p["nblkmem"] * 324
+            want = dict(zs=zb + h, h=h, u=u, v=v)
+            for fields in (("u",), ("zs", "h", "u", "v")):
+                out = {f: np.full(n, -7, T) for f in fields}
+                rc = bgf.lib().bgf_batch_get_state(b.h, mid, *[out[f].ctypes.data if f in out else None
+                                                               for f in ("zs", "h", "u", "v")])
+                assert rc == 0
+                for f in fields:
+                    assert np.array_equal(out[f][m], want[f][m]) and (out[f][~m] == -7).all(), f
+    b.close()
