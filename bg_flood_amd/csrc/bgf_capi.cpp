@@ -429,7 +429,7 @@ bgf_status setup_fix(bgf_handle h) {
 // src/ReadInput.cu:1282-1283 sets it, and epsbnd = calcres(dx, initlevel) with
 // initlevel 0), and the device table with the remainder (type aoibnd) last.
 // Without segments every boundary face is of type aoibnd and nothing is kept.
-bgf_status setup_segments(bgf_handle h) {
+bgf_status segment_table(bgf_handle h) {
     bgf::KParams& kp = h->kp;
     if (h->d_bseg) (void)hipFree(h->d_bseg);
     if (h->d_seg) (void)hipFree(h->d_seg);
@@ -442,7 +442,7 @@ bgf_status setup_segments(bgf_handle h) {
         (void)hipGraphExecDestroy(h->graph);
         h->graph = nullptr;
     }
-    if (h->segs.empty()) return setup_fix(h);
+    if (h->segs.empty()) return BGF_OK;
     const bgf_param& p = h->p;
     auto inT = [&](double v) { return h->prec == 0 ? v : (double)(float)v; };  // XBlock.xo is a T
     double xmax = -1e300, ymax = -1e300;
@@ -458,6 +458,7 @@ bgf_status setup_segments(bgf_handle h) {
         h->prec == 0 ? assign_segments<double>(p, h->active, h->h_level, h->h_xo, h->h_yo, h->h_nb, polys, h->cap)
                      : assign_segments<float>(p, h->active, h->h_level, h->h_xo, h->h_yo, h->h_nb, polys, h->cap);
     std::vector<bgf::BSeg> tab;
+    int open = 0, mapmax = 0;
     for (const HostSeg& g : h->segs) {
         bgf::BSeg b{};
         b.type = g.type == 4 ? 1 : g.type;  // type 4 acts as type 1 in engine 2's flux boundary
@@ -474,10 +475,10 @@ bgf_status setup_segments(bgf_handle h) {
         } else if (g.nt >= 2) {
             b.frames = g.d_frames;
             b.now = g.d_now;
-            kp.bmapmax = std::max(kp.bmapmax, g.nx * g.ny);
+            mapmax = std::max(mapmax, g.nx * g.ny);
         }
         b.on = b.n >= 2 || b.now ? 1 : 0;
-        kp.bopen |= b.type >= 2 ? 1 : 0;
+        open |= b.type >= 2 ? 1 : 0;
         tab.push_back(b);
     }
     bgf::BSeg rem{};
@@ -491,7 +492,16 @@ bgf_status setup_segments(bgf_handle h) {
     kp.bseg = h->d_bseg;
     kp.seg = h->d_seg;
     kp.nseg = (int)tab.size();
-    return setup_fix(h);
+    kp.bopen = open;
+    kp.bmapmax = mapmax;
+    return BGF_OK;
+}
+
+// The segments and the blocks whose advance waits for them, which the stage
+// takes from kp.bopen: the two agree also where the table could not be made.
+bgf_status setup_segments(bgf_handle h) {
+    const bgf_status s = segment_table(h), f = setup_fix(h);
+    return s != BGF_OK ? s : f;
 }
 
 // The rivers on the handle's current mesh (InitialConditions.cu:346-445):
@@ -1627,11 +1637,6 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
         const int* nb[8] = {b->LeftBot, b->LeftTop, b->RightBot, b->RightTop, b->TopLeft, b->TopRight, b->BotLeft, b->BotRight};
         for (int k = 0; k < 8; k++) h->h_nb[k].assign(nb[k], nb[k] + nbm);
     }
-    if (!h->riv_n.empty()) {
-        HIPCHK(hipStreamSynchronize(h->stream));
-        s = setup_rivers(h);  // the discharge cells of the new mesh
-        if (s != BGF_OK) return s;
-    }
     if (!h->segs.empty()) {
         HIPCHK(hipStreamSynchronize(h->stream));
         s = setup_segments(h);  // the boundary blocks of the new mesh
@@ -1639,6 +1644,11 @@ bgf_status bgf_remesh(bgf_handle h, const bgf_param* p, const bgf_blocks* b, con
         s = setup_fix(h);
     }
     if (s != BGF_OK) return s;
+    if (!h->riv_n.empty()) {
+        HIPCHK(hipStreamSynchronize(h->stream));
+        s = setup_rivers(h);  // the discharge cells of the new mesh
+        if (s != BGF_OK) return s;
+    }
     // the bed's halo on the new mesh (src/InitialConditions.cu:135-147)
     bgf::launch_amr_fill(prec, kp, h->d_zb, h->stream);
     // the statistics restart on the new mesh
