@@ -57,7 +57,10 @@
 // rewritten: it sees the prolonged value if that neighbour comes earlier in
 // the active list.  Only a halo cell of the coarser block beside a still
 // coarser one is ever rewritten, so with three levels the chain ends there and
-// a block evaluates that cell again (end_halo).  Every other stage only reads
+// a block evaluates that cell again (the EH_* cells of k_amr_stage).  The bed
+// of such a halo cell may be written by the coarser block's workgroup in the
+// same launch, but only with the bed of the cell that the evaluation takes
+// instead, so what was read of it is not used.  Every other stage only reads
 // cells that the same launch does not write, so blocks run in parallel.
 
 #include <hip/hip_runtime.h>
@@ -356,16 +359,9 @@ __device__ __forceinline__ void amr_halo_side(const KParams& P, T* h, T* u, T* v
     v[w] = vv;
 }
 template <class T>
-__device__ __forceinline__ void amr_halo(const KParams& P, T* h, T* u, T* v, const T* zb, const DevLoop* L, int corr,
-                                         int t, int vb) {
-    const int ib = quad_block(P, t, vb);
-    if (ib < 0) return;
-    if (L && stage_off(loop_of(P, const_cast<DevLoop*>(L), ib), corr)) return;
-    amr_halo_side<T>(P, h, u, v, zb, (t >> 4) & 3, t & 15, ib);
-}
-template <class T>
-__global__ __launch_bounds__(256) void k_amr_halo(KParams P, T* h, T* u, T* v, const T* zb, DevLoop* L, int corr) {
-    amr_halo<T>(P, h, u, v, zb, L, corr, threadIdx.x, blockIdx.x);
+__global__ __launch_bounds__(256) void k_amr_halo(KParams P, T* h, T* u, T* v, const T* zb) {
+    const int t = threadIdx.x, ib = quad_block(P, t, blockIdx.x);
+    if (ib >= 0) amr_halo_side<T>(P, h, u, v, zb, (t >> 4) & 3, t & 15, ib);
 }
 
 // Halo of one static field (the bed at set-up, src/InitialConditions.cu:135-147).
@@ -650,7 +646,7 @@ template <class T> struct StageLds {
         };
         T pt[4][4][NPT];         // h, u, v and the bed of the points
     };
-    Q4<T> fe[2 * BW];  // the seventeenth X faces, then Y faces (before that: four of each side's, see EndHalo)
+    Q4<T> fe[2 * BW];  // the seventeenth X faces, then Y faces (before that: the EH_* cells of side s from 4 s)
     T sh[4][BW], sz[4][BW];
     T red[4];
 };
@@ -1269,7 +1265,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 7) void k_amr_stage(KPara
         }
         wave_sync();
         // the linear reconstructions: lanes 0-15 of the halo cells, lanes 48-50 of C's halo at the end of
-        // the half (EndHalo)
+        // the half (the EH_* cells, to S.fe[4 s + EH_*])
         int p = s, jr = j;
         const int m = j / 2, lend = (int)(signed char)(ends >> RC_END);
         const bool lo = s == SL || s == SB;  // the side faces the neighbour's high end
@@ -1681,10 +1677,10 @@ void launch_amr_halo(int precision, const KParams& P, void* h, void* u, void* v,
     const dim3 quad((P.nblk + 3) / 4), tpb(256);
     if (precision == 0)
         hipLaunchKernelGGL(k_amr_halo<double>, quad, tpb, 0, st, P, (double*)h, (double*)u, (double*)v,
-                           (const double*)zb, (DevLoop*)nullptr, 0);
+                           (const double*)zb);
     else
         hipLaunchKernelGGL(k_amr_halo<float>, quad, tpb, 0, st, P, (float*)h, (float*)u, (float*)v,
-                           (const float*)zb, (DevLoop*)nullptr, 0);
+                           (const float*)zb);
 }
 
 }  // namespace bgf

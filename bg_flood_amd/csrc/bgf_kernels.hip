@@ -257,8 +257,7 @@ template <class T, bool ROW> struct Tile {
 
 // Strip slot k in [0, 128): waves 0 and 1 fetch the two-deep x strips (left,
 // right) and y strips (bottom, top) of the 20x20 tile.  strip_cell gives the
-// tile position, strip_src the source cell; a missing neighbour (the block
-// itself) maps to the block's own edge cell.
+// tile position.
 __device__ __forceinline__ int strip_off(int k) {
     const int s = (k >> 4) & 3;  // 0: -1, 1: -2, 2: 16, 3: 17
     return s < 2 ? -1 - s : 14 + s;
@@ -266,33 +265,6 @@ __device__ __forceinline__ int strip_off(int k) {
 __device__ __forceinline__ int strip_cell(int k) {
     const int j = k & 15, o = strip_off(k);
     return k < 64 ? tix(o, j) : tix(j, o);
-}
-struct StripCell {
-    int x, y, nb;
-};
-__device__ __forceinline__ StripCell strip_cell_src(int k, int ib, int nL, int nR, int nB, int nT) {
-    const int j = k & 15, o = strip_off(k);
-    const bool lo = o < 0;
-    StripCell c;
-    if (k < 64) {
-        c.nb = lo ? nL : nR;
-        c.x = c.nb == ib ? (lo ? 0 : BW - 1) : (lo ? BW + o : o - BW);
-        c.y = j;
-    } else {
-        c.nb = lo ? nB : nT;
-        c.x = j;
-        c.y = c.nb == ib ? (lo ? 0 : BW - 1) : (lo ? BW + o : o - BW);
-    }
-    return c;
-}
-__device__ __forceinline__ int strip_src(int k, int ib, int nL, int nR, int nB, int nT) {
-    const StripCell c = strip_cell_src(k, ib, nL, nR, nB, nT);
-    return memloc(c.x, c.y, c.nb);
-}
-// the same source cell in the interior-only layout of the tendency arrays
-__device__ __forceinline__ int strip_src_i(int k, int ib, int nL, int nR, int nB, int nT) {
-    const StripCell c = strip_cell_src(k, ib, nL, nR, nB, nT);
-    return c.nb * BSI + c.y * BW + c.x;
 }
 
 // The strip sources in a form that costs a few vector instructions per block:
