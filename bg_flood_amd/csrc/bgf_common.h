@@ -323,8 +323,7 @@ __device__ __forceinline__ float seg_level(const KParams& P, const BSeg& S, doub
         const double x2x1 = x2 - x1, y2y1 = y2 - y1, x2x = x2 - xi, y2y = y2 - yi, yy1 = yi - y1, xx1 = xi - x1;
         z = (float)(1.0 / (x2x1 * y2y1) * (q11 * x2x * y2y + q21 * xx1 * y2y + q12 * x2x * yy1 + q22 * xx1 * yy1));
     } else if (S.on) {
-        int k = 1;
-        while (k < S.n - 1 && S.t[k] - t < 0.0) k++;  // the reference does not stop at the end
+        const int k = series_entry<true>(S.t, 1, S.n, t);  // the reference does not stop at the end
         z = (float)(S.z[k - 1] + (t - S.t[k - 1]) / (S.t[k] - S.t[k - 1]) * (S.z[k] - S.z[k - 1]));
     } else {
         z = (float)S.zs0;

@@ -261,3 +261,30 @@ def test_segments_follow_the_remesh():
             lg.totaltime += lg.dt
             lo.totaltime += lo.dt
         compare(d, o)
+
+
+@pytest.mark.parametrize("mesh", ["one level", "three levels"])
+@pytest.mark.parametrize("n", [2, 3, 4, 2000])
+def test_long_level_series(n, mesh):
+    """Level series of few and many entries on two sides, from times before, on and between the entries and
+    past the last."""
+    sc = scenarios.gaussian_hump(n=48, dx=4.0, depth=1.0, amp=0.1, precision="fp64") if mesh == "one level" else \
+        scenarios.amr_basin(nbx=3, nby=3, precision="fp64", island=True, amp=0.1)
+    rng = np.random.default_rng(n)
+    t = np.cumsum(rng.uniform(0.5, 2.0, n))
+    d, o = domain_for(sc, precision="fp64"), oracle_for(sc, precision="fp64")
+    for x in (d, o):
+        x.set_boundary(0, 2, t, 0.3 * np.sin(t))
+        x.set_boundary(3, 3, t, 0.2 * np.cos(t))
+    lg = bgf.Loop(nextoutputtime=1e9, dt=0, dtmax=0, totaltime=0)
+    lo = po.OrcLoop(nextoutputtime=1e9, dt=0, dtmax=0, totaltime=0)
+    d.init_dt(lg)
+    o.init_loop(lo)
+    for at in sorted({t[0] - 0.1, t[0], t[1] - 0.01, t[n // 2], t[n // 2] - 0.02, t[-2], t[-1], t[-1] + 3.0}):
+        print("case level series of %d, %s, at %g" % (n, mesh, at), flush=True)
+        lg.totaltime = lo.totaltime = float(at)
+        d.run(lg, 3)
+        o.run(lo, 3)
+        assert (lg.dt, lg.totaltime) == (lo.dt, lo.totaltime)
+        compare(d, o)
+    d.close()
