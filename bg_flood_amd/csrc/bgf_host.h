@@ -136,8 +136,8 @@ inline bgf_status read_back(ReadBack& R, int prec, const std::vector<int>& activ
     return BGF_OK;
 }
 
-// Room for a multi-level mesh of cap block slots in one allocation (each costs
-// a growing mesh some 0.1 ms): its gather recipes and its list of fix-up blocks.
+// Room for the gather recipes and the list of fix-up blocks of a multi-level
+// batch of cap block slots, in one allocation.
 inline bool mesh_tables(size_t cap, int4** rcell, int2** rmeta, int** fix) {
     const size_t n = bgf::RECIPES * cap;
     if (hipMalloc((void**)rcell, n * (sizeof(int4) + sizeof(int2)) + cap * sizeof(int)) != hipSuccess) return false;

@@ -179,9 +179,10 @@ __device__ __forceinline__ bool kurg_face(const Cst<T>& C, const Q4<T>& qi, cons
 // times the half-cell increment of zs, since hl and hr lie as far below and
 // above h.  So a face keeps only F.b = up qp - w dF + k dq for cell i and
 // F.c = F.b + g/2 (hp^2 - hm^2) for cell n, and the cell adds one term
-// (cell_source): 50 instructions a face instead of 70, and no difference of
-// squares of whole depths is rounded; where the water is at rest both parts
-// are exactly zero.
+// (cell_source), and no difference of squares of whole depths is rounded; where
+// the water is at rest both parts are exactly zero.  With this and the exchange
+// along x between lanes the FAST predictor issues 267 vector instructions a
+// wave and block, 276 before, and 22 LDS instructions, 29 before.
 template <bool WANT_DT>
 __device__ __forceinline__ bool kurg_face_fast(const Cst<float>& C, const Q4<float>& qi, const Q4<float>& qn,
                                                const Q4<float>& si, const Q4<float>& sn, Q4<float>& F, float& dt) {
@@ -434,8 +435,9 @@ template <class T> __device__ __forceinline__ Q4<T> swap_uv(const Q4<T>& q) { re
 // registers.  FAST kernels exchange along x between lanes: with every exchange
 // through LDS the FAST predictor's 30 accesses of 16 bytes a lane, with their
 // bank conflicts, took all of its 655 us at 8192 x 8192 cells, 21 accesses and
-// 28 more vector instructions 622.  The exact kernels have the vector ALU busy
-// for nine tenths of their time and gain nothing from that trade.
+// 28 more vector instructions 622.  The exact FP32 kernels need 41 of their 48
+// us (1520 x 2032 cells) to issue vector instructions at the top clock of 2.4
+// GHz and gain nothing from that trade.
 template <class T> struct CellFaces {
     Q4<T> l, r, b, t;
 };
@@ -1408,11 +1410,15 @@ void launch_step(int precision, const KParams& P, const void* buffers, DevLoop* 
 // that a grid not asked for by wg_per_cu takes at the most.  The FP32
 // predictors fit seven by their registers, but the seventh starts late (its
 // first block waits for another workgroup's end, and the launch for it) and
-// more of them only lengthen the tail; six of the exact one and five of the
-// FAST one are as fast or faster at every size.  Ten steps, exact FP32: 720 x
-// 640 cells 392 -> 317 us, 1024 x 1024 557 -> 511, 2048 x 2048 1471 -> 1419,
-// 4096 x 4096 4763 -> 4786 (run to run: 1 %); FAST: 344 -> 262, 445 -> 378,
-// 1065 -> 1029, 3681 -> 3654.
+// more of them only lengthen the tail.  A step on rain, exact FP32, with seven,
+// six, five and four, us: 720 x 640 cells 41.4, 33.8, 34.2, 34.6; 1024 x 1024
+// 56.0, 50.4, 49.4, 49.3; 1520 x 1520 87.2, 80.4, 81.6, 83.9; 2048 x 2048 134,
+// 128.5, 131, 137; 4096 x 4096 478.6, 476.6, 487.4, 499; 8192 x 8192 1896,
+// 1899, 1943, 2002: six, within 0.2 % of the best from 1520 x 1520 on and 2 %
+// below.  FAST, seven, six, five, four: 33.0, 26.2, 25.6, 25.6; 45.2, 38.7,
+// 37.9, 37.4; 68.6, 63.2, 62.0, 61.7; 105.2, 102.2, 101.2, 100.9; 375, 374,
+// 372, 375; 1475, 1473, 1472, 1500: five, within 1.3 %.  Smaller grids have
+// fewer blocks than that.
 template <class K> int grid_for(K kernel, int nblk, int wg_per_cu, int most = 8) {
     int dev = 0, ncu = 0, occ = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
