@@ -629,7 +629,10 @@ bgf_status bgf_batch_get_state(bgf_batch b, int m, void* zs, void* hh, void* u, 
     if (s != BGF_OK) return s;
     const Member& M = b->members[m];
     void* const dst[4] = {zs, hh, u, v};
-    return read_back(*b->back, b->prec, M.active, M.off, b->d_active + active_offset(b, m), b->d_zb, b->d_h[0],
+    int most = 0;
+    for (const Member& x : b->members)
+        if (x.used) most = std::max(most, x.nblk);
+    return read_back(*b->back, b->prec, M.active, most, M.off, b->d_active + active_offset(b, m), b->d_zb, b->d_h[0],
                      b->d_u[0], b->d_v[0], dst, b->stream);
 }
 

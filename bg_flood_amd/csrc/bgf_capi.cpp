@@ -826,7 +826,7 @@ bgf_status bgf_get_state(bgf_handle h, void* zs, void* hh, void* u, void* v) {
     if (!h) return fail(BGF_ERR_INVALID_ARG, "null handle");
     if (h->pending_steps) return fail(BGF_ERR_STATE, "bgf_run_async pending: call bgf_sync first");
     void* const dst[4] = {zs, hh, u, v};
-    return read_back(*h->back, h->prec, h->active, 0, h->d_active, h->d_zb, h->d_h[0], h->d_u[0], h->d_v[0], dst,
+    return read_back(*h->back, h->prec, h->active, h->nblk, 0, h->d_active, h->d_zb, h->d_h[0], h->d_u[0], h->d_v[0], dst,
                      h->stream);
 }
 

@@ -59,7 +59,7 @@ inline bool device_accessible(const void* p) {
 // is written while the one before is spread, so the pinned memory stays small.
 // Copying whole arrays, with their halos and the bed, through pageable memory
 // took 3.48 ms for the eight members (25.6 MB of arrays) of an ensemble.  The
-// pieces are no larger than what was read through them needs, and one that
+// pieces are no larger than the largest read through them needs, and one that
 // suffices has no second: a domain of one block takes 8 KB, not 2 MB.
 struct ReadBack {
     static constexpr size_t PIECE = 1024 * 1024;  // bytes of one of the two pieces at the most, a power of two
@@ -77,9 +77,11 @@ struct ReadBack {
 
 // Fields dst = (zs, h, u, v; null: not wanted) of the blocks active (d_active:
 // the same list on the device), block ib going to place ib - off of dst.
-inline bgf_status read_back(ReadBack& R, int prec, const std::vector<int>& active, int off, const int* d_active,
-                            const void* zb, const void* h, const void* u, const void* v, void* const dst[4],
-                            hipStream_t st) {
+// most: the blocks of the largest such read to expect (the members of a batch
+// are read in turn).
+inline bgf_status read_back(ReadBack& R, int prec, const std::vector<int>& active, int most, int off,
+                            const int* d_active, const void* zb, const void* h, const void* u, const void* v,
+                            void* const dst[4], hipStream_t st) {
     const size_t es = prec == 0 ? sizeof(double) : sizeof(float);
     int fields = 0, nf = 0;
     for (int k = 0; k < 4; k++)
@@ -102,10 +104,10 @@ inline bgf_status read_back(ReadBack& R, int prec, const std::vector<int>& activ
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? hipEventRecord(R.ev[k & 1], st) : e;
     };
-    for (int k = 0; k < std::min(2, pieces); k++) {
+    for (int k = 0; k < (most > per ? 2 : 1); k++) {
         if (!R.ev[k]) HIPCHK(hipEventCreateWithFlags(&R.ev[k], hipEventDisableTiming));
         size_t need = 4096;  // doubled: at most eight times for a handle
-        while (need < (size_t)std::min(per, n) * nf * BSI * es) need *= 2;
+        while (need < (size_t)std::min(per, most) * nf * BSI * es) need *= 2;
         if (R.size[k] >= need) continue;
         if (R.mem[k]) (void)hipHostFree(R.mem[k]);
         R.mem[k] = nullptr;
